@@ -42,15 +42,19 @@ __host__ __device__ inline double det_log(double x) { return detm_log(x); }
 // reference calls it, src/mctsnc.py:1882): the 11 discarded bits are cleared, the remaining 53 significant bits are
 // exact in float64 (two conversions and one fused multiply-add, all exact), the narrowing rounds once to nearest even
 // as the reference's float32 cast does, and the scaling by 2^-64 is exact.  Five instructions per draw.
-__device__ __forceinline__ float uniform_from_bits(uint32_t lo, uint32_t hi) {
+__device__ __forceinline__ float uniform_scaled_from_bits(uint32_t lo, uint32_t hi) {   // times 2^64
     // (hi is usually the upper half of a 64-bit sum; without this the compiler converts that 64-bit value shifted down
     // instead, a longer sequence with an addition of zero that it does not fold)
     asm("" : "+v"(hi));
     const double d = __builtin_fma((double)hi, 4294967296.0, (double)(lo & 0xfffff800u));
-    return (float)d * 0x1p-64f;
+    return (float)d;
 }
+__device__ __forceinline__ float uniform_from_bits(uint32_t lo, uint32_t hi) { return uniform_scaled_from_bits(lo, hi) * 0x1p-64f; }
 
 // xoroshiro128+ step on 32-bit halves (the 64-bit shifts of the generic form are slow vector instructions)
+// (one instruction; the compiler makes two of a ^ b ^ c)
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96); }
+
 struct Rng32 { uint32_t s0l, s0h, s1l, s1h; };
 
 __device__ __forceinline__ void rng_next32(Rng32 &r, uint32_t &out_lo, uint32_t &out_hi) {
@@ -60,7 +64,7 @@ __device__ __forceinline__ void rng_next32(Rng32 &r, uint32_t &out_lo, uint32_t 
     // rotl(s0, 55) = rotr(s0, 9); t << 14; rotl(t, 36) = halves swapped, then rotl 4
     const uint32_t r0l = __builtin_amdgcn_alignbit(r.s0h, r.s0l, 9), r0h = __builtin_amdgcn_alignbit(r.s0l, r.s0h, 9);
     const uint32_t shl = tl << 14, shh = __builtin_amdgcn_alignbit(th, tl, 18);
-    r.s0l = r0l ^ tl ^ shl; r.s0h = r0h ^ th ^ shh;
+    r.s0l = xor3(r0l, tl, shl); r.s0h = xor3(r0h, th, shh);
     r.s1l = __builtin_amdgcn_alignbit(th, tl, 28); r.s1h = __builtin_amdgcn_alignbit(tl, th, 28);
 }
 
