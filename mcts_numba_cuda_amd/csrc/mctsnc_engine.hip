@@ -217,10 +217,11 @@ struct Budget {
 
 // Root of a Gomoku search: bitboards with bit = row * n + column; any arrangement of stones is accepted, as in the
 // reference (its outcome test only looks through the last stone placed).
-// Words per colour of a Gomoku position: 8 for boards of up to 16 x 16; beyond, 12 while the board has at most 384 cells
-// (the stone sets then still fit the 128-byte node record) and 16 up to the 512 cells the reference allows.
+// Words per colour of a Gomoku position: 8 for boards whose playouts fit the narrow format (all up to 16 x 15); beyond, 12
+// while the board has at most 384 cells (the stone sets then still fit the 128-byte node record) and 16 up to the 512 cells
+// the reference allows.
 int gomoku_words(const mctsnc_config &c) {
-    if (c.board_m <= 16 && c.board_n <= 16) return 8;
+    if (gomoku::narrow_playouts(c.board_m, c.board_n)) return 8;
     return c.board_m * c.board_n <= 384 ? 12 : 16;
 }
 
@@ -236,14 +237,17 @@ int gomoku_encode_root(const mctsnc_config &c, const int8_t *board, uint32_t *bb
     return MCTSNC_OK;
 }
 
-// Playouts a Gomoku workgroup runs at a time (a power of two, as n_playouts is: the kernel finds a playout's line words
-// with a shift): as many as there are playouts, up to 256, and no more than fit the LDS of a CU beside the kernel's own
-// 8 KB, 12 KB in the wide formats (16 x 16 boards: 128, 19 x 19 and beyond: 64; more playouts then run in rounds).
-int gomoku_block(const mctsnc_config &c) {
-    int slots = c.n_playouts < 64 ? 64 : (c.n_playouts > gomoku::kMaxThreads ? gomoku::kMaxThreads : c.n_playouts);
+// Playouts a Gomoku workgroup runs at a time, a power of two from 64 to its threads: one-child variants as many as there
+// are, all-children variants (whose workgroups play several children) as many as there are threads, and no more than fit
+// the LDS of a CU beside the kernel's own 6 KB, 14 KB in the wide formats (15 x 15: 256, two workgroups per CU; 19 x 19: 128).
+int gomoku_slots(const mctsnc_config &c) {
+    const bool acp = c.variant >= MCTSNC_ACP_THRIFTY;
+    const int wanted = acp ? c.n_playouts * c.max_actions : c.n_playouts;
+    int slots = 64;
+    while (slots < wanted && slots < gomoku::kMaxSlots) slots *= 2;
     const bool wide = gomoku_words(c) > 8;
-    const size_t lds_of_a_cu = 160 * 1024, kernels_own = (wide ? 12 : 8) * 1024;
-    while (slots > 64 && gomoku::playout_lds_bytes(c.board_m * c.board_n, 3 * (c.board_m + c.board_n) - 2, slots, wide) + kernels_own > lds_of_a_cu) slots /= 2;
+    const size_t lds_of_a_cu = 160 * 1024, kernels_own = (wide ? 14 : 6) * 1024;
+    while (slots > 64 && gomoku::playout_lds_bytes(c.board_m, c.board_n, slots, 1, wide) + kernels_own > lds_of_a_cu) slots /= 2;
     return slots;
 }
 
@@ -692,15 +696,21 @@ int run_many_gomoku(mctsnc_engine **engines, int n, const int8_t *boards, const 
 
     gomoku::SearchArgs args;
     args.refs = d_refs; args.n_refs = n_refs; args.m = c.board_m; args.n = c.board_n; args.P = c.n_playouts; args.G = e0->G; args.slots = e0->slots;
-    if (e0->slots < 64 || (e0->slots & (e0->slots - 1))) return fail(MCTSNC_E_STATE, "playouts per round (%d) must be a power of two >= 64", e0->slots);
+    if (e0->slots < 64 || e0->slots > e0->block || (e0->slots & (e0->slots - 1))) return fail(MCTSNC_E_STATE, "playouts per round (%d) must be a power of two from 64 to the workgroup's threads", e0->slots);
     args.S = (int32_t)c.max_tree_size; args.thrifty = e0->thrifty ? 1 : 0; args.ucb_c = c.ucb_c; args.abort_flag = e0->d_abort;
     args.stage_timing = e0->stage_timing ? 1 : 0;
     const int *opt = e0->options;
     args.agent_fences = opt[MCTSNC_OPT_AGENT_FENCES] ? 1 : 0;
     args.spin_limit = opt[MCTSNC_OPT_SPIN_LIMIT] > 0 ? (uint32_t)opt[MCTSNC_OPT_SPIN_LIMIT] : gomoku::kSpinLimit;
     args.prep_levels = opt[MCTSNC_OPT_PREP_LEVELS] >= 0 ? std::min(opt[MCTSNC_OPT_PREP_LEVELS], gomoku::kPrepLevels) : gomoku::kPrepLevels;
-    const dim3 block(e0->block);
-    const size_t lds = gomoku::playout_lds_bytes(cells, 3 * (c.board_m + c.board_n) - 2, e0->slots, wide);
+    // One-child trees that have a CU each: workgroups of 512 threads, whose two teams look for the ends of 64 playouts each,
+    // if there are that many and the second board of times fits.
+    int threads = e0->block, cus_now = 0;
+    HIP_TRY(hipDeviceGetAttribute(&cus_now, hipDeviceAttributeMultiprocessorCount, c.device));
+    size_t lds = gomoku::playout_lds_bytes(c.board_m, c.board_n, e0->slots, 1, wide);
+    const size_t lds_two = gomoku::playout_lds_bytes(c.board_m, c.board_n, e0->slots, 2, wide);
+    if (!e0->acp && n_refs <= cus_now && e0->slots > 64 && lds_two + (wide ? 14 : 6) * 1024 <= 160 * 1024) { threads = gomoku::kMaxThreads; lds = lds_two; }
+    const dim3 block(threads);
     // the kernel of this engine's variant and board format
     auto *const kernel = gomoku_kernel(e0->acp, W);
     // the limit is a setting of the kernel function, not of this engine: an engine of another shape may have changed it
@@ -866,10 +876,10 @@ int mctsnc_create(const mctsnc_config *cfg, mctsnc_engine **out) {
         e->block = c.n_playouts < 64 ? 64 : c.n_playouts;
     } else {
         e->G = e->acp ? (c.max_actions < 32 ? c.max_actions : 32) : 1;  // workgroups per tree; each takes every G-th child
-        e->slots = gomoku_block(c);
-        // one workgroup per tree (one-child variants): all 256 threads, whatever the playout count -- creating up to 225
-        // children and re-evaluating the path are shared by all of them
-        e->block = e->acp ? e->slots : gomoku::kMaxThreads;
+        e->slots = gomoku_slots(c);
+        // 256 threads, whatever the playout count: creating the children, re-evaluating the path and finding the ends of the
+        // games are shared by all of them
+        e->block = gomoku::kMaxSlots;
     }
     // tpb table of src/mctsnc.py:360-365 with cuda_tpb_default = 512: fixes which expand generators OCP uses
     const int tpb_board = next_pow2(c.board_m * c.board_n), tpb_extra = next_pow2(c.extra_info_memory), tpb_actions = next_pow2(c.max_actions);
@@ -949,7 +959,7 @@ static int init_device_impl(mctsnc_engine *e) {
         e->hg_refs = refs;
         // the playout state of a workgroup can need more LDS than the default limit allows
         const bool wide = gomoku_words(c) > 8;
-        const size_t lds = gomoku::playout_lds_bytes(c.board_m * c.board_n, 3 * (c.board_m + c.board_n) - 2, e->slots, wide);
+        const size_t lds = gomoku::playout_lds_bytes(c.board_m, c.board_n, e->slots, 1, wide);
         auto *const kernel = gomoku_kernel(e->acp, gomoku_words(c));
         HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         if (e->acp) {
