@@ -85,7 +85,6 @@ struct mctsnc_engine {
     mctsnc_config cfg;
     bool inited = false;
     bool acp = false, thrifty = false;
-    int slots = 0;   // Gomoku: playouts a workgroup runs at a time (its LDS is sized for them); <= block
     int G = 1, block = 64, tpb_e1 = 64;
     c4::Node *d_nodes = nullptr;
     c4::TreeHdr *d_hdrs = nullptr;
@@ -237,18 +236,26 @@ int gomoku_encode_root(const mctsnc_config &c, const int8_t *board, uint32_t *bb
     return MCTSNC_OK;
 }
 
-// Playouts a Gomoku workgroup runs at a time, a power of two from 64 to its threads: one-child variants as many as there
-// are, all-children variants (whose workgroups play several children) as many as there are threads, and no more than fit
-// the LDS of a CU beside the kernel's own 6 KB, 14 KB in the wide formats (15 x 15: 256, two workgroups per CU; 19 x 19: 128).
-int gomoku_slots(const mctsnc_config &c) {
-    const bool acp = c.variant >= MCTSNC_ACP_THRIFTY;
-    const int wanted = acp ? c.n_playouts * c.max_actions : c.n_playouts;
-    int slots = 64;
-    while (slots < wanted && slots < gomoku::kMaxSlots) slots *= 2;
-    const bool wide = gomoku_words(c) > 8;
-    const size_t lds_of_a_cu = 160 * 1024, kernels_own = (wide ? 14 : 6) * 1024;
-    while (slots > 64 && gomoku::playout_lds_bytes(c.board_m, c.board_n, slots, 1, wide) + kernels_own > lds_of_a_cu) slots /= 2;
-    return slots;
+// How a workgroup of a Gomoku search is laid out: its threads, the playouts it runs at a time (a power of two from 64 up) and
+// the boards of times it looks for their ends on (one per 256 threads at most), with the dynamic LDS these take.
+// All-children variants: 256 threads and as many playouts (a workgroup plays several children).  One-child variants: two
+// wavefronts draw 64 playouts, so 512 threads and up to 256 playouts while every tree has a CU to itself (the others create
+// the children and prepare the backup meanwhile), 256 threads and up to 128 playouts where two trees share one.  Fewer
+// boards and playouts where they do not fit the LDS of a CU beside the kernel's own 6 KB (8 and 10 KB in the wide formats).
+struct GomokuLayout { int threads, slots, teams; size_t lds; };
+GomokuLayout gomoku_layout(const mctsnc_config &c, bool acp, bool tree_per_cu) {
+    const int words = gomoku_words(c);
+    const bool wide = words > 8;
+    const int wanted = acp ? c.n_playouts * c.max_actions : c.n_playouts, most = acp || tree_per_cu ? gomoku::kMaxSlots : gomoku::kMaxSlots / 2;
+    GomokuLayout g{acp || !tree_per_cu ? gomoku::kMaxThreads / 2 : gomoku::kMaxThreads, 64, 0, 0};
+    while (g.slots < wanted && g.slots < most) g.slots *= 2;
+    g.teams = g.threads / 256;
+    for (;;) {
+        g.lds = gomoku::playout_lds_bytes(c.board_m, c.board_n, g.slots, g.teams, wide) + (acp ? 0 : (size_t)(g.slots / 64) * gomoku::kRingBytes);
+        if (g.lds + (size_t)(words > 12 ? 10 : wide ? 8 : 6) * 1024 <= 160 * 1024 || (g.slots == 64 && g.teams == 1)) return g;
+        if (g.teams > 1) g.teams = 1;
+        else g.slots /= 2;
+    }
 }
 
 // The search kernel of a variant and board format.
@@ -695,22 +702,19 @@ int run_many_gomoku(mctsnc_engine **engines, int n, const int8_t *boards, const 
     HIP_TRY(hipStreamSynchronize(stream));
 
     gomoku::SearchArgs args;
-    args.refs = d_refs; args.n_refs = n_refs; args.m = c.board_m; args.n = c.board_n; args.P = c.n_playouts; args.G = e0->G; args.slots = e0->slots;
-    if (e0->slots < 64 || e0->slots > e0->block || (e0->slots & (e0->slots - 1))) return fail(MCTSNC_E_STATE, "playouts per round (%d) must be a power of two from 64 to the workgroup's threads", e0->slots);
+    int cus_now = 0;
+    HIP_TRY(hipDeviceGetAttribute(&cus_now, hipDeviceAttributeMultiprocessorCount, c.device));
+    const GomokuLayout layout = gomoku_layout(c, e0->acp, n_refs <= cus_now);
+    args.refs = d_refs; args.n_refs = n_refs; args.m = c.board_m; args.n = c.board_n; args.P = c.n_playouts; args.G = e0->G;
+    args.slots = layout.slots; args.teams = layout.teams;
     args.S = (int32_t)c.max_tree_size; args.thrifty = e0->thrifty ? 1 : 0; args.ucb_c = c.ucb_c; args.abort_flag = e0->d_abort;
     args.stage_timing = e0->stage_timing ? 1 : 0;
     const int *opt = e0->options;
     args.agent_fences = opt[MCTSNC_OPT_AGENT_FENCES] ? 1 : 0;
     args.spin_limit = opt[MCTSNC_OPT_SPIN_LIMIT] > 0 ? (uint32_t)opt[MCTSNC_OPT_SPIN_LIMIT] : gomoku::kSpinLimit;
     args.prep_levels = opt[MCTSNC_OPT_PREP_LEVELS] >= 0 ? std::min(opt[MCTSNC_OPT_PREP_LEVELS], gomoku::kPrepLevels) : gomoku::kPrepLevels;
-    // One-child trees that have a CU each: workgroups of 512 threads, whose two teams look for the ends of 64 playouts each,
-    // if there are that many and the second board of times fits.
-    int threads = e0->block, cus_now = 0;
-    HIP_TRY(hipDeviceGetAttribute(&cus_now, hipDeviceAttributeMultiprocessorCount, c.device));
-    size_t lds = gomoku::playout_lds_bytes(c.board_m, c.board_n, e0->slots, 1, wide);
-    const size_t lds_two = gomoku::playout_lds_bytes(c.board_m, c.board_n, e0->slots, 2, wide);
-    if (!e0->acp && n_refs <= cus_now && e0->slots > 64 && lds_two + (wide ? 14 : 6) * 1024 <= 160 * 1024) { threads = gomoku::kMaxThreads; lds = lds_two; }
-    const dim3 block(threads);
+    const dim3 block(layout.threads);
+    const size_t lds = layout.lds;
     // the kernel of this engine's variant and board format
     auto *const kernel = gomoku_kernel(e0->acp, W);
     // the limit is a setting of the kernel function, not of this engine: an engine of another shape may have changed it
@@ -722,7 +726,7 @@ int run_many_gomoku(mctsnc_engine **engines, int n, const int8_t *boards, const 
     if (e0->acp) {
         int per_cu = 0, cus = 0;
         HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
-        HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, e0->block, lds));
+        HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, layout.threads, lds));
         const int64_t fit = (int64_t)per_cu * cus / e0->G;   // trees per launch
         if (fit < 1) return fail(MCTSNC_E_INVALID, "the device cannot hold the %d workgroups of a tree at once", e0->G);
         const int64_t n_groups = (n_refs + fit - 1) / fit;
@@ -876,10 +880,7 @@ int mctsnc_create(const mctsnc_config *cfg, mctsnc_engine **out) {
         e->block = c.n_playouts < 64 ? 64 : c.n_playouts;
     } else {
         e->G = e->acp ? (c.max_actions < 32 ? c.max_actions : 32) : 1;  // workgroups per tree; each takes every G-th child
-        e->slots = gomoku_slots(c);
-        // 256 threads, whatever the playout count: creating the children, re-evaluating the path and finding the ends of the
-        // games are shared by all of them
-        e->block = gomoku::kMaxSlots;
+        e->block = gomoku_layout(c, e->acp, false).threads;
     }
     // tpb table of src/mctsnc.py:360-365 with cuda_tpb_default = 512: fixes which expand generators OCP uses
     const int tpb_board = next_pow2(c.board_m * c.board_n), tpb_extra = next_pow2(c.extra_info_memory), tpb_actions = next_pow2(c.max_actions);
@@ -958,8 +959,7 @@ static int init_device_impl(mctsnc_engine *e) {
         HIP_TRY(hipMemcpy(e->g_refs, refs.data(), sizeof(gomoku::TreeRef) * T, hipMemcpyHostToDevice));
         e->hg_refs = refs;
         // the playout state of a workgroup can need more LDS than the default limit allows
-        const bool wide = gomoku_words(c) > 8;
-        const size_t lds = gomoku::playout_lds_bytes(c.board_m, c.board_n, e->slots, 1, wide);
+        const size_t lds = gomoku_layout(c, e->acp, false).lds;
         auto *const kernel = gomoku_kernel(e->acp, gomoku_words(c));
         HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         if (e->acp) {
