@@ -74,27 +74,102 @@ def reason(raw):
     return (int(raw) >> PACKED_REASON_SHIFT) & 0x3F
 
 
+# The arrays of a call: name -> (element type, shape).  A selection and its backup take a dozen microseconds on a GPU when
+# they are small, and a call used to spend twenty on looking its arrays over: one pass over them now, each attribute asked
+# once, and plain integers for ctypes.
+_TREES, _NODES, _EDGES, _WALKS, _PATHS = range(5)      # [trees], [trees, nodes], [.., edges], [trees, warps], [.., path_depth]
+_ARRAYS = {"edge_child": (np.int32, _EDGES), "edge_prior": (np.float32, _EDGES), "edge_w": (np.float32, _EDGES), "edge_n": (np.int32, _EDGES),
+           "edge_inflight": (np.int32, _EDGES), "node_inflight": (np.int32, _NODES), "node_expand_inflight": (np.int32, _NODES),
+           "node_expanded": (np.int32, _NODES), "node_count": (np.int32, _TREES), "out_selected": (np.int32, _WALKS),
+           "out_path": (np.int32, _PATHS), "out_len": (np.int32, _WALKS), "path_edge_values": (np.float32, _PATHS)}
+_SHAPE_TEXT = {_TREES: "[trees]", _NODES: "[trees, nodes]", _EDGES: "[trees, nodes, edges]", _WALKS: "[trees, warps]", _PATHS: "[trees, warps, path_depth]"}
+
+
+def _fields(*names):
+    """(fields in the order of a launcher's arguments, other arrays whose shape is checked if the dictionary has them)"""
+    checked = ("edge_prior", "edge_w", "edge_n", "edge_inflight", "node_expand_inflight", "node_expanded", "node_inflight", "node_count",
+               "out_selected", "out_len")
+    return tuple((n, *_ARRAYS[n]) for n in names), tuple((n, _ARRAYS[n][1]) for n in checked if n not in names)
+
+
+_SELECT = _fields("edge_child", "edge_prior", "edge_w", "edge_n", "edge_inflight", "node_expand_inflight", "node_expanded", "node_count",
+                  "out_selected", "out_path", "out_len")
+_NODE_SELECT = _fields("edge_child", "edge_prior", "edge_w", "edge_n", "node_inflight", "node_expand_inflight", "node_expanded", "node_count",
+                       "out_selected", "out_path", "out_len")
+_EDGE_BACKUP = _fields("edge_w", "edge_n", "edge_inflight", "node_expand_inflight", "node_count", "out_selected", "out_path", "out_len")
+_NODE_BACKUP = _fields("edge_child", "edge_w", "edge_n", "node_inflight", "node_expand_inflight", "node_count", "out_selected", "out_path", "out_len")
+_torch = None                 # the torch module, once a torch tensor has been seen
+_TORCH_TYPES = {}
+_raw_stream = None            # handle of a device's current stream, without a Stream object around it where torch offers that
+
+
+def _bind_torch():
+    global _torch, _raw_stream
+    if _torch is None:
+        import torch
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
+        _TORCH_TYPES.update({np.int32: torch.int32, np.float32: torch.float32})
+        _torch = torch
+    return _torch
+
+
 def _device_ptr(t, dtype, name):
     """Device address of a contiguous array of `dtype`: a hipmem.DeviceArray or a torch tensor on the GPU."""
     from .hipmem import DeviceArray
     if isinstance(t, DeviceArray):
         if t.dtype != np.dtype(dtype):
             raise ValueError(f"{name}: expected {np.dtype(dtype)}, got {t.dtype}")
-        return ctypes.c_void_p(t.data_ptr())
-    import torch
-    want = {np.int32: torch.int32, np.float32: torch.float32}[dtype]
+        return t.data_ptr()
+    torch = _bind_torch()
+    want = _TORCH_TYPES[dtype]
     if not isinstance(t, torch.Tensor) or not t.is_cuda or t.dtype != want or not t.is_contiguous():
         raise ValueError(f"{name}: expected a contiguous {want} tensor on the GPU")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+def _shape_error(name, kind):
+    if name in ("out_selected", "out_len"):
+        return ValueError("out_selected / out_len must have shape [trees, warps]")
+    return ValueError(f"{name} must have shape {_SHAPE_TEXT[kind]}")
+
+
+def _arguments(d, fields, values=None):
+    """(addresses of the arrays of `fields`, (trees, nodes, edges, warps, path_depth, stream)): everything a launcher takes
+    from the dictionary, checked.  `values`: path_edge_values, or None."""
+    trees, nodes, edges = d["edge_child"].shape
+    warps, path_depth = d["out_path"].shape[1], d["out_path"].shape[2]
+    shapes = ((trees,), (trees, nodes), (trees, nodes, edges), (trees, warps), (trees, warps, path_depth))
+    fields, others = fields
+    for name, kind in others:
+        if name in d and tuple(d[name].shape) != shapes[kind]:
+            raise _shape_error(name, kind)
+    out = []
+    tensor = _torch.Tensor if _torch is not None else None
+    for name, dtype, kind in fields:
+        t = d[name]
+        if t.__class__ is tensor:
+            if t.shape != shapes[kind] and name != "edge_child" and name != "out_path":
+                raise _shape_error(name, kind)
+            if t.dtype is not _TORCH_TYPES[dtype] or not t.is_cuda or not t.is_contiguous():
+                _device_ptr(t, dtype, name)      # (says what is wrong)
+            out.append(t.data_ptr())
+        else:
+            if tuple(t.shape) != shapes[kind] and name != "edge_child" and name != "out_path":
+                raise _shape_error(name, kind)
+            out.append(_device_ptr(t, dtype, name))
+            tensor = _torch.Tensor if _torch is not None else None
+    if values is not None:
+        if tuple(values.shape) != shapes[_PATHS]:
+            raise ValueError("path_edge_values must have shape [trees, warps, path_depth]")
+        values = _device_ptr(values, np.float32, "path_edge_values")
+    return out, values, trees, nodes, edges, warps, path_depth, _stream_handle(d)
 
 
 def _stream_handle(d):
     """torch's current stream when the arrays are torch tensors, the default stream otherwise."""
-    import sys
-    torch = sys.modules.get("torch")
-    if torch is not None and isinstance(d["edge_child"], torch.Tensor):
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return ctypes.c_void_p(0)
+    if _torch is not None and isinstance(d["edge_child"], _torch.Tensor):
+        return _raw_stream(_torch.cuda.current_device())
+    return 0
 
 
 def _check(code, what):
@@ -103,36 +178,12 @@ def _check(code, what):
         raise RuntimeError(f"PUCT {what} launch failed: {msg} ({code})")
 
 
-def _shape(d):
-    trees, nodes, edges = d["edge_child"].shape
-    warps, path_depth = d["out_path"].shape[1], d["out_path"].shape[2]
-    if tuple(d["out_selected"].shape) != (trees, warps) or tuple(d["out_len"].shape) != (trees, warps):
-        raise ValueError("out_selected / out_len must have shape [trees, warps]")
-    for k in ("edge_prior", "edge_w", "edge_n", "edge_inflight"):
-        if k in d and tuple(d[k].shape) != (trees, nodes, edges):
-            raise ValueError(f"{k} must have shape [trees, nodes, edges]")
-    for k in ("node_expand_inflight", "node_expanded", "node_inflight"):
-        if k in d and tuple(d[k].shape) != (trees, nodes):
-            raise ValueError(f"{k} must have shape [trees, nodes]")
-    if tuple(d["node_count"].shape) != (trees,):
-        raise ValueError("node_count must have shape [trees]")
-    return trees, nodes, edges, warps, path_depth
-
-
 def launch_select(d, cpuct=1.0, c_pw=1.0, alpha_pw=0.5, soft_winner=0):
     """Asynchronous PUCT selection on torch's current stream (src/puct/puct_gpu_v3_cpp.py:118-156)."""
-    trees, nodes, edges, warps, path_depth = _shape(d)
-    i32, f32 = np.int32, np.float32
-    code = _lib().puct_select_winner_recalc_launch(
-        cpuct, c_pw, alpha_pw, int(soft_winner),
-        _device_ptr(d["edge_child"], i32, "edge_child"), _device_ptr(d["edge_prior"], f32, "edge_prior"),
-        _device_ptr(d["edge_w"], f32, "edge_w"), _device_ptr(d["edge_n"], i32, "edge_n"),
-        _device_ptr(d["edge_inflight"], i32, "edge_inflight"),
-        _device_ptr(d["node_expand_inflight"], i32, "node_expand_inflight"),
-        _device_ptr(d["node_expanded"], i32, "node_expanded"), _device_ptr(d["node_count"], i32, "node_count"),
-        _device_ptr(d["out_selected"], i32, "out_selected"), _device_ptr(d["out_path"], i32, "out_path"),
-        _device_ptr(d["out_len"], i32, "out_len"), trees, nodes, edges, warps, path_depth, _stream_handle(d))
-    _check(code, "select")
+    arrays, _, *rest = _arguments(d, _SELECT)
+    code = (_LIB or _lib()).puct_select_winner_recalc_launch(cpuct, c_pw, alpha_pw, int(soft_winner), *arrays, *rest)
+    if code:
+        _check(code, "select")
 
 
 VARIANT_PRECLAIM, VARIANT_WINNER_RECALC = "preclaim", "winner_recalc"   # src/puct/test_puct_gpu_v2.py:317-352
@@ -142,57 +193,30 @@ def launch_node_select(d, cpuct=1.0, c_pw=1.0, alpha_pw=0.5, variant=VARIANT_PRE
     """Asynchronous PUCT selection with node-level virtual loss (d["node_inflight"], int32 [trees, nodes]): the two
     kernels of src/puct/puct_gpu_v2.py:573-840, chosen by `variant` as in the reference's launch helper
     (src/puct/test_puct_gpu_v2.py:317-352).  Selection words have the v2 layout (no reason field, no BUSY kind)."""
-    trees, nodes, edges, warps, path_depth = _shape(d)
-    i32, f32 = np.int32, np.float32
     if variant == VARIANT_PRECLAIM:
         fn = _lib().puct_node_select_preclaim_launch
     elif variant == VARIANT_WINNER_RECALC:
         fn = _lib().puct_node_select_winner_recalc_launch
     else:
         raise ValueError(f"unknown select variant: {variant}")
-    code = fn(cpuct, c_pw, alpha_pw,
-              _device_ptr(d["edge_child"], i32, "edge_child"), _device_ptr(d["edge_prior"], f32, "edge_prior"),
-              _device_ptr(d["edge_w"], f32, "edge_w"), _device_ptr(d["edge_n"], i32, "edge_n"),
-              _device_ptr(d["node_inflight"], i32, "node_inflight"),
-              _device_ptr(d["node_expand_inflight"], i32, "node_expand_inflight"),
-              _device_ptr(d["node_expanded"], i32, "node_expanded"), _device_ptr(d["node_count"], i32, "node_count"),
-              _device_ptr(d["out_selected"], i32, "out_selected"), _device_ptr(d["out_path"], i32, "out_path"),
-              _device_ptr(d["out_len"], i32, "out_len"), trees, nodes, edges, warps, path_depth, _stream_handle(d))
-    _check(code, "node select")
+    arrays, _, *rest = _arguments(d, _NODE_SELECT)
+    code = fn(cpuct, c_pw, alpha_pw, *arrays, *rest)
+    if code:
+        _check(code, "node select")
 
 
 def launch_edge_backup(d, path_edge_values=None, virtual_loss=1):
     """Releases the edge-level claims of launch_select; with `path_edge_values` (float32 [trees, warps, path_depth],
     already in the perspective of each edge's owner) it also adds one visit and the value to every path edge."""
-    trees, nodes, edges, warps, path_depth = _shape(d)
-    i32, f32 = np.int32, np.float32
-    values = ctypes.c_void_p(0)
-    if path_edge_values is not None:
-        if tuple(path_edge_values.shape) != (trees, warps, path_depth):
-            raise ValueError("path_edge_values must have shape [trees, warps, path_depth]")
-        values = _device_ptr(path_edge_values, f32, "path_edge_values")
-    code = _lib().puct_edge_backup_launch(
-        int(virtual_loss), _device_ptr(d["edge_w"], f32, "edge_w"), _device_ptr(d["edge_n"], i32, "edge_n"),
-        _device_ptr(d["edge_inflight"], i32, "edge_inflight"),
-        _device_ptr(d["node_expand_inflight"], i32, "node_expand_inflight"),
-        _device_ptr(d["node_count"], i32, "node_count"), _device_ptr(d["out_selected"], i32, "out_selected"),
-        _device_ptr(d["out_path"], i32, "out_path"), _device_ptr(d["out_len"], i32, "out_len"), values,
-        trees, nodes, edges, warps, path_depth, _stream_handle(d))
-    _check(code, "edge backup")
+    arrays, values, *rest = _arguments(d, _EDGE_BACKUP, path_edge_values)
+    code = (_LIB or _lib()).puct_edge_backup_launch(int(virtual_loss), *arrays, values, *rest)
+    if code:
+        _check(code, "edge backup")
 
 
 def launch_node_backup(d, path_edge_values, virtual_loss=1):
     """Backup with node-level virtual loss (d["node_inflight"]), src/puct/puct_gpu_v2.py:847-927."""
-    trees, nodes, edges, warps, path_depth = _shape(d)
-    i32, f32 = np.int32, np.float32
-    if tuple(path_edge_values.shape) != (trees, warps, path_depth):
-        raise ValueError("path_edge_values must have shape [trees, warps, path_depth]")
-    code = _lib().puct_node_backup_launch(
-        int(virtual_loss), _device_ptr(d["edge_child"], i32, "edge_child"), _device_ptr(d["edge_w"], f32, "edge_w"),
-        _device_ptr(d["edge_n"], i32, "edge_n"), _device_ptr(d["node_inflight"], i32, "node_inflight"),
-        _device_ptr(d["node_expand_inflight"], i32, "node_expand_inflight"),
-        _device_ptr(d["node_count"], i32, "node_count"), _device_ptr(d["out_selected"], i32, "out_selected"),
-        _device_ptr(d["out_path"], i32, "out_path"), _device_ptr(d["out_len"], i32, "out_len"),
-        _device_ptr(path_edge_values, f32, "path_edge_values"), trees, nodes, edges, warps, path_depth,
-        _stream_handle(d))
-    _check(code, "node backup")
+    arrays, values, *rest = _arguments(d, _NODE_BACKUP, path_edge_values)
+    code = (_LIB or _lib()).puct_node_backup_launch(int(virtual_loss), *arrays, values, *rest)
+    if code:
+        _check(code, "node backup")
