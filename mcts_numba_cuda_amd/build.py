@@ -1,8 +1,9 @@
-"""Builds libmctsnc_hip.so (search engine) and libpuct_hip.so (PUCT select/backup) for gfx950 with hipcc, in-tree,
-next to this file."""
+"""Builds libmctsnc_hip.so (search engine) and libpuct_hip.so (PUCT select/backup) for gfx950 with hipcc, and _puct_call
+(the Python side of a PUCT launch, host code only) with the C compiler, in-tree, next to this file."""
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -24,17 +25,30 @@ HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
 EXTRA_FLAGS = {PUCT_LIB: ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"]}
 
 
-def build_one(lib, sources, verbose=False):
-    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    cmd = [hipcc] + HIPCC_FLAGS + EXTRA_FLAGS.get(lib, []) + ["-o", lib] + [os.path.join(CSRC, s) for s in sources]
+HOST_MODULE = os.path.join(HERE, "_puct_call" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
+
+
+def run(cmd, what, verbose):
     if verbose:
         print(" ".join(cmd))
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     out = "\n".join(l for l in res.stdout.splitlines() if "packed-fp32-ops" not in l)
     if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + out)
+        raise RuntimeError(f"{what} failed:\n" + out)
     if verbose and out.strip():
         print(out)
+
+
+def build_host_module(verbose=False):
+    run([os.environ.get("CC", "gcc"), "-O2", "-Wall", "-fPIC", "-shared", "-I" + sysconfig.get_paths()["include"], "-o", HOST_MODULE,
+         os.path.join(CSRC, "puct_call.c")], "the C compiler", verbose)
+    return HOST_MODULE
+
+
+def build_one(lib, sources, verbose=False):
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    cmd = [hipcc] + HIPCC_FLAGS + EXTRA_FLAGS.get(lib, []) + ["-o", lib] + [os.path.join(CSRC, s) for s in sources]
+    run(cmd, "hipcc", verbose)
     return lib
 
 
@@ -43,6 +57,8 @@ def build(verbose=False, only=None):
     for lib, sources in LIBRARIES.items():
         if only is None or only == lib:
             build_one(lib, sources, verbose)
+    if only is None or only == HOST_MODULE:
+        build_host_module(verbose)
     return LIB
 
 

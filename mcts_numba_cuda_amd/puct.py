@@ -76,7 +76,8 @@ def reason(raw):
 
 # The arrays of a call: name -> (element type, shape).  A selection and its backup take a dozen microseconds on a GPU when
 # they are small, and a call used to spend twenty on looking its arrays over: one pass over them now, each attribute asked
-# once, and plain integers for ctypes.
+# once, and plain integers for ctypes.  The usual case, torch tensors that fit, goes through _puct_call (csrc/puct_call.c)
+# where it has been built, which makes the same checks in C.
 _TREES, _NODES, _EDGES, _WALKS, _PATHS = range(5)      # [trees], [trees, nodes], [.., edges], [trees, warps], [.., path_depth]
 _ARRAYS = {"edge_child": (np.int32, _EDGES), "edge_prior": (np.float32, _EDGES), "edge_w": (np.float32, _EDGES), "edge_n": (np.int32, _EDGES),
            "edge_inflight": (np.int32, _EDGES), "node_inflight": (np.int32, _NODES), "node_expand_inflight": (np.int32, _NODES),
@@ -85,21 +86,29 @@ _ARRAYS = {"edge_child": (np.int32, _EDGES), "edge_prior": (np.float32, _EDGES),
 _SHAPE_TEXT = {_TREES: "[trees]", _NODES: "[trees, nodes]", _EDGES: "[trees, nodes, edges]", _WALKS: "[trees, warps]", _PATHS: "[trees, warps, path_depth]"}
 
 
-def _fields(*names):
-    """(fields in the order of a launcher's arguments, other arrays whose shape is checked if the dictionary has them)"""
+def _fields(what, *names):
+    """(fields in the order of a launcher's arguments, other arrays whose shape is checked if the dictionary has them, and
+    both with the launcher's number as _puct_call takes them)"""
     checked = ("edge_prior", "edge_w", "edge_n", "edge_inflight", "node_expand_inflight", "node_expanded", "node_inflight", "node_count",
                "out_selected", "out_len")
-    return tuple((n, *_ARRAYS[n]) for n in names), tuple((n, _ARRAYS[n][1]) for n in checked if n not in names)
+    others = tuple(n for n in checked if n not in names)
+    return (tuple((n, *_ARRAYS[n]) for n in names), tuple((n, _ARRAYS[n][1]) for n in others), what,
+            tuple((n, int(_ARRAYS[n][0] is np.float32), _ARRAYS[n][1]) for n in names + others))
 
 
-_SELECT = _fields("edge_child", "edge_prior", "edge_w", "edge_n", "edge_inflight", "node_expand_inflight", "node_expanded", "node_count",
+_SELECT = _fields(0, "edge_child", "edge_prior", "edge_w", "edge_n", "edge_inflight", "node_expand_inflight", "node_expanded", "node_count",
                   "out_selected", "out_path", "out_len")
-_NODE_SELECT = _fields("edge_child", "edge_prior", "edge_w", "edge_n", "node_inflight", "node_expand_inflight", "node_expanded", "node_count",
+_NODE_SELECT = _fields(1, "edge_child", "edge_prior", "edge_w", "edge_n", "node_inflight", "node_expand_inflight", "node_expanded", "node_count",
                        "out_selected", "out_path", "out_len")
-_EDGE_BACKUP = _fields("edge_w", "edge_n", "edge_inflight", "node_expand_inflight", "node_count", "out_selected", "out_path", "out_len")
-_NODE_BACKUP = _fields("edge_child", "edge_w", "edge_n", "node_inflight", "node_expand_inflight", "node_count", "out_selected", "out_path", "out_len")
+_EDGE_BACKUP = _fields(2, "edge_w", "edge_n", "edge_inflight", "node_expand_inflight", "node_count", "out_selected", "out_path", "out_len")
+_NODE_BACKUP = _fields(3, "edge_child", "edge_w", "edge_n", "node_inflight", "node_expand_inflight", "node_count", "out_selected", "out_path", "out_len")
 _torch = None                 # the torch module, once a torch tensor has been seen
 _TORCH_TYPES = {}
+try:
+    from . import _puct_call
+except ImportError:           # (host code only: without it the launchers below do the same in Python)
+    _puct_call = None
+_ENTRIES = {}                 # launcher -> address
 _raw_stream = None            # handle of a device's current stream, without a Stream object around it where torch offers that
 
 
@@ -109,6 +118,8 @@ def _bind_torch():
         import torch
         _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
         _TORCH_TYPES.update({np.int32: torch.int32, np.float32: torch.float32})
+        if _puct_call is not None:
+            _puct_call.setup(torch.Tensor, torch.int32, torch.float32, getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device, _raw_stream)
         _torch = torch
     return _torch
 
@@ -139,7 +150,7 @@ def _arguments(d, fields, values=None):
     trees, nodes, edges = d["edge_child"].shape
     warps, path_depth = d["out_path"].shape[1], d["out_path"].shape[2]
     shapes = ((trees,), (trees, nodes), (trees, nodes, edges), (trees, warps), (trees, warps, path_depth))
-    fields, others = fields
+    fields, others = fields[:2]
     for name, kind in others:
         if name in d and tuple(d[name].shape) != shapes[kind]:
             raise _shape_error(name, kind)
@@ -178,45 +189,51 @@ def _check(code, what):
         raise RuntimeError(f"PUCT {what} launch failed: {msg} ({code})")
 
 
+def _launch(name, fields, d, values, whole, floats=(0.0, 0.0, 0.0)):
+    """Calls the launcher `name` with the arrays of d: `whole` is its soft_winner or virtual_loss, floats its cpuct, c_pw, alpha_pw."""
+    lib = _LIB or _lib()
+    code = None
+    if _torch is not None and _puct_call is not None:
+        entry = _ENTRIES.get(name)
+        if entry is None:
+            entry = _ENTRIES[name] = ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+        code = _puct_call.launch(fields[2], entry, fields[3], d, values, whole, *floats)
+    if code is None:
+        arrays, values, *rest = _arguments(d, fields, values)
+        args = {0: (*floats, whole, *arrays), 1: (*floats, *arrays)}.get(fields[2]) or (whole, *arrays, values)
+        code = getattr(lib, name)(*args, *rest)
+    if code:
+        _check(code, "edge backup" if name == "puct_edge_backup_launch" else "node backup" if name == "puct_node_backup_launch" else
+               "select" if name == "puct_select_winner_recalc_launch" else "node select")
+
+
 def launch_select(d, cpuct=1.0, c_pw=1.0, alpha_pw=0.5, soft_winner=0):
     """Asynchronous PUCT selection on torch's current stream (src/puct/puct_gpu_v3_cpp.py:118-156)."""
-    arrays, _, *rest = _arguments(d, _SELECT)
-    code = (_LIB or _lib()).puct_select_winner_recalc_launch(cpuct, c_pw, alpha_pw, int(soft_winner), *arrays, *rest)
-    if code:
-        _check(code, "select")
+    _launch("puct_select_winner_recalc_launch", _SELECT, d, None, int(soft_winner), (cpuct, c_pw, alpha_pw))
 
 
 VARIANT_PRECLAIM, VARIANT_WINNER_RECALC = "preclaim", "winner_recalc"   # src/puct/test_puct_gpu_v2.py:317-352
+_NODE_SELECTS = {VARIANT_PRECLAIM: "puct_node_select_preclaim_launch", VARIANT_WINNER_RECALC: "puct_node_select_winner_recalc_launch"}
 
 
 def launch_node_select(d, cpuct=1.0, c_pw=1.0, alpha_pw=0.5, variant=VARIANT_PRECLAIM):
     """Asynchronous PUCT selection with node-level virtual loss (d["node_inflight"], int32 [trees, nodes]): the two
     kernels of src/puct/puct_gpu_v2.py:573-840, chosen by `variant` as in the reference's launch helper
     (src/puct/test_puct_gpu_v2.py:317-352).  Selection words have the v2 layout (no reason field, no BUSY kind)."""
-    if variant == VARIANT_PRECLAIM:
-        fn = _lib().puct_node_select_preclaim_launch
-    elif variant == VARIANT_WINNER_RECALC:
-        fn = _lib().puct_node_select_winner_recalc_launch
-    else:
+    name = _NODE_SELECTS.get(variant)
+    if name is None:
         raise ValueError(f"unknown select variant: {variant}")
-    arrays, _, *rest = _arguments(d, _NODE_SELECT)
-    code = fn(cpuct, c_pw, alpha_pw, *arrays, *rest)
-    if code:
-        _check(code, "node select")
+    _launch(name, _NODE_SELECT, d, None, 0, (cpuct, c_pw, alpha_pw))
 
 
 def launch_edge_backup(d, path_edge_values=None, virtual_loss=1):
     """Releases the edge-level claims of launch_select; with `path_edge_values` (float32 [trees, warps, path_depth],
     already in the perspective of each edge's owner) it also adds one visit and the value to every path edge."""
-    arrays, values, *rest = _arguments(d, _EDGE_BACKUP, path_edge_values)
-    code = (_LIB or _lib()).puct_edge_backup_launch(int(virtual_loss), *arrays, values, *rest)
-    if code:
-        _check(code, "edge backup")
+    _launch("puct_edge_backup_launch", _EDGE_BACKUP, d, path_edge_values, int(virtual_loss))
 
 
 def launch_node_backup(d, path_edge_values, virtual_loss=1):
     """Backup with node-level virtual loss (d["node_inflight"]), src/puct/puct_gpu_v2.py:847-927."""
-    arrays, values, *rest = _arguments(d, _NODE_BACKUP, path_edge_values)
-    code = (_LIB or _lib()).puct_node_backup_launch(int(virtual_loss), *arrays, values, *rest)
-    if code:
-        _check(code, "node backup")
+    if path_edge_values is None:
+        raise ValueError("path_edge_values must have shape [trees, warps, path_depth]")
+    _launch("puct_node_backup_launch", _NODE_BACKUP, d, path_edge_values, int(virtual_loss))
