@@ -201,20 +201,28 @@ __device__ __forceinline__ int best_edge(const uint32_t (&keys)[S], int lane, in
 }
 
 // The claims in flight on one tree's edges, edge_inflight[tree, :, :].  While a launch runs they are read and changed by
-// the traversals of that tree only; when those are the wavefronts of one workgroup (up to 16 traversals per tree) and the
-// tree is small enough (nodes * edges words), the workgroup keeps them in LDS for the launch (LOCAL): loaded at the
-// start, stored at the end, every read of a node's row and every claim in between an LDS operation instead of an
-// agent-scope load and an atomic performed at the memory side.
+// the traversals of that tree only, so where they are kept depends on how many those are:
+//   * OWN: one.  Nobody else changes a claim between its read and the winner's, so the claim is an ordinary store, by the
+//     lane that reads that edge, and the row of claims one more load beside the row's other fields.  No LDS, so a CU holds
+//     32 such traversals, which is what hides the memory behind a level: each is a chain of dependent levels.
+//   * LDS: the wavefronts of one workgroup (up to 16), and the tree is small enough (nodes * edges words).  The workgroup
+//     keeps the claims in LDS for the launch: loaded at the start, stored at the end, every read of a node's row and every
+//     claim in between an LDS operation instead of an agent-scope load and an atomic performed at the memory side.
+//   * SHARED: otherwise, the agent-scope loads and atomics.
 typedef __attribute__((address_space(3))) int *LdsInts;
-template <bool LOCAL>
+enum class ClaimsIn { SHARED, LDS, OWN };
+template <ClaimsIn WHERE>
 struct EdgeClaims {
+    static constexpr bool LOCAL = WHERE == ClaimsIn::LDS;
     int *in_memory;     // edge_inflight + tree * nodes * edges
     LdsInts in_lds;     // the same counters, the workgroup's copy
     // (at: byte offset of the edge's slot in the tree, (node * edges + edge) * 4)
     __device__ __forceinline__ int peek(uint32_t at) const {
         if (LOCAL) return __hip_atomic_load(in_lds + (at >> 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (WHERE == ClaimsIn::OWN) return *at_bytes(in_memory, at);
         return load_relaxed(at_bytes(in_memory, at));
     }
+    __device__ __forceinline__ void set(uint32_t at, int v) const { *at_bytes(in_memory, at) = v; }   // OWN: by the lane that peeks there
     __device__ __forceinline__ void add(uint32_t at, int v) const {
         if (LOCAL) __hip_atomic_fetch_add(in_lds + (at >> 2), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         else atomicAdd(at_bytes(in_memory, at), v);
@@ -229,14 +237,15 @@ struct EdgeClaims {
 };
 
 // The path entries of a traversal are stored by lane 0 of its wavefront and read back by all its lanes past the L1
-// (load_relaxed), so all a rollback needs before it reads them is that the stores have reached the L2.  A device-scope fence
+// (load_relaxed), so all a rollback needs before it reads them is that the stores have reached the L2 (and with them the
+// claims that its atomics take back, where those were stores too).  A device-scope fence
 // would write the L2 back: with 1024 trees of 8 traversals, most of which give way to another, 8192 of those were five
 // sixths of a launch (122 us, 4097 nodes of 64 edges a tree, paths of two levels).
 __device__ __forceinline__ void wait_path_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // Takes back the virtual loss of the first `depth` path entries (src/puct/puct_gpu_v3_cpp.cu:206-217).
-template <bool LOCAL>
-__device__ __forceinline__ void rollback_path(const SelectArgs &a, const EdgeClaims<LOCAL> &claims, const int *path, int tree, int depth, int lane,
+template <ClaimsIn WHERE>
+__device__ __forceinline__ void rollback_path(const SelectArgs &a, const EdgeClaims<WHERE> &claims, const int *path, int tree, int depth, int lane,
                                               int node_cnt) {
     wait_path_stores();
     for (int d = lane; d < depth; d += kWave) {
@@ -251,8 +260,8 @@ __device__ __forceinline__ void rollback_path(const SelectArgs &a, const EdgeCla
 // number S of 64-edge slices that the node's expanded edges fill (1..4, the same for all lanes): these kernels are bound
 // by the wavefronts' instruction issue, vector and scalar together, and a level written for "up to four slices" spends a
 // third of it on finding out, slice by slice, that a slice is not there.
-template <bool LOCAL>
-__device__ __forceinline__ void select_traversal(const SelectArgs &a, const EdgeClaims<LOCAL> &claims, int tree, int wid, int lane) {
+template <ClaimsIn WHERE>
+__device__ __forceinline__ void select_traversal(const SelectArgs &a, const EdgeClaims<WHERE> &claims, int tree, int wid, int lane) {
     static_assert(kPasses == 4, "the levels below are written for one to four slices");
     const size_t out = (size_t)tree * a.warps + wid;
     int *path = a.out_path_eids + out * a.path_depth;
@@ -384,7 +393,7 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                 // what they read -- and three registers per lane; at 128 edges waiting for the word cost more than the row).
                 int best_eid = 0, held = 0, best_child = c0;   // (cur_expanded == 1: lane 0's is read below)
                 if (cur_expanded == 1) {
-                    if (lane == 0) claims.add(row4, 1);
+                    if (WHERE != ClaimsIn::OWN && lane == 0) claims.add(row4, 1);
                     held = 1;
                 } else {
                     // Winner-recalc claim, src/puct/puct_gpu_v3_cpp.cu:235-275: score all edges, try to move the winner's
@@ -421,13 +430,17 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                         }
                         best_eid = best_edge<S>(keys, lane, -1, tie_offset);
                         if (best_eid == kNoEdge) break;
-                        const int best_inflight = of_edge(f, best_eid);
                         if (best_eid < CS * kWave) {
                             best_child = __builtin_amdgcn_readlane(c[0], best_eid & (kWave - 1));
                             if (CS > 1 && best_eid >= kWave) best_child = __builtin_amdgcn_readlane(c[CS - 1], best_eid & (kWave - 1));
                         } else {
                             best_child = load_relaxed(at_bytes(tree_c, row4 + (uint32_t)best_eid * 4u));   // (every lane the same word)
                         }
+                        if (WHERE == ClaimsIn::OWN) {
+                            held = 1;
+                            break;
+                        }
+                        const int best_inflight = of_edge(f, best_eid);
                         int got = 0;
                         if (lane == 0) {
                             const int prev = claims.cas(row4 + (uint32_t)best_eid * 4u, best_inflight, best_inflight + 1);
@@ -436,7 +449,7 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                         held = __builtin_amdgcn_readfirstlane(got);
                         if (held) break;
                     }
-                    if (a.soft_winner != 0 && held == 0 && best_eid != kNoEdge) {
+                    if (WHERE != ClaimsIn::OWN && a.soft_winner != 0 && held == 0 && best_eid != kNoEdge) {
                         if (lane == 0) claims.add(row4 + (uint32_t)best_eid * 4u, 1);
                         held = 1;
                     }
@@ -453,11 +466,16 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
 
                 best_child = __builtin_amdgcn_readfirstlane(best_child);
                 if (best_child < 0 || best_child >= node_cnt) {
-                    if (lane == 0) claims.add(row4 + (uint32_t)best_eid * 4u, -1);
+                    if (WHERE != ClaimsIn::OWN && lane == 0) claims.add(row4 + (uint32_t)best_eid * 4u, -1);
                     rollback_path(a, claims, path, tree, depth, lane, node_cnt);
                     final_packed =
                         pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_CHILD_OOB);
                     return -1;
+                }
+                if (WHERE == ClaimsIn::OWN) {   // (the claim, now that the edge is known to lead somewhere)
+#pragma unroll
+                    for (int i = 0; i < S; ++i)
+                        if (lane + i * kWave == best_eid) claims.set(row4 + (uint32_t)best_eid * 4u, f[i] + 1);
                 }
                 if (lane == 0) path[depth] = (node << 8) | best_eid;
                 return best_child;

@@ -4,20 +4,21 @@
 namespace {
 using namespace puct;
 
-// LOCAL: the tree's traversals are this workgroup's wavefronts (grid.y == 1) and the claims on its edges are kept in
-// the workgroup's dynamic LDS for the launch (a.nodes * a.edges words).
-template <bool LOCAL>
+// LDS: the tree's traversals are this workgroup's wavefronts (grid.y == 1) and the claims on its edges are kept in
+// the workgroup's dynamic LDS for the launch (a.nodes * a.edges words).  OWN: the tree has one traversal.
+template <ClaimsIn WHERE>
 __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) __attribute__((amdgpu_waves_per_eu(8, 8))) void select_kernel(const SelectArgs a) {
     extern __shared__ int tree_claims[];
     const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave);   // the same in all lanes
+    constexpr bool LOCAL = WHERE == ClaimsIn::LDS;
     const int words = a.nodes * a.edges;
     int *const in_memory = a.edge_inflight + (size_t)blockIdx.x * a.nodes * a.edges;
-    const EdgeClaims<LOCAL> claims{in_memory, (LdsInts)tree_claims};
+    const EdgeClaims<WHERE> claims{in_memory, (LdsInts)tree_claims};
     if (LOCAL) {
         for (int i = threadIdx.x; i < words; i += blockDim.x) tree_claims[i] = in_memory[i];
         __syncthreads();
     }
-    if (LOCAL || wid < a.warps) select_traversal<LOCAL>(a, claims, blockIdx.x, wid, threadIdx.x & (kWave - 1));
+    if (LOCAL || wid < a.warps) select_traversal<WHERE>(a, claims, blockIdx.x, wid, threadIdx.x & (kWave - 1));
     if (LOCAL) {
         __syncthreads();
         for (int i = threadIdx.x; i < words; i += blockDim.x) in_memory[i] = tree_claims[i];
@@ -76,10 +77,14 @@ extern "C" int puct_select_winner_recalc_launch(float cpuct, float c_pw, float a
     launch_shape(trees, warps, grid, block);
     // (the claims of a tree in LDS: up to 8192 edge slots, so that a CU still holds four workgroups)
     const long long slots = (long long)nodes * edges;
-    if (grid.y == 1 && slots > 0 && slots <= kLocalClaimSlots)
-        hipLaunchKernelGGL(select_kernel<true>, grid, block, sizeof(int) * (size_t)slots, reinterpret_cast<hipStream_t>(stream), a);
+    // With larger trees a launch shares edge_inflight with other launches, also one of single traversals.
+    const bool exclusive = grid.y == 1 && slots > 0 && slots <= kLocalClaimSlots;
+    if (exclusive && warps == 1)
+        hipLaunchKernelGGL(select_kernel<ClaimsIn::OWN>, grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);
+    else if (exclusive)
+        hipLaunchKernelGGL(select_kernel<ClaimsIn::LDS>, grid, block, sizeof(int) * (size_t)slots, reinterpret_cast<hipStream_t>(stream), a);
     else
-        hipLaunchKernelGGL(select_kernel<false>, grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);
+        hipLaunchKernelGGL(select_kernel<ClaimsIn::SHARED>, grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);
     return static_cast<int>(hipGetLastError());
 }
 
