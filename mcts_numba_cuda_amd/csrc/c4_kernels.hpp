@@ -112,10 +112,19 @@ struct SearchArgs {
 struct Geometry {
     int m, n, H;
     uint64_t full;          // all playable cells
+    // A playout keeps a board as two 32-bit words.  On most boards a column can be kept in one word: the lower word takes
+    // as many columns as fit, moved up so that the last of them ends at bit 31.  If, besides, every row and diagonal of
+    // four starts (at its leftmost column) in the lower word, the test for four needs 20 instructions instead of 36
+    // (5 x 6, 6 x 7 and 7 x 7 boards; not 7 x 8, whose column 4 starts fours, nor 8 x 7, with three columns to a word).
+    int base;               // how far a playout's board is moved up
+    bool aligned;
     __device__ Geometry(int m_, int n_) : m(m_), n(n_), H(m_ + 1) {
         uint64_t f = 0;
         for (int c = 0; c < n; c++) f |= (((1ull << m) - 1ull) << (c * H));
         full = f;
+        const int low = 32 / H;   // columns of the lower word
+        aligned = H <= 8 && n - 3 <= low && (n - low) * H - 1 <= 32;   // (H <= 8: base + m fits a 4-bit field)
+        base = aligned ? 32 - low * H : 0;
     }
     __device__ __forceinline__ uint64_t col_mask(int c) const { return ((1ull << m) - 1ull) << (c * H); }
     __device__ __forceinline__ uint64_t bottom(int c) const { return 1ull << (c * H); }
@@ -221,8 +230,8 @@ __device__ __forceinline__ BB bb_shr(BB x, int s) {  // 0 < s < 32 (the largest 
 }
 __device__ __forceinline__ BB bb_and(BB a, BB b) { BB r; r.lo = a.lo & b.lo; r.hi = a.hi & b.hi; return r; }
 
-// four in a row anywhere in p (equals "through the last stone" while no earlier line exists)
-__device__ __forceinline__ bool bb_has_four(BB p, int H) {
+// Nonzero if there are four in a row anywhere in p (equals "through the last stone" while no earlier line exists).
+__device__ __forceinline__ uint32_t bb_fours(BB p, int H) {
     BB t = bb_and(p, bb_shr(p, 1));
     BB r = bb_and(t, bb_shr(t, 2));
     t = bb_and(p, bb_shr(p, H));
@@ -233,14 +242,43 @@ __device__ __forceinline__ bool bb_has_four(BB p, int H) {
     r.lo |= q.lo; r.hi |= q.hi;
     t = bb_and(p, bb_shr(p, H + 1));
     q = bb_and(t, bb_shr(t, 2 * (H + 1)));
-    return (r.lo | q.lo | r.hi | q.hi) != 0;
+    return r.lo | q.lo | r.hi | q.hi;
+}
+
+// The same on an aligned board (Geometry::aligned) whose last stone is in the upper word if `upper` is all ones, in the
+// lower one if it is 0: rows and diagonals start in the lower word, a column is within the stone's word.
+__device__ __forceinline__ uint32_t bb_fours_aligned(BB p, uint32_t upper, int H) {
+    const uint32_t w = __builtin_amdgcn_bitop3_b32(upper, p.hi, p.lo, 0xca);   // the stone's word
+    const uint32_t v = w & (w >> 1);
+    uint32_t r = v & (v >> 2);
+    const auto along = [&](int s) {   // 3 s < 32
+        return p.lo & __builtin_amdgcn_alignbit(p.hi, p.lo, s) & __builtin_amdgcn_alignbit(p.hi, p.lo, 2 * s) & __builtin_amdgcn_alignbit(p.hi, p.lo, 3 * s);
+    };
+    r |= along(H);
+    r |= along(H - 1);
+    r |= along(H + 1);
+    return r;
 }
 
 // What a playout of one node starts from: the stones of the side to move (a) and of the other side (b) as 32-bit halves,
-// the column fills and the ascending list of legal columns as 4-bit fields, the number of legal columns, and the side
-// to move (low byte) with the node's column (second byte) and the number of stones on the board (third byte).  Worked out once per node and step by the workgroup that searches a tree
-// alone, once per playout elsewhere.
-struct PoolChild { uint32_t a_lo, a_hi, b_lo, b_hi, fills, list; int32_t count; uint32_t turn_col; };
+// the column fills (counted from Geometry::base) and the ascending list of legal columns as 4-bit fields, the number of
+// legal columns times 2^-32, and the side to move (low byte) with the node's column (second byte) and the number of stones
+// on the board (third byte).  Both boards are moved up by Geometry::base.  Worked out once per node and step by the
+// workgroup that searches a tree alone, once per playout elsewhere.
+struct PoolChild { uint32_t a_lo, a_hi, b_lo, b_hi, fills, list; float count; uint32_t turn_col; };
+
+// A running playout, one per lane: column fills, legal columns and their number as in PoolChild, the generator, the number
+// it gives next, and the fours of the last move.
+struct Playout {
+    uint32_t fills, list;
+    float count;      // legal columns * 2^-32
+    Rng32 rng;
+    float draw;       // the next uniform times 2^32; 2^32 itself (the uniform rounded up to 1.0f) stops the playout
+    uint32_t fours;   // nonzero: the last move won
+    __device__ __forceinline__ bool running() const { return fours == 0 && count != 0.0f && draw < 4294967296.0f; }
+    __device__ __forceinline__ bool full() const { return count == 0.0f; }
+    __device__ __forceinline__ bool to_replay() const { return fours == 0 && count != 0.0f; }   // of a playout that stopped
+};
 
 // ------------------------------------------------------------------------------------------------------------------------
 // Connect 4 as the game of the bitboard step skeleton below (search_body): the five device functions of the reference's
@@ -249,11 +287,12 @@ struct PoolChild { uint32_t a_lo, a_hi, b_lo, b_hi, fills, list; int32_t count; 
 //   legal_actions   is_action_legal for all actions at once (bit a set = action a legal)
 //   child           take_action + compute_outcome: the position after `action` and its outcome (-1 / 0 / +1, 2 = ongoing)
 //   playout_start   legal_actions_playout: what a playout from a position starts from
-//   ply             take_action_playout + compute_outcome for one random move, free of branches
+//   begin, ply      take_action_playout + compute_outcome for one random move, free of branches
 //   fast_playout    a whole playout (start + plies); exact_playout: the byte-array emulation for draws that round up
 // ------------------------------------------------------------------------------------------------------------------------
 struct Connect4 {
     using Geometry = c4::Geometry;
+    using Playout = c4::Playout;
     using Exact = ExactScratch;
 
     static __device__ __forceinline__ uint32_t legal_actions(const Geometry &g, uint64_t pos, uint64_t neg) { return g.legal_cols(pos | neg); }
@@ -270,31 +309,52 @@ struct Connect4 {
 
     static __device__ __forceinline__ PoolChild playout_start(const Geometry &g, uint64_t cur, uint64_t opp, int turn, int column) {
         PoolChild pc;
-        pc.a_lo = (uint32_t)cur; pc.a_hi = (uint32_t)(cur >> 32); pc.b_lo = (uint32_t)opp; pc.b_hi = (uint32_t)(opp >> 32);
+        const uint64_t a = cur << g.base, b = opp << g.base;
+        pc.a_lo = (uint32_t)a; pc.a_hi = (uint32_t)(a >> 32); pc.b_lo = (uint32_t)b; pc.b_hi = (uint32_t)(b >> 32);
         const uint64_t occ = cur | opp;
         uint32_t fills = 0, list = 0; int count = 0;
         for (int c = 0; c < g.n; c++) {
             const int h = __popcll(occ & g.col_mask(c));
-            fills |= (uint32_t)h << (4 * c);
+            fills |= (uint32_t)(h + g.base) << (4 * c);
             if (h < g.m) { list |= (uint32_t)c << (4 * count); count++; }
         }
-        pc.fills = fills; pc.list = list; pc.count = count;
+        pc.fills = fills; pc.list = list; pc.count = (float)count * 0x1p-32f;
         pc.turn_col = (uint32_t)(turn & 0xff) | ((uint32_t)column << 8) | ((uint32_t)__popcll(occ) << 16);
         return pc;
     }
 
+    // The uniform that the generator gives in its present state, times 2^32.  The reference's float32 of the upper 53 bits
+    // of the sum, a single rounding, in four instructions without float64 (which took six, four of them conversions): the
+    // upper word's conversion rounds as the whole would if its last bit says whether anything follows, as long as at
+    // least two bits are dropped, that is from 2^25 on.  Below that the ordinal is 0 anyway: with at most 8 columns it
+    // is as long as the uniform is below 1/8.
+    static __device__ __forceinline__ float draw_of(const Rng32 &r) {
+        const uint64_t sum = (((uint64_t)r.s0h << 32) | r.s0l) + (((uint64_t)r.s1h << 32) | r.s1l);
+        const uint32_t rest = (uint32_t)sum >> 11;
+        return (float)((uint32_t)(sum >> 32) | (rest < 1u ? rest : 1u));
+    }
+
+    static __device__ __forceinline__ void begin(Playout &p, const PoolChild &pc, uint64_t s0, uint64_t s1) {
+        p.fills = pc.fills; p.list = pc.list; p.count = pc.count;
+        p.rng.s0l = (uint32_t)s0; p.rng.s0h = (uint32_t)(s0 >> 32); p.rng.s1l = (uint32_t)s1; p.rng.s1h = (uint32_t)(s1 >> 32);
+        p.draw = draw_of(p.rng);
+        p.fours = 0;
+    }
+
     // One random move of the side whose stones are `me` (the other side's stones are not needed: the column fills say
-    // where a stone lands); the caller alternates the two sides.  Returns 0 = game goes on, 1 = the mover won, 2 = board
-    // full, 3 = the drawn ordinal equals the count (the uniform rounded up to 1.0f).
-    static __device__ __forceinline__ int ply(int m, int H, BB &me, uint32_t &fills, uint32_t &list, int &count, Rng32 &r) {
-        uint32_t xl, xh;
-        rng_next32(r, xl, xh);
-        const float u = uniform_from_bits(xl, xh);
-        const int ord = (int)(u * (float)count);  // single-precision product, as the reference's float32 * int16
+    // where a stone lands) in a playout that is running; the caller alternates the two sides.  A ply is bound by its
+    // instructions, 60 on aligned boards (87 with the test over both words and the draw through float64, of which the
+    // flag word of the outcome took seven where now three comparisons meet in scalar registers); the next draw does not
+    // depend on the move and is made beside it.  512 trees x 7 x 256 playouts a step: 16.7 -> 14.7 ms per 500 steps; 64 searches
+    // of 4 trees in one pass: 32.0 -> 26.8 ms; 8 trees from the empty board, 20000 steps: 215 -> 193 ms.
+    static __device__ __forceinline__ void ply(bool aligned, int last_fill /* of a column: base + m - 1 */, int H, BB &me, Playout &p) {
+        const int ord = (int)(p.draw * p.count);  // single-precision product, as the reference's float32 * int16
+        rng_advance32(p.rng);
+        p.draw = draw_of(p.rng);
         const int sh = ord * 4;
-        const uint32_t c = (list >> sh) & 7u;
+        const uint32_t c = (p.list >> sh) & 7u;
         const uint32_t c4 = c * 4u;
-        const uint32_t h = (fills >> c4) & 15u;
+        const uint32_t h = (p.fills >> c4) & 15u;
         uint32_t pos;   // c * H + h at full rate (the compiler would take the 64-bit multiply-add, a quarter-rate instruction)
         asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(pos) : "v"(c), "s"(H), "v"(h));
         const uint32_t bit = 1u << (pos & 31u);
@@ -302,15 +362,23 @@ struct Connect4 {
         asm("" : "+v"(upper));                                      // (kept as a mask: two and-or instructions instead of compare and selects)
         me.lo |= bit & ~upper;
         me.hi |= bit & upper;
-        fills += 1u << c4;
-        const bool full = (h + 1u == (uint32_t)m);
+        p.fills += 1u << c4;
+        const bool full = h == (uint32_t)last_fill;
         const uint32_t low = (1u << sh) - 1u;
-        list = full ? ((list & low) | ((list >> 4) & ~low)) : list;  // a full column leaves the ascending list
-        const bool hit = ord >= count;
-        count -= full ? 1 : 0;
-        const bool win = bb_has_four(me, H);
-        if (!(hit || win || count == 0)) return 0;
-        return hit ? 3 : (win ? 1 : 2);
+        p.list = full ? ((p.list & low) | ((p.list >> 4) & ~low)) : p.list;  // a full column leaves the ascending list
+        p.count -= full ? 0x1p-32f : 0.0f;
+        p.fours = aligned ? bb_fours_aligned(me, upper, H) : bb_fours(me, H);
+    }
+
+    template <bool ALIGNED>
+    static __device__ __forceinline__ void play(const Geometry &g, BB &a, BB &b, Playout &p) {
+        int last_fill = g.base + g.m - 1, H = g.H;
+        asm("" : "+s"(last_fill), "+s"(H));   // the shifts are worked out here, not kept in scalar registers through the whole search
+        while (p.running()) {   // the two sides in turn
+            ply(ALIGNED, last_fill, H, a, p);
+            if (!p.running()) break;
+            ply(ALIGNED, last_fill, H, b, p);
+        }
     }
 
     // cur: stones of the side to move, opp: the other side's.  Returns -1 / 0 / +1, or 2 when a draw of the uniform
@@ -318,25 +386,17 @@ struct Connect4 {
     static __device__ __forceinline__ int fast_playout(const Geometry &g, uint64_t cur, uint64_t opp, int turn,
                                                        uint64_t &s0, uint64_t &s1, uint32_t &plies) {
         const PoolChild pc = playout_start(g, cur, opp, turn, 0);
+        if (pc.count == 0.0f) return 0;
         BB a = {pc.a_lo, pc.a_hi}, b = {pc.b_lo, pc.b_hi};
-        uint32_t fills = pc.fills, list = pc.list;
-        int count = pc.count;
-        if (count == 0) return 0;
-        const int m = g.m, H = g.H;
-        Rng32 r;
-        r.s0l = (uint32_t)s0; r.s0h = (uint32_t)(s0 >> 32); r.s1l = (uint32_t)s1; r.s1h = (uint32_t)(s1 >> 32);
-        int status;
-        for (;;) {   // the two sides in turn
-            status = ply(m, H, a, fills, list, count, r);
-            if (status != 0) break;
-            status = ply(m, H, b, fills, list, count, r);
-            if (status != 0) break;
-        }
-        s0 = ((uint64_t)r.s0h << 32) | r.s0l; s1 = ((uint64_t)r.s1h << 32) | r.s1l;
+        Playout p;
+        begin(p, pc, s0, s1);
+        if (g.aligned) play<true>(g, a, b, p);
+        else play<false>(g, a, b, p);
+        s0 = ((uint64_t)p.rng.s0h << 32) | p.rng.s0l; s1 = ((uint64_t)p.rng.s1h << 32) | p.rng.s1l;
         const uint32_t n = (uint32_t)(__popc(a.lo) + __popc(a.hi) + __popc(b.lo) + __popc(b.hi)) - (pc.turn_col >> 16);   // plies made
         plies += n;
         const int mover = (n & 1u) ? turn : -turn;  // side that made the last move
-        return status == 1 ? mover : (status == 2 ? 0 : 2);
+        return p.fours != 0 ? mover : (p.full() ? 0 : 2);
     }
 
     static __device__ __forceinline__ int exact_playout(Exact &s, const Geometry &g, uint64_t pos, uint64_t neg, int turn,
@@ -685,19 +745,20 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
             {
                 const int n_jobs = __builtin_amdgcn_readfirstlane(s_pool_n) * P;   // (the same in every lane: kept in a scalar register)
                 const int pshift = 31 - __clz(P);   // P is a power of two
-                const int m = geo.m, H = geo.H;
+                int last_fill = geo.base + geo.m - 1, H = geo.H;
+                asm("" : "+s"(last_fill), "+s"(H));   // (the playouts' shifts are worked out here, not kept through the search)
+                const bool aligned = geo.aligned;     // (a branch within the ply: two loops with the booking would not fit the registers)
+                constexpr uint32_t kNoJob = 0xffffffffu;
                 BB a = {0, 0}, b = {0, 0};
-                uint32_t fills = 0, list = 0, job_turn_col = 0, job_t = 0;
-                int count = 0;
-                Rng32 rg = {0, 0, 0, 0};
+                uint32_t job_turn_col = 0, job_t = kNoJob;   // kNoJob: nothing taken, or booked already
+                typename Game::Playout p = {};               // (count 0: not running)
                 auto take_job = [&](int j, BB &mover, BB &waiting) {   // j < n_jobs; mover: the stones of the side that moves next
                     const PoolChild pc = s_pool[j >> pshift];
                     job_t = (uint32_t)j & (uint32_t)(P - 1);
-                    mover.lo = pc.a_lo; mover.hi = pc.a_hi; waiting.lo = pc.b_lo; waiting.hi = pc.b_hi; fills = pc.fills; list = pc.list; count = pc.count;
+                    mover.lo = pc.a_lo; mover.hi = pc.a_hi; waiting.lo = pc.b_lo; waiting.hi = pc.b_hi;
                     job_turn_col = pc.turn_col;
                     const uint64_t *st = s_rng + 2 * ((size_t)((pc.turn_col >> 8) & 0xffu) * P + job_t);
-                    const uint64_t q0 = st[0], q1 = st[1];
-                    rg.s0l = (uint32_t)q0; rg.s0h = (uint32_t)(q0 >> 32); rg.s1l = (uint32_t)q1; rg.s1h = (uint32_t)(q1 >> 32);
+                    Game::begin(p, pc, st[0], st[1]);
                 };
                 // The wavefronts take jobs from one counter, in batches, as their lanes fall idle: how fast a wavefront gets
                 // through its playouts depends on how many wavefronts share its SIMD, which a workgroup cannot choose, and with
@@ -709,10 +770,10 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
                 };
                 int first = grab(kWave);
                 bool exhausted = first + kWave >= n_jobs;   // the counter has passed the end: nothing more to take
-                // per lane: 0 = its playout is running; 1 = it ended with a win of the mover, 2 = with the board full, 3 = with
-                // a draw that equalled the count (to be replayed), all three not booked yet; 4 = no playout
-                int state = first + lane < n_jobs ? 0 : 4;
-                if (state == 0) take_job(first + lane, a, b);
+                if (first + lane < n_jobs) take_job(first + lane, a, b);
+                // The lanes whose playouts are running, as a mask in scalar registers (a flag per lane that lives across
+                // iterations becomes a 0/1 register that is made and compared each time).
+                unsigned long long running = __ballot(p.running());
                 // Finished lanes are served in batches: booking a result and fetching the next job costs about 40
                 // instructions for the whole wavefront whenever it runs, and with 64 lanes some lane finishes in almost
                 // every iteration; so it runs only once kRefill lanes are waiting (or all are), and not at all once the
@@ -723,13 +784,15 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
                 // One iteration for the side whose stones are `me`, the same side in every lane (a job taken now starts
                 // with the next iteration, so its side to move goes where `other` is); true when the wavefront is done.
                 auto iteration = [&](BB &me, BB &other) -> bool {
-                    if (state == 0) state = Game::ply(m, H, me, fills, list, count, rg);
-                    const unsigned long long idle = __ballot(state != 0);
+                    if (__builtin_amdgcn_inverse_ballot_w64(running)) Game::ply(aligned, last_fill, H, me, p);
+                    running = __ballot(p.running());
+                    const unsigned long long idle = ~running;
                     const int n_idle = __builtin_popcountll(idle);
                     if (!(idle == ~0ull || (!exhausted && (uint32_t)n_idle >= (uint32_t)kRefill))) return false;
                     const int col = (int)((job_turn_col >> 8) & 0xffu), turn_a = (int)(int8_t)(job_turn_col & 0xffu);
+                    const bool ended = ((idle >> lane) & 1ull) && job_t != kNoJob, replay = ended && p.to_replay();
                     uint64_t *const st = s_rng + 2 * ((size_t)col * P + job_t);
-                    if (__ballot(state == 3) != 0ull) {  // rare: a draw rounded up to 1.0f; replay with the exact emulation, one playout at a time
+                    if (__ballot(replay) != 0ull) {  // rare: a draw rounded up to 1.0f; replay with the exact emulation, one playout at a time
                         if (lane == 0) {
                             uint32_t spins = 0;
                             while (atomicCAS(&s_lock, 0u, 1u) != 0u) {
@@ -738,14 +801,14 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
                             }
                         }
                         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                        unsigned long long redo = __ballot(state == 3);
+                        unsigned long long redo = __ballot(replay);
                         while (redo) {
                             const int l = (int)__ffsll((long long)redo) - 1;
                             redo &= redo - 1ull;
                             if (lane == l) {
                                 const PoolChild pc = s_pool[__popc(solo_played & ((1u << col) - 1u))];
                                 uint64_t q0 = st[0], q1 = st[1];   // the generator as it was when the playout started
-                                const uint64_t cur = ((uint64_t)pc.a_hi << 32) | pc.a_lo, opp = ((uint64_t)pc.b_hi << 32) | pc.b_lo;
+                                const uint64_t cur = (((uint64_t)pc.a_hi << 32) | pc.a_lo) >> geo.base, opp = (((uint64_t)pc.b_hi << 32) | pc.b_lo) >> geo.base;
                                 const uint64_t ppos = (turn_a == 1) ? cur : opp, pneg = (turn_a == 1) ? opp : cur;
                                 const int outcome = Game::exact_playout(s_exact_solo, geo, ppos, pneg, turn_a, q0, q1, plies, u1);
                                 st[0] = q0; st[1] = q1;
@@ -755,23 +818,24 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
                         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
                         if (lane == 0) atomicExch(&s_lock, 0u);
                     }
-                    if (state == 1 || state == 2) {
-                        st[0] = ((uint64_t)rg.s0h << 32) | rg.s0l; st[1] = ((uint64_t)rg.s1h << 32) | rg.s1l;
+                    if (ended && !replay) {
+                        st[0] = ((uint64_t)p.rng.s0h << 32) | p.rng.s0l; st[1] = ((uint64_t)p.rng.s1h << 32) | p.rng.s1l;
                         const uint32_t n = (uint32_t)(__popc(me.lo) + __popc(me.hi) + __popc(other.lo) + __popc(other.hi)) - (job_turn_col >> 16);   // plies made
                         plies += n;
-                        if (state == 1) {
+                        if (p.fours != 0) {
                             const int winner = (n & 1u) ? turn_a : -turn_a;   // the side that made the last move
                             atomicAdd(&s_cnt[col][winner == 1 ? 1 : 0], 1);
                         }
                     }
-                    state = state != 0 ? 4 : 0;
+                    if ((idle >> lane) & 1ull) job_t = kNoJob;
                     if (exhausted) return true;   // every lane is idle and there is nothing left to hand out
                     // the idle lanes take the next jobs in lane order
                     first = grab(n_idle);
                     exhausted = first + n_idle >= n_jobs;
                     const int mine = first + (int)__popcll(idle & ((1ull << lane) - 1ull));
-                    if (state != 0 && mine < n_jobs) { take_job(mine, other, me); state = 0; }
-                    return __ballot(state == 0) == 0ull;   // (the counter had passed the end already)
+                    if (((idle >> lane) & 1ull) && mine < n_jobs) take_job(mine, other, me);
+                    running = __ballot(p.running());
+                    return __ballot(job_t != kNoJob) == 0ull;   // (the counter had passed the end already)
                 };
                 for (;;) {
                     if (iteration(a, b)) break;

@@ -57,15 +57,20 @@ __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) { r
 
 struct Rng32 { uint32_t s0l, s0h, s1l, s1h; };
 
-__device__ __forceinline__ void rng_next32(Rng32 &r, uint32_t &out_lo, uint32_t &out_hi) {
-    const uint64_t sum = (((uint64_t)r.s0h << 32) | r.s0l) + (((uint64_t)r.s1h << 32) | r.s1l);
-    out_lo = (uint32_t)sum; out_hi = (uint32_t)(sum >> 32);
+// The state after a draw.
+__device__ __forceinline__ void rng_advance32(Rng32 &r) {
     const uint32_t tl = r.s1l ^ r.s0l, th = r.s1h ^ r.s0h;
     // rotl(s0, 55) = rotr(s0, 9); t << 14; rotl(t, 36) = halves swapped, then rotl 4
     const uint32_t r0l = __builtin_amdgcn_alignbit(r.s0h, r.s0l, 9), r0h = __builtin_amdgcn_alignbit(r.s0l, r.s0h, 9);
     const uint32_t shl = tl << 14, shh = __builtin_amdgcn_alignbit(th, tl, 18);
     r.s0l = xor3(r0l, tl, shl); r.s0h = xor3(r0h, th, shh);
     r.s1l = __builtin_amdgcn_alignbit(th, tl, 28); r.s1h = __builtin_amdgcn_alignbit(tl, th, 28);
+}
+
+__device__ __forceinline__ void rng_next32(Rng32 &r, uint32_t &out_lo, uint32_t &out_hi) {
+    const uint64_t sum = (((uint64_t)r.s0h << 32) | r.s0l) + (((uint64_t)r.s1h << 32) | r.s1l);
+    out_lo = (uint32_t)sum; out_hi = (uint32_t)(sum >> 32);
+    rng_advance32(r);
 }
 
 // UCB of one child with the reference's numba typing (src/mctsnc.py:1337): float64 arithmetic on

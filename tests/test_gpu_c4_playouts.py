@@ -1,0 +1,40 @@
+"""Connect 4 playouts at the edges of their two board layouts, engine against oracle, every array bit for bit (two searches
+in a row): boards whose columns each fit one of the two words and whose fours start in the lower one (4 x 4 to 7 x 7, a lower
+word of four to six columns, with and without free bits below them), the first ones that miss either condition, by teams, by
+one workgroup per tree and by teams with playout pools; and searches long enough to meet draws rounded up to 1.0f."""
+import numpy as np
+import pytest
+
+from helpers import compare_with_oracle, make_engine, random_c4_root
+from oracle.oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+FORMS = dict(teams=dict(solo_trees=0, team_pool=0), solo=dict(solo_trees=1), pools=dict(solo_trees=0, team_pool=1))
+BOARDS = [(4, 4), (6, 4), (5, 6), (4, 7), (5, 8), (6, 6), (7, 7), (7, 4), (8, 6), (6, 8), (4, 8)]
+LONG = [  # rows, columns, plies, variant, seed, steps: the oracle meets at least one such draw in each
+    (6, 7, 0, "acp_prodigal", 0, 150), (5, 6, 0, "acp_prodigal", 0, 150), (7, 8, 0, "acp_prodigal", 0, 150),
+    (6, 7, 2, "ocp_thrifty", 5, 600), (5, 6, 2, "ocp_thrifty", 5, 600),
+]
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("m,n", BOARDS)
+def test_playouts_on_both_board_layouts(m, n, form):
+    params = dict(n_trees=2, n_playouts=64, variant="acp_prodigal", device_memory=0.1, ucb_c=2.0, seed=3)
+    e = make_engine(params, board_shape=(m, n), extra=n, actions=n, options=FORMS[form])
+    o = Oracle("c4", (m, n), n, n, 2, 64, "acp_prodigal", ucb_c=2.0, seed=3, device_memory=0.1, threads=8)
+    rng = np.random.default_rng(10 * m + n)
+    for plies in (0, m * n // 2):
+        board, fills, turn = random_c4_root(rng, plies, m, n)
+        compare_with_oracle(e, o, board, fills, turn, steps=120)
+
+
+@pytest.mark.parametrize("m,n,plies,variant,seed,steps", LONG)
+def test_draws_rounded_up_are_replayed(m, n, plies, variant, seed, steps):
+    params = dict(n_trees=4, n_playouts=512, variant=variant, device_memory=0.3, ucb_c=2.0, seed=seed)
+    for options in FORMS.values() if variant.startswith("acp") else (None,):
+        e = make_engine(params, board_shape=(m, n), extra=n, actions=n, options=options)
+        o = Oracle("c4", (m, n), n, n, 4, 512, variant, ucb_c=2.0, seed=seed, device_memory=0.3, threads=8)
+        compare_with_oracle(e, o, *random_c4_root(np.random.default_rng(seed), plies, m, n), steps=steps)
+        assert o.u1_events > 0
