@@ -624,7 +624,6 @@ __device__ void expand_phase(const LoopArgs &g, StepLds &s, int tree, int wave, 
     const bool wants = kind == PUCT_SELECT_EXPAND && ticket_slot < n_legal;
     if (lane == 0) s.want[wave] = wants ? node : -1;
     __syncthreads();
-    if (FARM) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");   // the evaluators' priors of the step before (see search_kernel)
     const int other = lane < n_waves ? s.want[lane] : -1;
     const uint64_t all = __ballot(other >= 0), here = __ballot(other >= 0 && other == node);
     const int total = __popcll(all), before = __popcll(all & lanes_below(wave));
@@ -785,17 +784,14 @@ __global__ __launch_bounds__(kWave) void init_kernel(const LoopArgs g, const uin
     if (n_legal > 0) write_priors(g, tree, 0, board, lane, psyn_board_hash(psyn_tree_seed(g.seed, tree), board), n_legal);
 }
 
-// Makes the stores of a phase visible to the loads of the next one.  All wavefronts of a tree run on one CU and share
-// its write-through L1 and the L2 behind it, so no L2 write-back is needed; what is needed is (1) that every
-// wavefront's stores of the phase have been acknowledged by the L2 before any wavefront goes on -- a workgroup-scope
-// release fence does not wait for that on one CU (it lowers to no vector-memory wait) -- hence the explicit wait on the
-// wavefront's own outstanding vector memory operations; and (2) that the L1 drops the lines which other wavefronts have
-// changed underneath it: the agent-scope acquire.
-__device__ __forceinline__ void phase_barrier() {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+// Makes the stores of a phase visible to the loads of the next one.  All wavefronts of a tree run on one CU and share its
+// L1, which takes their loads and stores in order, so among themselves a workgroup barrier is all they need; nothing is
+// invalidated.  (An agent-scope acquire in every wavefront here made the CU's next load wait for sixteen invalidations:
+// 1.1 us instead of 0.15, twice a step.)  What other workgroups are told of next must also have been acknowledged by the L2
+// that they read, which a workgroup-scope release does not wait for.
+__device__ __forceinline__ void phase_barrier(bool for_evaluators) {
+    if (for_evaluators) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
 // What the traversals of a step ended with, between the launches of the stepwise mode and for the host to read.
@@ -1019,12 +1015,15 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
         if (farm) {
             // A node created in the step before can be expanded now at the earliest (selection hands out tickets without
             // looking at a node's priors), so this is where its priors must be there, not a step's length earlier.
+            // Selection has read rows of such nodes while they were being written: the L1 drops what it holds.  The first
+            // wavefront's acquire does that for all of them, which read no evaluator's work before expand_phase's barrier.
             if (threadIdx.x == 0) wait_for_evaluators(rq, s);
+            if (wave == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             expand_phase<true>(g, s, tree, wave, lane, n_waves, work.created);
         } else {
             expand_phase<false>(g, s, tree, wave, lane, n_waves, work.created);
         }
-        phase_barrier();   // the claims of the selection and the new nodes are in memory
+        phase_barrier(farm);   // the claims of the selection and the new nodes are in memory
         if (s.gave_up) break;
         if (farm && threadIdx.x == 0) {   // ... and the evaluators may start on this step's nodes
             rq.n = s.requests;
@@ -1042,7 +1041,7 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
         }
         if (wave == 0) t2 = wall_clock64();
         backup_phase(g, s, paths, tree, wave, lane, n_waves);
-        phase_barrier();
+        phase_barrier(false);
         if (wave == 0) {
             const uint64_t t3 = wall_clock64();
             work.ticks[0] += t1 - t0;
