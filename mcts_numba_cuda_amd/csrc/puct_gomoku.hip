@@ -39,6 +39,7 @@ constexpr int kTurnBit = 0x10000;
 
 constexpr int kTrav = kMaxWavesPerBlock;   // most traversals per tree: one wavefront each, one workgroup per tree
 constexpr int kSlices = kEdges / kWave;    // 64-edge slices of the widest node
+constexpr int kRow = 16;                   // lanes of a DPP row
 constexpr int kTally = 12;
 
 struct LoopArgs {
@@ -90,7 +91,7 @@ struct StepLds {
     int requested;       // ... and of all steps so far
     int gave_up;
     uint32_t board[kTrav][kBoardWords];
-    int stage[kTrav][kWave];   // per wavefront: edges on their way from four per lane to one per lane
+    alignas(16) int stage[kTrav][5 * kRow];   // per wavefront: edges on their way from four per lane to one per lane
 };
 
 __device__ __forceinline__ int pack_sel(int kind, int node, int slot) {
@@ -399,6 +400,90 @@ __device__ __forceinline__ void decide_in_turn(const LoopArgs &g, StepLds &s, in
     }
 }
 
+__device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {   // over the 16 lanes of each row
+    auto step = [](uint32_t x, auto ctrl) {
+        const uint32_t o = (uint32_t)dpp<decltype(ctrl)::value>((int)x);
+        return o > x ? o : x;
+    };
+    v = step(v, std::integral_constant<int, 0xB1>{});
+    v = step(v, std::integral_constant<int, 0x4E>{});
+    v = step(v, std::integral_constant<int, 0x141>{});
+    return step(v, std::integral_constant<int, 0x140>{});
+}
+
+// decide_in_turn for at most 16 edges, one per lane from lane 0 on, all of which lead to a node and have a finite score.  A
+// decision is a chain of dependent instructions on a lone wavefront, 0.5 us by decide_in_turn, most of it not the score:
+// here the maximum stays within a row of 16 lanes, the outcome is one register of the traversal's lane, and what the
+// traversals leave behind is written once, for all of them.  `single`: there is one edge to take.
+template <bool TICKETS>
+__device__ __forceinline__ void row_decisions(const EdgeSet<1> &e, uint64_t edges, uint32_t members, int lane, int expanded, float sqrt_lane, int allowed_lane,
+                                              bool single, int &tickets, uint32_t &with_ticket, int &den, int &mine) {
+    // (an empty lane's score is below every other, and finite)
+    const bool edge = e.eid[0] >= 0;
+    const float q = edge ? e.q[0] : -FLT_MAX, cp = edge ? e.cp[0] : 0.0f;
+    int claimed = 0;
+    uint32_t rest = members;
+    do {
+        const uint32_t bit = rest & (0u - rest);
+        rest ^= bit;
+        if (TICKETS && expanded + tickets < __builtin_amdgcn_readlane(allowed_lane, claimed)) {
+            with_ticket |= bit;
+            tickets += 1;
+        } else {
+            uint64_t first = 1ull;
+            if (!single) {
+                const float sqrt_parent = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), claimed));
+                const uint32_t b = __float_as_uint((q + cp * sqrt_parent / (float)den) + 0.0f);   // -0.0f counts as +0.0f
+                const uint32_t image = b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);           // score_image of a finite score
+                const uint32_t top = row_max_u32(image);
+                first = __builtin_amdgcn_uicmp(image, top, 32 /* == */) & edges;
+                if ((first & (first - 1)) != 0) {   // the rotated edge index decides, as in candidate_key
+                    int tie_offset = __builtin_ctz(bit);
+                    if (tie_offset >= expanded) tie_offset %= expanded;
+                    const int turned = e.eid[0] - tie_offset + (e.eid[0] < tie_offset ? expanded : 0);
+                    const uint32_t key = __builtin_amdgcn_inverse_ballot_w64(first) ? 0x10000u - (uint32_t)turned : 0u;
+                    const uint32_t top_key = row_max_u32(key);
+                    first &= __builtin_amdgcn_uicmp(key, top_key, 32);
+                }
+            }
+            den += __builtin_amdgcn_inverse_ballot_w64(first) ? 1 : 0;
+            mine = __builtin_amdgcn_inverse_ballot_w64(bit) ? __builtin_ctzll(first) : mine;
+            claimed += 1;
+        }
+    } while (rest != 0);
+}
+__device__ __forceinline__ void decide_in_row(const LoopArgs &g, StepLds &s, int *paths, int *next, Edge *row, const EdgeSet<1> &e, int node,
+                                              uint32_t members, int depth, int lane, int expanded, int legal, int total, int &tickets, bool single) {
+    const bool widening = expanded != 1 || g.c_pw != 0.0f;
+    const int eff_lane = widening ? (total + lane > 1 ? total + lane : 1) : 1;
+    const float sqrt_lane = widening ? sqrtf((float)eff_lane) : 1.0f;
+    const int allowed_lane = widening ? allowed_children(g.c_pw, g.alpha_pw, eff_lane, sqrt_lane, legal) : 1;
+    const int tickets_before = tickets;
+    int den = e.den[0], mine = -1;   // mine: lane of the edge that this lane's traversal takes
+    uint32_t with_ticket = 0;
+    const uint64_t edges = __ballot(e.eid[0] >= 0);
+    // (the limit grows with the claims: its largest value is the last one's)
+    if (expanded + tickets < __builtin_amdgcn_readlane(allowed_lane, __builtin_popcount(members) - 1))
+        row_decisions<true>(e, edges, members, lane, expanded, sqrt_lane, allowed_lane, single, tickets, with_ticket, den, mine);
+    else
+        row_decisions<false>(e, edges, members, lane, expanded, sqrt_lane, allowed_lane, single, tickets, with_ticket, den, mine);
+    const int from = (mine < 0 ? 0 : mine) << 2;
+    const int child = (int)((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)e.link[0]) >> 8);
+    const int eid = __builtin_amdgcn_ds_bpermute(from, e.eid[0]);
+    if (lane < kTrav && ((members >> lane) & 1u)) {
+        if ((with_ticket >> lane) & 1u) {
+            s.sel[lane] = pack_sel(PUCT_SELECT_EXPAND, node, expanded + tickets_before + __builtin_popcount(with_ticket & ((1u << lane) - 1u)));
+            s.len[lane] = depth + 1;
+            s.claims[lane] = depth;
+            next[lane] = -1;
+        } else {
+            paths[lane * g.path_depth + depth] = (node << 8) | eid;
+            next[lane] = child;
+        }
+    }
+    if (e.eid[0] >= 0 && den != e.den[0]) row[e.eid[0]].link = e.link[0] + (uint32_t)(den - e.den[0]);
+}
+
 // The traversals of a tree descend in lockstep, one level per round.  The traversals that stand on the same node are
 // served by one wavefront (that of the first of them), which loads the node's edges once and lets the traversals decide
 // one after another, wid ascending, on registers: every decision is the reference's (progressive widening, expansion
@@ -472,94 +557,127 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
         return allowed_children(g.c_pw, g.alpha_pw, eff_last, sqrtf((float)eff_last), legal) <= expanded;
     };
 
-    if (expanded <= kWave) {
-        bool taken = false;
-        if (n_members >= 3 && no_ticket_for_anyone()) {
-            // one edge per lane: which of them can come first for any of these traversals (the bounds of the wide case below)
-            uint64_t in = 1ull;   // (a node's only edge is taken whatever its score)
-            if (expanded > 1) {
-                const int now = total > 1 ? total : 1, then = total + n_members > 1 ? total + n_members : 1;
-                const uint32_t l = all.eid[0] >= 0 ? score_image(edge_score(all, 0, sqrtf((float)now), n_members)) : 0u;
-                const uint32_t h = all.eid[0] >= 0 ? score_image(edge_score(all, 0, sqrtf((float)then), 0)) : 0u;
-                const uint32_t low = wave_max_u32(l);
-                in = __ballot(low != 0 && h >= low && h != 0);
+    // decide_in_row's terms: every edge leads to a node and has a finite score
+    const auto fit_for_row = [&](const EdgeSet<1> &e) {
+        const int child = (int)(e.link[0] >> 8);
+        return __ballot(e.eid[0] >= 0 && !(child > 0 && child < g.max_nodes && fabsf(e.q[0]) < 1e30f && fabsf(e.cp[0]) < 1e30f && e.den[0] > 0)) == 0;
+    };
+    // Several traversals on a node with many edges: most edges cannot come first for any of them.  While these
+    // traversals decide, sqrt(parent) only grows (by their own claims) and an edge's claims only grow, and every
+    // operation of the score is monotonic, so an edge's score stays below its score at the largest sqrt(parent) and
+    // its present claims, and the best edge's score stays above the largest score at the present sqrt(parent) with
+    // all of these traversals' claims on it.  Edges whose upper bound is below that lower bound are out; when at
+    // most 64 remain they move to one edge per lane, and a decision costs one division instead of one per 64 edges.
+    // Returns false if nothing has been decided.
+    const auto decide_among_the_best = [&](auto slices) -> bool {
+        constexpr int NS = decltype(slices)::value;
+        const int now = total > 1 ? total : 1, then = total + n_members > 1 ? total + n_members : 1;
+        const float sqrt_now = sqrtf((float)now), sqrt_then = sqrtf((float)then);
+        uint32_t low = 0, high[NS];
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const uint32_t l = all.eid[i] >= 0 ? score_image(edge_score(all, i, sqrt_now, n_members)) : 0u;
+            high[i] = all.eid[i] >= 0 ? score_image(edge_score(all, i, sqrt_then, 0)) : 0u;
+            low = l > low ? l : low;
+        }
+        low = wave_max_u32(low);
+        if (low == 0) return false;
+        int kept = 0, place[NS];
+        uint64_t in_slice[NS];
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const uint64_t mask = __ballot(high[i] >= low);
+            in_slice[i] = mask;
+            place[i] = ((mask >> lane) & 1ull) ? kept + __popcll(mask & lanes_below(lane)) : -1;
+            kept += __popcll(mask);
+        }
+        // One edge left and no expansion ticket to be had: every one of these traversals takes that edge.
+        if (kept == 1 && no_ticket_for_anyone()) {
+#pragma unroll
+            for (int i = 0; i < NS; ++i)
+                if (in_slice[i] != 0) {
+                    const int at = __builtin_ctzll(in_slice[i]);
+                    take_all((uint32_t)__builtin_amdgcn_readlane((int)all.link[i], at), at + i * kWave);
+                }
+            return true;
+        }
+        int *stage = s.stage[wave];
+        EdgeSet<1> few{{0.0f}, {0.0f}, {1}, {0u}, {0u}, {-1}};
+        if (kept <= kRow) {   // through LDS into the first row, in one go
+#pragma unroll
+            for (int i = 0; i < NS; ++i)
+                if (place[i] >= 0) {
+                    *reinterpret_cast<int4 *>(stage + 4 * place[i]) = make_int4(__float_as_int(all.q[i]), __float_as_int(all.cp[i]), all.den[i], (int)all.link[i]);
+                    stage[4 * kRow + place[i]] = all.eid[i];
+                }
+            wave_lds_fence();
+            if (lane < kept) {
+                const int4 v = *reinterpret_cast<const int4 *>(stage + 4 * lane);
+                few = EdgeSet<1>{{__int_as_float(v.x)}, {__int_as_float(v.y)}, {v.z}, {(uint32_t)v.w}, {(uint32_t)v.w}, {stage[4 * kRow + lane]}};
             }
-            if (__popcll(in) == 1) {
-                const int at = __builtin_ctzll(in);
-                take_all((uint32_t)__builtin_amdgcn_readlane((int)all.link[0], at), at);
-                taken = true;
+            wave_lds_fence();
+            if (fit_for_row(few)) {
+                decide_in_row(g, s, paths, next, row, few, node, (uint32_t)members, depth, lane, expanded, legal, total, tickets, kept == 1);
+                return true;
+            }
+        } else {
+            if (NS == 1 || kept > kWave) return false;
+#pragma unroll
+            for (int f = 0; f < 5; ++f) {
+#pragma unroll
+                for (int i = 0; i < NS; ++i)
+                    if (place[i] >= 0)
+                        stage[place[i]] = f == 0 ? __float_as_int(all.q[i]) : f == 1 ? __float_as_int(all.cp[i]) : f == 2 ? all.den[i]
+                                        : f == 3 ? (int)all.link[i] : all.eid[i];
+                wave_lds_fence();
+                const int v = lane < kept ? stage[lane] : 0;
+                wave_lds_fence();
+                if (f == 0) few.q[0] = __int_as_float(v);
+                if (f == 1) few.cp[0] = __int_as_float(v);
+                if (f == 2) few.den[0] = lane < kept ? v : 1;
+                if (f == 3) few.link[0] = few.link_loaded[0] = (uint32_t)v;
+                if (f == 4) few.eid[0] = lane < kept ? v : -1;
             }
         }
-        if (!taken) {
-            EdgeSet<1> one{{all.q[0]}, {all.cp[0]}, {all.den[0]}, {all.link[0]}, {all.link_loaded[0]}, {all.eid[0]}};
+        decide_in_turn<1>(g, s, paths, next, few, node, members, depth, lane, expanded, legal, total, tickets, kept == 1);
+        if (few.eid[0] >= 0 && few.link[0] != few.link_loaded[0]) row[few.eid[0]].link = few.link[0];
+        return true;
+    };
+
+    EdgeSet<1> one{{all.q[0]}, {all.cp[0]}, {all.den[0]}, {all.link[0]}, {all.link_loaded[0]}, {all.eid[0]}};
+    const int allowed_now = expanded == 0 ? allowed_children(g.c_pw, g.alpha_pw, total > 1 ? total : 1, sqrtf((float)(total > 1 ? total : 1)), legal) : 0;
+    if (allowed_now > 0) {
+        // No edge to claim, so the widening limit stays as it is: the first of these traversals get the tickets that are
+        // left, the others find the node's children being created.
+        if (lane < kTrav && ((members >> lane) & 1ull)) {
+            const int slot = tickets + __popcll(members & lanes_below(lane));
+            const bool with_ticket = slot < allowed_now;
+            s.sel[lane] = with_ticket ? pack_sel(PUCT_SELECT_EXPAND, node, slot) : pack_sel(PUCT_SELECT_BUSY, node, 0);
+            s.len[lane] = with_ticket ? depth + 1 : 0;
+            s.claims[lane] = depth;
+            next[lane] = -1;
+        }
+        const int left = allowed_now - tickets > 0 ? allowed_now - tickets : 0;
+        tickets += n_members < left ? n_members : left;
+    } else {
+        bool decided = false;
+        if (n_members >= 3) {
+            if (expanded > kWave) {
+                decided = decide_among_the_best(std::integral_constant<int, kSlices>{});
+            } else if (expanded > 1) {
+                decided = decide_among_the_best(std::integral_constant<int, 1>{});
+            } else if (no_ticket_for_anyone()) {   // a node's only edge is taken whatever its score
+                take_all((uint32_t)__builtin_amdgcn_readlane((int)all.link[0], 0), 0);
+                decided = true;
+            }
+        }
+        if (decided) {
+        } else if (expanded >= 1 && expanded <= kRow && fit_for_row(one)) {
+            decide_in_row(g, s, paths, next, row, one, node, (uint32_t)members, depth, lane, expanded, legal, total, tickets, expanded == 1);
+        } else if (expanded <= kWave) {
             decide_in_turn<1>(g, s, paths, next, one, node, members, depth, lane, expanded, legal, total, tickets);
             if (one.link[0] != one.link_loaded[0]) row[lane].link = one.link[0];
-        }
-    } else {
-        // A wide node with several traversals on it: most edges cannot come first for any of them.  While these
-        // traversals decide, sqrt(parent) only grows (by their own claims) and an edge's claims only grow, and every
-        // operation of the score is monotonic, so an edge's score stays below its score at the largest sqrt(parent) and
-        // its present claims, and the best edge's score stays above the largest score at the present sqrt(parent) with
-        // all of these traversals' claims on it.  Edges whose upper bound is below that lower bound are out; when at
-        // most 64 remain they move to one edge per lane and a decision costs one division instead of four.
-        bool pruned = false;
-        if (n_members >= 3) {
-            const int now = total > 1 ? total : 1, then = total + n_members > 1 ? total + n_members : 1;
-            const float sqrt_now = sqrtf((float)now), sqrt_then = sqrtf((float)then);
-            uint32_t low = 0, high[kSlices];
-#pragma unroll
-            for (int i = 0; i < kSlices; ++i) {
-                const uint32_t l = all.eid[i] >= 0 ? score_image(edge_score(all, i, sqrt_now, n_members)) : 0u;
-                high[i] = all.eid[i] >= 0 ? score_image(edge_score(all, i, sqrt_then, 0)) : 0u;
-                low = l > low ? l : low;
-            }
-            low = wave_max_u32(low);
-            int kept = 0, place[kSlices];
-            uint64_t in_slice[kSlices];
-#pragma unroll
-            for (int i = 0; i < kSlices; ++i) {
-                const bool in = low != 0 && high[i] >= low && high[i] != 0;
-                const uint64_t mask = __ballot(in);
-                in_slice[i] = mask;
-                place[i] = in ? kept + __popcll(mask & lanes_below(lane)) : -1;
-                kept += __popcll(mask);
-            }
-            // One edge left and no expansion ticket to be had: every one of these traversals takes that edge.
-            if (kept == 1 && low != 0 && no_ticket_for_anyone()) {
-                pruned = true;
-#pragma unroll
-                for (int i = 0; i < kSlices; ++i)
-                    if (in_slice[i] != 0) {
-                        const int at = __builtin_ctzll(in_slice[i]);
-                        take_all((uint32_t)__builtin_amdgcn_readlane((int)all.link[i], at), at + i * kWave);
-                    }
-            }
-            if (!pruned && kept >= 1 && kept <= kWave && low != 0) {
-                pruned = true;
-                // through LDS into one edge per lane
-                EdgeSet<1> few{{0.0f}, {0.0f}, {1}, {0u}, {0u}, {-1}};
-                int *stage = s.stage[wave];
-#pragma unroll
-                for (int f = 0; f < 5; ++f) {
-#pragma unroll
-                    for (int i = 0; i < kSlices; ++i)
-                        if (place[i] >= 0)
-                            stage[place[i]] = f == 0 ? __float_as_int(all.q[i]) : f == 1 ? __float_as_int(all.cp[i]) : f == 2 ? all.den[i]
-                                            : f == 3 ? (int)all.link[i] : all.eid[i];
-                    wave_lds_fence();
-                    const int v = lane < kept ? stage[lane] : 0;
-                    wave_lds_fence();
-                    if (f == 0) few.q[0] = __int_as_float(v);
-                    if (f == 1) few.cp[0] = __int_as_float(v);
-                    if (f == 2) few.den[0] = lane < kept ? v : 1;
-                    if (f == 3) few.link[0] = few.link_loaded[0] = (uint32_t)v;
-                    if (f == 4) few.eid[0] = lane < kept ? v : -1;
-                }
-                decide_in_turn<1>(g, s, paths, next, few, node, members, depth, lane, expanded, legal, total, tickets, kept == 1);
-                if (few.eid[0] >= 0 && few.link[0] != few.link_loaded[0]) row[few.eid[0]].link = few.link[0];
-            }
-        }
-        if (!pruned) {
+        } else {
             decide_in_turn<kSlices>(g, s, paths, next, all, node, members, depth, lane, expanded, legal, total, tickets);
 #pragma unroll
             for (int i = 0; i < kSlices; ++i)
