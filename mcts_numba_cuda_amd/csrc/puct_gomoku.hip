@@ -972,67 +972,93 @@ extern __shared__ int dynamic_lds[];
 // The priors of a new node are a pure function of its position, and nothing reads them before the next step's
 // selection, so they need not be worked out on the compute unit that owns the tree: the tree's workgroup posts the
 // step's new nodes, goes on with its backup, and picks the results up before the next step.  An evaluator workgroup
-// takes two nodes at a time, four wavefronts and one cell per lane each; the slot of a cell is the number of larger keys
-// among the node's 256, counted from LDS.  Same priors, bit for bit, as write_priors().
+// takes up to four nodes at a time, four wavefronts and one cell per lane each.  A wavefront sorts its 64 keys in registers;
+// the slot of a cell is its place there and the number of larger keys in the three other wavefronts' lists, each a binary
+// search in LDS.  Same priors, bit for bit, as write_priors().  Bound by vector instructions: about 700 a wavefront and
+// node, 1200 when every lane compared its key with all 256; four evaluators of 8 wavefronts then took longer over a step's
+// sixteen nodes than the tree's own step.
+constexpr int kEvalParts = kEdges / kWave;              // wavefronts per node
+constexpr int kEvalNodes = kTrav / kEvalParts;          // nodes at a time, at most
 struct EvalLds {
-    uint32_t keys[2][kEdges];
-    unsigned long long weight[2][4];
-    int legal[2][4];
+    uint32_t keys[kEvalNodes][kEvalParts][kWave];
+    unsigned long long weight[kEvalNodes][kEvalParts];
+    int legal[kEvalNodes][kEvalParts];
     int tag;
 };
+__device__ __forceinline__ int eval_nodes_at_once() { return (int)blockDim.x / (kWave * kEvalParts); }   // (2 to 4: 8 to 16 wavefronts)
+
+// The wavefront's 64 keys, largest first: a bitonic sort with one key per lane.
+template <int SIZE, int DIST>
+__device__ __forceinline__ void sort64_step(uint32_t &v, int lane) {
+    constexpr auto takes_larger = [] {
+        uint64_t m = 0;
+        for (int i = 0; i < kWave; ++i) m |= (uint64_t)(((i & DIST) == 0) == ((i & SIZE) == 0)) << i;
+        return m;
+    }();
+    const uint32_t p = from_lane_xor<DIST>(v, lane);
+    const uint32_t hi = v > p ? v : p, lo = v > p ? p : v;
+    v = __builtin_amdgcn_inverse_ballot_w64(takes_larger) ? hi : lo;
+    if constexpr (DIST > 1) sort64_step<SIZE, DIST / 2>(v, lane);
+}
+template <int SIZE = 2>
+__device__ __forceinline__ void sort64_descending(uint32_t &v, int lane) {
+    sort64_step<SIZE, SIZE / 2>(v, lane);
+    if constexpr (SIZE < kWave) sort64_descending<2 * SIZE>(v, lane);
+}
 
 __device__ __forceinline__ int poll_word(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// Entries `first` and `first + 1` of the step, by wavefronts 0..3 and 4..7 of the workgroup; all eight must call it.
-__device__ void evaluate_pair(const LoopArgs &g, EvalLds &L, int tree, int first, int n, int wave, int lane) {
+// Entry `index` of the step (none if it is not below n) by four wavefronts, `part` = 0..3; the whole workgroup must call it.
+__device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index, int n, int group, int part, int lane) {
     const EvalRequests &rq = g.requests[tree];
-    const int group = wave >> 2, part = wave & 3, index = first + group;
     const int child = index < n ? rq.child[index] : -1;
     const bool active = child > 0;
     const size_t trow = (size_t)tree * g.max_nodes;
-    const int cell = part * kWave + lane;
-    uint32_t weight_key = 0;
-    bool legal = false;
+    uint32_t key = 0;
     if (active) {
+        const int cell = part * kWave + lane;
         const uint32_t w = lane < kBoardWords ? g.board[(trow + child) * kBoardWords + lane] : 0u;
         // words of the lane's cell: the same for each half of the wavefront
         uint32_t plus = (uint32_t)__builtin_amdgcn_readlane((int)w, 2 * part), minus = (uint32_t)__builtin_amdgcn_readlane((int)w, 8 + 2 * part);
         const uint32_t plus_hi = (uint32_t)__builtin_amdgcn_readlane((int)w, 2 * part + 1);
         const uint32_t minus_hi = (uint32_t)__builtin_amdgcn_readlane((int)w, 8 + 2 * part + 1);
         if (lane >= 32) plus = plus_hi, minus = minus_hi;
-        legal = cell < g.cells && !(((plus | minus) >> (lane & 31)) & 1u);
-        const uint64_t key = psyn_cell_key(rq.hash[index], cell);
+        const bool legal = cell < g.cells && !(((plus | minus) >> (lane & 31)) & 1u);
+        const uint64_t stream = psyn_cell_key(rq.hash[index], cell);
         bool pending = legal;
         for (int round = 0; __ballot(pending) != 0; ++round) {
             float x;
-            const int ok = psyn_gamma_round(g.dirichlet_alpha, key, round, &x);
+            const int ok = psyn_gamma_round(g.dirichlet_alpha, stream, round, &x);
             if (pending && (ok || round == PSYN_GAMMA_ROUNDS - 1)) {
-                weight_key = psyn_weight_key(x, cell);
+                key = psyn_weight_key(x, cell);
                 pending = false;
             }
         }
-    }
-    L.keys[group][cell] = weight_key;
-    const uint64_t part_sum = wave_sum64(weight_key ? psyn_key_weight(weight_key) : 0);
-    const int part_legal = __popcll(__ballot(legal));
-    if (lane == 0) {
-        L.weight[group][part] = part_sum;
-        L.legal[group][part] = part_legal;
+        const uint64_t part_sum = wave_sum64(key ? psyn_key_weight(key) : 0);
+        const int part_legal = __popcll(__ballot(legal));
+        if (lane == 0) {
+            L.weight[group][part] = part_sum;
+            L.legal[group][part] = part_legal;
+        }
+        sort64_descending(key, lane);   // (0: not a legal cell, last)
+        L.keys[group][part][lane] = key;
     }
     __syncthreads();
-    if (legal) {
+    if (key != 0) {
         const uint64_t sum = L.weight[group][0] + L.weight[group][1] + L.weight[group][2] + L.weight[group][3];
         const int n_legal = L.legal[group][0] + L.legal[group][1] + L.legal[group][2] + L.legal[group][3];
-        int slot = 0;
-        const uint4 *keys = reinterpret_cast<const uint4 *>(L.keys[group]);
-#pragma unroll 8
-        for (int c = 0; c < kEdges / 4; ++c) {
-            const uint4 k = keys[c];
-            slot += (k.x > weight_key) + (k.y > weight_key) + (k.z > weight_key) + (k.w > weight_key);
-        }
+        int larger[kEvalParts - 1] = {};   // keys above this one in the other parts' lists
+        const auto list = [&](int i) -> const uint32_t * { return L.keys[group][(part + 1 + i) & (kEvalParts - 1)]; };
+#pragma unroll
+        for (int d = kWave / 2; d > 0; d >>= 1)
+#pragma unroll
+            for (int i = 0; i < kEvalParts - 1; ++i) larger[i] += list(i)[larger[i] + d - 1] > key ? d : 0;
+        int slot = lane;
+#pragma unroll
+        for (int i = 0; i < kEvalParts - 1; ++i) slot += larger[i] + (list(i)[larger[i]] > key ? 1 : 0);
         const size_t e = (trow + child) * kEdges + slot;
-        store_edge(g.edges + e, 0, 0.0f, psyn_prior(psyn_key_weight(weight_key), sum, n_legal), 0u);
-        g.action[e] = (uint8_t)cell;
+        store_edge(g.edges + e, 0, 0.0f, psyn_prior(psyn_key_weight(key), sum, n_legal), 0u);
+        g.action[e] = (uint8_t)(255u - (key & 0xFFu));
     }
     __syncthreads();   // the keys are free again
 }
@@ -1061,9 +1087,12 @@ __device__ void evaluator_loop(const LoopArgs &g, EvalLds &L, int tree, int help
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         const int n = rq.n;
         int worked_off = 0;
-        for (int first = 2 * helper; first < n; first += 2 * g.evaluators) {
-            evaluate_pair(g, L, tree, first, n, wave, lane);
-            worked_off += n - first >= 2 ? 2 : 1;
+        // (the step's nodes are dealt to the evaluators one by one, so that a step with few of them keeps all busy)
+        const int at_once = eval_nodes_at_once();
+        for (int first = helper; first < n; first += at_once * g.evaluators) {
+            const int group = wave / kEvalParts;
+            evaluate_node(g, L, tree, first + group * g.evaluators, n, group, wave & (kEvalParts - 1), lane);
+            for (int i = 0; i < at_once; ++i) worked_off += first + i * g.evaluators < n ? 1 : 0;
         }
         // every wavefront's stores have reached the L2 before one of them reports; the release pushes them on
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1108,7 +1137,7 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
     }
     if (tree >= trees) return;
     if (role > 0) {
-        if (wave >= 8) return;   // an evaluator workgroup works with eight wavefronts
+        if (wave >= kEvalParts * eval_nodes_at_once()) return;
         evaluator_loop(g, eval_lds, tree, role - 1, wave, lane);
         return;
     }
