@@ -568,8 +568,9 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
     // its present claims, and the best edge's score stays above the largest score at the present sqrt(parent) with
     // all of these traversals' claims on it.  Edges whose upper bound is below that lower bound are out; when at
     // most 64 remain they move to one edge per lane, and a decision costs one division instead of one per 64 edges.
-    // Returns false if nothing has been decided.
-    const auto decide_among_the_best = [&](auto slices) -> bool {
+    // Returns how many remain if they are in `few` now, 0 if they are not, -1 if all is decided.
+    EdgeSet<1> few{{0.0f}, {0.0f}, {1}, {0u}, {0u}, {-1}};
+    const auto keep_the_best = [&](auto slices) -> int {
         constexpr int NS = decltype(slices)::value;
         const int now = total > 1 ? total : 1, then = total + n_members > 1 ? total + n_members : 1;
         const float sqrt_now = sqrtf((float)now), sqrt_then = sqrtf((float)then);
@@ -581,7 +582,7 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
             low = l > low ? l : low;
         }
         low = wave_max_u32(low);
-        if (low == 0) return false;
+        if (low == 0) return 0;
         int kept = 0, place[NS];
         uint64_t in_slice[NS];
 #pragma unroll
@@ -599,10 +600,9 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
                     const int at = __builtin_ctzll(in_slice[i]);
                     take_all((uint32_t)__builtin_amdgcn_readlane((int)all.link[i], at), at + i * kWave);
                 }
-            return true;
+            return -1;
         }
         int *stage = s.stage[wave];
-        EdgeSet<1> few{{0.0f}, {0.0f}, {1}, {0u}, {0u}, {-1}};
         if (kept <= kRow) {   // through LDS into the first row, in one go
 #pragma unroll
             for (int i = 0; i < NS; ++i)
@@ -616,12 +616,8 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
                 few = EdgeSet<1>{{__int_as_float(v.x)}, {__int_as_float(v.y)}, {v.z}, {(uint32_t)v.w}, {(uint32_t)v.w}, {stage[4 * kRow + lane]}};
             }
             wave_lds_fence();
-            if (fit_for_row(few)) {
-                decide_in_row(g, s, paths, next, row, few, node, (uint32_t)members, depth, lane, expanded, legal, total, tickets, kept == 1);
-                return true;
-            }
         } else {
-            if (NS == 1 || kept > kWave) return false;
+            if (NS == 1 || kept > kWave) return 0;
 #pragma unroll
             for (int f = 0; f < 5; ++f) {
 #pragma unroll
@@ -639,12 +635,9 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
                 if (f == 4) few.eid[0] = lane < kept ? v : -1;
             }
         }
-        decide_in_turn<1>(g, s, paths, next, few, node, members, depth, lane, expanded, legal, total, tickets, kept == 1);
-        if (few.eid[0] >= 0 && few.link[0] != few.link_loaded[0]) row[few.eid[0]].link = few.link[0];
-        return true;
+        return kept;
     };
 
-    EdgeSet<1> one{{all.q[0]}, {all.cp[0]}, {all.den[0]}, {all.link[0]}, {all.link_loaded[0]}, {all.eid[0]}};
     const int allowed_now = expanded == 0 ? allowed_children(g.c_pw, g.alpha_pw, total > 1 ? total : 1, sqrtf((float)(total > 1 ? total : 1)), legal) : 0;
     if (allowed_now > 0) {
         // No edge to claim, so the widening limit stays as it is: the first of these traversals get the tickets that are
@@ -660,24 +653,28 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
         const int left = allowed_now - tickets > 0 ? allowed_now - tickets : 0;
         tickets += n_members < left ? n_members : left;
     } else {
-        bool decided = false;
+        int edges = 0;   // how many there are in `few`, one per lane
         if (n_members >= 3) {
             if (expanded > kWave) {
-                decided = decide_among_the_best(std::integral_constant<int, kSlices>{});
+                edges = keep_the_best(std::integral_constant<int, kSlices>{});
             } else if (expanded > 1) {
-                decided = decide_among_the_best(std::integral_constant<int, 1>{});
+                edges = keep_the_best(std::integral_constant<int, 1>{});
             } else if (no_ticket_for_anyone()) {   // a node's only edge is taken whatever its score
                 take_all((uint32_t)__builtin_amdgcn_readlane((int)all.link[0], 0), 0);
-                decided = true;
+                edges = -1;
             }
         }
-        if (decided) {
-        } else if (expanded >= 1 && expanded <= kRow && fit_for_row(one)) {
-            decide_in_row(g, s, paths, next, row, one, node, (uint32_t)members, depth, lane, expanded, legal, total, tickets, expanded == 1);
-        } else if (expanded <= kWave) {
-            decide_in_turn<1>(g, s, paths, next, one, node, members, depth, lane, expanded, legal, total, tickets);
-            if (one.link[0] != one.link_loaded[0]) row[lane].link = one.link[0];
-        } else {
+        const bool only_one = edges == 1;
+        if (edges == 0 && expanded <= kWave) {
+            few = EdgeSet<1>{{all.q[0]}, {all.cp[0]}, {all.den[0]}, {all.link[0]}, {all.link_loaded[0]}, {all.eid[0]}};
+            edges = expanded;
+        }
+        if (edges >= 1 && edges <= kRow && fit_for_row(few)) {
+            decide_in_row(g, s, paths, next, row, few, node, (uint32_t)members, depth, lane, expanded, legal, total, tickets, edges == 1);
+        } else if (edges > 0 || expanded == 0) {
+            decide_in_turn<1>(g, s, paths, next, few, node, members, depth, lane, expanded, legal, total, tickets, only_one);
+            if (few.eid[0] >= 0 && few.link[0] != few.link_loaded[0]) row[few.eid[0]].link = few.link[0];
+        } else if (edges == 0) {
             decide_in_turn<kSlices>(g, s, paths, next, all, node, members, depth, lane, expanded, legal, total, tickets);
 #pragma unroll
             for (int i = 0; i < kSlices; ++i)
@@ -1123,6 +1120,8 @@ __device__ void wait_for_evaluators(EvalRequests &rq, StepLds &s) {
 // The whole search in one launch.  evaluators == 0: one workgroup per tree (grid = trees).  Otherwise every tree has
 // 1 + evaluators workgroups; those of one tree have the same blockIdx.x % 8, which is how workgroups are dealt to the
 // eight XCDs, so a tree's requests and results meet in one L2.
+// (FARM: with evaluators; two kernels because their code is 60 KB, the instruction cache of two CUs 64.)
+template <bool FARM>
 __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, int trees) {
     __shared__ StepLds s;
     __shared__ EvalLds eval_lds;
@@ -1130,19 +1129,19 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), n_waves = g.traversals;
     int tree = blockIdx.x, role = 0;
-    if (g.evaluators > 0) {
+    if (FARM) {
         const int per_tree = 1 + g.evaluators, nth = blockIdx.x / 8;
         tree = (int)(blockIdx.x % 8) + 8 * (nth / per_tree);
         role = nth % per_tree;
     }
     if (tree >= trees) return;
-    if (role > 0) {
+    if (FARM && role > 0) {
         if (wave >= kEvalParts * eval_nodes_at_once()) return;
         evaluator_loop(g, eval_lds, tree, role - 1, wave, lane);
         return;
     }
     if (wave >= n_waves) return;   // the launch's workgroups are as large as the larger of the two kinds needs
-    const bool farm = g.evaluators > 0;
+    constexpr bool farm = FARM;
     EvalRequests &rq = g.requests[tree];
     Work work;
     if (threadIdx.x == 0) {
@@ -1166,10 +1165,8 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
             // wavefront's acquire does that for all of them, which read no evaluator's work before expand_phase's barrier.
             if (threadIdx.x == 0) wait_for_evaluators(rq, s);
             if (wave == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            expand_phase<true>(g, s, tree, wave, lane, n_waves, work.created);
-        } else {
-            expand_phase<false>(g, s, tree, wave, lane, n_waves, work.created);
         }
+        expand_phase<FARM>(g, s, tree, wave, lane, n_waves, work.created);
         phase_barrier(farm);   // the claims of the selection and the new nodes are in memory
         if (s.gave_up) break;
         if (farm && threadIdx.x == 0) {   // ... and the evaluators may start on this step's nodes
@@ -1424,14 +1421,15 @@ extern "C" int puct_gomoku_run(puct_gomoku_engine *e, const int8_t *board, int32
             // resident: as many evaluators per tree as the device takes at once, none if it comes to that.
             int waves = c.traversals, per_cu = 0;
             if (g.evaluators > 0 && waves < 8) waves = 8;
-            hipDeviceProp_t prop;
-            HIP_TRY(hipGetDeviceProperties(&prop, c.device));
-            HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, search_kernel, waves * kWave, lds));
-            const long resident = (long)per_cu * prop.multiProcessorCount, groups = 8L * ((c.trees + 7) / 8);
+            int cus = 0;
+            HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
+            HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, search_kernel<true>, waves * kWave, lds));
+            const long resident = (long)per_cu * cus, groups = 8L * ((c.trees + 7) / 8);
             while (g.evaluators > 0 && groups * (1 + g.evaluators) > resident) g.evaluators -= 1;
-            if (g.evaluators == 0) waves = c.traversals;
-            const dim3 all(g.evaluators > 0 ? (unsigned)(groups * (1 + g.evaluators)) : (unsigned)c.trees);
-            hipLaunchKernelGGL(search_kernel, all, dim3(waves * kWave), lds, s, g, (int)c.trees);
+            if (g.evaluators > 0)
+                hipLaunchKernelGGL(search_kernel<true>, dim3((unsigned)(groups * (1 + g.evaluators))), dim3(waves * kWave), lds, s, g, (int)c.trees);
+            else
+                hipLaunchKernelGGL(search_kernel<false>, grid, block, lds, s, g, (int)c.trees);
             HIP_TRY(hipGetLastError());
         }
     } else {
