@@ -78,6 +78,8 @@ static_assert(sizeof(EvalRequests::xcc) == sizeof(int) * (1 + kMaxEvaluators), "
 __device__ __forceinline__ int my_xcc() { return (int)(__builtin_amdgcn_s_getreg(6164) & 0xfu); }   // HW_REG_XCC_ID, bits 3:0
 constexpr unsigned long long kWaitTicks = 300000000ull;   // 3 s of the 100 MHz clock: a partner that is not there
 
+constexpr int kReachedNothing = 0, kReachedValued = 1 /* by s.value */, kReachedPosition = 2, kReachedChild = 3, kReachedWin = 4, kReachedDraw = 5;
+
 // What a step keeps per traversal between its phases.  The paths ([traversals][path_depth] words) follow in dynamic LDS.
 struct StepLds {
     int cur[2][kTrav];   // node every traversal stands on, -1 once it has ended; double buffered by level parity
@@ -86,6 +88,9 @@ struct StepLds {
     int claims[kTrav];   // edges the traversal holds a claim on = path entries written
     float value[kTrav];  // of the reached node, for the player who moved into it
     int want[kTrav];     // node the traversal expands, -1 if none
+    int4 reached[kTrav]; // what the expansion makes of the traversal: kReached..., and of a new child its node, its edge
+                         // (parent << 8 | slot) and its NodeInfo::legal_turn
+    unsigned long long hash[kTrav];   // of the position on `board`
     int node_count;
     int requests;        // evaluation requests of this step
     int requested;       // ... and of all steps so far
@@ -118,22 +123,13 @@ __device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOM
 __device__ __forceinline__ bool stone_at(const uint32_t *colour, int cell) { return (colour[cell >> 5] >> (cell & 31)) & 1u; }
 
 // Does the stone just placed at `cell` complete a row of exactly five (src/mctsnc_game_mechanics.py:181-280: a longer
-// row does not win)?  Lanes 0..3 each scan one direction; the result is uniform.
+// row does not win)?  Lane 16 d + 5 + k looks at the cell k steps along direction d; the result is uniform.
 __device__ __forceinline__ bool makes_five(const uint32_t *mine, int cell, int m, int n, int lane) {
-    bool hit = false;
-    if (lane < 4) {
-        const int dr = lane == 0 ? 0 : 1, dc = lane == 0 ? 1 : (lane == 1 ? 0 : (lane == 2 ? 1 : -1));
-        const int r0 = cell / n, c0 = cell % n;
-        int run = 1;
-        for (int s = -1; s <= 1; s += 2)
-            for (int k = 1; k < 6; ++k) {
-                const int r = r0 + s * k * dr, c = c0 + s * k * dc;
-                if (r < 0 || r >= m || c < 0 || c >= n || !stone_at(mine, r * n + c)) break;
-                ++run;
-            }
-        hit = run == 5;
-    }
-    return __ballot(hit) != 0;
+    const int d = lane >> 4, k = (lane & 15) - 5;
+    const int r = cell / n + (d == 0 ? 0 : k), c = cell % n + (d == 0 || d == 2 ? k : (d == 1 ? 0 : -k));
+    const uint64_t like = __ballot(k <= 5 && r >= 0 && r < m && c >= 0 && c < n && stone_at(mine, r * n + c));
+    const uint32_t line = (uint32_t)(like >> (16 * (lane & 3))) & 0x7FFu;   // bit 5: the stone itself
+    return __ballot(1 + __builtin_clz(~(line << 27)) + __builtin_ctz(~(line >> 6)) == 5) != 0;
 }
 
 // Bitonic sort of the wavefront's 256 keys, largest first: element e = 4 * lane + k lives in v[k] of `lane`.  Partners
@@ -743,54 +739,71 @@ __device__ void expand_phase(const LoopArgs &g, StepLds &s, int tree, int wave, 
     const uint64_t all = __ballot(other >= 0), here = __ballot(other >= 0 && other == node);
     const int total = __popcll(all), before = __popcll(all & lanes_below(wave));
     const int rank = __popcll(here & lanes_below(wave)), siblings = __popcll(here);
-    const int base = s.node_count;
+    const int base = s.node_count;   // (wave 0 counts on behind the next barrier)
     const bool fits = base + total <= g.max_nodes;
-    __syncthreads();
-    if (wave == 0 && lane == 0) {
-        if (fits) s.node_count = base + total;
-        s.requests = fits ? total : 0;
-    }
-    if (wave == 0 && fits) created += (uint32_t)total;
 
-    float u = 0.0f;   // value of the reached node for the player who moved into it
+    int reached = kReachedNothing, child = 0, child_turn = 0, edge = 0;
     if (wants && fits) {
-        const int child = base + before, slot = ni.expanded + rank;
-        const size_t erow = (trow + node) * kEdges;
-        const int action = g.action[erow + slot];
+        const int slot = ni.expanded + rank;
+        child = base + before;
+        edge = (node << 8) | slot;
+        const int action = g.action[(trow + node) * kEdges + slot];
         uint32_t *mine = board + (turn > 0 ? 0 : 8);
         if (lane == 0) mine[action >> 5] |= 1u << (action & 31);
         wave_lds_fence();
-        const bool win = makes_five(mine, action, g.m, g.n, lane);
-        const int child_legal = n_legal - 1;
-        const bool terminal = win || child_legal == 0;
-        const uint64_t bh = psyn_board_hash(tree_seed, board);
-        const float v_child = win ? -1.0f : (terminal ? 0.0f : psyn_value(bh));
+        child_turn = (n_legal - 1) | (turn > 0 ? kTurnBit : 0);
+        reached = makes_five(mine, action, g.m, g.n, lane) ? kReachedWin : n_legal == 1 ? kReachedDraw : kReachedChild;
         if (lane < kBoardWords) g.board[(trow + child) * kBoardWords + lane] = board[lane];
-        if (lane == 0) {
-            *reinterpret_cast<uint4 *>(g.info + trow + child) =
-                make_uint4((uint32_t)(terminal ? PUCT_NODE_EXPANDED_TERMINAL : 0), 0u,
-                           (uint32_t)(child_legal | (turn > 0 ? kTurnBit : 0)), __float_as_uint(v_child));
-            Edge *e = g.edges + erow + slot;
-            e->n = 1;
-            e->w = -v_child;
-            e->link = (uint32_t)child << 8;
-            if (rank == 0) g.info[trow + node].expanded = ni.expanded + siblings;
-        }
-        if (FARM) {   // the child's priors are an evaluator workgroup's work
-            if (lane == 0) {
-                g.requests[tree].child[before] = terminal ? -1 : child;
-                g.requests[tree].hash[before] = bh;
-            }
-        } else if (!terminal) {
-            write_priors(g, tree, child, board, lane, bh, child_legal);
-        }
-        u = -v_child;
+        if (lane == 0 && rank == 0) g.info[trow + node].expanded = ni.expanded + siblings;
     } else if (kind == PUCT_SELECT_TERMINAL) {
-        u = ni.value;
+        reached = kReachedValued;
     } else if (has_node) {
-        u = psyn_value(psyn_board_hash(tree_seed, board));
+        reached = kReachedPosition;
     }
-    if (lane == 0) s.value[wave] = u;
+    if (lane == 0) {
+        s.reached[wave] = make_int4(reached, child, edge, child_turn);
+        s.value[wave] = ni.value;
+    }
+    __syncthreads();
+    // A position's hash is a chain of twenty 64-bit products, at a quarter of the rate whatever the number of lanes: one
+    // wavefront works out all of them, a traversal per lane, instead of each its own (four wavefronts on a SIMD: 2 us).
+    if (wave == 0) {
+        if (lane == 0) {
+            if (fits) s.node_count = base + total;
+            s.requests = fits ? total : 0;
+        }
+        if (fits) created += (uint32_t)total;
+        if (lane < n_waves) {
+            const int4 r = s.reached[lane];
+            float u = 0.0f;   // value of the reached node for the player who moved into it
+            if (r.x == kReachedValued) u = s.value[lane];
+            if (r.x >= kReachedPosition) {
+                const uint64_t bh = psyn_board_hash(tree_seed, s.board[lane]);
+                s.hash[lane] = bh;
+                const bool terminal = r.x == kReachedWin || r.x == kReachedDraw;
+                const float v = r.x == kReachedWin ? -1.0f : (terminal ? 0.0f : psyn_value(bh));
+                u = v;
+                if (r.x != kReachedPosition) {
+                    *reinterpret_cast<uint4 *>(g.info + trow + r.y) =
+                        make_uint4((uint32_t)(terminal ? PUCT_NODE_EXPANDED_TERMINAL : 0), 0u, (uint32_t)r.w, __float_as_uint(v));
+                    Edge *e = g.edges + (trow + (r.z >> 8)) * kEdges + (r.z & 0xFF);
+                    e->n = 1;
+                    e->w = -v;
+                    e->link = (uint32_t)r.y << 8;
+                    u = -v;
+                    if (FARM) {   // the child's priors are an evaluator workgroup's work
+                        g.requests[tree].child[r.y - base] = terminal ? -1 : r.y;
+                        g.requests[tree].hash[r.y - base] = bh;
+                    }
+                }
+            }
+            s.value[lane] = u;
+        }
+    }
+    if (!FARM) {
+        __syncthreads();
+        if (reached == kReachedChild) write_priors(g, tree, child, board, lane, s.hash[wave], n_legal - 1);
+    }
 }
 
 // ---- backup ----------------------------------------------------------------------------------------------------------
