@@ -548,7 +548,7 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
     // the claims, and its largest value, the one the last of them sees, does not exceed the children there are.
     const auto no_ticket_for_anyone = [&] {
         if (expanded < 1) return false;
-        if (expanded == 1 && g.c_pw == 0.0f) return true;
+        if (expanded >= legal || (expanded == 1 && g.c_pw == 0.0f)) return true;   // (the limit does not exceed the legal moves)
         const int eff_last = total + n_members - 1 > 1 ? total + n_members - 1 : 1;
         return allowed_children(g.c_pw, g.alpha_pw, eff_last, sqrtf((float)eff_last), legal) <= expanded;
     };
@@ -811,69 +811,56 @@ __device__ void expand_phase(const LoopArgs &g, StepLds &s, int tree, int wave, 
 // leaves a visit and the node's value, sign alternating, on every edge of the path (src/puct/puct_gpu_v2.py:847-927
 // moved to edge-level virtual loss), and an expansion returns its ticket.  Lane = (traversal, one of four depths): the
 // traversals whose paths share an edge at that depth meet inside a row of 16 lanes, and the last of them stores the
-// edge after adding the values in traversal order, so the float sums do not depend on timing.
+// edge after adding the values in traversal order, so the float sums do not depend on timing.  A step's paths are a few
+// levels, so this is one pass of one wavefront, as long as its chain of instructions: what the others of a row hold comes by
+// DPP broadcasts (by 48 LDS permutes it took 1.2 us longer), and the tickets go back by the last wavefront meanwhile.
+template <int J>
+__device__ __forceinline__ void meet_in_row(int enc, uint32_t &same) {   // bit j: traversal j of the row stands on this lane's edge
+    same |= dpp<0x150 + J>(enc) == enc ? 1u << J : 0u;                     // row_newbcast:J
+    if constexpr (J + 1 < kTrav) meet_in_row<J + 1>(enc, same);
+}
+template <int J>
+__device__ __forceinline__ void add_in_order(float val, uint32_t which, float &acc) {
+    const float with = acc + __int_as_float(dpp<0x150 + J>(__float_as_int(val)));
+    acc = (which >> J) & 1u ? with : acc;
+    if constexpr (J + 1 < kTrav) add_in_order<J + 1>(val, which, acc);
+}
 __device__ void backup_phase(const LoopArgs &g, StepLds &s, const int *paths, int tree, int wave, int lane, int n_waves) {
     const size_t trow = (size_t)tree * g.max_nodes;
     const int t = lane & (kTrav - 1), sub = lane >> 4;
     const int raw = s.sel[t], my_claims = s.claims[t];
     const int kind = (raw >> PUCT_GOMOKU_SEL_KIND_SHIFT) & 7;
-    const int counted = (kind == PUCT_SELECT_EXPAND || kind == PUCT_SELECT_TERMINAL || kind == PUCT_SELECT_DEPTH_LIMIT) ? 1 : 0;
+    const uint32_t counted = (uint32_t)__ballot(kind == PUCT_SELECT_EXPAND || kind == PUCT_SELECT_TERMINAL || kind == PUCT_SELECT_DEPTH_LIMIT) & 0xFFFFu;
     const float u = s.value[t];
-    int deepest = 0;
-    for (int j = 0; j < n_waves; ++j) deepest = s.claims[j] > deepest ? s.claims[j] : deepest;
+    const int deepest = __builtin_amdgcn_readfirstlane((int)row_max_u32((uint32_t)my_claims));
     for (int d0 = 4 * wave; d0 < deepest; d0 += 4 * n_waves) {
         const int d = d0 + sub;
         const int enc = d < my_claims ? paths[t * g.path_depth + d] : -1;
         const float val = ((my_claims - d) & 1) ? -u : u;   // a counted traversal's path has as many edges as claims
         Edge *e = nullptr;
-        int n_old = 0;
-        float acc = 0.0f;
-        uint32_t link_old = 0;
+        Edge old{0, 0.0f, 0.0f, 0u};
         if (enc >= 0) {
             e = g.edges + (trow + (enc >> 8)) * kEdges + (enc & 0xFF);
-            n_old = e->n;
-            acc = e->w;
-            link_old = e->link;
+            old = load_edge(e);
         }
-        int visits = 0, released = 0;
-        bool last = true;
-#pragma unroll
-        for (int j = 0; j < kTrav; ++j) {
-            const int src = ((lane & ~(kTrav - 1)) | j) << 2;
-            const int enc_j = __builtin_amdgcn_ds_bpermute(src, enc);
-            const float val_j = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(val)));
-            const int counted_j = __builtin_amdgcn_ds_bpermute(src, counted);
-            const bool same = enc >= 0 && enc_j == enc;
-            if (same && j <= t) {
-                released += 1;
-                if (counted_j) {
-                    acc += val_j;
-                    visits += 1;
-                }
-            }
-            if (same && j > t) last = false;
-        }
-        if (enc >= 0 && last) {
-            e->n = n_old + visits;
+        uint32_t same = 0;
+        meet_in_row<0>(enc, same);
+        const uint32_t upto = same & ((2u << t) - 1u);   // this traversal and those before it
+        float acc = old.w;
+        add_in_order<0>(val, upto & counted, acc);
+        if (enc >= 0 && upto == same) {   // the last of them
+            e->n = old.n + __builtin_popcount(upto & counted);
             e->w = acc;
-            e->link = link_old - (uint32_t)released;
+            e->link = old.link - (uint32_t)__builtin_popcount(upto);
         }
     }
-    if (wave == 0) {   // expansion tickets back, once per node
+    if (wave == n_waves - 1) {   // expansion tickets back, once per node
         const int sel_l = lane < n_waves ? s.sel[lane] : 0;
         const bool is_exp = lane < n_waves && ((sel_l >> PUCT_GOMOKU_SEL_KIND_SHIFT) & 7) == PUCT_SELECT_EXPAND;
-        const int node_l = sel_l & PUCT_GOMOKU_SEL_NODE_MASK;
-        int returned = 0;
-        bool first = true;
-        for (int j = 0; j < n_waves; ++j) {
-            const int node_j = __builtin_amdgcn_readlane(node_l, j);
-            const bool exp_j = (__ballot(is_exp) >> j) & 1ull;
-            if (exp_j && node_j == node_l) {
-                returned += 1;
-                if (j < lane) first = false;
-            }
-        }
-        if (is_exp && first) g.info[trow + node_l].tickets -= returned;
+        const int node_l = is_exp ? sel_l & PUCT_GOMOKU_SEL_NODE_MASK : -1;   // (the first row; the others hold none)
+        uint32_t same = 0;
+        meet_in_row<0>(node_l, same);
+        if (is_exp && (same & ((1u << lane) - 1u)) == 0) g.info[trow + node_l].tickets -= __builtin_popcount(same);
     }
 }
 
@@ -1090,11 +1077,11 @@ __device__ void evaluator_loop(const LoopArgs &g, EvalLds &L, int tree, int help
             }
             L.tag = tag;
         }
+        if (wave == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");   // for all of the workgroup's wavefronts, which share an L1
         __syncthreads();
         const int tag = L.tag;
         __syncthreads();
         if (tag < 0) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         const int n = rq.n;
         int worked_off = 0;
         // (the step's nodes are dealt to the evaluators one by one, so that a step with few of them keeps all busy)
