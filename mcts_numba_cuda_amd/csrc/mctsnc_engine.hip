@@ -556,6 +556,12 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
         if (opt[MCTSNC_OPT_TEAM_POOL_THREADS] > 0) threads = opt[MCTSNC_OPT_TEAM_POOL_THREADS];
         block = dim3(threads);
     }
+    // A step's other work (child records, exploration terms, levels of the path) is spread over a workgroup's wavefronts, so
+    // searches of few playouts get more wavefronts than those need, while every workgroup has a CU to itself.  us a step,
+    // 64 / 128 / 256 / 512 threads: one child, 32 playouts, 1 tree 9.6 / 8.4 / 8.1 / 8.3, 8 trees 10.3 / 9.3 / 8.8 / 9.2;
+    // all children, 32 playouts, 4 trees 10.1 / 9.2 / 9.4 / 9.6, 64 playouts 10.0 / 9.2 / 9.3 / 9.5 (more to meet at each barrier).
+    const unsigned least_threads = e0->acp ? 128 : 256;
+    if (!solo && !team_pool && block.x < least_threads && e0->G * n_refs <= cus_now) block = dim3(least_threads);
     const size_t lds = solo ? c4::solo_lds_bytes(c.board_m, c.board_n, c.n_playouts)
                             : (team_pool ? c4::team_pool_lds_bytes(c.board_m, c.board_n, c.n_playouts) : c4::search_lds_bytes(c.board_m, c.board_n));
     const auto solo_kernel = c4::search_kernel_solo;
