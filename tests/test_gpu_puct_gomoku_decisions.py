@@ -1,0 +1,27 @@
+"""Gomoku PUCT loop: the ways a group of traversals decides on a node, GPU against host oracle, array for array: no edge yet
+(tickets, and too few of them), one edge, up to a row of 16, up to 64, more; every score equal (no exploration: the rotated
+order decides), scores beyond what a row of lanes takes, no widening, and numbers of traversals that leave an evaluator two,
+three or four nodes at a time."""
+import numpy as np
+import pytest
+
+from helpers import random_gomoku_root
+from oracle import puct_oracle as po
+from test_gpu_puct_gomoku import assert_same_trees, read_all
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape,traversals,cpuct,c_pw,steps", [
+    ((15, 15), 16, 0.0, 16.0, 120), ((15, 15), 16, 0.0, 1.0, 200), ((9, 9), 12, 1e31, 4.0, 150), ((15, 15), 9, 1e36, 16.0, 100),
+    ((15, 15), 16, 1.5, 0.0, 150), ((12, 12), 3, 1.5, 0.3, 400), ((15, 15), 4, 1e-3, 40.0, 250), ((8, 8), 2, 3.0, 5.0, 400),
+    ((6, 6), 12, 0.5, 7.5, 250), ((16, 16), 16, 50.0, 40.0, 120)])
+def test_every_way_of_deciding_equals_the_oracle(shape, traversals, cpuct, c_pw, steps):
+    from mcts_numba_cuda_amd.puct_gomoku import PUCTGomoku
+    board, turn = random_gomoku_root(np.random.default_rng(traversals), shape[0], shape[1], 4)
+    kw = dict(trees=2, traversals=traversals, max_nodes=8192, path_depth=64, cpuct=cpuct, c_pw=c_pw, dirichlet_alpha=0.3, seed=5)
+    want = po.gomoku_search(board, turn, steps, **kw)
+    for fused, evaluators in ((True, 3), (True, 1), (True, 0), (False, 0)):
+        with PUCTGomoku(board_shape=shape, evaluators=evaluators, **kw) as e:
+            e.run(board, turn, steps, fused=fused)
+            assert_same_trees(read_all(e), want)
