@@ -176,9 +176,10 @@ int mctsnc_run_batch_noalloc(mctsnc_engine **engines, int32_t n, const int8_t *b
  *   MCTSNC_OPT_PROBE_STEPS        Connect 4 pass with more trees than stay resident: steps every tree runs before the
  *                                 searches are put in the order of what they cost; 0 = keep the order by stones,
  *                                 -1 (default) = a thirty-second of the step budget, 16 to 128
- *   MCTSNC_OPT_SPIN_LIMIT         polls after which a workgroup's wait for the others of its tree gives up and ends the
- *                                 launch (MCTSNC_E_DEVICE_SYNC); 0 (default) = 2^24.  1 makes the first wait that is not
- *                                 met at once give up: the hook with which the tests drive that path.
+ *   MCTSNC_OPT_SPIN_LIMIT         polls after which a workgroup's wait for the others of its tree, or a wavefront's for
+ *                                 the one it shares its playouts with (one-child Gomoku), gives up and ends the launch
+ *                                 (MCTSNC_E_DEVICE_SYNC); 0 (default) = 2^24.  1 makes the first wait that is not met at
+ *                                 once give up: the hook with which the tests drive that path.
  * After MCTSNC_E_DEVICE_SYNC the search is void, the engines stay usable and their random streams are back at their
  * seeds (as after mctsnc_reseed). */
 #define MCTSNC_OPT_AGENT_FENCES 0

@@ -53,6 +53,29 @@ def test_abandoned_search_reports_and_leaves_a_fresh_engine(game, variant):
         assert_same(snapshot(e, params["n_trees"]), snapshot(fresh, params["n_trees"]))
 
 
+@pytest.mark.parametrize("variant,shape,trees,playouts", [("ocp_prodigal", (15, 15), 2, 256), ("ocp_thrifty", (15, 15), 2, 512),
+                                                         ("ocp_thrifty", (15, 15), 300, 128), ("ocp_thrifty", (19, 19), 2, 128)])
+def test_one_child_gomoku_gives_up_on_its_playouts(variant, shape, trees, playouts):
+    """Two wavefronts draw 64 playouts of a one-child tree and wait for each other, for 2 to 16 polls at the busiest places
+    here: in one round, in two, two trees to a CU, and on two-byte cells."""
+    from mcts_numba_cuda_amd import _lib
+    params = dict(n_trees=trees, n_playouts=playouts, variant=variant, device_memory=0.5, ucb_c=2.0, seed=5)
+    mk = lambda: make_engine(params, board_shape=shape, extra=0, actions=shape[0] * shape[1], game="gomoku")
+    board, turn = random_gomoku_root(np.random.default_rng(5), *shape, 6)
+    e = mk()
+    e.run(board, None, turn, forced_search_steps_limit=12)
+    e.set_option("spin_limit", 1)
+    with pytest.raises(_lib.EngineError) as err:
+        e.run(board, None, turn, forced_search_steps_limit=12)
+    assert err.value.code == -5 and "timed out" in str(err.value)
+    e.set_option("spin_limit", 0)
+    fresh = mk()
+    for _ in range(2):
+        e.run(board, None, turn, forced_search_steps_limit=12)
+        fresh.run(board, None, turn, forced_search_steps_limit=12)
+        assert_same(snapshot(e, 2), snapshot(fresh, 2))
+
+
 def test_option_values_are_checked():
     from mcts_numba_cuda_amd import _lib
     e = make_engine(dict(n_trees=1, n_playouts=32, variant="ocp_thrifty", device_memory=0.05, ucb_c=2.0, seed=0))
