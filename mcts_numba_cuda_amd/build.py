@@ -1,6 +1,7 @@
 """Builds libmctsnc_hip.so (search engine) and libpuct_hip.so (PUCT select/backup) for gfx950 with hipcc, and _puct_call
 (the Python side of a PUCT launch, host code only) with the C compiler, in-tree, next to this file."""
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -39,9 +40,25 @@ def run(cmd, what, verbose):
         print(out)
 
 
-def build_host_module(verbose=False):
-    run([os.environ.get("CC", "gcc"), "-O2", "-Wall", "-fPIC", "-shared", "-I" + sysconfig.get_paths()["include"], "-o", HOST_MODULE,
-         os.path.join(CSRC, "puct_call.c")], "the C compiler", verbose)
+def build_host_module(verbose=False, optional=False):
+    """Compiles _puct_call; `optional`: where there is no C compiler or no Python.h (3.9 or later) the package does without it
+    (puct.py makes the same checks in Python), and one left from an earlier build goes, since its source may have been another."""
+    compiler, include = os.environ.get("CC") or "gcc", sysconfig.get_paths()["include"]
+    missing = None
+    if shutil.which(compiler.split()[0]) is None:
+        missing = f"no C compiler ({compiler})"
+    elif not os.path.exists(os.path.join(include, "Python.h")):
+        missing = f"no Python.h in {include}"
+    elif sys.version_info < (3, 9):
+        missing = "it calls functions of Python 3.9"
+    if missing and optional:
+        print(f"{os.path.basename(HOST_MODULE)} is not built: {missing}; a PUCT launch on torch tensors takes a few microseconds longer", file=sys.stderr)
+        if os.path.exists(HOST_MODULE):
+            os.remove(HOST_MODULE)
+        return None
+    if missing:
+        raise RuntimeError(f"{os.path.basename(HOST_MODULE)} cannot be built: {missing}")
+    run(compiler.split() + ["-O2", "-Wall", "-fPIC", "-shared", "-I" + include, "-o", HOST_MODULE, os.path.join(CSRC, "puct_call.c")], "the C compiler", verbose)
     return HOST_MODULE
 
 
@@ -53,12 +70,12 @@ def build_one(lib, sources, verbose=False):
 
 
 def build(verbose=False, only=None):
-    """Compiles every library (or the one whose path is `only`); returns the search engine's path."""
+    """Compiles every library (or the one whose path is `only`), and _puct_call where that can be done; returns the search engine's path."""
     for lib, sources in LIBRARIES.items():
         if only is None or only == lib:
             build_one(lib, sources, verbose)
     if only is None or only == HOST_MODULE:
-        build_host_module(verbose)
+        build_host_module(verbose, optional=only is None)
     return LIB
 
 
