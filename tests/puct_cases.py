@@ -371,6 +371,20 @@ def case_deep_chain_terminal(r):
     assert inflight_sum(r.release()) == 0
 
 
+def case_same_edge_again(r):
+    """Both edges of the root lead back to the root, with equal values and priors: a traversal sees its own claims, so it takes
+    them in turn (a tie goes to edge 0, then edge 0 is one claim behind), up to the depth limit, and gives all of them back."""
+    c = make_case(nodes=2, actions=4, path_depth=6)
+    c["node_expanded"][0, 0] = 2
+    c["edge_child"][0, 0, :2] = 0
+    c["edge_n"][0, 0, :2] = 1
+    c["edge_prior"][0, 0, :2] = 0.5
+    h = r.select(c, c_pw=0.0)
+    assert decode(h["out_selected"][0, 0]) == (DEPTH_LIMIT, 0, 0) and h["out_len"][0, 0] == 7
+    assert h["out_path"][0, 0].tolist() == [0, 1, 0, 1, 0, 1] and h["edge_inflight"][0, 0, :2].tolist() == [3, 3]
+    assert inflight_sum(r.release()) == 0
+
+
 REFERENCE_CASES = [case_fresh_root_expand, case_terminal_root, case_invalid_child_rolls_back,
                    case_child_beyond_node_count, case_progressive_widening_unique_slots, case_single_edge_contention,
                    case_full_ticket_quota_falls_through, case_strict_winner, case_soft_winner,
@@ -378,7 +392,7 @@ REFERENCE_CASES = [case_fresh_root_expand, case_terminal_root, case_invalid_chil
                    case_zero_n_edge_selectable, case_encoding_boundaries]
 ARITHMETIC_CASES = [case_hand_computed_scores, case_virtual_loss_lowers_score, case_tie_rotation_by_wid,
                     case_tie_rotation_across_slices_and_around, case_wide_node_beyond_one_wavefront, case_nan_and_minus_inf_never_win, case_deep_chain_rollback,
-                    case_deep_chain_terminal]
+                    case_deep_chain_terminal, case_same_edge_again]
 ALL_CASES = REFERENCE_CASES + ARITHMETIC_CASES
 
 
@@ -438,4 +452,26 @@ def wide_forest(rng, trees, nodes, actions, warps, path_depth, hubs=2, claims=0.
     if claims:
         held = rng.random(c["edge_inflight"].shape) < claims
         c["edge_inflight"][held] = rng.integers(1, 4, int(held.sum()))
+    return c
+
+
+def recurrent_forest(rng, trees, nodes, actions, path_depth, claims=0.1, dead_ends=0.02):
+    """Few nodes with many edges, for one traversal a tree: every node has 1 to `actions` expanded edges (the root all of them,
+    others mostly more than half), each to any node of the tree, the root included, so that a path comes back to nodes and edges it
+    has taken; a share of the edges leads nowhere, a few nodes are ends, and a share `claims` of the edges is claimed already.
+    Value sums are sixty-fourths, so that adding such values to one edge several times is exact in any order."""
+    c = make_case(trees=trees, nodes=nodes, actions=actions, warps=1, path_depth=path_depth)
+    shape = (trees, nodes, actions)
+    c["node_expanded"][:] = np.where(rng.random((trees, nodes)) < 0.3, rng.integers(1, actions + 1, (trees, nodes)), rng.integers((actions + 1) // 2, actions + 1, (trees, nodes)))
+    c["node_expanded"][:, 0] = actions
+    ends = rng.random((trees, nodes)) < 0.02
+    ends[:, 0] = False
+    c["node_expanded"][ends] = TERMINAL
+    c["edge_child"][:] = rng.integers(0, nodes, shape)
+    c["edge_child"][rng.random(shape) < dead_ends / 8] = -1
+    c["edge_n"][:] = np.where(rng.random(shape) < 0.8, rng.integers(0, 20, shape), 0)
+    c["edge_w"][:] = np.floor(rng.uniform(-64, 64, shape)) / 64 * c["edge_n"]
+    c["edge_prior"][:] = np.where(rng.random(shape) < 0.5, rng.choice([0.1, 0.25, 0.5, 1.0], shape), rng.uniform(0.01, 1.0, shape))
+    held = rng.random(shape) < claims
+    c["edge_inflight"][held] = rng.integers(1, 4, int(held.sum()))
     return c

@@ -56,8 +56,8 @@ def test_known_answers(case):
 def test_single_traversal_matches_oracle_exactly(actions, nodes, depth, cpuct, c_pw):
     """One traversal per tree is deterministic: every array must equal the oracle's, over several select/backup
     rounds on the same trees (the statistics drift apart as soon as one score comparison differs).  (Up to 8192 edge
-    slots per tree the kernel keeps a tree's claims in LDS during a launch, beyond that in device memory: the last two
-    cases sit on either side.)"""
+    slots per tree a single traversal's claims are plain stores, beyond that atomics: the last two cases sit on either
+    side.)"""
     rng = np.random.default_rng(actions * 1000 + nodes)
     case = pc.random_forest(rng, trees=64, nodes=nodes, actions=actions, warps=1, path_depth=depth)
     h = copy.deepcopy(case)
@@ -95,6 +95,36 @@ def test_wide_nodes_with_claims_in_flight_match_oracle_exactly(actions, nodes, h
         po.backup(h, values)
         for k in h:
             assert np.array_equal(got[k], h[k], equal_nan=True), (rnd, k)
+
+
+@pytest.mark.parametrize("actions,nodes,depth,claims,cpuct,c_pw,soft", [
+    (256, 30, 40, 0.1, 1.5, 0.0, 0), (256, 32, 64, 0.3, 0.5, 0.0, 1), (256, 33, 40, 0.1, 1.5, 0.0, 0), (193, 42, 100, 0.1, 1.0, 0.0, 0), (192, 42, 40, 0.0, 0.5, 2.0, 0),
+    (129, 63, 200, 0.05, 1.5, 0.0, 1), (128, 64, 40, 0.3, 0.2, 1.2, 0), (65, 126, 64, 0.1, 1.5, 0.0, 0), (64, 128, 40, 0.1, 1.0, 0.0, 1), (64, 129, 40, 0.1, 1.0, 0.0, 0),
+    (5, 3, 90, 0.0, 1.0, 0.0, 0)])
+def test_single_traversals_of_recurrent_trees_match_oracle_exactly(actions, nodes, depth, claims, cpuct, c_pw, soft):
+    """One traversal a tree on few nodes of one to four 64-edge slices, with claims already held, some of them on the edges
+    that win; paths come back to edges that they hold a claim on, and some end at an edge that leads nowhere and give all of
+    it back.  nodes * edges lies on both sides of 8192, where the claims change from plain stores to atomics."""
+    rng = np.random.default_rng(actions * 1000 + nodes)
+    case = pc.recurrent_forest(rng, trees=48, nodes=nodes, actions=actions, path_depth=depth, claims=claims, dead_ends=1.0 / min(depth, actions))
+    h = copy.deepcopy(case)
+    r = HipRunner()
+    again = given_back = 0
+    for rnd in range(4):
+        got = r.select(case if rnd == 0 else to_host(r.d), cpuct=cpuct, c_pw=c_pw, soft_winner=soft)
+        po.select(h, cpuct=cpuct, c_pw=c_pw, soft_winner=soft)
+        for k in h:
+            assert np.array_equal(got[k], h[k], equal_nan=True), (rnd, k)
+        for t in range(48):
+            path = h["out_path"][t, 0, :max(0, h["out_len"][t, 0] - 1)]
+            again += len(set(path.tolist())) < len(path)
+            given_back += pc.decode(h["out_selected"][t, 0])[0] == pc.INVALID
+        values = (np.floor(rng.uniform(-64, 64, h["out_path"].shape)) / 64).astype(np.float32)
+        got = r.backup(values)
+        po.backup(h, values)
+        for k in h:
+            assert np.array_equal(got[k], h[k], equal_nan=True), (rnd, k)
+    assert given_back > 0 and (again > 0 or c_pw > 0)   # (with widening the paths are short)
 
 
 @pytest.mark.parametrize("trees,warps,soft", [(16, 8, 0), (16, 16, 0), (4, 40, 0), (16, 16, 1), (128, 4, 0)])
