@@ -59,10 +59,11 @@ extern "C" {
  * Replaces puct_select_winner_recalc_launch of src/puct/puct_gpu_v3_cpp.cu:450-481 (kernel :277-448): same
  * signature, same semantics, same packing.  The reference launches `trees` blocks of `warps * 32` threads; this
  * library launches one 64-lane wavefront per (tree, wid) and splits trees with more than 16 traversals over several
- * workgroups, so `warps` is not limited to 32.  With up to 16 traversals per tree and nodes * edges <= 8192 a launch
- * keeps every tree's edge_inflight in the LDS of the one workgroup that runs the tree's traversals (read at the start,
- * written back at the end; the claims in between are LDS operations).  As with any output array, nothing else on the
- * device may read or write edge_inflight while the launch runs; launches on one stream, or ordered by events, are fine.
+ * workgroups, so `warps` is not limited to 32.  As with any output array, nothing else on the device may read or write
+ * edge_inflight while the launch runs, whatever the size of the trees; launches on one stream, or ordered by events, are
+ * fine.  (With nodes * edges <= 8192 a launch relies on it: with 2 to 16 traversals per tree it keeps every tree's
+ * edge_inflight in the LDS of the one workgroup that runs them, read at the start and written back at the end, and with one
+ * traversal per tree the claims are ordinary stores.)
  */
 int puct_select_winner_recalc_launch(float cpuct, float c_pw, float alpha_pw, int soft_winner,
                                      const int *edge_child_id, const float *edge_prior, const float *edge_W,

@@ -75,13 +75,17 @@ extern "C" int puct_select_winner_recalc_launch(float cpuct, float c_pw, float a
                  trees,        nodes,         edges,           warps,                path_depth};
     dim3 grid, block;
     launch_shape(trees, warps, grid, block);
-    // (the claims of a tree in LDS: up to 8192 edge slots, so that a CU still holds four workgroups)
+    // The claims of a tree in LDS: up to 8192 edge slots, so that a CU still holds four workgroups.  A single traversal needs
+    // none of it: its claims are plain stores, which at the sizes of this rule beat both other forms at every width (plain
+    // stores / atomics / LDS, ms a launch of 512 levels: 16384 trees of 65 x 64 edges 2.33 / 2.91 / 6.11, of 128 x 64 2.35 /
+    // 2.92 / 11.9; 8192 trees of 64 x 128 1.98 / 2.05 / 8.06; 4096 trees of 32 x 256 1.96 / 1.97 / 5.28).  Larger trees go
+    // by atomics, with one traversal too: there it depends on the width which is ahead (plain stores / atomics: 16384 trees of
+    // 129 x 64 2.27 / 2.91; with 1024 levels 8192 trees of 129 x 128 4.47 / 4.57, 4096 trees of 257 x 256 4.67 / 4.58).
     const long long slots = (long long)nodes * edges;
-    // With larger trees a launch shares edge_inflight with other launches, also one of single traversals.
-    const bool exclusive = grid.y == 1 && slots > 0 && slots <= kLocalClaimSlots;
-    if (exclusive && warps == 1)
+    const bool small = grid.y == 1 && slots > 0 && slots <= kLocalClaimSlots;
+    if (small && warps == 1)
         hipLaunchKernelGGL(select_kernel<ClaimsIn::OWN>, grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);
-    else if (exclusive)
+    else if (small)
         hipLaunchKernelGGL(select_kernel<ClaimsIn::LDS>, grid, block, sizeof(int) * (size_t)slots, reinterpret_cast<hipStream_t>(stream), a);
     else
         hipLaunchKernelGGL(select_kernel<ClaimsIn::SHARED>, grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);
