@@ -19,6 +19,7 @@
 //   * OCP: one workgroup per tree does everything, no inter-workgroup synchronisation.
 //   * blockIdx is decoded so that the workgroups of one tree share blockIdx % 8, i.e. the same XCD and L2.
 #pragma once
+#include "c4_draw.h"
 #include "mctsnc_common.hpp"
 
 namespace mctsnc {
@@ -323,15 +324,9 @@ struct Connect4 {
         return pc;
     }
 
-    // The uniform that the generator gives in its present state, times 2^32.  The reference's float32 of the upper 53 bits
-    // of the sum, a single rounding, in four instructions without float64 (which took six, four of them conversions): the
-    // upper word's conversion rounds as the whole would if its last bit says whether anything follows, as long as at
-    // least two bits are dropped, that is from 2^25 on.  Below that the ordinal is 0 anyway: with at most 8 columns it
-    // is as long as the uniform is below 1/8.
+    // The uniform that the generator gives in its present state, times 2^32.
     static __device__ __forceinline__ float draw_of(const Rng32 &r) {
-        const uint64_t sum = (((uint64_t)r.s0h << 32) | r.s0l) + (((uint64_t)r.s1h << 32) | r.s1l);
-        const uint32_t rest = (uint32_t)sum >> 11;
-        return (float)((uint32_t)(sum >> 32) | (rest < 1u ? rest : 1u));
+        return c4_draw((((uint64_t)r.s0h << 32) | r.s0l) + (((uint64_t)r.s1h << 32) | r.s1l));
     }
 
     static __device__ __forceinline__ void begin(Playout &p, const PoolChild &pc, uint64_t s0, uint64_t s1) {
