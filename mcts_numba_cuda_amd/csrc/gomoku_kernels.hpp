@@ -63,6 +63,9 @@ template <int W> struct Board {
 //     from the last note before the end.
 // Boards of the narrow format are laid out with rows of at most 15 cells (on their side, if need be), so that a row's masks
 // of both colours share a dword; cells and times are bytes.  Wide ones are laid on their longer side: at most 22 rows.
+// 16 x 16 has no side of 15 cells and is wide, with two-byte cells, though its cells would fit a byte: it gained less than its
+// neighbours when playouts began to draw first, but gained (before, in the narrow format, ply by ply / now: one child, 4 trees x 128
+// playouts, 500 steps 29.1 / 14.7 ms, all children, 8 x 128, 60 steps 26.9 / 17.5; 16 x 15 27.3 / 12.6 and 25.2 / 11.2).
 constexpr int kMaxRowsWide = 22;
 struct PlayoutShape {
     int rows, cols, stride;   // of the board of times: a cell's row is row * stride + column, "never" in the columns beside the board

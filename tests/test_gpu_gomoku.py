@@ -198,8 +198,8 @@ def test_gomoku_wide_board_other_playout_counts_and_batches():
 
 @pytest.mark.parametrize("variant,steps", [("ocp_prodigal", 20), ("acp_thrifty", 3)])
 def test_gomoku_largest_board_with_256_playouts(variant, steps):
-    """On 16x16 the lists and line words of 256 playouts do not fit the LDS of a CU: the workgroup then holds 128 at a
-    time and plays 256 in two rounds."""
+    """On 16x16 the lists (two-byte cells) of 256 playouts and a board of times do not fit the LDS of a CU: the workgroup
+    then holds 128 at a time and plays 256 in two rounds."""
     e, o = engines(variant, 2, 256, 16, 16, seed=8)
     board, turn = random_gomoku_root(np.random.default_rng(3), 16, 16, 30)
     compare_with_oracle(e, o, board, None, turn, steps)
@@ -227,8 +227,8 @@ def test_gomoku_many_trees(variant, T, steps):
 
 def test_gomoku_engines_of_different_shapes_alive_together():
     """The dynamic-LDS limit is a setting of the kernel function, not of an engine: an engine created earlier, whose
-    playouts need more LDS than the latest one's, must still launch.  Three engines (16 x 16 with 128 slots: 81 KB;
-    6 x 6: 3 KB; 19 x 19 in the other board format: 104 KB) are created first and then used in turn, twice."""
+    playouts need more LDS than the latest one's, must still launch.  Three engines (16 x 16 with 128 slots: 103 KB;
+    6 x 6: 52 KB; 19 x 19 with 128 slots: 143 KB) and a fourth (15 x 15: 70 KB) are created first and then used in turn, twice."""
     rng = np.random.default_rng(31)
     made = []
     for variant, (m, n), P, steps in (("acp_thrifty", (16, 16), 256, 2), ("ocp_prodigal", (6, 6), 64, 60), ("acp_prodigal", (19, 19), 64, 2),
