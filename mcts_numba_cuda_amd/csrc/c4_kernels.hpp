@@ -1142,7 +1142,7 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
 // apart and meet in one L2.  Set u starts on tree u; when a launch has more trees than sets (a large batch of
 // searches), a set that has finished its tree takes the next one from the queue: workgroup 0 draws the index and
 // leaves it in the finished tree's header for the others.  Five wavefronts per SIMD (at most 96 vector registers: none
-// spilled by the team kernel, two dwords by the one with playout pools) let five workgroups share a CU in such batches; a
+// spilled by the team kernel, eleven dwords by the one with playout pools) let five workgroups share a CU in such batches; a
 // single search is no slower for it.
 template <class Game, bool ACP, bool SOLO, bool POOL = false>
 __device__ __forceinline__ void search_trees(const SearchArgs &args) {
@@ -1182,7 +1182,7 @@ template <bool ACP>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5, 5))) search_kernel(SearchArgs args) { search_trees<Connect4, ACP, false>(args); }
 
 // One-child playouts: one workgroup per tree and never more than two of them on a CU, so the register budget of four
-// wavefronts per SIMD costs nothing (with 96 registers this variant spills 13 dwords).
+// wavefronts per SIMD costs nothing (with 96 registers this variant spills 18 dwords).
 template <>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) search_kernel<false>(SearchArgs args) { search_trees<Connect4, false, false>(args); }
 

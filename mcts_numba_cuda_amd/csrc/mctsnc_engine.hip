@@ -530,7 +530,14 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
     // the queue: the form for many hundreds of trees (from 3.5 trees per CU on in a batch; in one search from 1.4 trees
     // per CU on, and between 0.8 and 1).  Between the two, teams whose workgroups play their child's playouts as a pool of
     // jobs on half as many lanes: half the wavefronts per tree, so twice as many trees resident, and no idle lanes, at a
-    // step 1.4 times as long (from 1.75 trees per CU on).  MCTSNC_OPT_SOLO_TREES and MCTSNC_OPT_TEAM_POOL override the choice.
+    // step 1.3 times as long (from 1.75 trees per CU on).  MCTSNC_OPT_SOLO_TREES and MCTSNC_OPT_TEAM_POOL override the choice.
+    // Teams / pools / one workgroup per tree on 256 CUs, ms (4 x 256 playouts, 5000 steps): passes of 64 searches of 4 trees
+    // 54 / 80 / 112, 96: 76 / 83 / 112, 112: 86 / 86 / 125, 128: 94 / 84 / 123, 192: 138 / 111 / 117, 224: 162 / 126 / 114, 256: 183 /
+    // 142 / 115, 384: 270 / 207 / 160, 512: 356 / 273 / 170.  One search from the empty board, trees: 192: 115 / 133 / 142, 208: 117 /
+    // 135 / 142, 256: 141 / 158 / 142, 288: 155 / 160 / 199, 352: 173 / 185 / 204, 360: 207 / 185 / 208, 384: 214 / 207 / 208, 448:
+    // 239 / 229 / 208.  The lines for one search were drawn when a ply had 87 instructions (208 trees: 151 / 151 / 151, 256: 187 /
+    // 184 / 152, 288: 207 / 185 / 233, 352: 244 / 217 / 241): every form gained since, teams the most, and teams are ahead
+    // up to 1.35 trees per CU now; the lines have not been moved.
     int cus_now = 0;
     HIP_TRY(hipDeviceGetAttribute(&cus_now, hipDeviceAttributeMultiprocessorCount, c.device));
     bool solo = e0->acp && (n > 1 ? 2 * n_refs >= 7 * cus_now : (10 * n_refs >= 14 * cus_now || (10 * n_refs >= 8 * cus_now && n_refs <= cus_now)));
