@@ -551,7 +551,7 @@ def bench_gomoku_acp(args):
            "stage_ms_per_mcts_step": {k: v / mcts_steps * 1e3 for k, v in stage.items()},
            "stage_achieved_gbs": {k: alg[k] / stage[k] / 1e9 for k in stage if stage[k]},
            "roofline_valu": valu_roofline((prof or {}).get("sq_insts_valu_per_launch"), dev / steps, prof or {},
-                                          "one search, gomoku::search_kernel_for<Gomoku, true, 8> on 512 workgroups of 128 threads"),
+                                          "one search, gomoku::search_kernel_for<Gomoku, true, 8> on 512 workgroups of 256 threads"),
            "roofline": {"bound": "hbm", "achieved": alg["total"] / dev / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": alg["total"] / dev / 1e9 / HBM_PEAK_GBS, "traffic": (prof or {}).get("traffic_bytes_per_launch"),
                         "traffic_source": {"file": prof["file"], "commit": prof.get("commit"), "stale": prof.get("stale")} if prof else None,
