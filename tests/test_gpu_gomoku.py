@@ -73,8 +73,8 @@ def test_gomoku_one_child_backup_of_paths_too_deep_to_prepare(levels):
 
 @pytest.mark.parametrize("P", [1, 8, 32, 256])
 def test_gomoku_one_child_other_playout_counts(P):
-    """A one-child workgroup has 256 threads whatever the playout count: with fewer playouts the other wavefronts help
-    (LDS columns, children, the backup's arg-max), with 256 every wavefront plays and none is left to help."""
+    """A one-child workgroup has 512 threads whatever the playout count, two wavefronts of which draw 64 playouts: the others
+    help (children, the backup's arg-max), with 256 playouts every wavefront draws and none is left to help."""
     e, o = engines("ocp_thrifty", 2, P, 9, 9, seed=4)
     board, turn = random_gomoku_root(np.random.default_rng(P), 9, 9, 6)
     compare_with_oracle(e, o, board, None, turn, 60 if P < 256 else 25)
@@ -94,7 +94,7 @@ def test_gomoku_tree_full_path():
 
 
 def test_gomoku_large_playout_count_runs_in_rounds():
-    """n_playouts = 512 exceeds the 256 threads of a workgroup; the playouts then run in two rounds."""
+    """n_playouts = 512 exceeds the 256 playouts that a workgroup holds; they then run in two rounds."""
     e, o = engines("ocp_thrifty", 1, 512, 15, 15)
     board, turn = random_gomoku_root(np.random.default_rng(2), 15, 15, 8)
     compare_with_oracle(e, o, board, None, turn, 12)
@@ -171,7 +171,7 @@ def test_gomoku_wide_board_children_that_complete_lines():
 
 
 def test_gomoku_wide_board_other_playout_counts_and_batches():
-    """19 x 19 with 256 playouts (the workgroup holds 64 at a time: four rounds) and with 16; three searches in one
+    """19 x 19 with 256 playouts (the workgroup holds 128 at a time: two rounds) and with 16; three searches in one
     pass against separate runs."""
     from mcts_numba_cuda_amd import MCTSNC, run_batch
     rng = np.random.default_rng(23)
