@@ -370,18 +370,22 @@ __device__ __forceinline__ void set_lds_count(uint32_t *p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 // A wavefront's wait for its partner's next chunk.  The two belong to one workgroup, so both run, and neither waits for
-// anything else; bounded all the same, like the waits between workgroups.  One that gives up leaves the rest of its playouts
-// undone and says so: its partner, the workgroup at the end of the step, and the host.
+// anything else; bounded all the same, like the waits between workgroups.  One that gives up draws nothing more and says so to
+// its partner and, at the end of the step, to the workgroup, which tells the host.  (The wait is met at once as a rule: what
+// giving up needs stands in LDS and not in scalar registers, of which these kernels have none to spare, and has no way out of
+// its own in the loops around it.  us a step without a bound / so / with both: 15 x 15, 4 trees x 128 playouts 24.2 / 24.0 / 24.4,
+// 19 x 19 45.2 / 45.5 / 46.3, 9 x 9, 2 x 64 13.3 / 13.2 / 13.5, 22 x 22, 2 x 128 76.7 / 77.8 / 78.4.)
 struct RingWait {
-    int32_t *gave_up;      // of the workgroup, in LDS
-    int32_t *abort_flag;   // of the launch
-    uint32_t spin_limit;
+    int32_t *gave_up;             // of the workgroup
+    const uint32_t *spin_limit;   // polls
     __device__ __forceinline__ bool operator()(const uint32_t *p, uint32_t v) const {
-        uint32_t spins = 0;
-        while ((int32_t)(lds_count(p) - v) < 0) {
-            const bool bad = ++spins >= spin_limit;
-            if (bad) { *gave_up = 1; __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-            if (bad || ((spins & 1023u) == 0 && __hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0)) return false;
+        if (__builtin_expect((int32_t)(lds_count(p) - v) < 0, 0)) {
+            uint32_t left = *spin_limit;
+            do {
+                left--;
+                if (left == 0) *gave_up = 1;
+                if (left == 0 || ((left & 1023u) == 0 && __hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0)) return false;
+            } while ((int32_t)(lds_count(p) - v) < 0);
         }
         asm volatile("" ::: "memory");
         return true;
@@ -397,7 +401,7 @@ __device__ __forceinline__ float make_offsets(u32x2 *ring, uint32_t *made, const
         mark[s] = rg;
         for (int k = s * STEP; k < min(count, (s + 1) * STEP); k += kChunk) {
             const uint32_t chunk = (uint32_t)k / kChunk;
-            if (k >= kRingChunks * kChunk && !await(taken, chunk + 1 - kRingChunks)) return u_max;
+            if (k >= kRingChunks * kChunk && !await(taken, chunk + 1 - kRingChunks)) { count = 0; break; }
             float left = (float)(count - k) * 0x1p-64f;
             auto offset = [&]() __attribute__((always_inline)) -> uint32_t {
                 uint32_t lo, hi;
@@ -434,7 +438,7 @@ __device__ __forceinline__ void walk_list(Cell *list, Cell *my_times, const u32x
     auto at = [=](uint32_t offset) -> Cell * { return reinterpret_cast<Cell *>(reinterpret_cast<unsigned char *>(list) + offset); };
     for (int k0 = 0; k0 < whole; k0 += kChunk) {
         const uint32_t chunk = (uint32_t)k0 / kChunk;
-        if (!await(made, chunk + 1)) return;
+        if (!await(made, chunk + 1)) { count = 0; break; }
         u32x2 pair[kChunk / 4];
 #pragma unroll
         for (int q = 0; q < kChunk / 4; q++) pair[q] = ring[((chunk % kRingChunks) * (kChunk / 4) + q) * 64];
@@ -713,8 +717,10 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
     __shared__ int32_t s_pbase[ACP ? 1 : kPrepLevels];
     __shared__ Stat s_pstat[ACP ? 1 : kPrepLevels + 1];
     __shared__ int32_t s_flag, s_chosen, s_abort, s_njobs;
+    __shared__ uint32_t s_spin_limit;
 
     if (tid == 0) s_abort = 0;
+    if (!ACP && tid == 0) s_spin_limit = args.spin_limit;
     uint64_t e0 = 0, e1 = 0;
     if (!ACP && tid == 0) { e0 = ref.rng_expand[0]; e1 = ref.rng_expand[1]; }
     // One-child playouts that fit one round use the same generators, thread for thread, in every step: their states
@@ -735,7 +741,7 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
     bool xcd_local = false;
     const uint32_t my_xcc = (uint32_t)__builtin_amdgcn_s_getreg(6164) & 0xfu;   // HW_REG_XCC_ID, bits 3:0
     if (ACP && tid == 0) atomic_store_relaxed(&hdr->xcc[g], my_xcc);
-    const RingWait ring_wait{&s_abort, args.abort_flag, args.spin_limit};
+    const RingWait ring_wait{&s_abort, &s_spin_limit};
     // row of a cell in the board of times, which is what a legal list holds
     auto time_row = [=](uint32_t c) -> uint32_t {
         const uint32_t i = (c * div_n) >> 16, jj = c - i * (uint32_t)n;
@@ -1322,7 +1328,10 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
         } else {
             __threadfence_block();
             __syncthreads();
-            if (s_abort) break;   // (set before this step's last barriers, if at all)
+            if (s_abort) {   // (set before this step's last barriers, if at all)
+                if (tid == 0) __hip_atomic_store(args.abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
         }
         if (timing) { const unsigned long long t2 = wall_clock64(); tk_backup += t2 - tk; tk = t2; }
     }
