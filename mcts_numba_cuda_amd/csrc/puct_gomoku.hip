@@ -415,7 +415,8 @@ __device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {   // over the 16 l
 template <bool TICKETS>
 __device__ __forceinline__ void row_decisions(const EdgeSet<1> &e, uint64_t edges, uint32_t members, int lane, int expanded, float sqrt_lane, int allowed_lane,
                                               bool single, int &tickets, uint32_t &with_ticket, int &den, int &mine) {
-    prow_terms terms = prow_terms_of(e.eid[0] >= 0, e.q[0], e.cp[0], e.den[0]);
+    const bool edge = e.eid[0] >= 0;
+    const float q = prow_q(edge, e.q[0]), cp = prow_cp(edge, e.cp[0]);
     int claimed = 0;
     uint32_t rest = members;
     do {
@@ -428,7 +429,8 @@ __device__ __forceinline__ void row_decisions(const EdgeSet<1> &e, uint64_t edge
             uint64_t first = 1ull;
             if (!single) {
                 const float sqrt_parent = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), claimed));
-                const uint32_t image = prow_image(prow_score(terms, sqrt_parent));   // (score_image of a finite score)
+                const uint32_t b = __float_as_uint(prow_score(q, cp, sqrt_parent, den) + 0.0f);   // -0.0f counts as +0.0f
+                const uint32_t image = b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);           // score_image of a finite score
                 const uint32_t top = row_max_u32(image);
                 first = __builtin_amdgcn_uicmp(image, top, 32 /* == */) & edges;
                 if ((first & (first - 1)) != 0) {   // the rotated edge index decides, as in candidate_key
@@ -440,12 +442,11 @@ __device__ __forceinline__ void row_decisions(const EdgeSet<1> &e, uint64_t edge
                     first &= __builtin_amdgcn_uicmp(key, top_key, 32);
                 }
             }
-            terms.den += __builtin_amdgcn_inverse_ballot_w64(first) ? 1 : 0;
+            den += __builtin_amdgcn_inverse_ballot_w64(first) ? 1 : 0;
             mine = __builtin_amdgcn_inverse_ballot_w64(bit) ? __builtin_ctzll(first) : mine;
             claimed += 1;
         }
     } while (rest != 0);
-    den = terms.den;
 }
 __device__ __forceinline__ void decide_in_row(const LoopArgs &g, StepLds &s, int *paths, int *next, Edge *row, const EdgeSet<1> &e, int node,
                                               uint32_t members, int depth, int lane, int expanded, int legal, int total, int &tickets, bool single) {
@@ -454,7 +455,7 @@ __device__ __forceinline__ void decide_in_row(const LoopArgs &g, StepLds &s, int
     const float sqrt_lane = widening ? sqrtf((float)eff_lane) : 1.0f;
     const int allowed_lane = widening ? allowed_children(g.c_pw, g.alpha_pw, eff_lane, sqrt_lane, legal) : 1;
     const int tickets_before = tickets;
-    int den = 1, mine = -1;   // den: of this lane's edge after the claims; mine: lane of the edge that this lane's traversal takes
+    int den = prow_den(e.eid[0] >= 0, e.den[0]), mine = -1;   // mine: lane of the edge that this lane's traversal takes
     uint32_t with_ticket = 0;
     const uint64_t edges = __ballot(e.eid[0] >= 0);
     // (the limit grows with the claims: its largest value is the last one's)

@@ -6,8 +6,6 @@
 #ifndef MCTSNC_PUCT_ROW_H
 #define MCTSNC_PUCT_ROW_H
 #include <float.h>
-#include <stdint.h>
-#include <string.h>
 
 #if defined(__HIPCC__)
 #define PROW_FN __host__ __device__ inline
@@ -15,25 +13,11 @@
 #define PROW_FN static inline
 #endif
 
-typedef struct { float q, cp; int den; } prow_terms;   /* mean value, cpuct * prior, visits + claims in flight + 1 */
-
-/* Terms of a lane.  A lane without an edge has loaded a slot that nobody may have written yet: none of its words counts, and
- * its score is finite and below that of every edge (whose terms are below 1e30 and whose den is positive). */
-PROW_FN prow_terms prow_terms_of(int has_edge, float q, float cp, int den) {
-    prow_terms t;
-    t.q = has_edge ? q : -FLT_MAX;
-    t.cp = has_edge ? cp : 0.0f;
-    t.den = has_edge ? den : 1;
-    return t;
-}
-
-PROW_FN float prow_score(prow_terms t, float sqrt_parent) { return t.q + t.cp * sqrt_parent / (float)t.den; }
-
-/* Order-preserving integer image of a finite score; -0.0f counts as +0.0f. */
-PROW_FN uint32_t prow_image(float score) {
-    const float s = score + 0.0f;
-    uint32_t b;
-    memcpy(&b, &s, sizeof b);
-    return b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
-}
+/* The terms of a lane's score: mean value, cpuct * prior, and visits + claims in flight + 1.  A lane without an edge has loaded a
+ * slot that nobody may have written yet: none of its words counts, and its score is finite and below that of every edge (whose
+ * terms are below 1e30 and whose denominator is positive). */
+PROW_FN float prow_q(int has_edge, float q) { return has_edge ? q : -FLT_MAX; }
+PROW_FN float prow_cp(int has_edge, float cp) { return has_edge ? cp : 0.0f; }
+PROW_FN int prow_den(int has_edge, int den) { return has_edge ? den : 1; }
+PROW_FN float prow_score(float q, float cp, float sqrt_parent, int den) { return q + cp * sqrt_parent / (float)den; }
 #endif
