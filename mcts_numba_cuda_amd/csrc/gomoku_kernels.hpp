@@ -54,8 +54,9 @@ template <int W> struct Board {
 //     takes the place the list has just given up: entry E - 1 - k is the cell of ply k in the end.
 //   * To find the end of 64 playouts the workgroup scatters the plies into a board of times T (one row of 64 entries per
 //     cell; stones that were there before count as times 0 and 1, ply k as k + 2; the parity of a time is its colour), makes
-//     a bit mask of the odd times per board row, and ANDs the masks of both colours into the starts of all runs of five
-//     same-coloured cells on the full board.  Of the 572 windows of a 15 x 15 board about 36 are such candidates.  A
+//     bit masks of the odd and of the even times per board row, and ANDs the masks of both colours into the starts of all runs
+//     of five same-coloured cells.  Of the 572 windows of a 15 x 15 board about 36 are such candidates on the full board, about
+//     14 by the limit up to which they are looked for first (time_offset).  A
 //     candidate is complete at the latest of its five times, and it is exactly five (the reference's rule) if neither
 //     neighbouring cell held its colour by then: seven reads and a dozen instructions.  The earliest complete five is the
 //     end of the game.  A wavefront takes one of the four directions.
@@ -90,6 +91,18 @@ __host__ __device__ inline PlayoutShape playout_shape(int m, int n, bool wide) {
 __host__ __device__ inline size_t playout_lds_bytes(int m, int n, int slots, int teams, bool wide) {
     const PlayoutShape s = playout_shape(m, n, wide);
     return ((size_t)s.list_rows * slots + (size_t)s.time_rows * 64 * teams) * (wide ? 2 : 1);
+}
+// Few games last until the board is nearly full: one in a thousand ends with more stones on the board than 60 and 9 / 16 of
+// its cells (186 of 225; one in two with 113).  So find_ends looks at the runs that are complete by then first, (186 / 225)^5 =
+// 0.4 of the candidates and (263 / 361)^5 = 0.2 of those of 19 x 19, and looks again, at all of them, where 64 playouts hold a game that
+// outlasted the limit.  ms a search with the base at 50 / 60 / 70: one child, 15 x 15, 4 x 128, 48.3 / 46.6 / 46.6 (49.4
+// without a limit and with the parities read a playout at a time); all children, 8 x 128, 40.8 / 39.5 / 39.8 (44.7); 19 x 19, 4 x 128, 13.9 / 13.2 / 13.1 (14.5).
+// Times are written with an even offset that gives those beyond the limit a mark of their own, the two upper bits of a byte or
+// the uppermost of 16; 0: no limit, where it would spare nothing (boards of up to 155 cells, a few plies).
+__host__ __device__ inline uint32_t time_offset(int cells, int E, bool wide) {
+    const int before = cells - E, stones = 60 + cells * 9 / 16, top = wide ? 0x7fff : 0xbf;
+    const int last = (stones - before) | 1, kept = last < top - 2 ? last : top - 2;   // time of the last ply within the limit: odd
+    return stones >= cells - 8 || last < E / 2 || (!wide && E + 1 + top - kept > 0xfe) ? 0u : (uint32_t)(top - kept);
 }
 constexpr int kLevels = 8;         // path levels whose arg-max the backup evaluates together
 constexpr int kPrepLevels = 48;    // path levels whose arg-max the one-child variants prepare during the playouts (deeper paths: as above)
@@ -430,10 +443,10 @@ __device__ __forceinline__ float make_offsets(u32x2 *ring, uint32_t *made, const
 // become free, as in draw_list, or (DIRECT) their times go straight to the board of times.  A draw's two reads are issued before
 // the writes of the draw before it, and put right where they crossed them.
 template <class Cell, bool DIRECT>
-__device__ __forceinline__ void walk_list(Cell *list, Cell *my_times, const u32x2 *ring, const uint32_t *made, uint32_t *taken, RingWait await, int count) {
+__device__ __forceinline__ void walk_list(Cell *list, Cell *my_times, const u32x2 *ring, const uint32_t *made, uint32_t *taken, RingWait await, int count, uint32_t time) {
     constexpr uint32_t kRow = 64 * sizeof(Cell);   // bytes of a row
     Cell *last = list + (count - kChunk) * 64;     // the lowest of the next sixteen places that the list gives up
-    uint32_t time = 2, last_row = (uint32_t)(count - 1) * kRow;
+    uint32_t last_row = (uint32_t)(count - 1) * kRow;
     const int whole = count & ~(kChunk - 1);
     auto at = [=](uint32_t offset) -> Cell * { return reinterpret_cast<Cell *>(reinterpret_cast<unsigned char *>(list) + offset); };
     for (int k0 = 0; k0 < whole; k0 += kChunk) {
@@ -479,7 +492,7 @@ __device__ __forceinline__ void walk_list(Cell *list, Cell *my_times, const u32x
 // The runs of five along one direction (DIR 0: right, 1: down, 2: down right, 3: up right) of one playout on the full board,
 // and the earliest ply whose stone made one of them an exact five (all ones: none).  masks: see find_ends.
 template <int W, int DIR>
-__device__ __forceinline__ uint32_t earliest_five(const uint32_t *masks, uint32_t *starts, const typename Board<W>::Cell *my_times, const PlayoutShape &shape) {
+__device__ __forceinline__ uint32_t earliest_five(const uint32_t *masks, uint32_t *starts, const typename Board<W>::Cell *my_times, const PlayoutShape &shape, uint32_t offset /* of the times */) {
     using Cell = typename Board<W>::Cell;
     constexpr bool WIDE = Board<W>::kWide;
     constexpr int kWords = WIDE ? 2 : 1, kRows = WIDE ? kMaxRowsWide : 16, kLines = DIR == 0 ? kRows : kRows - 4;
@@ -537,21 +550,22 @@ __device__ __forceinline__ uint32_t earliest_five(const uint32_t *masks, uint32_
             // ("never", beside the board, is later than any time); a run of stones from before the playout is no end of it
             // (its last - 2 is no ply but a number beyond all plies)
             const bool longer = min((last - n0) & 0x80000001u, (last - n1) & 0x80000001u) == 0;
-            end = min(end, longer ? ~0u : last - 2u);
+            end = min(end, longer ? ~0u : last - (2u + offset));
         }
     }
     return end;
 }
 
 // Where the games of 64 playouts end, by a team of wavefronts of which this is number `wave` (every thread of the workgroup
-// calls it; two barriers inside, one at the end).  If there is something to do for the team: `list` holds the finished
+// calls it; all end up on the same barriers).  If there is something to do for the team: `list` holds the finished
 // orders of E cells each, `times` is the team's board of times at cell 0 (timed: the drawn cells' times are there already), own_row the row of the one stone that playout
 // `lane` has beside its node's (of the side that does not move first; ~0: none).  ends[lane] becomes the ply whose stone
-// completes the first exact five of playout `lane`, all ones (or a number beyond all plies) if there is none.  The lists
-// are used up.
+// completes the first exact five of playout `lane`, all ones (or a number beyond all plies) if there is none; 0 for a playout that
+// is not wanted.  ends is one of the `teams` rows of all_ends, null beside them; offset as time_offset gives it.  The lists are used up.
 template <int W>
 __device__ __forceinline__ void find_ends(bool work, bool timed, typename Board<W>::Cell *list, typename Board<W>::Cell *times, uint32_t *ends,
-                                          const PlayoutShape &shape, int E, uint32_t own_row, bool flip, int wave, int nwaves, int lane) {
+                                          const PlayoutShape &shape, int E, uint32_t own_row, bool flip, int wave, int lane,
+                                          bool wanted, const uint32_t (*all_ends)[64], int teams, uint32_t offset) {
     using Cell = typename Board<W>::Cell;
     constexpr bool WIDE = Board<W>::kWide;
     constexpr int kWords = WIDE ? 2 : 1;   // mask words of a board row: even and odd times, as halves of one dword on narrow boards
@@ -561,68 +575,104 @@ __device__ __forceinline__ void find_ends(bool work, bool timed, typename Board<
     Cell *const my_times = times + lane;
     uint32_t *const masks = reinterpret_cast<uint32_t *>(list) + lane;   // [kRows + 1][kWords][64], in the lists' place
     uint32_t *const starts = masks + (kRows + 1) * kWords * 64;          // of the directions across rows: [3][kRows - 3][64]
+    bool first = true;
     if (work && !timed) {
         const Cell *from = list + (wave * 64 + lane);
-        uint32_t t = (uint32_t)(E + 1 - wave);   // entry i is ply E - 1 - i
+        uint32_t t = (uint32_t)(E + 1 - wave) + offset;   // entry i is ply E - 1 - i
         int i = wave;
-        for (; i + (kBatch - 1) * nwaves < E; i += kBatch * nwaves) {
+        for (; i + (kBatch - 1) * 4 < E; i += kBatch * 4) {
             uint32_t row[kBatch];
 #pragma unroll
-            for (int k = 0; k < kBatch; k++) row[k] = from[k * nwaves * 64];
+            for (int k = 0; k < kBatch; k++) row[k] = from[k * 4 * 64];
 #pragma unroll
-            for (int k = 0; k < kBatch; k++) my_times[row[k] * 64] = (Cell)(t - k * nwaves);
-            from += kBatch * nwaves * 64; t -= kBatch * nwaves;
+            for (int k = 0; k < kBatch; k++) my_times[row[k] * 64] = (Cell)(t - k * 4);
+            from += kBatch * 4 * 64; t -= kBatch * 4;
         }
-        for (; i < E; i += nwaves) { my_times[(uint32_t)*from * 64] = (Cell)t; from += nwaves * 64; t -= nwaves; }
+        for (; i < E; i += 4) { my_times[(uint32_t)*from * 64] = (Cell)t; from += 4 * 64; t -= 4; }
     }
-    if (work && wave == 0 && own_row != ~0u) my_times[own_row * 64] = 1;
+    if (work && wave == 0 && own_row != ~0u) my_times[own_row * 64] = (Cell)(offset + 1);
     __syncthreads();
-    if (work) {
-        const uint32_t full = cols == 32 ? ~0u : (1u << cols) - 1u;
-        // (parities come in from the top of the word, N cells of a row at a time, so that all their times are read together; the
-        // columns of a wide board are 16 to 32)
-        auto odd_times = [&](int r, auto n) __attribute__((always_inline)) -> uint32_t {
-            constexpr int N = decltype(n)::value;
-            const Cell *const t = my_times + r * stride * 64;
-            uint32_t time[N], odd = 0;
+    const uint32_t full = cols == 32 ? ~0u : (1u << cols) - 1u;
+    for (bool limited = offset != 0;; limited = false) {
+        if (work) {
+            if constexpr (WIDE) {
+                // (marks and parities go through words, N cells of a row at a time, so that all their times are read together; the
+                // columns of a wide board are 16 to 32)
+                auto mask_row = [&](int r, auto n) __attribute__((always_inline)) {
+                    constexpr int N = decltype(n)::value;
+                    const int16_t *const t = reinterpret_cast<const int16_t *>(my_times) + r * stride * 64;
+                    int32_t time[N]; uint32_t odd = 0, late = 0;
 #pragma unroll
-            for (int k = 0; k < N; k++) time[k] = t[k * 64];
+                    for (int k = 0; k < N; k++) time[k] = t[k * 64];
 #pragma unroll
-            for (int k = 0; k < N; k++) odd = __builtin_amdgcn_alignbit(time[k], odd, 1);
-            return odd >> (32 - N);
-        };
-        if constexpr (WIDE) {
-            for (int r = wave; r < rows; r += nwaves) {
-                const uint32_t odd = cols <= 16 ? odd_times(r, std::integral_constant<int, 16>{}) : cols <= 24 ? odd_times(r, std::integral_constant<int, 24>{})
-                                                                                                                : odd_times(r, std::integral_constant<int, 32>{});
-                masks[2 * r * 64] = ~odd & full; masks[(2 * r + 1) * 64] = odd & full;
+                    for (int k = 0; k < N; k++) odd = __builtin_amdgcn_alignbit((uint32_t)time[k], odd, 1);
+#pragma unroll
+                    for (int k = N - 1; k >= 0; k--) late = __builtin_amdgcn_alignbit(late, (uint32_t)time[k], 31);
+                    odd >>= 32 - N;
+                    const uint32_t seen = limited ? full & ~late : full;
+                    masks[2 * r * 64] = seen & ~odd; masks[(2 * r + 1) * 64] = seen & odd;
+                };
+                for (int r = wave; r < rows; r += 4) {
+                    if (cols <= 16) mask_row(r, std::integral_constant<int, 16>{});
+                    else if (cols <= 24) mask_row(r, std::integral_constant<int, 24>{});
+                    else mask_row(r, std::integral_constant<int, 32>{});
+                }
+            } else {
+                // A lane reads one row of four playouts, a dword a cell: a quarter of the reads of a playout a lane, and two
+                // instructions a cell for the parities of four.  The four rows of a wavefront start at different columns, or their
+                // lanes would meet in the same banks.
+                const int r = wave * 4 + (lane >> 4), skew = lane >> 4;
+                const uint32_t *const t = reinterpret_cast<const uint32_t *>(times) + r * 256 + (lane & 15);
+                uint32_t time[16], odd[2] = {0, 0}, late[2] = {0, 0};
+#pragma unroll
+                for (int k = 0; k < 16; k++) time[k] = t[((k + skew) & 15) * 16];
+#pragma unroll
+                for (int k = 0; k < 16; k++) {
+                    odd[k / 8] |= (time[k] & 0x01010101u) << (k & 7);
+                    late[k / 8] |= (time[k] & (time[k] << 1) & 0x80808080u) >> (7 - (k & 7));
+                }
+                typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+                u32x4 word;
+                const uint32_t both = full | (full << 16), first_late = limited ? ~0u : 0u;
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const uint32_t sel = 0x04000400u + 0x01010101u * p;   // byte p of both words, twice
+                    uint32_t o = __builtin_amdgcn_perm(odd[1], odd[0], sel), l = __builtin_amdgcn_perm(late[1], late[0], sel) & first_late;
+                    o = __builtin_amdgcn_alignbit(o, o, 32 - skew); l = __builtin_amdgcn_alignbit(l, l, 32 - skew);
+                    word[p] = both & ~l & (o ^ 0xffffu);
+                }
+                *reinterpret_cast<u32x4 *>(reinterpret_cast<uint32_t *>(list) + r * 64 + (lane & 15) * 4) = word;
             }
-        } else {
-#pragma unroll 2
-            for (int r = wave; r < 16; r += nwaves) {
-                const uint32_t odd = odd_times(r, std::integral_constant<int, 16>{});
-                masks[r * 64] = (~odd & full) | ((odd & full) << 16);
+        }
+        if (wave == 0 && first && ends != nullptr) {
+            ends[lane] = work && wanted ? ~0u : 0u;
+            if (work) {
+                for (int c = 0; c < kWords; c++) masks[(kRows * kWords + c) * 64] = 0;   // the empty line beyond all others
+                for (int d = 0; d < 3; d++) starts[(d * (kRows - 3) + kRows - 4) * 64] = 0;
             }
         }
-        if (wave == 0) {
-            ends[lane] = ~0u;
-            for (int c = 0; c < kWords; c++) masks[(kRows * kWords + c) * 64] = 0;   // the empty line beyond all others
-            for (int d = 0; d < 3; d++) starts[(d * (kRows - 3) + kRows - 4) * 64] = 0;
+        __syncthreads();
+        if (work && wanted) {
+            uint32_t end = ~0u;
+            {   // a wavefront a direction; the two teams of a CU in opposite order
+                const int dir = flip ? 3 - wave : wave;
+                if (dir == 0) end = min(end, earliest_five<W, 0>(masks, nullptr, my_times, shape, offset));
+                else if (dir == 1) end = min(end, earliest_five<W, 1>(masks, starts, my_times, shape, offset));
+                else if (dir == 2) end = min(end, earliest_five<W, 2>(masks, starts + (kRows - 3) * 64, my_times, shape, offset));
+                else end = min(end, earliest_five<W, 3>(masks, starts + 2 * (kRows - 3) * 64, my_times, shape, offset));
+            }
+            if (end != ~0u) atomicMin(&ends[lane], end);
         }
+        __syncthreads();
+        if (!limited) break;
+        // games that had not ended by the limit are looked at again, with all times (an end beyond all plies is a run of stones
+        // from before the playout)
+        bool open = false;
+        for (int t = 0; t < teams; t++) open = open || all_ends[t][lane] >= (uint32_t)E;
+        if (__ballot(open) == 0) break;
+        wanted = work && ends[lane] >= (uint32_t)E;
+        first = false;
     }
-    __syncthreads();
-    if (work) {
-        uint32_t end = ~0u;
-        for (int turn = wave; turn < 4; turn += nwaves) {   // a wavefront a direction; the two teams of a CU in opposite order
-            const int dir = flip ? 3 - turn : turn;
-            if (dir == 0) end = min(end, earliest_five<W, 0>(masks, nullptr, my_times, shape));
-            else if (dir == 1) end = min(end, earliest_five<W, 1>(masks, starts, my_times, shape));
-            else if (dir == 2) end = min(end, earliest_five<W, 2>(masks, starts + (kRows - 3) * 64, my_times, shape));
-            else end = min(end, earliest_five<W, 3>(masks, starts + 2 * (kRows - 3) * 64, my_times, shape));
-        }
-        if (end != ~0u) atomicMin(&ends[lane], end);
-    }
-    __syncthreads();
 }
 
 // Arg-max key of a child: UCB, then the reference's tie rule (smallest bit-reversed action index among the maxima of its
@@ -971,12 +1021,13 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
         if (njobs > 0) {
             const int E = empties - (with_stone ? 1 : 0);   // cells that each playout draws
             const int p_shift = __builtin_ctz(P), total = njobs << p_shift;
+            const uint32_t offset = time_offset(cells, E, WIDE);
             // times of the node's stones: 0 for the side to move in the playouts, 1 for the other (they stay until the next step)
             if (team < teams)
             for (int i = tid & 255; i < (cells - empties) * kRowDwords; i += 256) {
                 const uint32_t stone = s_cells[B::kCells - i / kRowDwords];
                 reinterpret_cast<uint32_t *>(team_times)[(int)(stone & 0xffffu) * kRowDwords + i % kRowDwords] =
-                    (stone >> 31) == (pturn == -1 ? 1u : 0u) ? 0u : kCopies;
+                    ((stone >> 31) == (pturn == -1 ? 1u : 0u) ? offset : offset + 1u) * kCopies;
             }
             for (int round0 = 0; round0 < total; round0 += nslots) {
                 // the job of playout i of the sequence (slots beyond the last repeat it, to no effect), and its child's ordinal
@@ -1029,8 +1080,8 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
                 } else if (wave < 2 * n_makers) {
                     const int grp = wave - n_makers;
                     const u32x2 *const ring = s_ring + grp * (kRingBytes / 8) + lane;
-                    if (timed) walk_list<Cell, true>(my_list, s_times + (grp * shape.time_rows + shape.origin) * 64 + lane, ring, &s_made[grp], &s_taken[grp], ring_wait, E);
-                    else walk_list<Cell, false>(my_list, nullptr, ring, &s_made[grp], &s_taken[grp], ring_wait, E);
+                    if (timed) walk_list<Cell, true>(my_list, s_times + (grp * shape.time_rows + shape.origin) * 64 + lane, ring, &s_made[grp], &s_taken[grp], ring_wait, E, offset + 2u);
+                    else walk_list<Cell, false>(my_list, nullptr, ring, &s_made[grp], &s_taken[grp], ring_wait, E, 0u);
                 } else if (round0 == 0) {
                     const int first = 2 * n_makers;
                     if (deferred) create_children(tid - first * 64, nthreads - first * 64, chosen_j);
@@ -1049,8 +1100,9 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
                 const int groups = (min(nslots, total - round0) + 63) >> 6;
                 for (int g0 = 0; g0 < groups; g0 += teams) {
                     const int grp = g0 + team;
-                    find_ends<W>(grp < groups && team < teams, timed, s_list + (size_t)grp * shape.list_rows * 64, team_times, s_end[team < teams ? team : 0], shape, E,
-                                 with_stone ? time_row((uint32_t)s_actions[ordinal_of(round0 + grp * 64 + lane)]) : ~0u, (team & 1) != 0, wave & 3, min(nwaves, 4), lane);
+                    find_ends<W>(grp < groups && team < teams, timed, s_list + (size_t)grp * shape.list_rows * 64, team_times, team < teams ? s_end[team] : nullptr, shape, E,
+                                 with_stone ? time_row((uint32_t)s_actions[ordinal_of(round0 + grp * 64 + lane)]) : ~0u, (team & 1) != 0, wave & 3, lane,
+                                 round0 + grp * 64 + lane < total, s_end, teams, offset);
                     if (wave - g0 < teams && wave >= g0 && wave < groups) end_ply = s_end[wave - g0][lane];
                 }
 

@@ -29,3 +29,18 @@ def test_playouts_at_the_edges_of_their_formats(m, n, stones, variant, trees, pl
     for _ in range(2):
         board, turn = random_gomoku_root(rng, m, n, stones)
         compare_with_oracle(e, o, board, None, turn, steps)
+
+
+# boards around the fewest cells for which ends are looked for up to a limit first (155 and 156), the largest ones whose marked
+# times fit a byte, roots that leave few plies to the limit, and enough playouts that many outlast it
+LONG_GAMES = [
+    (5, 31, 0, "acp_prodigal", 2, 64, 4), (12, 13, 0, "ocp_thrifty", 4, 256, 12), (12, 13, 30, "acp_thrifty", 3, 64, 6), (13, 13, 60, "acp_prodigal", 2, 128, 4),
+    (15, 15, 0, "ocp_prodigal", 4, 256, 16), (15, 15, 90, "acp_prodigal", 2, 64, 6), (15, 15, 14, "acp_thrifty", 2, 32, 8), (16, 15, 0, "acp_thrifty", 1, 64, 5),
+    (15, 16, 1, "ocp_thrifty", 3, 128, 12), (16, 16, 0, "acp_prodigal", 1, 64, 4), (19, 19, 100, "acp_prodigal", 1, 32, 3), (19, 19, 2, "ocp_thrifty", 4, 128, 12),
+    (22, 23, 0, "ocp_thrifty", 2, 256, 6),
+]
+
+
+@pytest.mark.parametrize("m,n,stones,variant,trees,playouts,steps", LONG_GAMES)
+def test_games_that_outlast_the_first_look_for_their_end(m, n, stones, variant, trees, playouts, steps):
+    test_playouts_at_the_edges_of_their_formats(m, n, stones, variant, trees, playouts, steps)
