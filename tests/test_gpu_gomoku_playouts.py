@@ -31,14 +31,15 @@ def test_playouts_at_the_edges_of_their_formats(m, n, stones, variant, trees, pl
         compare_with_oracle(e, o, board, None, turn, steps)
 
 
-# boards around the fewest cells for which ends are looked for up to a limit first (155 and 156), the largest ones whose marked
-# times fit a byte, roots that leave few plies to the limit, and enough playouts that many outlast it
+# boards around the fewest cells for which ends are looked for up to a limit first (169 and 170), the largest ones whose marked
+# times fit a byte, roots that leave few plies to the limit, draws on either side of a chunk and of what is worth leaving, more
+# groups of 64 playouts than boards of times, and enough playouts that many outlast the limit
 LONG_GAMES = [
-    (5, 31, 0, "acp_prodigal", 2, 64, 4), (12, 13, 0, "ocp_thrifty", 4, 256, 12), (12, 13, 30, "acp_thrifty", 3, 64, 6), (13, 13, 60, "acp_prodigal", 2, 128, 4),
+    (10, 17, 0, "acp_prodigal", 2, 64, 4), (13, 13, 0, "ocp_thrifty", 4, 256, 12), (13, 13, 30, "acp_thrifty", 3, 64, 6), (13, 14, 60, "acp_prodigal", 2, 128, 4),
     (15, 15, 0, "ocp_prodigal", 4, 256, 16), (15, 15, 90, "acp_prodigal", 2, 64, 6), (15, 15, 14, "acp_thrifty", 2, 32, 8), (16, 15, 0, "acp_thrifty", 1, 64, 5),
     (15, 16, 1, "ocp_thrifty", 3, 128, 12), (16, 16, 0, "acp_prodigal", 1, 64, 4), (19, 19, 100, "acp_prodigal", 1, 32, 3), (19, 19, 2, "ocp_thrifty", 4, 128, 12),
-    (22, 23, 0, "ocp_thrifty", 2, 256, 6),
-]
+    (22, 23, 0, "ocp_thrifty", 2, 256, 6), (16, 14, 0, "ocp_prodigal", 300, 128, 4), (15, 15, 9, "ocp_thrifty", 2, 512, 12), (32, 16, 40, "ocp_prodigal", 1, 256, 6),
+] + [(15, 14, stones, "ocp_thrifty", 3, 256, 5) for stones in (20, 27, 28, 100, 130, 140)] + [(17, 17, stones, "ocp_prodigal", 3, 128, 5) for stones in (0, 7, 150, 200)]
 
 
 @pytest.mark.parametrize("m,n,stones,variant,trees,playouts,steps", LONG_GAMES)
