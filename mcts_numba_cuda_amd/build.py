@@ -1,5 +1,6 @@
 """Builds libmctsnc_hip.so (search engine) and libpuct_hip.so (PUCT select/backup) for gfx950 with hipcc, and _puct_call
 (the Python side of a PUCT launch, host code only) with the C compiler, in-tree, next to this file."""
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -58,8 +59,26 @@ def build_host_module(verbose=False, optional=False):
         return None
     if missing:
         raise RuntimeError(f"{os.path.basename(HOST_MODULE)} cannot be built: {missing}")
-    run(compiler.split() + ["-O2", "-Wall", "-fPIC", "-shared", "-I" + include, "-o", HOST_MODULE, os.path.join(CSRC, "puct_call.c")], "the C compiler", verbose)
+    command = compiler.split() + ["-O2", "-Wall", "-fPIC", "-shared", "-I" + include, "-o", HOST_MODULE, os.path.join(CSRC, "puct_call.c")]
+    exchange = dlpack_flags()
+    try:
+        run(command + exchange, "the C compiler", verbose)
+    except RuntimeError:
+        if not exchange:
+            raise
+        run(command, "the C compiler", verbose)   # (without torch's exchange table: by the tensors' attributes)
     return HOST_MODULE
+
+
+def dlpack_flags():
+    """Flags with which _puct_call reads tensors through the exchange table that torch publishes, where torch's DLPack header has it."""
+    spec = importlib.util.find_spec("torch")
+    include = os.path.join(os.path.dirname(spec.origin), "include") if spec is not None and spec.origin else ""
+    header = os.path.join(include, "ATen", "dlpack.h")
+    if not include or not os.path.exists(header):
+        return []
+    with open(header, errors="replace") as f:
+        return ["-I" + include, "-DPUCT_CALL_DLPACK=<ATen/dlpack.h>"] if "DLPackExchangeAPI" in f.read() else []
 
 
 def build_one(lib, sources, verbose=False):

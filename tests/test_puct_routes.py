@@ -101,22 +101,26 @@ def outcome(library, launcher, d, v):
     return None, "", list(library.calls)
 
 
+@pytest.mark.parametrize("table", [False, True])
 @pytest.mark.parametrize("launcher", LAUNCHERS)
-def test_both_routes_take_and_refuse_the_same(library, monkeypatch, launcher):
-    accepted = refused = 0
+def test_both_routes_take_and_refuse_the_same(library, monkeypatch, launcher, table):
+    """table: the tensors are described by an exchange table, as torch's are, else by their attributes."""
+    accepted = refused = asked = 0
     for code in (0, 700):
         library.code[0] = code
         for what, d, v in spoilt():
-            with pr.routes() as call:
+            described = [] if table else None
+            with pr.routes(described=described) as call:
                 if call is None:
                     pytest.skip("_puct_call is not built")
                 by_c = outcome(library, launcher, d, v)
                 puct._puct_call = None
                 by_python = outcome(library, launcher, d, v)
+            asked += len(described or ())
             assert by_c == by_python, what
             assert (by_c[0] is None) == (len(by_c[2]) == 1 and code == 0), what
             accepted, refused = accepted + len(by_c[2]), refused + (not by_c[2])
-    assert accepted > 2 and refused > 2
+    assert accepted > 2 and refused > 2 and (asked > 100 or not table or not build.dlpack_flags())
 
 
 @pytest.mark.parametrize("launcher", LAUNCHERS)
