@@ -836,25 +836,34 @@ struct BackupArgs {
 // src/puct/test_puct_gpu_v3.py:297-302.
 template <bool NODE_LEVEL>
 __device__ __forceinline__ void backup_traversal(const BackupArgs &a, int tree, int wid, int lane) {
-    const int node_limit = a.node_count[tree];
-    if (node_limit <= 0 || node_limit > a.nodes || node_limit > PUCT_PACKED_NODE_LIMIT) return;
-
+    // All that a path of up to 64 levels needs is requested at once: a launch of few traversals is as long as its chain of loads,
+    // which was four long, each asked for when the one before was known to matter (16 trees x 8 traversals 3.5 -> 2.7 us, 1024 x 8
+    // 4.1 -> 3.8).
     const size_t out = (size_t)tree * a.warps + wid;
-    const int raw = a.out_selected_node[out];
+    const int *const path = a.out_path_eids + out * a.path_depth;
+    const float *const values = a.path_edge_values == nullptr ? nullptr : a.path_edge_values + out * a.path_depth;
+    const int node_limit = a.node_count[tree], raw = a.out_selected_node[out], plen = a.out_path_len[out];
+    int encoded = lane < a.path_depth ? path[lane] : -1;
+    float value = values != nullptr && lane < a.path_depth ? values[lane] : 0.0f;
+    asm volatile("" ::: "memory");
+    if (node_limit <= 0 || node_limit > a.nodes || node_limit > PUCT_PACKED_NODE_LIMIT) return;
     if (raw < 0) return;
     const int kind = NODE_LEVEL ? raw >> PUCT_PACKED_KIND_SHIFT : (raw >> PUCT_PACKED_KIND_SHIFT) & PUCT_PACKED_KIND_MASK;
     if (kind == PUCT_SELECT_INVALID) return;
     if (!NODE_LEVEL && kind == PUCT_SELECT_BUSY) return;
-    const int plen = a.out_path_len[out];
     if (plen <= 0) return;
 
     int edge_count = plen - 1;
     if (edge_count > a.path_depth) edge_count = a.path_depth;
-    const int *path = a.out_path_eids + out * a.path_depth;
     for (int d = lane; d < edge_count; d += kWave) {
-        const int encoded = path[d];
-        if (encoded < 0) continue;
-        const int parent = encoded >> 8, slot = encoded & 0xFF;
+        const int here = encoded;
+        const float v = value;
+        if (d + kWave < edge_count) {   // (the next 64 levels, on their way meanwhile)
+            encoded = path[d + kWave];
+            if (values != nullptr) value = values[d + kWave];
+        }
+        if (here < 0) continue;
+        const int parent = here >> 8, slot = here & 0xFF;
         if (parent >= node_limit || slot >= a.edges) continue;
         const size_t e = ((size_t)tree * a.nodes + parent) * a.edges + slot;
         if (NODE_LEVEL) {
@@ -864,9 +873,9 @@ __device__ __forceinline__ void backup_traversal(const BackupArgs &a, int tree, 
         } else {
             atomicSub(&a.edge_inflight[e], a.virtual_loss);
         }
-        if (a.path_edge_values != nullptr) {
+        if (values != nullptr) {
             atomicAdd(&a.edge_N[e], 1);
-            unsafeAtomicAdd(&a.edge_W[e], a.path_edge_values[out * a.path_depth + d]);
+            unsafeAtomicAdd(&a.edge_W[e], v);
         }
     }
 

@@ -46,7 +46,7 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) __attribute__((amdgpu_wav
 
 template <bool NODE_LEVEL>
 __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void backup_kernel(const BackupArgs a) {
-    const int wid = blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave;
+    const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave);   // the same in all lanes
     if (wid >= a.warps) return;
     backup_traversal<NODE_LEVEL>(a, blockIdx.x, wid, threadIdx.x & (kWave - 1));
 }
