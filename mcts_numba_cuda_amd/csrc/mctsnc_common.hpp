@@ -67,6 +67,14 @@ __device__ __forceinline__ void rng_advance32(Rng32 &r) {
     r.s1l = __builtin_amdgcn_alignbit(th, tl, 28); r.s1h = __builtin_amdgcn_alignbit(tl, th, 28);
 }
 
+// The state before a draw that led to (s0, s1).
+__device__ __forceinline__ void rng_back(uint64_t &s0, uint64_t &s1) {
+    const uint64_t t = rotl64(s1, 64 - 36);
+    const uint64_t r = s0 ^ t ^ (t << 14);
+    s0 = rotl64(r, 64 - 55);
+    s1 = t ^ s0;
+}
+
 __device__ __forceinline__ void rng_next32(Rng32 &r, uint32_t &out_lo, uint32_t &out_hi) {
     const uint64_t sum = (((uint64_t)r.s0h << 32) | r.s0l) + (((uint64_t)r.s1h << 32) | r.s1l);
     out_lo = (uint32_t)sum; out_hi = (uint32_t)(sum >> 32);
@@ -95,6 +103,22 @@ __device__ __forceinline__ uint32_t max_over_8_lanes(uint32_t key) {
     o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key, 0x4E, 0xf, 0xf, true); key = o > key ? o : key;
     o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key, 0x141, 0xf, 0xf, true); key = o > key ? o : key;
     return key;
+}
+
+// The same for the bits set in any of them.
+__device__ __forceinline__ uint32_t or_over_8_lanes(uint32_t bits) {
+    bits |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)bits, 0xB1, 0xf, 0xf, true);
+    bits |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)bits, 0x4E, 0xf, 0xf, true);
+    bits |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)bits, 0x141, 0xf, 0xf, true);
+    return bits;
+}
+
+// A pointer read from memory, known to point to device memory: it is then not looked up among LDS and scratch addresses too
+// (a "flat" access, which is slower and waits for LDS accesses as well).
+template <class T>
+__device__ __forceinline__ T *device_memory(T *const &p) {
+    typedef __attribute__((address_space(1))) T *Pointer;
+    return (T *)*reinterpret_cast<const Pointer *>(&p);
 }
 
 // ---- agent-scope synchronisation between workgroups --------------------------------------------

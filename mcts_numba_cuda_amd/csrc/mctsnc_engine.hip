@@ -517,7 +517,7 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
     HIP_TRY(hipStreamSynchronize(stream));
 
     c4::SearchArgs args;
-    args.refs = d_refs; args.n_refs = n_refs; args.m = c.board_m; args.n = c.board_n; args.P = c.n_playouts; args.G = e0->G;
+    args.refs = d_refs; args.n_refs = n_refs; args.m = c.board_m; args.n = c.board_n; args.P = c.n_playouts; args.G = e0->G; args.parts = 1;
     args.S = (int32_t)c.max_tree_size; args.thrifty = e0->thrifty ? 1 : 0; args.ucb_c = c.ucb_c; args.abort_flag = e0->d_abort;
     args.stage_timing = e0->stage_timing ? 1 : 0;
     const int *opt = e0->options;
@@ -569,10 +569,23 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
     // all children, 32 playouts, 4 trees 10.1 / 9.2 / 9.4 / 9.6, 64 playouts 10.0 / 9.2 / 9.3 / 9.5 (more to meet at each barrier).
     const unsigned least_threads = e0->acp ? 128 : 256;
     if (!solo && !team_pool && block.x < least_threads && e0->G * n_refs <= cus_now) block = dim3(least_threads);
+    // Playouts split over wavefronts (see c4::Split), while every workgroup has a CU to itself: 64 of them to a workgroup, so
+    // a column of a team has up to four.  28 workgroups take 0.4 us longer than 7 to exchange a step's results, so the longest
+    // playouts must be long enough: with fewer than 16 cells left on the boards on average, most of such searches lose 2 to 5 %
+    // (6 x 7, 4 trees of 64 to 256: 0.95 to 1.01 of the time at 8 to 16 cells, 1.05 at 24; 5 x 6, one tree of 256, 8 / 12 / 16 / 18 /
+    // 20 / 24 cells: 0.95 / 0.99 / 0.99 / 1.06 / 1.08 / 1.17).
+    const int parts = e0->acp ? std::max(1, c.n_playouts / kWave) : 1;
+    int64_t stones = 0;
+    for (int r = 0; r < n_refs; r++) stones += __builtin_popcountll(bb[2 * (size_t)r]) + __builtin_popcountll(bb[2 * (size_t)r + 1]);
+    const bool split = !solo && !team_pool && (e0->acp ? e0->G * parts <= c4::kMaxWide && (int64_t)n_refs * mn - stones >= (int64_t)16 * n_refs : c.n_playouts <= kWave) &&
+                       e0->G * parts * (8 * ((n_refs + 7) / 8)) <= cus_now;
+    if (split) { args.G = e0->G * parts; args.parts = parts; block = dim3(c4::kSplitThreads); }
     const size_t lds = solo ? c4::solo_lds_bytes(c.board_m, c.board_n, c.n_playouts)
-                            : (team_pool ? c4::team_pool_lds_bytes(c.board_m, c.board_n, c.n_playouts) : c4::search_lds_bytes(c.board_m, c.board_n));
+                            : (team_pool ? c4::team_pool_lds_bytes(c.board_m, c.board_n, c.n_playouts)
+                               : split   ? c4::split_lds_bytes(c.board_m, c.board_n) : c4::search_lds_bytes(c.board_m, c.board_n));
     const auto solo_kernel = c4::search_kernel_solo;
-    const auto team_kernel = team_pool ? c4::search_kernel_team_pool : c4::search_kernel<true>;
+    const auto team_kernel = team_pool ? c4::search_kernel_team_pool : split ? c4::search_kernel_split<true> : c4::search_kernel<true>;
+    const auto one_child_kernel = split ? c4::search_kernel_split<false> : c4::search_kernel<false>;
     if (solo) HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(solo_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     // Sets of G workgroups (8 sets per grid row, one per XCD).  The all-children kernel is launched cooperatively, so
     // all its workgroups must be resident together: a batch with more trees than resident sets starts one tree per
@@ -624,7 +637,7 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
                 }
             }
         } else {
-            hipLaunchKernelGGL(c4::search_kernel<false>, grid, block, lds, stream, args);
+            hipLaunchKernelGGL(one_child_kernel, grid, block, lds, stream, args);
             HIP_TRY(hipGetLastError());
         }
         return MCTSNC_OK;

@@ -1,7 +1,8 @@
 """Connect 4 playouts at the edges of their two board layouts, engine against oracle, every array bit for bit (two searches
 in a row): boards whose columns each fit one of the two words and whose fours start in the lower one (4 x 4 to 7 x 7, a lower
 word of four to six columns, with and without free bits below them), the first ones that miss either condition, by teams, by
-one workgroup per tree and by teams with playout pools; and searches long enough to meet draws rounded up to 1.0f."""
+one workgroup per tree and by teams with playout pools; and searches long enough to meet draws rounded up to 1.0f; playouts
+split over wavefronts, in each number of workgroups to a column, on full and nearly decided boards."""
 import numpy as np
 import pytest
 
@@ -37,4 +38,25 @@ def test_draws_rounded_up_are_replayed(m, n, plies, variant, seed, steps):
         e = make_engine(params, board_shape=(m, n), extra=n, actions=n, options=options)
         o = Oracle("c4", (m, n), n, n, 4, 512, variant, ucb_c=2.0, seed=seed, device_memory=0.3, threads=8)
         compare_with_oracle(e, o, *random_c4_root(np.random.default_rng(seed), plies, m, n), steps=steps)
+        assert o.u1_events > 0
+
+
+SPLIT = [  # rows, columns, variant, trees, playouts, plies, steps, memory (GiB), seed
+    (6, 7, "acp_prodigal", 4, 256, 0, 150, 0.3, 5), (7, 8, "acp_thrifty", 4, 256, 0, 150, 0.3, 5), (6, 7, "ocp_thrifty", 8, 64, 0, 900, 0.3, 5),
+    (8, 6, "ocp_prodigal", 9, 32, 1, 400, 0.3, 1), (4, 4, "ocp_thrifty", 1, 1, 9, 200, 0.1, 2), (6, 7, "acp_thrifty", 8, 128, 5, 200, 0.3, 3),
+    (4, 4, "acp_prodigal", 3, 64, 0, 700, 0.1, 4), (5, 8, "acp_prodigal", 2, 128, 22, 400, 0.1, 6), (6, 7, "acp_prodigal", 2, 256, 26, 1500, 0.1, 7),
+    (6, 7, "acp_thrifty", 4, 256, 26, 900, 0.001, 8), (7, 4, "acp_prodigal", 8, 2, 3, 300, 0.1, 9),
+]
+
+
+@pytest.mark.parametrize("m,n,variant,trees,playouts,plies,steps,memory,seed", SPLIT)
+def test_playouts_split_over_wavefronts(m, n, variant, trees, playouts, plies, steps, memory, seed):
+    """The first three meet a draw rounded up to 1.0f; those with many stones end at terminal nodes for long stretches, in which
+    teams stop exchanging results; the one with little memory fills its pool."""
+    params = dict(n_trees=trees, n_playouts=playouts, variant=variant, device_memory=memory, ucb_c=2.0, seed=seed)
+    e = make_engine(params, board_shape=(m, n), extra=n, actions=n)
+    o = Oracle("c4", (m, n), n, n, trees, playouts, variant, ucb_c=2.0, seed=seed, device_memory=memory, threads=8)
+    for extra in (0, 1):
+        compare_with_oracle(e, o, *random_c4_root(np.random.default_rng(seed + extra), plies, m, n), steps=steps)
+    if seed == 5:
         assert o.u1_events > 0
