@@ -299,7 +299,7 @@ struct Chooser { uint32_t fills, list; float count; };
 // empty board: moves chosen after 3900, fours looked for 4900, ends known 5600; one wavefront took 10200.
 // 8 trees, 20000 steps: 186 -> 132 ms; 32 playouts of one child, 100 steps: 1.00 -> 0.78 ms; 2 trees of 128 on 7 x 8: 163 -> 102 ms.
 // (Draws made ahead alone, the rest left to one wavefront, gained a search nothing.)
-struct Split {
+struct alignas(16) Split {
     static constexpr int kRing = 128;     // draws per playout (a playout takes up to 57, and as many may have been made ahead of it)
     static constexpr int kWords = 16;     // moves of a playout, four to a word
     static constexpr uint32_t kNone = 0xffu, kNotYet = 0xffffffffu, kEnd = 0xfffffffeu, kReplayed = 0x8000u;
@@ -309,8 +309,8 @@ struct Split {
     uint32_t looked[2][kWave];            // per side: index of the move that made four (kNone) | words looked at << 8
     uint32_t bad[kWave];                  // first word for whose moves a draw had rounded up to 1.0f, times four (kNotYet: none)
     uint32_t used[kWave];                 // draws the playout took; of one that was replayed: place of the next draw << 16 | kReplayed
+    ExactScratch exact;                   // of a replay
     uint32_t stop;                        // every playout's end is known
-    uint32_t pad[3];
 
     static __device__ __forceinline__ uint32_t get(const uint32_t &x) { return __hip_atomic_load(&x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
     static __device__ __forceinline__ void set(uint32_t &x, uint32_t v) { __hip_atomic_store(&x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
@@ -666,7 +666,7 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
     Split &s_split = *reinterpret_cast<Split *>(s_dyn);   // SPLIT
     char *const s_step = reinterpret_cast<char *>(s_dyn) + (SPLIT ? sizeof(Split) : 0);
     double (*const s_explore)[8] = reinterpret_cast<double (*)[8]>(s_step);
-    typename Game::Exact &s_exact = *reinterpret_cast<typename Game::Exact *>(s_step);
+    typename Game::Exact &s_exact = SPLIT ? s_split.exact : *reinterpret_cast<typename Game::Exact *>(s_step);
     uint32_t (*const s_rec)[kRecDwords] = reinterpret_cast<uint32_t (*)[kRecDwords]>(s_step + explore_bytes(args.m, args.n));
     uint64_t *const s_rng = reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(s_dyn) + search_lds_bytes(args.m, args.n));   // SOLO: [column][playout][2]
     typename Game::Exact &s_exact_solo = *reinterpret_cast<typename Game::Exact *>(s_rng + (size_t)(POOL ? 1 : args.n) * args.P * 2);
@@ -1096,12 +1096,32 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
                 if (do_playouts) { res_neg = s_cnt[0][0]; res_pos = s_cnt[0][1]; }
             }
         }
+        // ---- exploration terms of the path nodes' children after this step ----
+        // The visit counts after the backup are known before the playout results of the other workgroups arrive (the
+        // wins are not), so the expensive part of every UCB that has to be re-evaluated is computed before that, by the
+        // wavefronts that do not take part in the exchange.  Where nothing is exchanged and playouts are split, the wavefront that
+        // has chosen their moves does it while the others finish (32 playouts of one child: 100 steps 0.79 -> 0.74 ms, 8 trees,
+        // 1999 steps: 11.6 -> 10.8 ms; a team's step got 0.6 us longer that way).
+        const int n_tot_known = (ACP && mode == kModeExpand) ? P * k_exp : P;
+        const int n_levels = (mode == kModeExpand) ? L + 1 : L;
+        const auto explore = [&](int first, int workers) __attribute__((always_inline)) {
+            for (int i = first; i < n_levels * 8; i += workers) {
+                const int lvl = i >> 3, a = i & 7;
+                int n;
+                if (lvl == L) n = ACP ? (((expmask >> a) & 1u) ? P : 0) : ((a == chosen) ? P : 0);
+                else n = (int)s_rec[lvl][kDwNs + a] + ((a == (int)s_pslot[lvl + 1]) ? n_tot_known : 0);
+                const int N = ((lvl == 0) ? s_t.root_ns : (int)s_rec[lvl - 1][kDwNs + s_pslot[lvl]]) + n_tot_known;
+                s_explore[lvl][a] = (n > 0) ? (double)args.ucb_c * __dsqrt_rn(det_log((double)N) / (double)n) : 0.0;
+            }
+        };
         if (SPLIT && do_playouts) {  // uniform over the workgroup
             const int n_moves = most_moves - (int)__popcll(pl_cur | pl_opp), n_words = (n_moves + 3) >> 2;   // as far as a playout can go
             int chosen_words = 0;
             bool ok = true;
-            if (wave == kChooser) chosen_words = split_choose<Game>(geo, pl_cur, pl_opp, s_split, lane, ring_at, n_words);
-            else if (wave == kFirst || wave == kSecond) {
+            if (wave == kChooser) {
+                chosen_words = split_choose<Game>(geo, pl_cur, pl_opp, s_split, lane, ring_at, n_words);
+                if (!ACP) explore(lane, kWave);
+            } else if (wave == kFirst || wave == kSecond) {
                 const int side = wave == kFirst ? 0 : 1;
                 const uint64_t stones = wave == kFirst ? pl_cur : pl_opp;
                 ok = geo.aligned ? split_look<Game, true>(geo, stones, side, s_split, lane, n_words, args.spin_limit)
@@ -1189,24 +1209,9 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
         if (timing) { const unsigned long long t2 = wall_clock64(); tk_playout += t2 - tk; tk = t2; }
         st_levels += L; st_expanded += k_exp; st_played += do_playouts && part == 0 ? 1 : 0;
 
-        // ---- exploration terms of the path nodes' children after this step ----
-        // The visit counts after the backup are known before the playout results of the other workgroups arrive (the
-        // wins are not), so the expensive part of every UCB that has to be re-evaluated is computed here, by the
-        // wavefronts that do not take part in the exchange.
-        const int n_tot_known = (ACP && mode == kModeExpand) ? P * k_exp : P;
-        const int n_levels = (mode == kModeExpand) ? L + 1 : L;
         {
             const int first = (nwaves > 1 && !SOLO) ? kWave : 0, workers = blockDim.x - first;
-            if (tid >= first) {
-                for (int i = tid - first; i < n_levels * 8; i += workers) {
-                    const int lvl = i >> 3, a = i & 7;
-                    int n;
-                    if (lvl == L) n = ACP ? (((expmask >> a) & 1u) ? P : 0) : ((a == chosen) ? P : 0);
-                    else n = (int)s_rec[lvl][kDwNs + a] + ((a == (int)s_pslot[lvl + 1]) ? n_tot_known : 0);
-                    const int N = ((lvl == 0) ? s_t.root_ns : (int)s_rec[lvl - 1][kDwNs + s_pslot[lvl]]) + n_tot_known;
-                    s_explore[lvl][a] = (n > 0) ? (double)args.ucb_c * __dsqrt_rn(det_log((double)N) / (double)n) : 0.0;
-                }
-            }
+            if (tid >= first && !(SPLIT && !ACP && do_playouts)) explore(tid - first, workers);
             if (!ACP || SOLO) {
                 // every wavefront of a workgroup that searches a tree alone stored child records earlier in the step; the
                 // next walk reads records past the L1, so the stores must have been acknowledged by the L2 (long since)
