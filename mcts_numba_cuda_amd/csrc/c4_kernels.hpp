@@ -147,11 +147,6 @@ struct Geometry {
         r |= t & (t >> (2 * (H + 1)));
         return r != 0;
     }
-    __device__ __forceinline__ uint32_t legal_cols(uint64_t all) const {
-        uint32_t l = 0;
-        for (int c = 0; c < n; c++) l |= (uint32_t)(((all >> (c * H + m - 1)) & 1ull) ^ 1ull) << c;
-        return l;
-    }
 };
 
 // ---- exact emulation of one reference playout on byte arrays ------------------------------------
@@ -336,9 +331,8 @@ struct Connect4 {
     using Playout = c4::Playout;
     using Exact = ExactScratch;
 
-    static __device__ __forceinline__ uint32_t legal_actions(const Geometry &g, uint64_t pos, uint64_t neg) { return g.legal_cols(pos | neg); }
-    // the same, a lane per column (all lanes of the wavefront active)
-    static __device__ __forceinline__ uint32_t legal_actions_of_wave(const Geometry &g, uint64_t pos, uint64_t neg, int lane) {
+    // (a lane per column; all lanes of the wavefront are active)
+    static __device__ __forceinline__ uint32_t legal_actions(const Geometry &g, uint64_t pos, uint64_t neg, int lane) {
         const uint32_t top = (uint32_t)lane * (uint32_t)g.H + (uint32_t)g.m - 1u;
         return (uint32_t)__ballot(lane < g.n && !(((pos | neg) >> (top & 63u)) & 1ull));
     }
@@ -353,33 +347,21 @@ struct Connect4 {
         outcome = win ? mover : (((all | newbit) == g.full) ? 0 : 2);
     }
 
-    static __device__ __forceinline__ PoolChild playout_start(const Geometry &g, uint64_t cur, uint64_t opp, int turn, int column) {
+    // Worked out by the eight lanes that have the position in common, a column each (all lanes of the wavefront are active), in a
+    // fifth of the instructions that a lane for all columns takes, which stood before every step's playouts: 64 searches of 4
+    // trees, 2000 steps, 28.0 -> 26.9 ms, 512 trees, 500 steps, 18.3 -> 18.0, one child, 2 trees of 128 from 13 stones 20.5 -> 18.9.
+    static __device__ __forceinline__ PoolChild playout_start(const Geometry &g, uint64_t cur, uint64_t opp, int turn, int column, int lane) {
         PoolChild pc;
         const uint64_t a = cur << g.base, b = opp << g.base;
         pc.a_lo = (uint32_t)a; pc.a_hi = (uint32_t)(a >> 32); pc.b_lo = (uint32_t)b; pc.b_hi = (uint32_t)(b >> 32);
-        const uint64_t occ = cur | opp;
-        uint32_t fills = 0, list = 0; int count = 0;
-        for (int c = 0; c < g.n; c++) {
-            const int h = __popcll(occ & g.col_mask(c));
-            fills |= (uint32_t)(h + g.base) << (4 * c);
-            if (h < g.m) { list |= (uint32_t)c << (4 * count); count++; }
-        }
-        pc.fills = fills; pc.list = list; pc.count = (float)count * 0x1p-32f;
-        pc.turn_col = (uint32_t)(turn & 0xff) | ((uint32_t)column << 8) | ((uint32_t)__popcll(occ) << 16);
-        return pc;
-    }
-
-    // The same with the columns of one position worked out by eight lanes each (all lanes of the wavefront get the result; no
-    // side, column or stones): a third of the instructions that one lane after the other's columns takes.
-    static __device__ __forceinline__ PoolChild playout_start_of_wave(const Geometry &g, uint64_t cur, uint64_t opp, int lane) {
-        PoolChild pc = {};
         const uint32_t c = (uint32_t)lane & 7u;
         const uint32_t h = (uint32_t)__popc((uint32_t)((cur | opp) >> ((c * (uint32_t)g.H) & 63u)) & ((1u << g.m) - 1u));
         const bool exists = (int)c < g.n, open = exists && (int)h < g.m;
-        const uint32_t legal = (uint32_t)__ballot(open) & 0xffu;
+        const uint32_t legal = (uint32_t)(__ballot(open) >> (lane & 56)) & 0xffu;
         pc.fills = or_over_8_lanes(exists ? (h + (uint32_t)g.base) << (4u * c) : 0u);
         pc.list = or_over_8_lanes(open ? c << (4u * (uint32_t)__popc(legal & ((1u << c) - 1u))) : 0u);
         pc.count = (float)__popc(legal) * 0x1p-32f;
+        pc.turn_col = (uint32_t)(turn & 0xff) | ((uint32_t)column << 8) | ((uint32_t)__popcll(cur | opp) << 16);
         return pc;
     }
 
@@ -437,9 +419,7 @@ struct Connect4 {
 
     // cur: stones of the side to move, opp: the other side's.  Returns -1 / 0 / +1, or 2 when a draw of the uniform
     // rounded up to 1.0f (the caller then replays the playout with exact_playout).
-    static __device__ __forceinline__ int fast_playout(const Geometry &g, uint64_t cur, uint64_t opp, int turn,
-                                                       uint64_t &s0, uint64_t &s1, uint32_t &plies) {
-        const PoolChild pc = playout_start(g, cur, opp, turn, 0);
+    static __device__ __forceinline__ int fast_playout(const Geometry &g, const PoolChild &pc, int turn, uint64_t &s0, uint64_t &s1, uint32_t &plies) {
         if (pc.count == 0.0f) return 0;
         BB a = {pc.a_lo, pc.a_hi}, b = {pc.b_lo, pc.b_hi};
         Playout p;
@@ -580,7 +560,7 @@ __device__ __forceinline__ int split_choose(const typename Game::Geometry &g, ui
     };
     float d[4];
     read_four(d);
-    const PoolChild pc = Game::playout_start_of_wave(g, cur, opp, lane);
+    const PoolChild pc = Game::playout_start(g, cur, opp, 0, 0, lane);
     Chooser p{pc.fills, pc.list, pc.count};
     asm volatile("" : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]));   // (waited for here, so that the loop waits for nothing at its head)
     int t = 0;
@@ -875,7 +855,7 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
         int mode; uint32_t expmask = 0, legal = 0;
         if (leaf.flags & kTerminal) mode = kModeTerminal;
         else {
-            legal = SPLIT ? Game::legal_actions_of_wave(geo, leaf.bb_pos, leaf.bb_neg, lane) : Game::legal_actions(geo, leaf.bb_pos, leaf.bb_neg);
+            legal = Game::legal_actions(geo, leaf.bb_pos, leaf.bb_neg, lane);
             int room = S - size; if (room < 0) room = 0;
             expmask = legal;
             while ((int)__popc(expmask) > room) expmask &= ~(1u << (31 - __clz(expmask)));  // children beyond the pool end are dropped
@@ -916,22 +896,17 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
             // two thirds of the time).  What a playout starts from (stones, column fills, the ascending list of legal
             // columns) is worked out once per node here instead of once per playout.
             if (wave == 0) {
-                const int a = lane & 7;
-                bool playable = false;
-                uint64_t cur = 0, opp = 0; int turn_a = 0;
-                if (lane < kMaxCols) {
-                    if (mode == kModeExpand) {
-                        playable = a < ncols && ((expmask >> a) & 1u) && solo_outcome_l == 2;   // terminal child: stored outcome times P (src/mctsnc.py:1842-1846)
-                        turn_a = -mover; cur = (turn_a == 1) ? cpos_l : cneg_l; opp = (turn_a == 1) ? cneg_l : cpos_l;
-                    } else if (mode == kModeFull) {  // pool exhausted: the selected node itself is played out, with the generators of column 0
-                        playable = a == 0;
-                        turn_a = mover; cur = (mover == 1) ? leaf.bb_pos : leaf.bb_neg; opp = (mover == 1) ? leaf.bb_neg : leaf.bb_pos;
-                    }
-                }
+                const int a = lane & 7, k = lane >> 3;   // eight lanes work out what the playouts of node k start from
+                const bool playable = lane < kMaxCols && (mode == kModeExpand ? a < ncols && ((expmask >> a) & 1u) && solo_outcome_l == 2   // terminal child: stored outcome times P (src/mctsnc.py:1842-1846)
+                                                                              : mode == kModeFull && a == 0);   // pool exhausted: the selected node itself is played out, with the generators of column 0
                 const uint32_t pmask = (uint32_t)__ballot(playable) & 0xffu;
-                if (playable) {
-                    s_pool[__popc(pmask & ((1u << a) - 1u))] = Game::playout_start(geo, cur, opp, turn_a, a);
-                    s_cnt[a][0] = 0; s_cnt[a][1] = 0;
+                const int turn_k = mode == kModeExpand ? -mover : mover;
+                const uint64_t pos = mode == kModeExpand ? (uint64_t)__shfl((unsigned long long)cpos_l, k) : leaf.bb_pos;
+                const uint64_t neg = mode == kModeExpand ? (uint64_t)__shfl((unsigned long long)cneg_l, k) : leaf.bb_neg;
+                const PoolChild pc = Game::playout_start(geo, turn_k == 1 ? pos : neg, turn_k == 1 ? neg : pos, turn_k, k, lane);
+                if (a == 0 && ((pmask >> k) & 1u)) {
+                    s_pool[__popc(pmask & ((1u << k) - 1u))] = pc;
+                    s_cnt[k][0] = 0; s_cnt[k][1] = 0;
                 }
                 if (lane == 0) { s_pool_n = __popc(pmask); s_pool_mask = pmask; s_pool_next = 0; }
             }
@@ -947,9 +922,10 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
             } else if (mode == kModeFull && column == 0) {  // pool exhausted: the selected node itself is played out
                 do_playouts = true; pl_turn = mover; pl_cur = (mover == 1) ? leaf.bb_pos : leaf.bb_neg; pl_opp = (mover == 1) ? leaf.bb_neg : leaf.bb_pos;
             }
-            if (POOL && tid == 0) {   // this workgroup's node as the pool's only one (its generators are the pool's column 0)
-                if (do_playouts) { s_pool[0] = Game::playout_start(geo, pl_cur, pl_opp, pl_turn, 0); s_cnt[0][0] = 0; s_cnt[0][1] = 0; }
-                s_pool_n = do_playouts ? 1 : 0; s_pool_mask = do_playouts ? 1u : 0u; s_pool_next = 0;
+            if (POOL && wave == 0) {   // this workgroup's node as the pool's only one (its generators are the pool's column 0)
+                const PoolChild pc = Game::playout_start(geo, pl_cur, pl_opp, pl_turn, 0, lane);
+                if (do_playouts && lane == 0) { s_pool[0] = pc; s_cnt[0][0] = 0; s_cnt[0][1] = 0; }
+                if (lane == 0) { s_pool_n = do_playouts ? 1 : 0; s_pool_mask = do_playouts ? 1u : 0u; s_pool_next = 0; }
             }
         } else {
             if (mode == kModeExpand) {
@@ -1180,8 +1156,9 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
             int outcome = 0; bool redo = false;
             const uint64_t s0_start = s0, s1_start = s1;
             const uint32_t plies_start = plies;
+            const PoolChild start = Game::playout_start(geo, pl_cur, pl_opp, pl_turn, 0, lane);
             if (tid < P) {
-                outcome = Game::fast_playout(geo, pl_cur, pl_opp, pl_turn, s0, s1, plies);
+                outcome = Game::fast_playout(geo, start, pl_turn, s0, s1, plies);
                 redo = outcome == 2;
             }
             const int par = step & 1;
