@@ -16,7 +16,9 @@
 //     tree redundantly (read-only, deterministic), creates and plays out its own child, publishes its result
 //     and reads the results of the tree's other workgroups (one exchange per step), then applies the backup
 //     to its own LDS copy of the path records and writes its share of them back;
-//   * OCP: one workgroup per tree does everything, no inter-workgroup synchronisation.
+//   * OCP: one workgroup per tree does everything, no inter-workgroup synchronisation;
+//   * where CUs would idle, 64 playouts to a workgroup, each split over four wavefronts (Split), and several workgroups to a
+//     child, which exchange results in both variants.
 //   * blockIdx is decoded so that the workgroups of one tree share blockIdx % 8, i.e. the same XCD and L2.
 #pragma once
 #include "c4_draw.h"
@@ -324,7 +326,8 @@ struct alignas(16) Split {
 //   child           take_action + compute_outcome: the position after `action` and its outcome (-1 / 0 / +1, 2 = ongoing)
 //   playout_start   legal_actions_playout: what a playout from a position starts from
 //   begin, ply      take_action_playout + compute_outcome for one random move, free of branches
-//   fast_playout    a whole playout (start + plies); exact_playout: the byte-array emulation for draws that round up
+//   fast_playout    a whole playout after its start; exact_playout: the byte-array emulation for draws that round up
+//   choose, put     a ply in two halves, for playouts split over wavefronts
 // ------------------------------------------------------------------------------------------------------------------------
 struct Connect4 {
     using Geometry = c4::Geometry;
