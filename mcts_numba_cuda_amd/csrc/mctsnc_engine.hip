@@ -574,28 +574,17 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
     // playouts must be long enough: with fewer than 16 cells left on the boards on average, most of such searches lose 2 to 5 %
     // (6 x 7, 4 trees of 64 to 256: 0.95 to 1.01 of the time at 8 to 16 cells, 1.05 at 24; 5 x 6, one tree of 256, 8 / 12 / 16 / 18 /
     // 20 / 24 cells: 0.95 / 0.99 / 0.99 / 1.06 / 1.08 / 1.17).
-    const int parts = std::max(1, c.n_playouts / kWave);
+    const int parts = e0->acp ? std::max(1, c.n_playouts / kWave) : 1;
     int64_t stones = 0;
     for (int r = 0; r < n_refs; r++) stones += __builtin_popcountll(bb[2 * (size_t)r]) + __builtin_popcountll(bb[2 * (size_t)r + 1]);
-    const int64_t left = (int64_t)n_refs * mn - stones;
-    const bool roomy = !solo && !team_pool && e0->G * parts <= c4::kMaxWide && e0->G * parts * (8 * ((n_refs + 7) / 8)) <= cus_now;
-    const bool split = roomy && (e0->acp ? left >= (int64_t)16 * n_refs : parts == 1);
-    // One child's playouts shared by several workgroups, which makes every step one of exchanging results as well: with two thirds
-    // of the cells left, and only where steps play out.  What a search is like shows in its first 64 steps: it goes on with one
-    // workgroup to a tree if these took fewer than 7 plies a playout, counting steps that ended at a terminal node as none.
-    // Searches too short for that go by their stones.  (us a step, one workgroup / shared, 6 x 7, 4 trees of 128: 34 cells
-    // left 9.2 / 7.5, 28 7.7 / 6.8, 24 6.6 / 6.4; decided positions 2.1 / 2.4; trying takes 0.1 ms.)
-    const double step_budget = bud.forced < INFINITY ? bud.forced : bud.steps_limit;
-    constexpr int kTrySteps = 64;
-    const bool try_shared = step_budget >= 4.0 * kTrySteps;
-    bool shared = roomy && !e0->acp && parts > 1 && 3 * left >= 2 * (int64_t)n_refs * mn && (try_shared || 4 * stones <= (int64_t)n_refs * mn);
+    const bool split = !solo && !team_pool && (e0->acp ? e0->G * parts <= c4::kMaxWide && (int64_t)n_refs * mn - stones >= (int64_t)16 * n_refs : c.n_playouts <= kWave) &&
+                       e0->G * parts * (8 * ((n_refs + 7) / 8)) <= cus_now;
     if (split) { args.G = e0->G * parts; args.parts = parts; block = dim3(c4::kSplitThreads); }
     const size_t lds = solo ? c4::solo_lds_bytes(c.board_m, c.board_n, c.n_playouts)
                             : (team_pool ? c4::team_pool_lds_bytes(c.board_m, c.board_n, c.n_playouts)
                                : split   ? c4::split_lds_bytes(c.board_m, c.board_n) : c4::search_lds_bytes(c.board_m, c.board_n));
     const auto solo_kernel = c4::search_kernel_solo;
     const auto team_kernel = team_pool ? c4::search_kernel_team_pool : split ? c4::search_kernel_split<true> : c4::search_kernel<true>;
-    const auto shared_kernel = c4::search_kernel_shared;
     const auto one_child_kernel = split ? c4::search_kernel_split<false> : c4::search_kernel<false>;
     if (solo) HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(solo_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     // Sets of G workgroups (8 sets per grid row, one per XCD).  The all-children kernel is launched cooperatively, so
@@ -624,7 +613,6 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
         probe_steps = budget < 32.0 * 128.0 ? (budget < 32.0 * 16.0 ? 16 : (int32_t)(budget / 32.0)) : 128;
         if (opt[MCTSNC_OPT_PROBE_STEPS] >= 0) probe_steps = opt[MCTSNC_OPT_PROBE_STEPS];
     }
-    if (shared && try_shared) probe_steps = kTrySteps;
     const bool plain_launch = opt[MCTSNC_OPT_PLAIN_LAUNCH] != 0;
     static std::atomic<uint32_t> launch_counter{0};
     int64_t steps; double dev_time, time_loop;
@@ -649,15 +637,7 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
                 }
             }
         } else {
-            if (shared) {   // (fewer workgroups than CUs, which wait for each other)
-                c4::SearchArgs of_team = args;
-                of_team.G = of_team.parts = parts;
-                void *kargs[] = {&of_team};
-                const dim3 team_grid(parts * sets), team_block(c4::kSplitThreads);
-                const size_t team_lds = c4::split_lds_bytes(c.board_m, c.board_n);
-                if (plain_launch) hipLaunchKernelGGL(shared_kernel, team_grid, team_block, team_lds, stream, of_team);
-                else HIP_TRY(hipLaunchCooperativeKernel(reinterpret_cast<void *>(shared_kernel), team_grid, team_block, kargs, (unsigned)team_lds, stream));
-            } else hipLaunchKernelGGL(one_child_kernel, grid, block, lds, stream, args);
+            hipLaunchKernelGGL(one_child_kernel, grid, block, lds, stream, args);
             HIP_TRY(hipGetLastError());
         }
         return MCTSNC_OK;
@@ -669,12 +649,6 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
         std::vector<unsigned long long> plies((size_t)n_refs);
         HIP_TRY(hipMemcpyAsync(plies.data(), d_plies, sizeof(unsigned long long) * n_refs, hipMemcpyDeviceToHost, stream));
         HIP_TRY(hipStreamSynchronize(stream));
-        if (!e0->acp) {
-            unsigned long long played = 0;
-            for (const unsigned long long p : plies) played += p;
-            shared = played >= 7ull * kTrySteps * (unsigned long long)c.n_playouts * (unsigned long long)n_refs;
-            return MCTSNC_OK;
-        }
         std::vector<unsigned long long> cost((size_t)n, 0);
         std::vector<int> by_cost((size_t)n);
         for (int j = 0; j < n; j++) { by_cost[j] = j; for (int t = 0; t < T; t++) cost[j] += plies[(size_t)j * T + t]; }
