@@ -165,6 +165,11 @@ int mctsnc_run_batch_noalloc(mctsnc_engine **engines, int32_t n, const int8_t *b
  *   MCTSNC_OPT_TEAM_POOL          Connect 4, all children: a team's workgroups play their playouts as a pool of jobs on
  *                                 fewer lanes; 1 / 0 = always / never, -1 (default) = by the number of trees
  *   MCTSNC_OPT_TEAM_POOL_THREADS  lanes of such a workgroup, a multiple of 64 up to 512; 0 (default) = half the playouts
+ *   MCTSNC_OPT_SPLIT              Connect 4, teams without pools and one child: playouts split over four wavefronts, in
+ *                                 workgroups that have a CU each; 0 = never, 1 = wherever that fits (a CU for every
+ *                                 workgroup of the pass, at most 32 workgroups to a tree; one child: up to 64 playouts),
+ *                                 -1 (default) = of those, one-child searches and teams with 16 empty cells or more on
+ *                                 average
  *   MCTSNC_OPT_PREP_LEVELS        Gomoku, one child: the backup of paths up to this many levels is prepared during the
  *                                 playouts (at most 48); -1 (default) = 48
  *   MCTSNC_OPT_PLAIN_LAUNCH       1: the all-children kernels, whose workgroups wait for each other, are launched as
@@ -177,7 +182,7 @@ int mctsnc_run_batch_noalloc(mctsnc_engine **engines, int32_t n, const int8_t *b
  *                                 searches are put in the order of what they cost; 0 = keep the order by stones,
  *                                 -1 (default) = a thirty-second of the step budget, 16 to 128
  *   MCTSNC_OPT_SPIN_LIMIT         polls after which a workgroup's wait for the others of its tree, or a wavefront's for
- *                                 the one it shares its playouts with (one-child Gomoku), gives up and ends the launch
+ *                                 those it shares its playouts with (one-child Gomoku, split Connect 4), gives up and ends the launch
  *                                 (MCTSNC_E_DEVICE_SYNC); 0 (default) = 2^24.  1 makes the first wait that is not met at
  *                                 once give up: the hook with which the tests drive that path.
  * After MCTSNC_E_DEVICE_SYNC the search is void, the engines stay usable and their random streams are back at their
@@ -191,7 +196,8 @@ int mctsnc_run_batch_noalloc(mctsnc_engine **engines, int32_t n, const int8_t *b
 #define MCTSNC_OPT_PLAIN_LAUNCH 6
 #define MCTSNC_OPT_PROBE_STEPS 7
 #define MCTSNC_OPT_SPIN_LIMIT 8
-#define MCTSNC_OPT_COUNT 9
+#define MCTSNC_OPT_SPLIT 9
+#define MCTSNC_OPT_COUNT 10
 int mctsnc_set_option(mctsnc_engine *e, int32_t option, int32_t value);
 
 /* Switches the per-stage device timers on (default) or off. */

@@ -45,7 +45,7 @@ ARRAYS = {  # name -> (id, dtype, trailing shape builder)
 
 # mctsnc_set_option(): names of the MCTSNC_OPT_* constants of include/mctsnc_hip.h
 OPTIONS = {"agent_fences": 0, "solo_trees": 1, "solo_threads": 2, "team_pool": 3, "team_pool_threads": 4, "prep_levels": 5,
-           "plain_launch": 6, "probe_steps": 7, "spin_limit": 8}
+           "plain_launch": 6, "probe_steps": 7, "spin_limit": 8, "split": 9}
 
 _lib = None
 

@@ -98,7 +98,7 @@ struct mctsnc_engine {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     bool has_run = false;
     bool stage_timing = true;
-    int options[MCTSNC_OPT_COUNT] = {0, -1, 0, -1, 0, -1, 0, -1, 0};   // mctsnc_set_option(): defaults, see include/mctsnc_hip.h
+    int options[MCTSNC_OPT_COUNT] = {0, -1, 0, -1, 0, -1, 0, -1, 0, -1};   // mctsnc_set_option(): defaults, see include/mctsnc_hip.h
     std::vector<uint64_t> rng_init_playout, rng_init_expand;  // the streams as seeded, kept for reseed()
     std::vector<c4::TreeRef> h_refs;          // host copies of the per-tree pointer records (a batch gathers them)
     std::vector<gomoku::TreeRef> hg_refs;
@@ -577,8 +577,9 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
     const int parts = e0->acp ? std::max(1, c.n_playouts / kWave) : 1;
     int64_t stones = 0;
     for (int r = 0; r < n_refs; r++) stones += __builtin_popcountll(bb[2 * (size_t)r]) + __builtin_popcountll(bb[2 * (size_t)r + 1]);
-    const bool split = !solo && !team_pool && (e0->acp ? e0->G * parts <= c4::kMaxWide && (int64_t)n_refs * mn - stones >= (int64_t)16 * n_refs : c.n_playouts <= kWave) &&
-                       e0->G * parts * (8 * ((n_refs + 7) / 8)) <= cus_now;
+    const bool splits = !solo && !team_pool && (e0->acp ? e0->G * parts <= c4::kMaxWide : c.n_playouts <= kWave) && e0->G * parts * (8 * ((n_refs + 7) / 8)) <= cus_now;
+    bool split = splits && (!e0->acp || (int64_t)n_refs * mn - stones >= (int64_t)16 * n_refs);
+    if (opt[MCTSNC_OPT_SPLIT] >= 0) split = splits && opt[MCTSNC_OPT_SPLIT] != 0;
     if (split) { args.G = e0->G * parts; args.parts = parts; block = dim3(c4::kSplitThreads); }
     const size_t lds = solo ? c4::solo_lds_bytes(c.board_m, c.board_n, c.n_playouts)
                             : (team_pool ? c4::team_pool_lds_bytes(c.board_m, c.board_n, c.n_playouts)
@@ -1053,7 +1054,7 @@ int mctsnc_set_option(mctsnc_engine *e, int32_t option, int32_t value) {
     switch (option) {
     case MCTSNC_OPT_AGENT_FENCES: case MCTSNC_OPT_PLAIN_LAUNCH: ok = value == 0 || value == 1; break;
     case MCTSNC_OPT_SOLO_TREES: case MCTSNC_OPT_PROBE_STEPS: ok = value >= -1; break;
-    case MCTSNC_OPT_TEAM_POOL: ok = value >= -1 && value <= 1; break;
+    case MCTSNC_OPT_TEAM_POOL: case MCTSNC_OPT_SPLIT: ok = value >= -1 && value <= 1; break;
     case MCTSNC_OPT_PREP_LEVELS: ok = value >= -1; break;
     case MCTSNC_OPT_SOLO_THREADS: case MCTSNC_OPT_TEAM_POOL_THREADS: ok = value == 0 || (value >= 64 && value <= 512 && value % 64 == 0); break;
     case MCTSNC_OPT_SPIN_LIMIT: ok = value >= 0; break;

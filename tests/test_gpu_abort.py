@@ -25,13 +25,16 @@ def assert_same(a, b):
             np.testing.assert_array_equal(a[key], b[key], err_msg=str(key))
 
 
-@pytest.mark.parametrize("game,variant", [("c4", "acp_prodigal"), ("c4", "acp_thrifty"), ("gomoku", "acp_prodigal")])
-def test_abandoned_search_reports_and_leaves_a_fresh_engine(game, variant):
+@pytest.mark.parametrize("game,variant,split,playouts", [
+    ("c4", "acp_prodigal", 0, 64), ("c4", "acp_thrifty", 0, 64), ("c4", "acp_prodigal", 1, 64), ("c4", "acp_thrifty", 1, 256),
+    ("c4", "ocp_thrifty", 1, 64), ("c4", "ocp_prodigal", 1, 32), ("gomoku", "acp_prodigal", None, 64)])
+def test_abandoned_search_reports_and_leaves_a_fresh_engine(game, variant, split, playouts):
+    """Connect 4 with split = 1: the wavefronts that share a playout wait for each other as well, also in one-child variants."""
     from mcts_numba_cuda_amd import _lib
     rng = np.random.default_rng(5)
     if game == "c4":
-        params = dict(n_trees=3, n_playouts=64, variant=variant, device_memory=0.25, ucb_c=2.0, seed=5)
-        mk = lambda: make_engine(params)
+        params = dict(n_trees=3, n_playouts=playouts, variant=variant, device_memory=0.25, ucb_c=2.0, seed=5)
+        mk = lambda: make_engine(params, options=dict(split=split))
         board, fills, turn = random_c4_root(rng, 9)
         root, steps = (board, fills, turn), 300
     else:
@@ -79,7 +82,7 @@ def test_one_child_gomoku_gives_up_on_its_playouts(variant, shape, trees, playou
 def test_option_values_are_checked():
     from mcts_numba_cuda_amd import _lib
     e = make_engine(dict(n_trees=1, n_playouts=32, variant="ocp_thrifty", device_memory=0.05, ucb_c=2.0, seed=0))
-    for name, value in (("solo_threads", 100), ("solo_threads", 1024), ("team_pool", 2), ("agent_fences", 3), ("spin_limit", -1)):
+    for name, value in (("solo_threads", 100), ("solo_threads", 1024), ("team_pool", 2), ("split", 2), ("split", -2), ("agent_fences", 3), ("spin_limit", -1)):
         with pytest.raises(_lib.EngineError):
             e.set_option(name, value)
     with pytest.raises(ValueError):
