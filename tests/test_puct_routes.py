@@ -105,6 +105,8 @@ def outcome(library, launcher, d, v):
 @pytest.mark.parametrize("launcher", LAUNCHERS)
 def test_both_routes_take_and_refuse_the_same(library, monkeypatch, launcher, table):
     """table: the tensors are described by an exchange table, as torch's are, else by their attributes."""
+    if table and not build.dlpack_flags():
+        pytest.skip("_puct_call is built without torch's exchange table here")
     accepted = refused = asked = 0
     for code in (0, 700):
         library.code[0] = code
@@ -120,7 +122,7 @@ def test_both_routes_take_and_refuse_the_same(library, monkeypatch, launcher, ta
             assert by_c == by_python, what
             assert (by_c[0] is None) == (len(by_c[2]) == 1 and code == 0), what
             accepted, refused = accepted + len(by_c[2]), refused + (not by_c[2])
-    assert accepted > 2 and refused > 2 and (asked > 100 or not table or not build.dlpack_flags())
+    assert accepted > 2 and refused > 2 and (not table or asked > 100)
 
 
 @pytest.mark.parametrize("launcher", LAUNCHERS)
