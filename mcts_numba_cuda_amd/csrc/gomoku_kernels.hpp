@@ -560,7 +560,7 @@ __device__ __forceinline__ uint32_t earliest_five(const uint32_t *masks, uint32_
             if constexpr (DIR == 0) { const uint32_t y = masks[(line * kWords + colour) * 64]; return run_of_five(y, y, y, y, y); }
             else return starts[line * 64];
         };
-        auto first = [](uint32_t bits) -> uint32_t { return (uint32_t)__builtin_amdgcn_ubfe(__builtin_ctz(bits), 0, 5); };   // (any line if there is none)
+        auto first = [](uint32_t bits) -> uint32_t { return bits == 0 ? 32u : (uint32_t)__builtin_ctz(bits); };   // (32 if there is none)
         uint32_t line = first(some), x = line_word(line);
         const Cell *at_line = my_times + (int)line * (stride * 64) + low;
         some &= some - 1;

@@ -1,0 +1,82 @@
+"""The Gomoku search kernels on the CPU (tests/simt: lanes that meet where the device's do, wavefronts in any order between
+barriers), against the oracle."""
+import ctypes
+import functools
+
+import numpy as np
+import pytest
+
+import simt_build
+from helpers import random_gomoku_root
+from oracle.oracle import Oracle
+
+needs_clang = pytest.mark.skipif(simt_build.CLANG is None, reason="no clang++")
+
+
+@functools.lru_cache(None)
+def library(path):
+    lib = ctypes.CDLL(path)
+    lib.simt_gomoku.argtypes = [ctypes.c_int] * 11 + [ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_uint, ctypes.c_void_p, ctypes.c_int] + [ctypes.c_void_p] * 6
+    return lib
+
+
+def words_of(m, n):
+    if m <= 16 and n <= 16 and m * n <= 240:
+        return 8
+    return 12 if m * n <= 384 else 16
+
+
+def compare(path, m, n, stones, variant, trees, playouts, steps, groups=3, per_cu=True, launches=1, prep=48, xccs=1, seed=7, room=None):
+    acp, thrifty, W, A = variant.startswith("acp"), variant.endswith("thrifty"), words_of(m, n), m * n
+    S = room or 1 + A * steps * launches
+    o = Oracle("gomoku", (m, n), 0, A, trees, playouts, variant, ucb_c=2.0, seed=seed, max_tree_size_override=S, threads=1)
+    board, turn = random_gomoku_root(np.random.default_rng(seed), m, n, stones)
+    rng = o.rng_states("playout").copy()
+    # (the expansion generators are those of the same seed's stream that start a tree's threads)
+    tpb = 1
+    while tpb < max(m * n, A):
+        tpb *= 2
+    tpb = min(tpb, 512)
+    streams = Oracle("gomoku", (m, n), 0, A, trees * 8, 64, "acp_prodigal", seed=seed, max_tree_size_override=1).rng_states("playout")
+    expand = np.ascontiguousarray(streams[np.arange(trees) * tpb])
+    bits = np.zeros((2, 32 * W), np.uint8)
+    bits[0, :A], bits[1, :A] = board.ravel() == 1, board.ravel() == -1
+    bb = np.packbits(bits, axis=1, bitorder="little").view(np.uint32)
+    rec = 256 if W > 12 else 128
+    nodes, stats = np.zeros((trees, S, rec), np.uint8), np.zeros((trees, S, 4), np.int32)
+    sizes, layout = np.zeros(trees, np.int32), np.zeros(3, np.int32)
+    rc = library(path).simt_gomoku(m, n, trees, playouts, acp, thrifty, groups, per_cu, S, steps, launches, 2.0, prep, xccs, seed, bb.ctypes.data, turn,
+                                        rng.ctypes.data, expand.ctypes.data, nodes.ctypes.data, stats.ctypes.data, sizes.ctypes.data, layout.ctypes.data)
+    assert rc == 0
+    o.run(board, None, turn, steps * launches)
+    for t in range(trees):
+        sz = o.tree_size(t)
+        assert sizes[t] == sz, (t, sizes[t], sz)
+        np.testing.assert_array_equal(stats[t, :sz, 0], o.tree(t, "ns"), err_msg=f"ns[{t}]")
+        np.testing.assert_array_equal(stats[t, :sz, 1], o.tree(t, "ns_wins"), err_msg=f"wins[{t}]")
+        head = nodes[t, :sz].view(np.int32)
+        np.testing.assert_array_equal(head[:, 1], o.tree(t, "trees")[:, 0], err_msg=f"parents[{t}]")
+        np.testing.assert_array_equal(nodes[t, :sz, 16:18].copy().view(np.int16)[:, 0], o.tree(t, "depths"))
+        np.testing.assert_array_equal(nodes[t, 1:sz, 19].view(np.int8), o.tree(t, "outcomes")[1:])
+    np.testing.assert_array_equal(rng, o.rng_states("playout"), err_msg="generators")
+    return layout
+
+
+# rows, columns, stones, variant, trees, playouts, steps, and how the search is laid out: formats of either side of the limit on times,
+# several rounds, two trees to a CU, full pools, paths beyond what is prepared, workgroups on one XCC and on several
+CASES = [
+    (5, 5, 0, "acp_prodigal", 2, 64, 3, dict(groups=5, xccs=8)), (5, 32, 0, "ocp_thrifty", 1, 128, 3, {}), (9, 9, 6, "acp_thrifty", 1, 64, 4, dict(xccs=3)),
+    (11, 11, 0, "acp_prodigal", 2, 32, 3, dict(groups=4, xccs=8)), (13, 13, 30, "acp_prodigal", 1, 32, 3, {}), (13, 14, 0, "ocp_prodigal", 2, 256, 4, {}),
+    (15, 15, 0, "ocp_thrifty", 1, 512, 3, {}), (15, 15, 0, "ocp_prodigal", 2, 128, 6, dict(per_cu=False, launches=2)), (15, 15, 90, "acp_prodigal", 2, 32, 2, {}),
+    (15, 14, 130, "ocp_thrifty", 1, 64, 8, dict(prep=2)), (10, 16, 0, "acp_thrifty", 1, 64, 2, {}), (16, 15, 3, "acp_prodigal", 1, 32, 2, dict(xccs=8)),
+    (16, 16, 0, "ocp_prodigal", 1, 128, 3, {}), (17, 17, 7, "acp_prodigal", 1, 16, 2, {}), (19, 19, 100, "ocp_thrifty", 1, 128, 4, dict(prep=0)),
+    (22, 23, 0, "ocp_prodigal", 1, 256, 2, {}), (32, 16, 40, "acp_thrifty", 1, 8, 2, {}), (6, 7, 40, "acp_prodigal", 1, 8, 12, {}),
+    (9, 9, 4, "acp_prodigal", 1, 16, 6, dict(room=90)), (8, 8, 4, "ocp_thrifty", 1, 64, 8, dict(room=100)), (7, 7, 0, "acp_thrifty", 1, 4, 3, dict(room=1)),
+]
+
+
+@needs_clang
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_searches_on_the_cpu_equal_the_oracle(case):
+    """With one draw in 4096 rounded up to 1.0f, so that playouts are replayed all the time."""
+    simt_build.run_apart(compare, simt_build.checked("gomoku_host"), *case[:-1], **case[-1])
