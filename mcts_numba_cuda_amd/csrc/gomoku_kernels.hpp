@@ -1327,7 +1327,7 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
                     hdr->depth_sum += (int64_t)k_exp * (L + 1);
                     if (L + 1 > hdr->max_depth) hdr->max_depth = L + 1;
                 }
-                hdr->po_neg = neg_tot; hdr->po_pos = pos_tot;
+                if (!ACP || mode != kModeFull) { hdr->po_neg = neg_tot; hdr->po_pos = pos_tot; }   // (else they are what was read, and others may still read)
                 hdr->selected = leaf.node; hdr->path_len = L + 1; hdr->mode = mode;
             }
             // trees_actions_expanded[ti] with the reference's semantics (entries a step does not write keep their value)

@@ -6,6 +6,7 @@ import os
 import re
 import shutil
 import subprocess
+import sys
 import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -106,3 +107,23 @@ def run_apart(function, libraries, *args, **kw):
         child.join()
         raise AssertionError("has not ended")
     assert child.exitcode == 0, f"exit code {child.exitcode}"
+
+
+def thread_sanitizer():
+    """ThreadSanitizer's runtime library, or None."""
+    path = CLANG and subprocess.run([CLANG, "-print-file-name=libclang_rt.tsan-x86_64.so"], stdout=subprocess.PIPE, text=True).stdout.strip()
+    return path if path and os.path.isabs(path) and os.path.exists(path) else None
+
+
+def races(source, module, cases, known=""):
+    """What ThreadSanitizer has to say about module.compare(library, *case, **last of case) of the cases, in a process of its own: a
+    wavefront is one thread to it, barriers and what is published between workgroups order them.  known: a function to pass over."""
+    folder = tempfile.mkdtemp()
+    lib = build(source, folder, ["-fsanitize=thread", "-mllvm", "-tsan-instrument-func-entry-exit=0"], ["-fsanitize=thread", "-shared-libsan"])
+    passed_over = os.path.join(folder, "known")
+    with open(passed_over, "w") as f:
+        f.write(f"race:{known}\n" if known else "")
+    env = dict(os.environ, LD_PRELOAD=thread_sanitizer(), TSAN_OPTIONS=f"exitcode=66 suppressions={passed_over}", OMP_NUM_THREADS="1")
+    code = f"import sys; sys.path[:0] = {[os.path.dirname(HERE), HERE]!r}; import {module} as t\nfor c in {cases!r}: t.compare({lib!r}, *c[:-1], **c[-1])"
+    res = subprocess.run([sys.executable, "-c", code], env=env, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=600)
+    return res.returncode, res.stdout

@@ -80,3 +80,10 @@ CASES = [
 def test_searches_on_the_cpu_equal_the_oracle(case):
     """With one draw in 4096 rounded up to 1.0f, so that playouts are replayed all the time."""
     simt_build.run_apart(compare, simt_build.checked("gomoku_host"), *case[:-1], **case[-1])
+
+
+@pytest.mark.skipif(simt_build.thread_sanitizer() is None, reason="no ThreadSanitizer")
+def test_wavefronts_do_not_race():
+    """No two wavefronts touch the same LDS or memory, one of them writing, without a barrier or a published word in between."""
+    code, output = simt_build.races("gomoku_host", "test_simt_gomoku", CASES)
+    assert code == 0, output[-6000:]
