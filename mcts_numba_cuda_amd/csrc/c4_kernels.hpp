@@ -390,8 +390,8 @@ struct Connect4 {
         const int ord = (int)(p.draw * p.count);  // single-precision product, as the reference's float32 * int16
         rng_advance32(p.rng);
         p.draw = draw_of(p.rng);
-        const int sh = ord * 4;
-        const uint32_t c = (p.list >> sh) & 7u;
+        const int sh = ord * 4;   // (32 if one of eight columns was drawn with a uniform rounded up: some column then, the playout is replayed)
+        const uint32_t c = __builtin_amdgcn_ubfe(p.list, (uint32_t)sh, 3);   // (takes sh modulo 32)
         const uint32_t c4 = c * 4u;
         const uint32_t h = (p.fills >> c4) & 15u;
         uint32_t pos;   // c * H + h at full rate (the compiler would take the 64-bit multiply-add, a quarter-rate instruction)
@@ -403,7 +403,7 @@ struct Connect4 {
         me.hi |= bit & upper;
         p.fills += 1u << c4;
         const bool full = h == (uint32_t)last_fill;
-        const uint32_t low = (1u << sh) - 1u;
+        const uint32_t low = __builtin_amdgcn_ubfe(~0u, 0, (uint32_t)sh);
         p.list = full ? ((p.list & low) | ((p.list >> 4) & ~low)) : p.list;  // a full column leaves the ascending list
         p.count -= full ? 0x1p-32f : 0.0f;
         p.fours = aligned ? bb_fours_aligned(me, upper, H) : bb_fours(me, H);
@@ -441,14 +441,14 @@ struct Connect4 {
     // legal column is left.
     static __device__ __forceinline__ uint32_t choose(int last_fill, int H, float draw, Chooser &p) {
         const int ord = (int)(draw * p.count);
-        const int sh = ord * 4;
-        const uint32_t c = (p.list >> sh) & 7u, c4 = c * 4u;
+        const int sh = ord * 4;   // (as in ply)
+        const uint32_t c = __builtin_amdgcn_ubfe(p.list, (uint32_t)sh, 3), c4 = c * 4u;
         const uint32_t h = (p.fills >> c4) & 15u;
         uint32_t pos;
         asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(pos) : "v"(c), "s"(H), "v"(h));
         p.fills += 1u << c4;
         const bool full = h == (uint32_t)last_fill;
-        const uint32_t low = (1u << sh) - 1u;
+        const uint32_t low = __builtin_amdgcn_ubfe(~0u, 0, (uint32_t)sh);
         p.list = full ? ((p.list & low) | ((p.list >> 4) & ~low)) : p.list;
         p.count -= full ? 0x1p-32f : 0.0f;
         return pos;
