@@ -1,5 +1,6 @@
 """Builds the search kernels for the CPU (tests/simt): the sources as they are, with LDS variables made variables of a workgroup's
 thread and inline assembly replaced by what it does."""
+import atexit
 import functools
 import multiprocessing
 import os
@@ -42,6 +43,12 @@ def rewritten(text, rewrites=REWRITES):
         text = re.sub(pattern, to, text)
     assert rewrites is not REWRITES or "asm(" not in text and "asm volatile" not in text and "__shared__" not in text, re.findall(r".*(?:\basm\b|__shared__).*", text)
     return text
+
+
+def folder_for_this_run():
+    folder = tempfile.mkdtemp()
+    atexit.register(shutil.rmtree, folder, True)
+    return folder
 
 
 def run(command):
@@ -87,7 +94,7 @@ CHECKED = ["-fsanitize=undefined", "-fno-sanitize=function,vptr,alignment", "-fs
 def checked(source):
     """The library of tests/simt/<source>.cpp with FREQUENT draws that ends at undefined behaviour (an index beyond an array's bounds
     among it), and the oracle that goes with it."""
-    folder = tempfile.mkdtemp()
+    folder = folder_for_this_run()
     return build(source, folder, CHECKED, frequent=True), build_oracle(folder)
 
 
@@ -118,7 +125,7 @@ def thread_sanitizer():
 def races(source, module, cases, known=""):
     """What ThreadSanitizer has to say about module.compare(library, *case, **last of case) of the cases, in a process of its own: a
     wavefront is one thread to it, barriers and what is published between workgroups order them.  known: a function to pass over."""
-    folder = tempfile.mkdtemp()
+    folder = folder_for_this_run()
     lib = build(source, folder, ["-fsanitize=thread", "-mllvm", "-tsan-instrument-func-entry-exit=0"], ["-fsanitize=thread", "-shared-libsan"])
     passed_over = os.path.join(folder, "known")
     with open(passed_over, "w") as f:
