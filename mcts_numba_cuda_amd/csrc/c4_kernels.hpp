@@ -297,7 +297,7 @@ struct Chooser { uint32_t fills, list; float count; };
 // 8 trees, 20000 steps: 186 -> 132 ms; 32 playouts of one child, 100 steps: 1.00 -> 0.78 ms; 2 trees of 128 on 7 x 8: 163 -> 102 ms.
 // (Draws made ahead alone, the rest left to one wavefront, gained a search nothing.)
 struct alignas(16) Split {
-    static constexpr int kRing = 128;     // draws per playout (a playout takes up to 57, and as many may have been made ahead of it)
+    static constexpr int kRing = 128;     // draws per playout (a playout takes up to 56, and as many more may have been made ahead)
     static constexpr int kWords = 16;     // moves of a playout, four to a word
     static constexpr uint32_t kNone = 0xffu, kNotYet = 0xffffffffu, kEnd = 0xfffffffeu, kReplayed = 0x8000u;
     static constexpr uint32_t kApart = kWave * sizeof(float), kRingMask = kRing * kApart - 1u;   // places in `draws`: bytes
@@ -1240,9 +1240,10 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
                         __hip_atomic_store(&mail[g], v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
                     }
                 }
-                // Every look of a workgroup at the results line delays the others' stores to it: with 14 or 28 of them the first
-                // comes after 1150 clocks, about when the last result may be there (8 trees of 28, 20000 steps, after 0 / 500 / 750 /
-                // 900 / 1000 / 1300 / 1500 clocks: 145 / 145 / 141 / 139 / 136 / 135 / 136 ms).
+                // Every look of a workgroup at the results line delays the others' stores to it: where a column has several, the first
+                // comes after 1150 clocks, about when the last result may be there.  5000 steps, first look after 0 / 580 / 1150 / 1730
+                // clocks, ms: 4 trees of 14 workgroups 35.4 / 35.6 / 33.7 / 34.4, 8 of 16 (7 x 8) 42.4 / 41.5 / 41.3 / 42.5, 8 of 28 37.6 /
+                // 36.0 / 33.8 / 34.8, 8 of 32 (7 x 8) 43.5 / 42.5 / 41.5 / 42.3.
                 if (SPLIT && parts > 1) __builtin_amdgcn_s_sleep(18);
                 unsigned long long v = 0;
                 bool bad = false;
@@ -1483,8 +1484,8 @@ __device__ __forceinline__ void search_body(const SearchArgs &args, const int r,
 // XCD-aware decode: consecutive blockIdx values go to different XCDs, so the G workgroups of one set are spaced 8
 // apart and meet in one L2.  Set u starts on tree u; when a launch has more trees than sets (a large batch of
 // searches), a set that has finished its tree takes the next one from the queue: workgroup 0 draws the index and
-// leaves it in the finished tree's header for the others.  Five wavefronts per SIMD (at most 96 vector registers: none
-// spilled by the team kernel, eleven dwords by the one with playout pools) let five workgroups share a CU in such batches; a
+// leaves it in the finished tree's header for the others.  Five wavefronts per SIMD (at most 96 vector registers: five
+// dwords spilled by the team kernel, thirteen by the one with playout pools) let five workgroups share a CU in such batches; a
 // single search is no slower for it.
 template <class Game, bool ACP, bool SOLO, bool POOL = false, bool SPLIT = false>
 __device__ __forceinline__ void search_trees(const SearchArgs &args) {

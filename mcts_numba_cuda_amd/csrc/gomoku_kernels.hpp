@@ -520,8 +520,9 @@ __device__ __forceinline__ float draw_rest(Cell *list, Cell *my_times, int from,
     return u_max;
 }
 
-// The runs of five along one direction (DIR 0: right, 1: down, 2: down right, 3: up right) of one playout on the full board,
-// and the earliest ply whose stone made one of them an exact five (all ones: none).  masks: see find_ends.
+// The runs of five along one direction (DIR 0: right, 1: down, 2: down right, 3: up right) of one playout among the stones that the
+// masks hold (those up to the limit, or all: see find_ends), and the earliest ply whose stone made one of them an exact five (all
+// ones: none).
 template <int W, int DIR>
 __device__ __forceinline__ uint32_t earliest_five(const uint32_t *masks, uint32_t *starts, const typename Board<W>::Cell *my_times, const PlayoutShape &shape, uint32_t offset /* of the times */) {
     using Cell = typename Board<W>::Cell;
@@ -827,8 +828,9 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
     const bool keep_rng = !ACP && P <= nslots;
     uint64_t k0 = 0, k1 = 0;
     // What the last step's playouts made of them is worked out while the next step selects, `made` draws from k0, k1 on by the notes
-    // taken of them (0: nothing), up to 16 steps of the generator that were a twentieth of a step of the search: 15 x 15, 4 trees x
-    // 128 playouts, 2000 steps 45.2 -> 42.9 ms, 19 x 19, 300 steps, 11.8 -> 11.4 ms.
+    // taken of them (0: nothing): up to 15 steps of the generator for a game that ended among the first draws, and for one that
+    // outlasted them, of which there are few, as many as it drew beyond.  They were a twentieth of a step of the search: 15 x 15,
+    // 4 trees x 128 playouts, 2000 steps 45.2 -> 42.9 ms, 19 x 19, 300 steps, 11.8 -> 11.4 ms.
     Rng32 notes[ACP ? 1 : B::kCells / kChunk + 1];   // (in memory: a store per chunk and one load cost less than 64 registers)
     int made_last = 0, noted_last = 0;
     auto step_on = [&]() __attribute__((always_inline)) {
@@ -1276,7 +1278,10 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
                 }
                 s_flag = (prev == (uint32_t)(G - 1));
             }
-            // (one wavefront's acquire serves the workgroup, which shares an L1: invalidations take the L2's time too)
+            // (One wavefront's acquire serves the workgroup, which shares an L1: invalidations take the L2's time too.  The others'
+            // loads come after the barrier, so behind the invalidation in the CU's one queue to the L1, which is what the
+            // compiler's model of this chip relies on where an acquire is handed on through a workgroup's barrier.  The walk and the
+            // node records of the backup are read by that wavefront itself.)
             if (wave == 0) fence_acquire_agent();
             __syncthreads();
             leader = s_flag != 0;

@@ -571,9 +571,10 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
     if (!solo && !team_pool && block.x < least_threads && e0->G * n_refs <= cus_now) block = dim3(least_threads);
     // Playouts split over wavefronts (see c4::Split), while every workgroup has a CU to itself: 64 of them to a workgroup, so
     // a column of a team has up to four.  28 workgroups take 0.4 us longer than 7 to exchange a step's results, so the longest
-    // playouts must be long enough: with fewer than 16 cells left on the boards on average, most of such searches lose 2 to 5 %
-    // (6 x 7, 4 trees of 64 to 256: 0.95 to 1.01 of the time at 8 to 16 cells, 1.05 at 24; 5 x 6, one tree of 256, 8 / 12 / 16 / 18 /
-    // 20 / 24 cells: 0.95 / 0.99 / 0.99 / 1.06 / 1.08 / 1.17).
+    // playouts must be long enough: with fewer than 16 cells left on the boards on average, most of such searches lose up to 5 %
+    // (6 x 7, 4 trees of 64 to 256: 0.95 to 1.01 times as fast at 8 to 16 cells, 1.05 at 24; 5 x 6, one tree of 256, 8 / 12 / 16 / 18 /
+    // 20 / 24 cells: 0.95 / 0.99 / 0.99 / 1.06 / 1.08 / 1.17).  The line at a CU each is where the chip ends, not where the form does:
+    // 8 trees of 256 from the empty board take 33.8 ms for 5000 steps, 9, which run unsplit, 46.
     const int parts = e0->acp ? std::max(1, c.n_playouts / kWave) : 1;
     int64_t stones = 0;
     for (int r = 0; r < n_refs; r++) stones += __builtin_popcountll(bb[2 * (size_t)r]) + __builtin_popcountll(bb[2 * (size_t)r + 1]);
