@@ -716,7 +716,7 @@ def bench_c4_many(args):
            "roofline": {"bound": "hbm", "achieved": abytes / dev / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": abytes / dev / 1e9 / HBM_PEAK_GBS,
                         "traffic": (prof or {}).get("traffic_bytes_per_launch") if n == (prof or {}).get("searches") else None,
-                        "kernel": "mctsnc::c4::search_kernel_solo (batches of 896 trees or more), mctsnc::c4::search_kernel<true> below",
+                        "kernel": "mctsnc::c4::search_kernel_solo (batches of 896 trees or more), search_kernel_team_pool (448 or more), search_kernel<true> below",
                         "algorithmic_bytes_per_launch": abytes, "avg_launch_ms": dev * 1e3},
            "roofline_valu": valu_roofline((prof or {}).get("sq_insts_valu_per_pass") if n == (prof or {}).get("searches") else None, dev, prof or {},
                                           f"one pass over {n} searches"),
@@ -872,18 +872,18 @@ def main():
                 # HBM bytes per launch from the rocprofv3 FETCH_SIZE / WRITE_SIZE runs summarised in the named file
                 "traffic": (prof or {}).get("traffic_bytes_per_launch"),
                 "traffic_source": {"file": prof["file"], "commit": prof.get("commit"), "launches": prof.get("traffic_launches")} if prof else None,
-                "kernel": "mctsnc::c4::search_kernel<true>", "algorithmic_bytes_per_launch": alg["total"] / launches,
+                "kernel": "mctsnc::c4::search_kernel_split<true>", "algorithmic_bytes_per_launch": alg["total"] / launches,
                 "avg_launch_ms": dev_time / launches * 1e3,
                 "stage_bytes_per_launch": {k: v / launches for k, v in alg.items() if k != "total"},
                 "playout_plies_per_s": plies / dev_time,
-                "note": "latency-bound pointer chasing plus integer playouts on 28 workgroups: a few KB of tree data per step"}
+                "note": "latency-bound pointer chasing plus integer playouts on 112 workgroups: a few KB of tree data per step"}
 
     # vector-ALU side: the counted instructions of the timed roots over their kernel time
     per_root = (prof or {}).get("sq_insts_valu_per_root")
     roofline_valu = None
     if per_root and len(per_root) == len(roots):
         roofline_valu = valu_roofline(sum(per_root[k % len(roots)] for k in range(args.steps)), dev_time, prof,
-                                      "the timed single searches, search_kernel<true> on 28 of 256 CUs")
+                                      "the timed single searches, search_kernel_split<true> on 112 of 256 CUs")
 
     cpu_baseline = None
     if not args.no_cpu_baseline:
