@@ -116,10 +116,14 @@ def run_apart(function, libraries, *args, **kw):
     assert child.exitcode == 0, f"exit code {child.exitcode}"
 
 
+@functools.lru_cache(None)
 def thread_sanitizer():
-    """ThreadSanitizer's runtime library, or None."""
+    """ThreadSanitizer's runtime library, or None where there is none or it does not run."""
     path = CLANG and subprocess.run([CLANG, "-print-file-name=libclang_rt.tsan-x86_64.so"], stdout=subprocess.PIPE, text=True).stdout.strip()
-    return path if path and os.path.isabs(path) and os.path.exists(path) else None
+    if not path or not os.path.isabs(path) or not os.path.exists(path):
+        return None
+    tried = subprocess.run([sys.executable, "-c", "pass"], env=dict(os.environ, LD_PRELOAD=path), stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    return path if tried.returncode == 0 else None
 
 
 def races(source, module, cases, known=""):
