@@ -541,7 +541,10 @@ __device__ __forceinline__ uint32_t earliest_five(const uint32_t *masks, uint32_
         uint32_t row[kRows];   // (rows beyond the board hold anything; no run starts or ends there)
 #pragma unroll
         for (int i = 0; i < kRows; i++) row[i] = masks[(i * kWords + colour) * 64];
-        uint32_t some = 1u << kLines;   // bit i: a run starts in line i; the line beyond all others is empty and ends the search
+        // bit i: a run starts in line i; the line beyond all others is empty and ends the search, before bit 31, which stays, so that
+        // there is always a first bit
+        constexpr uint32_t kEnds = (1u << kLines) | (1u << 31);
+        uint32_t some = kEnds;
 #pragma unroll
         for (int i = 0; i < kLines; i++) {
             if (WIDE && i % 4 == 0 && i >= lines) break;
@@ -553,7 +556,7 @@ __device__ __forceinline__ uint32_t earliest_five(const uint32_t *masks, uint32_
             if constexpr (DIR != 0) starts[i * 64] = x;
             some |= min(x, 1u) << i;
         }
-        some &= ((1u << lines) - 1u) | (1u << kLines);
+        some &= ((1u << lines) - 1u) | kEnds;
         // Candidates, one per lane and turn, in straight code (a branch costs a wavefront that is alone on its SIMD as much as
         // the instructions it skips): x, the starts left in the present line; ahead, those of the next, the first in `some`,
         // read while the times of the candidate before are.
@@ -561,7 +564,7 @@ __device__ __forceinline__ uint32_t earliest_five(const uint32_t *masks, uint32_
             if constexpr (DIR == 0) { const uint32_t y = masks[(line * kWords + colour) * 64]; return run_of_five(y, y, y, y, y); }
             else return starts[line * 64];
         };
-        auto first = [](uint32_t bits) -> uint32_t { return bits == 0 ? 32u : (uint32_t)__builtin_ctz(bits); };   // (32 if there is none)
+        auto first = [](uint32_t bits) -> uint32_t { return (uint32_t)__builtin_ctz(bits); };
         uint32_t line = first(some), x = line_word(line);
         const Cell *at_line = my_times + (int)line * (stride * 64) + low;
         some &= some - 1;
