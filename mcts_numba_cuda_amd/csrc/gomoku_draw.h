@@ -21,8 +21,6 @@
 /* z + most * 385 / 2^32, times 2^32, for a list of count cells, at most `most` <= 4096: the ordinal is the upper word, unless the lower
  * one is below gomoku_unsure(most). */
 GDRAW_FN uint64_t gomoku_place(uint64_t output, uint32_t count, uint32_t most) {
-    const uint32_t rest = (uint32_t)output >> 11;   /* (of the 53 bits, those that nothing here depends on) */
-    (void)rest;
     return (uint64_t)(uint32_t)(output >> 32) * count + (uint64_t)(most * 385u);
 }
 GDRAW_FN uint32_t gomoku_unsure(uint32_t most) { return most * (384u + 385u); }

@@ -63,7 +63,7 @@ def compare(path, m, n, stones, variant, trees, playouts, steps, groups=3, per_c
 
 
 # rows, columns, stones, variant, trees, playouts, steps, and how the search is laid out: formats of either side of the limit on times,
-# several rounds, two trees to a CU, full pools, paths beyond what is prepared, workgroups on one XCC and on several
+# several rounds, two trees to a CU, all wavefronts on one board of times, full pools, paths beyond what is prepared, workgroups on one XCC and on several
 CASES = [
     (5, 5, 0, "acp_prodigal", 2, 64, 3, dict(groups=5, xccs=8)), (5, 32, 0, "ocp_thrifty", 1, 128, 3, {}), (9, 9, 6, "acp_thrifty", 1, 64, 4, dict(xccs=3)),
     (11, 11, 0, "acp_prodigal", 2, 32, 3, dict(groups=4, xccs=8)), (13, 13, 30, "acp_prodigal", 1, 32, 3, {}), (13, 14, 0, "ocp_prodigal", 2, 256, 4, {}),
@@ -72,6 +72,7 @@ CASES = [
     (16, 16, 0, "ocp_prodigal", 1, 128, 3, {}), (17, 17, 7, "acp_prodigal", 1, 16, 2, {}), (19, 19, 100, "ocp_thrifty", 1, 128, 4, dict(prep=0)),
     (22, 23, 0, "ocp_prodigal", 1, 256, 2, {}), (32, 16, 40, "acp_thrifty", 1, 8, 2, {}), (6, 7, 40, "acp_prodigal", 1, 8, 12, {}),
     (9, 9, 4, "acp_prodigal", 1, 16, 6, dict(room=90)), (8, 8, 4, "ocp_thrifty", 1, 64, 8, dict(room=100)), (7, 7, 0, "acp_thrifty", 1, 4, 3, dict(room=1)),
+    (13, 13, 0, "ocp_thrifty", 1, 32, 3, {}), (16, 16, 9, "ocp_prodigal", 1, 64, 3, {}), (32, 16, 90, "ocp_thrifty", 1, 64, 2, {}),
 ]
 
 
