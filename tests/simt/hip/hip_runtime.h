@@ -43,7 +43,8 @@ inline uint32_t perm(uint32_t s0, uint32_t s1, uint32_t sel) {
     return r;
 }
 inline int dpp(int v, int control) {
-    const int l = where.lane;
+    const int l = where.lane, n = control & 15;
+    if (control > 0x110 && control < 0x120) { const int o = from(kDpp, v, l >= n ? l - n : l); return (l & 15) >= n ? o : 0; }   // (row_shr)
     return from(kDpp, v, control == 0xB1 ? l ^ 1 : control == 0x4E ? l ^ 2 : (l & ~7) | (7 - (l & 7)));
 }
 inline uint64_t ballot(bool v) {
