@@ -1107,7 +1107,8 @@ __global__ void __launch_bounds__(ACP ? kMaxSlots : kMaxThreads) search_kernel_f
                     if (outcome != 2) {
                         const int neg = outcome == -1 ? P : 0, pos = outcome == 1 ? P : 0;
                         *(DeviceQuads)(stats + size + j) = i32x4{P, mover == -1 ? neg : pos, a, 0};
-                        ref.poc[2 * a] = neg; ref.poc[2 * a + 1] = pos;
+                        __attribute__((address_space(1))) int32_t *const poc = (__attribute__((address_space(1))) int32_t *)ref.poc + 2 * a;
+                        poc[0] = neg; poc[1] = pos;
                         ended += (outcome == -1 ? 1u : 0u) | (outcome == 1 ? 0x10000u : 0u);
                     }
                 } else if (j != played) *(DeviceQuads)(stats + size + j) = i32x4{0, 0, a, 0};
