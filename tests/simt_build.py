@@ -34,6 +34,7 @@ REWRITES = [
 FREQUENT = [
     (r"return \(float\)\(\(double\)\((mo_)?rng_next\((s0, s1|s)\) >> 11\)", r"const uint64_t x = \1rng_next(\2); if (x >> 52 == 0xfffu) return 1.0f; return (float)((double)(x >> 11)"),
     (r"( +const double d = __builtin_fma\(\(double\)hi)", r"    if (hi >> 20 == 0xfffu) return 0x1p64f;\n\1"),
+    (r"( +const uint32_t rest = \(uint32_t\)output >> 11;)", r"    if (output >> 52 == 0xfffu) return 0x1p32f;\n\1"),
     (r"( +return \(uint64_t\)\(uint32_t\)\(output >> 32\) \* count)", r"    if (output >> 52 == 0xfffu) return 0;\n\1"),
 ]
 
