@@ -62,8 +62,10 @@ __device__ __forceinline__ void rng_advance32(Rng32 &r) {
     const uint32_t tl = r.s1l ^ r.s0l, th = r.s1h ^ r.s0h;
     // rotl(s0, 55) = rotr(s0, 9); t << 14; rotl(t, 36) = halves swapped, then rotl 4
     const uint32_t r0l = __builtin_amdgcn_alignbit(r.s0h, r.s0l, 9), r0h = __builtin_amdgcn_alignbit(r.s0l, r.s0h, 9);
-    const uint32_t shl = tl << 14, shh = __builtin_amdgcn_alignbit(th, tl, 18);
-    r.s0l = xor3(r0l, tl, shl); r.s0h = xor3(r0h, th, shh);
+    const uint64_t t = ((uint64_t)th << 32) | tl;
+    uint64_t shifted;   // t << 14 in one instruction, which takes as long as one of the two that the compiler makes of it
+    asm("v_lshlrev_b64 %0, 14, %1" : "=v"(shifted) : "v"(t));
+    r.s0l = xor3(r0l, tl, (uint32_t)shifted); r.s0h = xor3(r0h, th, (uint32_t)(shifted >> 32));
     r.s1l = __builtin_amdgcn_alignbit(th, tl, 28); r.s1h = __builtin_amdgcn_alignbit(tl, th, 28);
 }
 

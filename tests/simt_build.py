@@ -24,6 +24,7 @@ REWRITES = [
     (r'asm volatile\("s_waitcnt vmcnt\(0\)" ::: "memory"\);', ";"),
     (r'asm volatile\("" ::: "memory"\);', "simt::together_only();"),   # (the lanes are in step wherever this stands)
     (r'asm\("v_mad_u32_u24 %0, %1, %2, %3" : "=v"\((\w+)\) : "v"\((\w+)\), "s"\((\w+)\), "v"\((\w+)\)\);', r"\1 = simt::mad24(\2, (uint32_t)\3, \4);"),
+    (r'asm\("v_lshlrev_b64 %0, 14, %1" : "=v"\((\w+)\) : "v"\((\w+)\)\);', r"\1 = \2 << 14;"),
     (r'asm(?: volatile)?\("" : [^;]*\);', ";"),
     (r"if \(xcd_local\) wait_own_stores_at_l2\(\);", "simt::together_only();"),   # (a store of all lanes before one of the first)
     # (one lane reads others' registers: all lanes take part)
