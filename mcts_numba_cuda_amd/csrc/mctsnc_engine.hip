@@ -238,7 +238,8 @@ int gomoku_encode_root(const mctsnc_config &c, const int8_t *board, uint32_t *bb
 
 // How a workgroup of a Gomoku search is laid out: its threads, the playouts it runs at a time (a power of two from 64 up) and
 // the boards of times it looks for their ends on (at most one per 256 threads and per 64 playouts), with the dynamic LDS these take.
-// All-children variants: 256 threads and as many playouts (a workgroup plays several children).  One-child variants: two
+// All-children variants: 256 threads and as many playouts (a workgroup plays several children), 512 threads on wide boards, of which
+// a CU holds one workgroup.  One-child variants: two
 // wavefronts draw 64 playouts, so 512 threads and up to 256 playouts while every tree has a CU to itself (the others create
 // the children and prepare the backup meanwhile), 256 threads and up to 128 playouts where two trees share one.  Fewer
 // boards and playouts where they do not fit the LDS of a CU beside the kernel's own 6 KB (8 and 10 KB in the wide formats).
@@ -247,9 +248,9 @@ GomokuLayout gomoku_layout(const mctsnc_config &c, bool acp, bool tree_per_cu) {
     const int words = gomoku_words(c);
     const bool wide = words > 8;
     const int wanted = acp ? c.n_playouts * c.max_actions : c.n_playouts, most = acp || tree_per_cu ? gomoku::kMaxSlots : gomoku::kMaxSlots / 2;
-    GomokuLayout g{acp || !tree_per_cu ? gomoku::kMaxThreads / 2 : gomoku::kMaxThreads, 64, 0, 0};
+    GomokuLayout g{(acp ? !wide : !tree_per_cu) ? gomoku::kMaxThreads / 2 : gomoku::kMaxThreads, 64, 0, 0};
     while (g.slots < wanted && g.slots < most) g.slots *= 2;
-    g.teams = std::min(g.threads / 256, g.slots / 64);
+    g.teams = acp ? 1 : std::min(g.threads / 256, g.slots / 64);
     for (;;) {
         g.lds = gomoku::playout_lds_bytes(c.board_m, c.board_n, g.slots, g.teams, wide, acp) + (acp ? 0 : (size_t)(g.slots / 64) * gomoku::kRingBytes);
         if (g.lds + (size_t)(words > 12 ? 10 : wide ? 8 : 6) * 1024 <= 160 * 1024 || (g.slots == 64 && g.teams == 1)) return g;

@@ -73,6 +73,7 @@ CASES = [
     (22, 23, 0, "ocp_prodigal", 1, 256, 2, {}), (32, 16, 40, "acp_thrifty", 1, 8, 2, {}), (6, 7, 40, "acp_prodigal", 1, 8, 12, {}),
     (9, 9, 4, "acp_prodigal", 1, 16, 6, dict(room=90)), (8, 8, 4, "ocp_thrifty", 1, 64, 8, dict(room=100)), (7, 7, 0, "acp_thrifty", 1, 4, 3, dict(room=1)),
     (13, 13, 0, "ocp_thrifty", 1, 32, 3, {}), (16, 16, 9, "ocp_prodigal", 1, 64, 3, {}), (32, 16, 90, "ocp_thrifty", 1, 64, 2, {}),
+    (16, 16, 200, "acp_thrifty", 1, 128, 3, dict(groups=5, xccs=8)), (22, 22, 440, "acp_prodigal", 1, 2, 3, {}),
 ]
 
 
