@@ -115,11 +115,17 @@ __host__ __device__ inline PlayoutShape playout_shape(int m, int n, bool wide, b
     s.origin = s.stride + 1; s.time_rows = s.origin + (wide ? s.rows + 1 : s.rows + 1 > 16 ? s.rows + 1 : 16) * s.stride;
     return s;
 }
-// Dynamic LDS of the search kernel: the lists of `slots` playouts, then for each team of four wavefronts the board of times
-// of the 64 playouts whose ends it looks for.
+// Where two wavefronts draw 64 playouts (one-child variants, wide boards), they share a ring of offsets, two bytes a draw (make_offsets).
+constexpr int kRingChunks = 2;
+constexpr int kRingBytes = kRingChunks * kChunk * 64 * 2;   // per 64 playouts
+// Dynamic LDS of the search kernel: the lists of `slots` playouts, then for each team of wavefronts the board of times of the 64
+// playouts whose ends it looks for, then the rings.  All-children variants keep the rings in the place of the one board that they
+// have, and beyond its end where they need more: 5 x 17 and 17 x 5 with 256 playouts (16384 bytes against 16256).
 __host__ __device__ inline size_t playout_lds_bytes(int m, int n, int slots, int teams, bool wide, bool acp) {
     const PlayoutShape s = playout_shape(m, n, wide, acp);
-    return ((size_t)s.list_rows * slots + (size_t)s.time_rows * 64 * teams) * (wide ? 2 : 1);
+    const size_t cell = wide ? 2 : 1, lists = (size_t)s.list_rows * slots * cell, times = (size_t)s.time_rows * 64 * teams * cell;
+    const size_t rings = !acp || wide ? (size_t)(slots / 64) * kRingBytes : 0;
+    return lists + (acp ? (times > rings ? times : rings) : times + rings);
 }
 constexpr int kLevels = 8;         // path levels whose arg-max the backup evaluates together
 constexpr int kPrepLevels = 48;    // path levels whose arg-max the one-child variants prepare during the playouts (deeper paths: as above)
@@ -430,9 +436,8 @@ __device__ __forceinline__ float draw_list(Cell *list, int count, Rng32 &rg, Rng
 // ordinals (gomoku_draw.h) instead of uniforms by way of float64; 109 -> 88 the walker, which reads each list entry when the write
 // before it is on its way and not a draw ahead (no reads to put right), and its offsets long before it needs them.
 // 15 x 15, 4 trees x 128 playouts: draws 20.9 -> 18.9 thousand clocks a step.
-constexpr int kRingChunks = 2;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-constexpr int kRingBytes = kRingChunks * kChunk / 4 * 64 * (int)sizeof(u32x2);   // per 64 playouts
+static_assert(kRingBytes == kRingChunks * kChunk / 4 * 64 * (int)sizeof(u32x2), "four draws of a lane are an entry of the ring");
 __device__ __forceinline__ uint32_t lds_count(const uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 __device__ __forceinline__ void set_lds_count(uint32_t *p, uint32_t v) {
     asm volatile("" ::: "memory");
@@ -874,7 +879,7 @@ __global__ void __launch_bounds__(ACP && W == 8 ? kMaxSlots : kMaxThreads) searc
     const int teams = args.teams, team_waves = teams == 1 ? nwaves : 4, team = team_waves == 8 ? 0 : wave >> 2;
     Cell *const team_times = s_times + (team * shape.time_rows + shape.origin) * 64;   // (row of cell 0)
     // where two wavefronts draw, per 64 playouts kRingBytes: behind the boards of times, all-children variants in the place of the one that
-    // they have (29 KB at least)
+    // they have (playout_lds_bytes counts the larger of the two)
     u32x2 *const s_ring = reinterpret_cast<u32x2 *>(ACP ? s_times : s_times + teams * shape.time_rows * 64);
     constexpr int kPack = 4 / (int)sizeof(Cell);                                // playouts whose entries share a dword
     constexpr uint32_t kCopies = WIDE ? 0x00010001u : 0x01010101u;

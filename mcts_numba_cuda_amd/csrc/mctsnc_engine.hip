@@ -252,7 +252,7 @@ GomokuLayout gomoku_layout(const mctsnc_config &c, bool acp, bool tree_per_cu) {
     while (g.slots < wanted && g.slots < most) g.slots *= 2;
     g.teams = acp ? 1 : std::min(g.threads / 256, g.slots / 64);
     for (;;) {
-        g.lds = gomoku::playout_lds_bytes(c.board_m, c.board_n, g.slots, g.teams, wide, acp) + (acp ? 0 : (size_t)(g.slots / 64) * gomoku::kRingBytes);
+        g.lds = gomoku::playout_lds_bytes(c.board_m, c.board_n, g.slots, g.teams, wide, acp);
         if (g.lds + (size_t)(words > 12 ? 10 : wide ? 8 : 6) * 1024 <= 160 * 1024 || (g.slots == 64 && g.teams == 1)) return g;
         if (g.teams > 1) g.teams = 1;
         else g.slots /= 2;

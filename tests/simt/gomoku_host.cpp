@@ -16,6 +16,20 @@ struct Reset { const gomoku::TreeRef *refs; int n; const uint32_t *bb; const int
 void reset(const void *args) { const Reset &r = *static_cast<const Reset *>(args); gomoku::reset_kernel(r.refs, r.n, r.bb, r.turns); }
 }
 
+// The layout of a search: threads, slots, boards of times, dynamic LDS; and what the kernel puts there, in bytes: the lists, the boards
+// of times, a ring of offsets for every 64 slots (counted from playout_shape and the ring's format).
+extern "C" void simt_gomoku_layout(int m, int n, int P, int acp, int tree_per_cu, int64_t *out) {
+    mctsnc_config c = {};
+    c.board_m = m; c.board_n = n; c.max_actions = m * n; c.n_playouts = P;
+    const bool wide = gomoku_words(c) > 8;
+    const GomokuLayout layout = gomoku_layout(c, acp != 0, tree_per_cu != 0);
+    const gomoku::PlayoutShape shape = gomoku::playout_shape(m, n, wide, acp != 0);
+    const int64_t cell = wide ? 2 : 1;
+    out[0] = layout.threads; out[1] = layout.slots; out[2] = layout.teams; out[3] = (int64_t)layout.lds;
+    out[4] = cell * shape.list_rows * layout.slots; out[5] = cell * shape.time_rows * 64 * layout.teams;
+    out[6] = (int64_t)(layout.slots / 64) * gomoku::kRingChunks * gomoku::kChunk / 4 * 64 * (int64_t)sizeof(gomoku::u32x2);
+}
+
 // One search of `trees` trees of a workgroup count G each, `launches` times nsteps steps.  nodes: per tree S records of
 // node_bytes; stats: per tree S times 4 int32; sizes: nodes of each tree; rng_*: states, before and after.  0, or -1: given up.
 extern "C" int simt_gomoku(int m, int n, int trees, int P, int acp, int thrifty, int G, int tree_per_cu, int S, int nsteps, int launches, float ucb_c, int prep_levels, int xccs, unsigned seed,

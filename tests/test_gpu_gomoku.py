@@ -125,6 +125,14 @@ def test_gomoku_boards_beyond_sixteen(variant, steps):
             compare_with_oracle(e, o, board, None, turn, max(2, int(steps * scale)))
 
 
+@pytest.mark.parametrize("m,n,variant,playouts", [(5, 17, "acp_prodigal", 64), (17, 5, "acp_thrifty", 128), (17, 5, "acp_prodigal", 2), (5, 17, "ocp_thrifty", 256)])
+def test_gomoku_boards_whose_offsets_outgrow_the_board_of_times(m, n, variant, playouts):
+    """All children: the smallest wide boards, whose rings of offsets do not fit the board of times in whose place they are."""
+    e, o = engines(variant, 2, playouts, m, n, seed=5)
+    board, turn = random_gomoku_root(np.random.default_rng(17), m, n, 6)
+    compare_with_oracle(e, o, board, None, turn, 6)
+
+
 @pytest.mark.parametrize("variant,steps", [("ocp_thrifty", 30), ("ocp_prodigal", 30), ("acp_thrifty", 2), ("acp_prodigal", 2)])
 def test_gomoku_boards_up_to_the_references_caps(variant, steps):
     """Boards of more than 384 cells need 16 words per colour and a 256-byte node record: 22 x 22, the two extreme shapes

@@ -74,6 +74,7 @@ CASES = [
     (9, 9, 4, "acp_prodigal", 1, 16, 6, dict(room=90)), (8, 8, 4, "ocp_thrifty", 1, 64, 8, dict(room=100)), (7, 7, 0, "acp_thrifty", 1, 4, 3, dict(room=1)),
     (13, 13, 0, "ocp_thrifty", 1, 32, 3, {}), (16, 16, 9, "ocp_prodigal", 1, 64, 3, {}), (32, 16, 90, "ocp_thrifty", 1, 64, 2, {}),
     (16, 16, 200, "acp_thrifty", 1, 128, 3, dict(groups=5, xccs=8)), (22, 22, 440, "acp_prodigal", 1, 2, 3, {}),
+    (5, 17, 0, "acp_prodigal", 1, 64, 2, {}), (17, 5, 0, "acp_thrifty", 1, 128, 2, {}),   # (rings larger than the board of times in whose place they are)
 ]
 
 
@@ -82,6 +83,28 @@ CASES = [
 def test_searches_on_the_cpu_equal_the_oracle(case):
     """With one draw in 4096 rounded up to 1.0f, so that playouts are replayed all the time."""
     simt_build.run_apart(compare, simt_build.checked("gomoku_host"), *case[:-1], **case[-1])
+
+
+@needs_clang
+def test_every_layout_holds_what_the_kernel_puts_there():
+    """For all boards and numbers of playouts that an engine takes: the lists, the boards of times and, where two wavefronts draw, the rings of
+    offsets lie within the LDS that is asked for, the rings behind the boards or (all children) in the place of the one there is."""
+    layout_of = ctypes.CDLL(simt_build.checked("gomoku_host")[0]).simt_gomoku_layout
+    out = (ctypes.c_int64 * 7)()
+    tight = set()
+    for m, n in ((m, n) for m in range(5, 33) for n in range(5, 33) if m * n <= 512):
+        for playouts, acp, per_cu in ((1 << k, acp, per_cu) for k in range(10) for acp in (0, 1) for per_cu in (0, 1)):
+            layout_of(m, n, playouts, acp, per_cu, out)
+            threads, slots, teams, lds, lists, times, rings = out
+            wide = words_of(m, n) > 8
+            two_draw = wide or not acp
+            assert threads in (256, 512) and slots in (64, 128, 256) and (2 if two_draw else 1) * slots <= threads, (m, n, playouts, acp, per_cu)
+            assert 1 <= teams <= max(1, threads // 256) and (teams == 1 or not acp), (m, n, playouts, acp, per_cu)
+            needed = lists + (times + rings if not acp else max(times, rings if wide else 0))
+            assert lds >= needed, (m, n, playouts, acp, per_cu, lds, needed)
+            if acp and wide and rings > times:
+                tight.add((m, n))
+    assert tight == {(5, 17), (17, 5)}
 
 
 @pytest.mark.skipif(simt_build.thread_sanitizer() is None, reason="no ThreadSanitizer")
