@@ -127,6 +127,11 @@ __host__ __device__ inline size_t playout_lds_bytes(int m, int n, int slots, int
     const size_t rings = !acp || wide ? (size_t)(slots / 64) * kRingBytes : 0;
     return lists + (acp ? (times > rings ? times : rings) : times + rings);
 }
+// LDS of a CU, of which a workgroup can have all, and the most that the search kernels of a board format declare for themselves beside the
+// dynamic part: one child 6192, 8384 and 9824 bytes for 8, 12 and 16 words, all children 5632, 8112 and 9808 (a test compares the
+// built library with these).  No rounder: one child on 9 x 18 with 256 playouts leaves 8448, all children on 11 x 21 with 256 leave 8320.
+constexpr size_t kLdsBytes = 160 * 1024;
+__host__ __device__ inline size_t kernel_lds_bytes(int words, bool acp) { return words > 12 ? 9984 : words > 8 ? (acp ? 8192 : 8448) : (acp ? 6144 : 6272); }
 constexpr int kLevels = 8;         // path levels whose arg-max the backup evaluates together
 constexpr int kPrepLevels = 48;    // path levels whose arg-max the one-child variants prepare during the playouts (deeper paths: as above)
 constexpr int kMaxSlots = 256;    // playouts beyond this run in several rounds of the same workgroup

@@ -242,7 +242,7 @@ int gomoku_encode_root(const mctsnc_config &c, const int8_t *board, uint32_t *bb
 // a CU holds one workgroup.  One-child variants: two
 // wavefronts draw 64 playouts, so 512 threads and up to 256 playouts while every tree has a CU to itself (the others create
 // the children and prepare the backup meanwhile), 256 threads and up to 128 playouts where two trees share one.  Fewer
-// boards and playouts where they do not fit the LDS of a CU beside the kernel's own 6 KB (8 and 10 KB in the wide formats).
+// boards and playouts where they do not fit the LDS of a CU beside what the kernel declares (kernel_lds_bytes).
 struct GomokuLayout { int threads, slots, teams; size_t lds; };
 GomokuLayout gomoku_layout(const mctsnc_config &c, bool acp, bool tree_per_cu) {
     const int words = gomoku_words(c);
@@ -253,7 +253,7 @@ GomokuLayout gomoku_layout(const mctsnc_config &c, bool acp, bool tree_per_cu) {
     g.teams = acp ? 1 : std::min(g.threads / 256, g.slots / 64);
     for (;;) {
         g.lds = gomoku::playout_lds_bytes(c.board_m, c.board_n, g.slots, g.teams, wide, acp);
-        if (g.lds + (size_t)(words > 12 ? 10 : wide ? 8 : 6) * 1024 <= 160 * 1024 || (g.slots == 64 && g.teams == 1)) return g;
+        if (g.lds + gomoku::kernel_lds_bytes(words, acp) <= gomoku::kLdsBytes || (g.slots == 64 && g.teams == 1)) return g;   // (64 playouts fit every board)
         if (g.teams > 1) g.teams = 1;
         else g.slots /= 2;
     }

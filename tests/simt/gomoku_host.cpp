@@ -16,6 +16,9 @@ struct Reset { const gomoku::TreeRef *refs; int n; const uint32_t *bb; const int
 void reset(const void *args) { const Reset &r = *static_cast<const Reset *>(args); gomoku::reset_kernel(r.refs, r.n, r.bb, r.turns); }
 }
 
+extern "C" int64_t simt_gomoku_kernel_lds(int words, int acp) { return (int64_t)gomoku::kernel_lds_bytes(words, acp != 0); }
+extern "C" int64_t simt_gomoku_cu_lds() { return (int64_t)gomoku::kLdsBytes; }
+
 // The layout of a search: threads, slots, boards of times, dynamic LDS; and what the kernel puts there, in bytes: the lists, the boards
 // of times, a ring of offsets for every 64 slots (counted from playout_shape and the ring's format).
 extern "C" void simt_gomoku_layout(int m, int n, int P, int acp, int tree_per_cu, int64_t *out) {

@@ -2,14 +2,21 @@
 barriers), against the oracle."""
 import ctypes
 import functools
+import os
+import re
+import struct
+import subprocess
 
 import numpy as np
 import pytest
 
 import simt_build
 from helpers import random_gomoku_root
+from mcts_numba_cuda_amd import _lib
+from mcts_numba_cuda_amd.build import LIB
 from oracle.oracle import Oracle
 
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 needs_clang = pytest.mark.skipif(simt_build.CLANG is None, reason="no clang++")
 
 
@@ -88,8 +95,10 @@ def test_searches_on_the_cpu_equal_the_oracle(case):
 @needs_clang
 def test_every_layout_holds_what_the_kernel_puts_there():
     """For all boards and numbers of playouts that an engine takes: the lists, the boards of times and, where two wavefronts draw, the rings of
-    offsets lie within the LDS that is asked for, the rings behind the boards or (all children) in the place of the one there is."""
-    layout_of = ctypes.CDLL(simt_build.checked("gomoku_host")[0]).simt_gomoku_layout
+    offsets lie within the LDS that is asked for, the rings behind the boards or (all children) in the place of the one there is; and a CU
+    has that much beside what the kernel declares for itself."""
+    lib = ctypes.CDLL(simt_build.checked("gomoku_host")[0])
+    layout_of, of_kernel, of_cu = lib.simt_gomoku_layout, lib.simt_gomoku_kernel_lds, lib.simt_gomoku_cu_lds()
     out = (ctypes.c_int64 * 7)()
     tight = set()
     for m, n in ((m, n) for m in range(5, 33) for n in range(5, 33) if m * n <= 512):
@@ -102,9 +111,35 @@ def test_every_layout_holds_what_the_kernel_puts_there():
             assert 1 <= teams <= max(1, threads // 256) and (teams == 1 or not acp), (m, n, playouts, acp, per_cu)
             needed = lists + (times + rings if not acp else max(times, rings if wide else 0))
             assert lds >= needed, (m, n, playouts, acp, per_cu, lds, needed)
+            assert lds + of_kernel(words_of(m, n), acp) <= of_cu, (m, n, playouts, acp, per_cu, lds)
             if acp and wide and rings > times:
                 tight.add((m, n))
     assert tight == {(5, 17), (17, 5)}
+
+
+@needs_clang
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_the_kernels_declare_no_more_lds_than_layouts_leave_them(tmp_path):
+    """The built library's own figures (its code objects' notes) against kernel_lds_bytes."""
+    _lib.lib()
+    with open(LIB, "rb") as f:
+        data = f.read()
+    at = data.index(b"__CLANG_OFFLOAD_BUNDLE__")
+    entries, found = at + 32, {}
+    for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):   # (offset, size, length of the target's name; the name)
+        offset, size, length = struct.unpack_from("<QQQ", data, entries)
+        if b"gfx950" in data[entries + 24:entries + 24 + length]:
+            (tmp_path / "code").write_bytes(data[at + offset:at + offset + size])
+            notes = subprocess.check_output([READELF, "--notes", str(tmp_path / "code")], text=True)
+            for kernel in re.split(r"\n  - ", notes):
+                name = re.search(r"\.name: +\S*search_kernel_forINS0_6GomokuELb([01])ELi(\d+)E", kernel)
+                if name:
+                    found[int(name[1]), int(name[2])] = int(re.search(r"\.group_segment_fixed_size: (\d+)", kernel)[1])
+        entries += 24 + length
+    assert sorted(found) == [(acp, words) for acp in (0, 1) for words in (8, 12, 16)]
+    most = ctypes.CDLL(simt_build.checked("gomoku_host")[0]).simt_gomoku_kernel_lds
+    for (acp, words), declared in found.items():
+        assert 4096 < declared <= most(words, acp), (acp, words, declared, most(words, acp))
 
 
 @pytest.mark.skipif(simt_build.thread_sanitizer() is None, reason="no ThreadSanitizer")
