@@ -40,9 +40,12 @@ FREQUENT = [
 ]
 
 
-def rewritten(text, rewrites=REWRITES):
-    for pattern, to in rewrites:
-        text = re.sub(pattern, to, text)
+def rewritten(text, rewrites=REWRITES, counts=None):
+    """`counts`: how often each pattern has matched, added up."""
+    for i, (pattern, to) in enumerate(rewrites):
+        text, matches = re.subn(pattern, to, text)
+        if counts is not None:
+            counts[i] += matches
     assert rewrites is not REWRITES or "asm(" not in text and "asm volatile" not in text and "__shared__" not in text, re.findall(r".*(?:\basm\b|__shared__).*", text)
     return text
 
@@ -62,8 +65,9 @@ def build_oracle(folder):
     """The oracle with draws as in build(frequent=True)."""
     source, lib = os.path.join(folder, "oracle.c"), os.path.join(folder, "liboracle.so")
     with open(os.path.join(os.path.dirname(HERE), "oracle", "mctsnc_oracle.c")) as f, open(source, "w") as out:
-        text = f.read()
-        out.write(rewritten(text, FREQUENT[:1]))
+        counts = [0]
+        out.write(rewritten(f.read(), FREQUENT[:1], counts))
+    assert all(counts), "the oracle's draws are not rounded up"
     run(["gcc", "-O2", "-std=gnu99", "-fPIC", "-fopenmp", "-ffp-contract=off", "-shared", "-o", lib, source, "-lm"])
     return lib
 
@@ -71,11 +75,13 @@ def build_oracle(folder):
 def build(source, folder, flags=(), libraries=(), frequent=False):
     """Compiles tests/simt/<source>.cpp and returns the shared library's path (`flags`: sanitizers, for the kernels alone;
     `frequent`: with FREQUENT draws)."""
+    counts = [0] * len(FREQUENT)
     for name in os.listdir(CSRC):
         if name.endswith((".h", ".hpp")):
             with open(os.path.join(CSRC, name)) as f, open(os.path.join(folder, name), "w") as out:
-                text = f.read()
-                out.write(rewritten(rewritten(text), FREQUENT) if frequent else rewritten(text))
+                text = rewritten(f.read())
+                out.write(rewritten(text, FREQUENT, counts) if frequent else text)
+    assert not frequent or all(counts), [pattern for (pattern, _), n in zip(FREQUENT, counts) if n == 0]
     with open(os.path.join(CSRC, "mctsnc_engine.hip")) as f:
         engine = f.read()
     words, layout = re.search(r"^int gomoku_words\(.*?^}", engine, re.M | re.S), re.search(r"^struct GomokuLayout .*?^}", engine, re.M | re.S)
