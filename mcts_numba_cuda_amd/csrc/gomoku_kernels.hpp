@@ -680,7 +680,7 @@ __device__ __forceinline__ uint32_t earliest_five(const uint32_t *masks, uint32_
 // orders of E cells each of which the first `drawn` have been drawn (ACP: all), `times` is the team's board of times at cell 0 (timed: the drawn cells' times are there already), own_row the row of the one stone that playout
 // `lane` has beside its node's (of the side that does not move first; ~0: none).  ends[lane] becomes the ply whose stone
 // completes the first exact five of playout `lane`, all ones (or a number beyond all plies) if there is none; 0 for a playout that
-// is not wanted.  ends is one of the `teams` rows of all_ends, null beside them; offset as time_offset or first_offset gives it.  The lists are used up from mask_row on; draw_rest is
+// is not wanted.  ends is the team's row of the `teams` of all_ends; offset as time_offset or first_offset gives it.  The lists are used up from mask_row on; draw_rest is
 // called before a second look, if there is one, and puts the times of the plies that were not drawn on the boards.
 template <bool ACP, int W, class Rest>
 __device__ __forceinline__ void find_ends(int team_waves, bool work, bool timed, typename Board<W>::Cell *list, typename Board<W>::Cell *times, uint32_t *ends,
@@ -782,7 +782,7 @@ __device__ __forceinline__ void find_ends(int team_waves, bool work, bool timed,
                 *reinterpret_cast<u32x4 *>(all_masks + r * 64 + (lane & 15) * 4) = word;
             }
         }
-        if (wave == 0 && first && ends != nullptr) {
+        if (wave == 0 && first) {
             ends[lane] = work && wanted ? ~0u : 0u;
             if (work) {
                 for (int c = 0; c < kWords; c++) masks[(kRows * kWords + c) * 64] = 0;   // the empty line beyond all others
@@ -1233,12 +1233,11 @@ __global__ void __launch_bounds__(ACP && W == 8 ? kMaxSlots : kMaxThreads) searc
             const uint32_t offset = ACP ? time_offset(cells, E, WIDE) : first_offset(first, E, WIDE);
             // times of the node's stones: 0 for the side to move in the playouts, 1 for the other (they stay until the next step)
             auto put_stones = [=]() {
-                if (team < teams)
-                    for (int i = tid & (64 * team_waves - 1); i < (cells - empties) * kRowDwords; i += 64 * team_waves) {
-                        const uint32_t stone = s_cells[B::kCells - i / kRowDwords];
-                        reinterpret_cast<uint32_t *>(team_times)[(int)(stone & 0xffffu) * kRowDwords + i % kRowDwords] =
-                            ((stone >> 31) == (pturn == -1 ? 1u : 0u) ? offset : offset + 1u) * kCopies;
-                    }
+                for (int i = tid & (64 * team_waves - 1); i < (cells - empties) * kRowDwords; i += 64 * team_waves) {
+                    const uint32_t stone = s_cells[B::kCells - i / kRowDwords];
+                    reinterpret_cast<uint32_t *>(team_times)[(int)(stone & 0xffffu) * kRowDwords + i % kRowDwords] =
+                        ((stone >> 31) == (pturn == -1 ? 1u : 0u) ? offset : offset + 1u) * kCopies;
+                }
             };
             if (!(ACP && kTwoDraw)) put_stones();
             for (int round0 = 0; round0 < total; round0 += nslots) {
@@ -1323,7 +1322,7 @@ __global__ void __launch_bounds__(ACP && W == 8 ? kMaxSlots : kMaxThreads) searc
                                 u_max = draw_rest<Cell>(my_list, s_times + ((wave - g0) * shape.time_rows + shape.origin) * 64 + lane, first, E, offset + 2u, rg, u_max);
                         }
                     };
-                    find_ends<ACP, W>(team_waves, grp < groups && team < teams, !ACP && g0 == 0, s_list + (size_t)grp * shape.list_rows * 64, team_times, team < teams ? s_end[team] : nullptr, shape, E, first,
+                    find_ends<ACP, W>(team_waves, grp < groups, !ACP && g0 == 0, s_list + (size_t)grp * shape.list_rows * 64, team_times, s_end[team], shape, E, first,
                                  with_stone ? time_row((uint32_t)s_actions[ordinal_of(round0 + grp * 64 + lane)]) : ~0u, (team & 1) != 0, wave & (team_waves - 1), lane,
                                  round0 + grp * 64 + lane < total, s_end, teams, offset, draw_rest_now);
                     if (wave - g0 < teams && wave >= g0 && wave < groups) end_ply = s_end[wave - g0][lane];
