@@ -47,6 +47,7 @@ template <int W> struct Board {
 // full (src/mctsnc.py:1877-1895 and its all-children twins).  What it draws does not depend on the stones, so a lane draws
 // the whole permutation of the node's E empty cells without looking at the board, and the ply that ended the game is found
 // afterwards, from the time at which each cell was taken.
+//     Two wavefronts share the draws of 64 playouts where a workgroup has a CU to itself (kTwoDraw, in the kernel).
 //   * A draw is a generator step, its conversion to an ordinal, two list reads and two writes: 30 instructions, against 110
 //     to 125 of a ply that also kept the line words of the board and tested them, in a loop that runs until the longest of
 //     64 playouts has ended (165 plies of 15 x 15 where the mean is 103).  All lanes draw the same number of cells, so
@@ -62,14 +63,14 @@ template <int W> struct Board {
 //     neighbouring cell held its colour by then: seven reads and a dozen instructions.  The earliest complete five is the
 //     end of the game.  A wavefront takes one of the four directions.
 //   * The generator is left where the game ended: its state is noted every sixteenth draw and stepped on from the last note
-//     before the end; in one-child searches while the next step selects.
+//     before the end; in one-child searches whose playouts fit one round while the next step selects.
 // Boards of the narrow format are laid out with rows of at most 15 cells (on their side, if need be), so that a row's masks
 // of both colours share a dword; cells and times are bytes.  Wide ones are laid on their longer side: at most 22 rows.
 // 16 x 16 has no side of 15 cells and is wide, with two-byte cells, though its cells would fit a byte: it gained less than its
 // neighbours when playouts began to draw first, but gained (before, in the narrow format, ply by ply / now: one child, 4 trees x 128
 // playouts, 500 steps 29.1 / 14.7 ms, all children, 8 x 128, 60 steps 26.9 / 17.5; 16 x 15 27.3 / 12.6 and 25.2 / 11.2).
 constexpr int kMaxRowsWide = 22;
-constexpr int kChunk = 16;   // draws that the wavefronts of a one-child playout hand on at a time
+constexpr int kChunk = 16;   // draws between two notes of a generator, and those that one of two drawing wavefronts hands to the other at a time
 // Few games last until the board is nearly full: one in a thousand ends with more stones on the board than 60 and 9 / 16 of
 // its cells (186 of 225; one in two with 113).  So find_ends looks at the runs that are complete by about then first, (192 / 225)^5 =
 // 0.45 of the candidates and (269 / 361)^5 = 0.23 of those of 19 x 19, and looks again, at all of them, where 64 playouts hold a game
@@ -208,8 +209,8 @@ struct SearchArgs {
     int32_t m, n;
     int32_t P;
     int32_t G;              // workgroups per tree
-    int32_t slots;          // playouts a workgroup runs at a time (a power of two from 64 to its threads)
-    int32_t teams;          // boards of times: one per 256 threads, if the LDS holds them (one at least)
+    int32_t slots;          // playouts a workgroup runs at a time (a power of two from 64 to its threads, to half of them where two wavefronts draw)
+    int32_t teams;          // boards of times: one per 256 threads and 64 slots, if the LDS holds them (one at least; all children: one)
     int32_t S;
     int32_t nsteps;
     int32_t thrifty;
@@ -498,7 +499,7 @@ __device__ __forceinline__ float make_offsets(u32x2 *ring, uint32_t *made, const
                 o[i] = (uint32_t)(place >> 32);
                 closest = min(closest, (uint32_t)place);
             }
-            if (__builtin_expect(__ballot(closest < gomoku_unsure(most)) != 0, 0)) {   // one time in 2^16 / most: all four as the reference does
+            if (__builtin_expect(__ballot(closest < gomoku_unsure(most)) != 0, 0)) {   // one time in 2^14.4 / most (64 lanes of four draws, 769 most / 2^32 each): all four as the reference does
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const float u = uniform_scaled_from_bits(lo[i], hi[i]);
@@ -835,10 +836,13 @@ __global__ void __launch_bounds__(ACP && W == 8 ? kMaxSlots : kMaxThreads) searc
     using B = Board<W>;
     constexpr bool WIDE = B::kWide;
     constexpr int QBITS = WIDE ? 9 : 8;
-    // Two wavefronts draw 64 playouts (make_offsets, walk_list) where a CU has one workgroup, which then has eight: one-child variants, and
-    // all-children ones on wide boards, whose lists leave no room for another (19 x 19, 4 trees x 128 playouts, 60 steps: 16.8 -> 14.1 ms;
-    // 22 x 22, 8 x 256, 4 steps: 10.8 -> 9.2).  On narrow boards two workgroups of four wavefronts share a CU, each drawing for itself:
-    // two of eight take as long with 8 trees of 15 x 15 (39.5 ms against 38.5) and 12 % longer with 4 x 256 playouts of 9 x 9.
+    // Two wavefronts draw 64 playouts (make_offsets, walk_list) in one-child variants, and in all-children ones on wide boards, whose lists
+    // leave a CU room for one workgroup, which has eight wavefronts (19 x 19, 4 trees x 128 playouts, 60 steps: 16.8 -> 14.1 ms;
+    // 22 x 22, 8 x 256, 4 steps: 10.8 -> 9.2).  The smallest wide boards, us a step with four wavefronts / with eight: 5 x 18, 8 trees x 1
+    // playout (one playout on about 100 cells: the only layouts of which the LDS held two) 43.1 / 34.7, 4 x 32 29.4 / 29.5, 4 x 256 66.9 / 65.8;
+    // 6 x 17, 4 x 32 30.5 / 31.0, 4 x 64 32.5 / 31.8; 12 x 17, 4 x 256 179.6 / 165.9.  So the line is the format's, though four are up to
+    // 2 % ahead on boards of 90 to 108 cells with 16 or 32 playouts.  On narrow boards two workgroups of four wavefronts share a CU, each
+    // drawing for itself: two of eight take as long with 8 trees of 15 x 15 (39.5 ms against 38.5) and 12 % longer with 4 x 256 playouts of 9 x 9.
     constexpr bool kTwoDraw = !ACP || WIDE;
     constexpr unsigned long long kQMask = (1ull << QBITS) - 1ull;
     // The G workgroups of a tree are consecutive, and consecutive blockIdx values go to different XCDs: every tree is
@@ -935,7 +939,7 @@ __global__ void __launch_bounds__(ACP && W == 8 ? kMaxSlots : kMaxThreads) searc
     // taken of them (0: nothing): up to 15 steps of the generator for a game that ended among the first draws, and for one that
     // outlasted them, of which there are few, as many as it drew beyond.  They were a twentieth of a step of the search: 15 x 15,
     // 4 trees x 128 playouts, 2000 steps 45.2 -> 42.9 ms, 19 x 19, 300 steps, 11.8 -> 11.4 ms.
-    Rng32 notes[kTwoDraw ? B::kCells / kChunk + 1 : 1];   // (in memory: a store per chunk and one load cost less than 64 registers)
+    Rng32 notes[kTwoDraw ? B::kCells / kChunk + 1 : 1];   // (in memory, 288, 416 or 544 bytes a lane: a store per chunk and one load cost less than 64 registers)
     int made_last = 0, noted_last = 0;
     auto step_on = [&]() __attribute__((always_inline)) {
         Rng32 rg = notes[noted_last];
