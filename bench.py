@@ -473,8 +473,8 @@ def bench_gomoku(args):
                         "kernel": "mctsnc::gomoku::search_kernel_for<Gomoku, false, 8>", "algorithmic_bytes_per_launch": alg["total"] / steps,
                         "avg_launch_ms": dev / steps * 1e3,
                         "stage_bytes_per_launch": {k: v / steps for k, v in alg.items() if k != "total"},
-                        "note": "four workgroups of two wavefronts: bound by the length of the longest playout "
-                                "(about 105 instructions per ply on a lone wavefront), not by memory"},
+                        "note": "four workgroups of eight wavefronts: bound by the chain of draws that two of them make for 64 playouts "
+                                "and by the search for the games' ends in LDS, not by memory"},
            "cpu_baseline": cpu}
     e._release()
     print(json.dumps(out))
