@@ -61,9 +61,9 @@ extern "C" {
  * library launches one 64-lane wavefront per (tree, wid) and splits trees with more than 16 traversals over several
  * workgroups, so `warps` is not limited to 32.  As with any output array, nothing else on the device may read or write
  * edge_inflight while the launch runs, whatever the size of the trees; launches on one stream, or ordered by events, are
- * fine.  (With nodes * edges <= 8192 a launch relies on it: with 2 to 16 traversals per tree it keeps every tree's
- * edge_inflight in the LDS of the one workgroup that runs them, read at the start and written back at the end, and with one
- * traversal per tree the claims are ordinary stores.)
+ * fine.  (A launch relies on it: with 2 to 16 traversals per tree and nodes * edges <= 8192
+ * it keeps every tree's edge_inflight in the LDS of the one workgroup that runs them, read at the start and written back at
+ * the end, and with one traversal per tree the claims are ordinary stores.)
  */
 int puct_select_winner_recalc_launch(float cpuct, float c_pw, float alpha_pw, int soft_winner,
                                      const int *edge_child_id, const float *edge_prior, const float *edge_W,

@@ -45,15 +45,6 @@ struct SelectArgs {
     int *out_path_eids;
     int *out_path_len;
     int trees, nodes, edges, warps, path_depth;
-    // Optional per-node limit on the number of children, int32 [trees, nodes]; NULL = `edges` for every node, which is
-    // the reference's behaviour.  A caller whose nodes have fewer possible children than `edges` (legal moves) passes
-    // it so that progressive widening stops asking for slots a node cannot have.
-    const int *node_capacity = nullptr;
-    // Attempts of the winner-recalc claim per level; the reference has 2 compiled in.
-    int recalc_attempts = kRecalcAttempts;
-    // Optional work counters, uint64 [trees, 8]: entry 6 of a tree's row gains the tree levels its traversals read,
-    // entry 7 the expanded edges examined on those levels (what the algorithmic byte count of a selection is made of).
-    unsigned long long *work = nullptr;
 };
 
 // ---- cross-lane reductions -------------------------------------------------------------------------------------
@@ -116,15 +107,13 @@ __device__ __forceinline__ int pack_selection(int kind, int node, int slot, int 
            node;
 }
 
-// src/puct/puct_gpu_v3_cpp.cu:43-49
-__device__ __forceinline__ bool valid_select_shape(int path_depth, int nodes, int node_cnt, int edges) {
-    return path_depth >= 1 && nodes > 0 && node_cnt > 0 && node_cnt <= nodes && node_cnt <= PUCT_PACKED_NODE_LIMIT &&
-           edges > 0 && edges <= PUCT_PACKED_EDGE_MASK + 1;
-}
+// src/puct/puct_gpu_v3_cpp.cu:43-49, in two parts: what the launch says and what the tree does
+__device__ __forceinline__ bool valid_select_shape(int path_depth, int nodes, int edges) { return path_depth >= 1 && nodes > 0 && edges > 0 && edges <= PUCT_PACKED_EDGE_MASK + 1; }
+__device__ __forceinline__ bool valid_node_count(int node_cnt, int nodes) { return node_cnt > 0 && node_cnt <= nodes && node_cnt <= PUCT_PACKED_NODE_LIMIT; }
 
 // Progressive widening, src/puct/puct_gpu_v3_cpp.cu:150-157.
 __device__ __forceinline__ int allowed_children(float c_pw, float alpha_pw, int n_node, int edges, float sqrt_n_node) {
-    const float val = (alpha_pw == 0.5f) ? c_pw * sqrt_n_node : c_pw * powf((float)n_node, alpha_pw);
+    const float val = __builtin_expect(alpha_pw == 0.5f, 1) ? c_pw * sqrt_n_node : c_pw * powf((float)n_node, alpha_pw);
     if (val >= (float)edges) return edges;
     const int allowed = (int)ceilf(val);
     return allowed > 1 ? allowed : 1;
@@ -236,20 +225,33 @@ struct EdgeClaims {
     }
 };
 
-// The path entries of a traversal are stored by lane 0 of its wavefront and read back by all its lanes past the L1
-// (load_relaxed), so all a rollback needs before it reads them is that the stores have reached the L2 (and with them the
-// claims that its atomics take back, where those were stores too).  A device-scope fence
-// would write the L2 back: with 1024 trees of 8 traversals, most of which give way to another, 8192 of those were five
-// sixths of a launch (122 us, 4097 nodes of 64 edges a tree, paths of two levels).
+// The path of a traversal: lane l holds entry l of the 64 it is in the middle of, and they are stored together when they are
+// complete and when the traversal ends (a store by one lane at every level was as many instructions as four levels' tests for an end).
+// A traversal that gives way takes its claims back by them, and reads back only what it has stored before, past the L1: all it has to wait
+// for is that the stores have reached the L2 (and with them the claims that its atomics take back, where those were stores too).  A
+// device-scope fence would write the L2 back: with 1024 trees of 8 traversals, most of which give way to another, 8192 of those
+// were five sixths of a launch (122 us, 4097 nodes of 64 edges a tree, paths of two levels).
 __device__ __forceinline__ void wait_path_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+struct Path {
+    int *entries;
+    int mine = 0;   // entry lane + 64 i, where 64 i .. depth - 1 have not been stored yet
+    __device__ __forceinline__ void append(int depth, int encoded, int lane) {
+        mine = lane == (depth & (kWave - 1)) ? encoded : mine;
+        if ((depth & (kWave - 1)) == kWave - 1) entries[depth - (kWave - 1) + lane] = mine;
+    }
+    __device__ __forceinline__ void finish(int depth, int lane) const {
+        if (lane < (depth & (kWave - 1))) entries[(depth & ~(kWave - 1)) + lane] = mine;
+    }
+};
 
 // Takes back the virtual loss of the first `depth` path entries (src/puct/puct_gpu_v3_cpp.cu:206-217).
 template <ClaimsIn WHERE>
-__device__ __forceinline__ void rollback_path(const SelectArgs &a, const EdgeClaims<WHERE> &claims, const int *path, int tree, int depth, int lane,
-                                              int node_cnt) {
-    wait_path_stores();
+__device__ __forceinline__ void rollback_path(const SelectArgs &a, const EdgeClaims<WHERE> &claims, const Path &path, int depth, int lane, int node_cnt) {
+    const int stored = depth & ~(kWave - 1);
+    if (WHERE == ClaimsIn::OWN || stored > 0) wait_path_stores();
     for (int d = lane; d < depth; d += kWave) {
-        const int encoded = load_relaxed(path + d);
+        const int encoded = d < stored ? load_relaxed(path.entries + d) : path.mine;
         const int parent = encoded >> 8, slot = encoded & 0xFF;
         if (parent >= 0 && parent < node_cnt && slot < a.edges)
             claims.add(((uint32_t)parent * (uint32_t)a.edges + (uint32_t)slot) * 4u, -1);
@@ -263,60 +265,59 @@ __device__ __forceinline__ void rollback_path(const SelectArgs &a, const EdgeCla
 template <ClaimsIn WHERE>
 __device__ __forceinline__ void select_traversal(const SelectArgs &a, const EdgeClaims<WHERE> &claims, int tree, int wid, int lane) {
     static_assert(kPasses == 4, "the levels below are written for one to four slices");
-    const size_t out = (size_t)tree * a.warps + wid;
-    int *path = a.out_path_eids + out * a.path_depth;
-    const int node_cnt = a.tree_nodes[tree];
+    const size_t out = (uint64_t)(uint32_t)tree * (uint32_t)a.warps + (uint32_t)wid;
+    int *const entries = a.out_path_eids + out * (uint32_t)a.path_depth;
     const int nodes = a.nodes, edges = a.edges;
-
-    int final_packed = pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_UNKNOWN);
+    int final_packed = pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_SHAPE);
     int final_len = 0;
-    int levels = 0, edges_seen = 0;
 
-    if (!valid_select_shape(a.path_depth, nodes, node_cnt, edges)) {
-        final_packed = pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_SHAPE);
-    } else {
-        const size_t tree_edges = (size_t)tree * nodes * edges;
-        const int *const tree_n = a.edge_N + tree_edges, *const tree_c = a.edge_child_id + tree_edges;
+    if (valid_select_shape(a.path_depth, nodes, edges)) {
+        const size_t tree_nodes = (uint64_t)(uint32_t)tree * (uint32_t)nodes, tree_edges = tree_nodes * (uint32_t)edges;
+        const int *const tree_n = a.edge_N + tree_edges, *const tree_c = a.edge_child_id + tree_edges, *const tree_expanded = a.node_expanded + tree_nodes;
         const float *const tree_p = a.edge_prior + tree_edges, *const tree_w = a.edge_W + tree_edges;
-        int node = 0, depth = 0;
+        int *const tree_tickets = a.node_expand_inflight + tree_nodes;
+        const int asked_node_cnt = load_relaxed(a.tree_nodes + tree);
+        int node = 0, depth = 0, node_cnt = 0;
+        Path path{entries};
         while (true) {
             // (the same in all lanes; said so that the level's addresses and branches are worked out once per wavefront)
             node = __builtin_amdgcn_readfirstlane(node), depth = __builtin_amdgcn_readfirstlane(depth);
-            levels += 1;
-            const size_t nrow = (size_t)tree * nodes + node;
-            const uint32_t row4 = (uint32_t)node * (uint32_t)edges * 4u;   // byte offset of the node's edges in the tree's fields
+            const uint32_t node4 = (uint32_t)node * 4u, row4 = node4 * (uint32_t)edges;   // byte offsets of the node, and of its edges, in the tree's fields
 
             // Everything a level can need from the first 64 edges, requested in one go, before the node's width is known
             // (lanes beyond the row read its last edge and take no part); the edges of wider nodes follow once it is
-            // and stay in registers for the rest of the level.
+            // and stay in registers for the rest of the level.  (Requested at the end of the level before, which moves the claims
+            // apart from the rest: deep trees a quarter slower.)
             const uint32_t at0 = row4 + (uint32_t)(lane < edges ? lane : edges - 1) * 4u;
             const int n0 = *at_bytes(tree_n, at0), f0 = claims.peek(at0), c0 = *at_bytes(tree_c, at0);
             const float p0 = *at_bytes(tree_p, at0), w0 = *at_bytes(tree_w, at0);
-            const int node_info = a.node_expanded[nrow];
-            const int expand_inflight = load_relaxed(a.node_expand_inflight + nrow);
-            const int capacity = a.node_capacity ? a.node_capacity[nrow] : edges;
+            const int node_info = *at_bytes(tree_expanded, node4);
+            const int tickets = load_relaxed(at_bytes(tree_tickets, node4));
 
+            // Where the traversal goes on, or the complement of its selection word where it ends.
+            int next;
+            if (depth == 0) {   // (how many nodes the tree has is not waited for before the root's row is on its way)
+                int count = asked_node_cnt;
+                asm volatile("" : "+v"(count));
+                node_cnt = __builtin_amdgcn_readfirstlane(count);
+                if (!valid_node_count(node_cnt, nodes)) break;
+            }
             if (node_info == PUCT_NODE_EXPANDED_TERMINAL) {
                 final_packed = pack_selection(PUCT_SELECT_TERMINAL, node, 0, PUCT_REASON_OK_TERMINAL);
-                final_len = depth + 1;
                 break;
             }
             if (node_info < 0 || node_info > edges) {
-                rollback_path(a, claims, path, tree, depth, lane, node_cnt);
-                final_packed =
-                    pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_NODE_INFO);
+                final_packed = pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_NODE_INFO);
                 break;
             }
             if (depth >= a.path_depth) {
                 final_packed = pack_selection(PUCT_SELECT_DEPTH_LIMIT, node, 0, PUCT_REASON_OK_DEPTH_LIMIT);
-                final_len = depth + 1;
                 break;
             }
 
             const int cur_expanded = node_info;
-            edges_seen += cur_expanded;
 
-            // The level proper; returns the child the traversal moves on to, or -1 when it ends here.
+            // The level proper.
             auto level = [&](auto slices) __attribute__((always_inline)) -> int {
                 constexpr int S = decltype(slices)::value;   // (S - 1) * 64 < cur_expanded <= S * 64, or no edge at all (S = 1)
                 constexpr int CS = S <= 2 ? S : 1;   // slices whose row of children is requested with the scores' fields (see best_child below)
@@ -340,42 +341,36 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
 
                 int parent_eff = 1, allowed = 1;
                 float sqrt_parent = 1.0f;
-                if (cur_expanded != 1 || a.c_pw != 0.0f) {
+                if (S == 1 && cur_expanded == 0) {   // no visits: 1 ** alpha_pw is 1, whatever alpha_pw is
+                    allowed = allowed_children(a.c_pw, 0.5f, 1, edges, 1.0f);
+                } else if (cur_expanded != 1 || a.c_pw != 0.0f) {
                     int total = 0;
 #pragma unroll
                     for (int i = 0; i < S; ++i) total += in_node[i] ? n[i] + f[i] : 0;
                     total = wave_sum(total);
                     parent_eff = total > 1 ? total : 1;
                     sqrt_parent = sqrtf((float)parent_eff);
-                    allowed = allowed_children(a.c_pw, a.alpha_pw, parent_eff, capacity, sqrt_parent);
+                    allowed = allowed_children(a.c_pw, a.alpha_pw, parent_eff, edges, sqrt_parent);
                 }
 
                 if (allowed > cur_expanded) {
                     // Expansion ticket, src/puct/puct_gpu_v3_cpp.cu:219-233.
                     int expand_slot = -1;
-                    if (cur_expanded + expand_inflight < allowed) {
+                    if (cur_expanded + tickets < allowed) {
                         if (lane == 0) {
-                            const int slot = cur_expanded + atomicAdd(&a.node_expand_inflight[nrow], 1);
+                            const int slot = cur_expanded + atomicAdd(at_bytes(tree_tickets, node4), 1);
                             if (slot < allowed)
                                 expand_slot = slot;
                             else
-                                atomicSub(&a.node_expand_inflight[nrow], 1);
+                                atomicSub(at_bytes(tree_tickets, node4), 1);
                         }
                         expand_slot = __builtin_amdgcn_readfirstlane(expand_slot);
                     }
-                    if (expand_slot >= 0) {
-                        final_packed = pack_selection(PUCT_SELECT_EXPAND, node, expand_slot, PUCT_REASON_OK_EXPAND);
-                        final_len = depth + 1;
-                        return -1;
-                    }
-                    if (cur_expanded == 0) {
-                        rollback_path(a, claims, path, tree, depth, lane, node_cnt);
-                        final_packed = pack_selection(PUCT_SELECT_BUSY, node, 0, PUCT_REASON_BUSY_EXPAND_INFLIGHT);
-                        return -1;
-                    }
+                    if (expand_slot >= 0) return ~pack_selection(PUCT_SELECT_EXPAND, node, expand_slot, PUCT_REASON_OK_EXPAND);
+                    if (cur_expanded == 0) return ~pack_selection(PUCT_SELECT_BUSY, node, 0, PUCT_REASON_BUSY_EXPAND_INFLIGHT);
                 }
 
-                int tie_offset = wid;
+                int tie_offset = WHERE == ClaimsIn::OWN ? 0 : wid;
                 if (tie_offset >= cur_expanded) tie_offset %= cur_expanded;
 
                 auto of_edge = [&](const int (&v)[S], int eid) {
@@ -404,9 +399,9 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                     float q[S], num[S];
 #pragma unroll
                     for (int i = 0; i < S; ++i) {
-                        // (a slice none of whose edges has a visit or a value has q = +0 without dividing)
+                        // (of a node of several slices, one none of whose edges has a visit or a value has q = +0 without dividing)
                         q[i] = 0.0f;
-                        if (__builtin_amdgcn_ballot_w64(n[i] > 0 && __float_as_uint(w[i]) != 0u) != 0) q[i] = n[i] > 0 ? w[i] / (float)n[i] : 0.0f;
+                        if (S == 1 || __builtin_amdgcn_ballot_w64(n[i] > 0 && __float_as_uint(w[i]) != 0u) != 0) q[i] = n[i] > 0 ? w[i] / (float)n[i] : 0.0f;
                         num[i] = a.cpuct * p[i] * sqrt_parent;
                     }
                     uint32_t keys[S];
@@ -414,7 +409,7 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                         return in_node[i] ? score_key(q[i] + num[i] / (float)(n[i] + inflight + 1)) : 0u;
                     };
                     best_eid = kNoEdge;
-                    for (int attempt = 0; attempt < a.recalc_attempts; ++attempt) {
+                    for (int attempt = 0; attempt < kRecalcAttempts; ++attempt) {
                         if (attempt == 0) {
 #pragma unroll
                             for (int i = 0; i < S; ++i) keys[i] = score_slice(i, f[i]);
@@ -455,51 +450,45 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                     }
                 }
 
-                if (held == 0) {
-                    rollback_path(a, claims, path, tree, depth, lane, node_cnt);
-                    final_packed =
-                        best_eid == kNoEdge
-                            ? pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_NO_VALID_EDGE)
-                            : pack_selection(PUCT_SELECT_BUSY, node, 0, PUCT_REASON_BUSY_WINNER_RECALC);
-                    return -1;
-                }
+                if (held == 0)
+                    return best_eid == kNoEdge ? ~pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_NO_VALID_EDGE)
+                                               : ~pack_selection(PUCT_SELECT_BUSY, node, 0, PUCT_REASON_BUSY_WINNER_RECALC);
 
                 best_child = __builtin_amdgcn_readfirstlane(best_child);
                 if (best_child < 0 || best_child >= node_cnt) {
                     if (WHERE != ClaimsIn::OWN && lane == 0) claims.add(row4 + (uint32_t)best_eid * 4u, -1);
-                    rollback_path(a, claims, path, tree, depth, lane, node_cnt);
-                    final_packed =
-                        pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_CHILD_OOB);
-                    return -1;
+                    return ~pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_CHILD_OOB);
                 }
                 if (WHERE == ClaimsIn::OWN) {   // (the claim, now that the edge is known to lead somewhere)
 #pragma unroll
                     for (int i = 0; i < S; ++i)
                         if (lane + i * kWave == best_eid) claims.set(row4 + (uint32_t)best_eid * 4u, f[i] + 1);
                 }
-                if (lane == 0) path[depth] = (node << 8) | best_eid;
+                path.append(depth, (node << 8) | best_eid, lane);
                 return best_child;
             };
 
             const int slices = (cur_expanded + kWave - 1) / kWave;
-            int next;
             if (slices <= 1) next = level(std::integral_constant<int, 1>{});
             else if (slices == 2) next = level(std::integral_constant<int, 2>{});
             else if (slices == 3) next = level(std::integral_constant<int, 3>{});
             else next = level(std::integral_constant<int, 4>{});
-            if (next < 0) break;
+            if (next < 0) {
+                final_packed = ~next;
+                break;
+            }
             node = next;
             depth += 1;
         }
+        const int kind = (final_packed >> PUCT_PACKED_KIND_SHIFT) & PUCT_PACKED_KIND_MASK;
+        if (kind == PUCT_SELECT_INVALID || kind == PUCT_SELECT_BUSY) rollback_path(a, claims, path, depth, lane, node_cnt);
+        else final_len = depth + 1;
+        path.finish(depth, lane);
     }
 
     if (lane == 0) {
         a.out_selected_node[out] = final_packed;
         a.out_path_len[out] = final_len;
-        if (a.work != nullptr) {
-            atomicAdd(&a.work[(size_t)tree * 8 + 6], (unsigned long long)levels);
-            atomicAdd(&a.work[(size_t)tree * 8 + 7], (unsigned long long)edges_seen);
-        }
     }
 }
 

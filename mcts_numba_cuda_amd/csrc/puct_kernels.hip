@@ -4,24 +4,56 @@
 namespace {
 using namespace puct;
 
+inline __host__ __device__ int traversals_of_block(int warps) { return warps < kMaxWavesPerBlock ? warps : kMaxWavesPerBlock; }
+
+// Has a launch's arguments read at once: the compiler asks for them where they are used, three waits one after the other (16 trees of
+// 257 x 64 edges, 8 traversals, a selection and its backup: 9.7 us, 8.8 with this and with the traversal's own scalar work below).
+__device__ __forceinline__ void fetch_arguments(const SelectArgs &a) {
+    asm volatile("" ::"s"(a.edge_child_id), "s"(a.edge_prior), "s"(a.edge_W), "s"(a.edge_N), "s"(a.edge_inflight), "s"(a.node_expand_inflight), "s"(a.node_expanded),
+                 "s"(a.tree_nodes), "s"(a.out_selected_node), "s"(a.out_path_eids), "s"(a.out_path_len), "s"(a.nodes), "s"(a.edges), "s"(a.warps), "s"(a.path_depth),
+                 "s"(a.cpuct), "s"(a.c_pw), "s"(a.alpha_pw), "s"(a.soft_winner));
+}
+__device__ __forceinline__ void fetch_arguments(const BackupArgs &a) {
+    asm volatile("" ::"s"(a.edge_child_id), "s"(a.edge_W), "s"(a.edge_N), "s"(a.edge_inflight), "s"(a.node_inflight), "s"(a.node_expand_inflight), "s"(a.node_count),
+                 "s"(a.out_selected_node), "s"(a.out_path_eids), "s"(a.out_path_len), "s"(a.path_edge_values), "s"(a.virtual_loss), "s"(a.nodes), "s"(a.edges), "s"(a.warps),
+                 "s"(a.path_depth));
+}
+
+// `words` words by the whole workgroup, eight reads of a lane in flight where there are as many.
+__device__ __forceinline__ void copy_words(int *to, const int *from, int words) {
+    constexpr int kBatch = 8;
+    const int threads = blockDim.x;
+    int i = threadIdx.x;
+    for (; i + (kBatch - 1) * threads < words; i += kBatch * threads) {
+        int v[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) v[k] = from[i + k * threads];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) to[i + k * threads] = v[k];
+    }
+#pragma unroll 1
+    for (; i < words; i += threads) to[i] = from[i];
+}
+
 // LDS: the tree's traversals are this workgroup's wavefronts (grid.y == 1) and the claims on its edges are kept in
 // the workgroup's dynamic LDS for the launch (a.nodes * a.edges words).  OWN: the tree has one traversal.
 template <ClaimsIn WHERE>
 __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) __attribute__((amdgpu_waves_per_eu(8, 8))) void select_kernel(const SelectArgs a) {
+    fetch_arguments(a);
     extern __shared__ int tree_claims[];
-    const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave);   // the same in all lanes
+    const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * traversals_of_block(a.warps) + threadIdx.x / kWave);   // the same in all lanes
     constexpr bool LOCAL = WHERE == ClaimsIn::LDS;
     const int words = a.nodes * a.edges;
-    int *const in_memory = a.edge_inflight + (size_t)blockIdx.x * a.nodes * a.edges;
+    int *const in_memory = a.edge_inflight + (uint64_t)blockIdx.x * (uint32_t)a.nodes * (uint32_t)a.edges;
     const EdgeClaims<WHERE> claims{in_memory, (LdsInts)tree_claims};
     if (LOCAL) {
-        for (int i = threadIdx.x; i < words; i += blockDim.x) tree_claims[i] = in_memory[i];
+        copy_words(tree_claims, in_memory, words);
         __syncthreads();
     }
     if (LOCAL || wid < a.warps) select_traversal<WHERE>(a, claims, blockIdx.x, wid, threadIdx.x & (kWave - 1));
     if (LOCAL) {
         __syncthreads();
-        for (int i = threadIdx.x; i < words; i += blockDim.x) in_memory[i] = tree_claims[i];
+        copy_words(in_memory, tree_claims, words);
     }
 }
 
@@ -46,7 +78,8 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) __attribute__((amdgpu_wav
 
 template <bool NODE_LEVEL>
 __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void backup_kernel(const BackupArgs a) {
-    const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave);   // the same in all lanes
+    fetch_arguments(a);
+    const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * traversals_of_block(a.warps) + threadIdx.x / kWave);   // the same in all lanes
     if (wid >= a.warps) return;
     backup_traversal<NODE_LEVEL>(a, blockIdx.x, wid, threadIdx.x & (kWave - 1));
 }
@@ -75,15 +108,15 @@ extern "C" int puct_select_winner_recalc_launch(float cpuct, float c_pw, float a
                  trees,        nodes,         edges,           warps,                path_depth};
     dim3 grid, block;
     launch_shape(trees, warps, grid, block);
-    // The claims of a tree in LDS: up to 8192 edge slots, so that a CU still holds four workgroups.  A single traversal needs
-    // none of it: its claims are plain stores, which at the sizes of this rule beat both other forms at every width (plain
-    // stores / atomics / LDS, ms a launch of 512 levels: 16384 trees of 65 x 64 edges 2.33 / 2.91 / 6.11, of 128 x 64 2.35 /
-    // 2.92 / 11.9; 8192 trees of 64 x 128 1.98 / 2.05 / 8.06; 4096 trees of 32 x 256 1.96 / 1.97 / 5.28).  Larger trees go
-    // by atomics, with one traversal too: there it depends on the width which is ahead (plain stores / atomics: 16384 trees of
-    // 129 x 64 2.27 / 2.91; with 1024 levels 8192 trees of 129 x 128 4.47 / 4.57, 4096 trees of 257 x 256 4.67 / 4.58).
+    // A single traversal's claims are plain stores, whatever the size of the tree (plain stores / atomics, us a selection and its backup:
+    // 512 trees of 4097 x 64, two levels, 8.9 / 10.4; 64 trees of 1500 x 200 8.6 / 9.5; 512 levels, 16384 trees of 129 x 64 2630 / 3047,
+    // 2048 trees of 257 x 256 1790 / 1990).  The claims of a tree with more of them in LDS: up to 8192 edge slots, so that a CU still holds
+    // four workgroups.  (In rows of LDS given to the nodes as they are visited, trees of any size: no faster.  16 trees of 257 x 64
+    // with 8 traversals 9.9 against 9.5, 1024 of 4097 x 64 18.9 against 17.1: what the claims gain, clearing the rows and adding
+    // them up afterwards costs.)  Larger trees go by atomics.
     const long long slots = (long long)nodes * edges;
     const bool small = grid.y == 1 && slots > 0 && slots <= kLocalClaimSlots;
-    if (small && warps == 1)
+    if (warps == 1)
         hipLaunchKernelGGL(select_kernel<ClaimsIn::OWN>, grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);
     else if (small)
         hipLaunchKernelGGL(select_kernel<ClaimsIn::LDS>, grid, block, sizeof(int) * (size_t)slots, reinterpret_cast<hipStream_t>(stream), a);
