@@ -823,14 +823,14 @@ struct BackupArgs {
 // selection word has no reason field).  NODE_LEVEL = false: the same conversion of virtual visits into real ones for
 // the edge-level virtual loss of select_kernel; BUSY selections hold nothing and are skipped, as in
 // src/puct/test_puct_gpu_v3.py:297-302.
-template <bool NODE_LEVEL>
-__device__ __forceinline__ void backup_traversal(const BackupArgs &a, int tree, int wid, int lane) {
+template <bool NODE_LEVEL, bool COUNTED = false>
+__device__ __forceinline__ void backup_traversal(const BackupArgs &a, LdsInts counted, int tree, int wid, int lane) {
     // All that a path of up to 64 levels needs is requested at once: a launch of few traversals is as long as its chain of loads,
     // which was four long, each asked for when the one before was known to matter (16 trees x 8 traversals 3.5 -> 2.7 us, 1024 x 8
     // 4.1 -> 3.8).
-    const size_t out = (size_t)tree * a.warps + wid;
-    const int *const path = a.out_path_eids + out * a.path_depth;
-    const float *const values = a.path_edge_values == nullptr ? nullptr : a.path_edge_values + out * a.path_depth;
+    const size_t out = (uint64_t)(uint32_t)tree * (uint32_t)a.warps + (uint32_t)wid, first = out * (uint32_t)a.path_depth;
+    const int *const path = a.out_path_eids + first;
+    const float *const values = a.path_edge_values == nullptr ? nullptr : a.path_edge_values + first;
     const int node_limit = a.node_count[tree], raw = a.out_selected_node[out], plen = a.out_path_len[out];
     int encoded = lane < a.path_depth ? path[lane] : -1;
     float value = values != nullptr && lane < a.path_depth ? values[lane] : 0.0f;
@@ -855,7 +855,9 @@ __device__ __forceinline__ void backup_traversal(const BackupArgs &a, int tree, 
         const int parent = here >> 8, slot = here & 0xFF;
         if (parent >= node_limit || slot >= a.edges) continue;
         const size_t e = ((size_t)tree * a.nodes + parent) * a.edges + slot;
-        if (NODE_LEVEL) {
+        if (COUNTED) {
+            __hip_atomic_fetch_add(counted + (parent * a.edges + slot), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        } else if (NODE_LEVEL) {
             const int child = a.edge_child_id[e];
             if (child >= 0 && child < node_limit)
                 atomicSub(&a.node_inflight[(size_t)tree * a.nodes + child], a.virtual_loss);
@@ -863,7 +865,7 @@ __device__ __forceinline__ void backup_traversal(const BackupArgs &a, int tree, 
             atomicSub(&a.edge_inflight[e], a.virtual_loss);
         }
         if (values != nullptr) {
-            atomicAdd(&a.edge_N[e], 1);
+            if (!COUNTED) atomicAdd(&a.edge_N[e], 1);
             unsafeAtomicAdd(&a.edge_W[e], v);
         }
     }

@@ -81,7 +81,45 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void backup_kernel(const 
     fetch_arguments(a);
     const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * traversals_of_block(a.warps) + threadIdx.x / kWave);   // the same in all lanes
     if (wid >= a.warps) return;
-    backup_traversal<NODE_LEVEL>(a, blockIdx.x, wid, threadIdx.x & (kWave - 1));
+    backup_traversal<NODE_LEVEL>(a, nullptr, blockIdx.x, wid, threadIdx.x & (kWave - 1));
+}
+
+// The backup of small trees with long paths, whose traversals are wavefronts of this workgroup (grid.y == 1): how often each edge is passed
+// is counted in LDS (a.nodes * a.edges words, and at node level a.nodes more), and the edges that were passed, and the nodes that they
+// lead to, are then updated in one sweep, an atomic each and lanes side by side, instead of one a level wherever the path leads.  (Values
+// are added one by one, in the order in which they come, as before.)  Bound by the lines that the sweep updates: 16384 trees of 65 x 64
+// edges with one path of 512 levels, some 0.55 GB in 86 us, where 8.4 M scattered atomics took 324.  Loads and stores in the sweep
+// instead of atomics: 100 us, with values 463 instead of 580, but then two launches on the same trees would no longer add up.
+template <bool NODE_LEVEL>
+__global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void counted_backup_kernel(const BackupArgs a) {
+    fetch_arguments(a);
+    extern __shared__ int times_passed[];
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), words = a.nodes * a.edges, threads = blockDim.x;
+    int *const times_reached = times_passed + words;
+    const int node_limit = a.node_count[blockIdx.x];
+    for (int i = threadIdx.x; i < words + (NODE_LEVEL ? a.nodes : 0); i += threads) times_passed[i] = 0;
+    __syncthreads();
+    if (wid < a.warps) backup_traversal<NODE_LEVEL, true>(a, (LdsInts)times_passed, blockIdx.x, wid, threadIdx.x & (kWave - 1));
+    __syncthreads();
+    const uint64_t first_node = (uint64_t)blockIdx.x * (uint32_t)a.nodes, first = first_node * (uint32_t)a.edges;
+    for (int i = threadIdx.x; i < words; i += threads) {
+        const int passed = times_passed[i];
+        if (passed == 0) continue;
+        if (!NODE_LEVEL) {
+            atomicAdd(&a.edge_inflight[first + i], (int)(0u - (uint32_t)passed * (uint32_t)a.virtual_loss));
+        } else {
+            const int child = a.edge_child_id[first + i];
+            if (child >= 0 && child < node_limit) __hip_atomic_fetch_add((LdsInts)times_reached + child, passed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        if (a.path_edge_values != nullptr) atomicAdd(&a.edge_N[first + i], passed);
+    }
+    if (NODE_LEVEL) {
+        __syncthreads();
+        for (int c = threadIdx.x; c < a.nodes; c += threads) {
+            const int reached = times_reached[c];
+            if (reached != 0) atomicAdd(&a.node_inflight[first_node + c], (int)(0u - (uint32_t)reached * (uint32_t)a.virtual_loss));
+        }
+    }
 }
 
 constexpr int kLocalVisitNodes = 16384;   // (what a selection word can name; 64 KB of LDS, two workgroups per CU: still ahead of counters in memory)
@@ -168,6 +206,30 @@ extern "C" int puct_node_select_winner_recalc_launch(float cpuct, float c_pw, fl
                                      out_path_len, trees, nodes, edges, warps, path_depth, stream);
 }
 
+namespace {
+template <bool NODE_LEVEL>
+int launch_backup(const BackupArgs &a, hipStream_t stream) {
+    dim3 grid, block;
+    launch_shape(a.trees, a.warps, grid, block);
+    // Counted in LDS where paths can only be that long by coming back to nodes, so that they pass a good part of a small tree's edges, and
+    // where there are many of them.  Atomics on scattered words go at 25 G a second, whatever the occupancy, one for a release and
+    // three with values.  us, atomics / counted, release and with values: 16384 trees of 65 x 64, paths of 512 324 / 86 and 1043 / 580, of
+    // 128 81 / 50 and 255 / 187; of 91 x 90 (512 threads) 316 / 131 and 1038 / 649; of 21 x 20, paths of 64, 39 / 18 and 122 / 71; 2048
+    // trees of 65 x 64 with 8 traversals of up to 512 98 / 15 and 309 / 144.  Few trees, which take a few us: 64 of 65 x 64 with one path
+    // of 128 4.3 / 6.4, with 8 traversals 4.6 / 5.1.  (Threads, us a release of 16384 x 512 by loads and stores with 64 / 128 / 256 / 512:
+    // 65 x 64 179 / 124 / 98 / 116, 91 x 90 627 / 415 / 291 / 213.)
+    const long long slots = (long long)a.nodes * a.edges, walked = (long long)a.warps * a.path_depth;
+    if (grid.y == 1 && slots > 0 && slots <= kLocalClaimSlots && a.path_depth >= a.nodes && walked * 40 >= slots && a.trees * walked >= 1 << 19) {
+        const unsigned threads = slots <= 4608 ? 256 : 512;
+        hipLaunchKernelGGL(counted_backup_kernel<NODE_LEVEL>, grid, dim3(block.x < threads ? threads : block.x),
+                           sizeof(int) * (size_t)(slots + (NODE_LEVEL ? a.nodes : 0)), stream, a);
+    } else {
+        hipLaunchKernelGGL(backup_kernel<NODE_LEVEL>, grid, block, 0, stream, a);
+    }
+    return static_cast<int>(hipGetLastError());
+}
+}  // namespace
+
 extern "C" const char *puct_cpp_cuda_error_string(int code) { return hipGetErrorString(static_cast<hipError_t>(code)); }
 
 extern "C" int puct_edge_backup_launch(int virtual_loss, float *edge_W, int *edge_N, int *edge_inflight,
@@ -177,10 +239,7 @@ extern "C" int puct_edge_backup_launch(int virtual_loss, float *edge_W, int *edg
     BackupArgs a{virtual_loss, nullptr,    edge_W,           edge_N,        edge_inflight, nullptr,
                  node_expand_inflight, node_count, out_selected_node, out_path_eids, out_path_len, path_edge_values,
                  trees,        nodes,      edges,            warps,         path_depth};
-    dim3 grid, block;
-    launch_shape(trees, warps, grid, block);
-    hipLaunchKernelGGL(backup_kernel<false>, grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);
-    return static_cast<int>(hipGetLastError());
+    return launch_backup<false>(a, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int puct_node_backup_launch(int virtual_loss, const int *edge_child_id, float *edge_W, int *edge_N,
@@ -191,8 +250,5 @@ extern "C" int puct_node_backup_launch(int virtual_loss, const int *edge_child_i
     BackupArgs a{virtual_loss, edge_child_id, edge_W,        edge_N,        nullptr,       node_inflight,
                  node_expand_inflight, node_count, out_selected_node, out_path_eids, out_path_len, path_edge_values,
                  trees,        nodes,         edges,         warps,         path_depth};
-    dim3 grid, block;
-    launch_shape(trees, warps, grid, block);
-    hipLaunchKernelGGL(backup_kernel<true>, grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);
-    return static_cast<int>(hipGetLastError());
+    return launch_backup<true>(a, reinterpret_cast<hipStream_t>(stream));
 }

@@ -127,6 +127,48 @@ def test_single_traversals_of_recurrent_trees_match_oracle_exactly(actions, node
     assert given_back > 0 and (again > 0 or c_pw > 0)   # (with widening the paths are short)
 
 
+@pytest.mark.parametrize("trees,actions,nodes,depth,warps,counted", [
+    (4096, 9, 10, 128, 1, True), (1030, 64, 65, 512, 1, True), (1024, 90, 91, 130, 8, True), (4096, 20, 21, 70, 3, True), (600, 33, 34, 130, 16, True),
+    (16, 64, 65, 300, 4, False), (4095, 9, 10, 128, 1, False), (8, 90, 92, 200, 16, False)])
+def test_backup_of_long_paths_matches_oracle(trees, actions, nodes, depth, warps, counted):
+    """Paths that come back to the nodes of a small tree, longer than a wavefront, by one to sixteen traversals; those that give way or end
+    nowhere hold nothing.  On either side of where the backup counts in LDS what was passed (`counted`).  Values are multiples of 1/64
+    small enough for their sums to be exact, so that every order of adding them gives the same."""
+    from mcts_numba_cuda_amd import puct
+    from mcts_numba_cuda_amd.hipmem import DeviceArray
+    assert counted == (nodes * actions <= 8192 and depth >= nodes and 40 * warps * depth >= nodes * actions and trees * warps * depth >= 1 << 19)
+    rng = np.random.default_rng(trees + actions * 1000 + warps)
+    case = pc.recurrent_forest(rng, trees=trees, nodes=nodes, actions=actions, path_depth=depth, claims=0.1, dead_ends=0.5 / depth)
+    case["out_selected"], case["out_len"] = np.zeros((trees, warps), np.int32), np.zeros((trees, warps), np.int32)
+    case["out_path"] = np.full((trees, warps, depth), -1, np.int32)
+    r = HipRunner()
+    for rnd, with_values in enumerate((True, False)):
+        before = int((case if rnd == 0 else h)["edge_inflight"].sum())
+        h = r.select(case if rnd == 0 else h, cpuct=1.5, c_pw=0.0, soft_winner=rnd)
+        kinds = (h["out_selected"] >> 22) & 7
+        holding = (kinds == pc.EXPAND) | (kinds == pc.TERMINAL_KIND) | (kinds == pc.DEPTH_LIMIT)
+        assert holding.any() and np.all(h["out_len"][~holding] == 0) and h["out_len"].max() > 65
+        assert int(h["edge_inflight"].sum()) - before == int((h["out_len"][holding] - 1).sum())   # (what gave way has taken all of it back)
+        values = (np.floor(rng.uniform(-64, 64, h["out_path"].shape)) / 64).astype(np.float32) if with_values else None
+        got = r.backup(values)
+        at_nodes = copy.deepcopy(h)
+        po.backup(h, values)
+        for k in h:
+            assert np.array_equal(got[k], h[k], equal_nan=True), (rnd, k)
+        # the same paths, as selections with node-level virtual loss report them
+        del at_nodes["edge_inflight"]
+        at_nodes["node_inflight"] = rng.integers(0, 1000, (trees, nodes)).astype(np.int32)
+        at_nodes["out_selected"] = np.where(holding, at_nodes["out_selected"] & ((1 << 25) - 1), 0x3FFF).astype(np.int32)
+        d = to_device(at_nodes)
+        values = (np.floor(rng.uniform(-64, 64, h["out_path"].shape)) / 64).astype(np.float32)
+        puct.launch_node_backup(d, DeviceArray(values))
+        synchronize()
+        got = to_host(d)
+        po.backup(at_nodes, values, node_level=True)
+        for k in at_nodes:
+            assert np.array_equal(got[k], at_nodes[k], equal_nan=True), (rnd, k)
+
+
 @pytest.mark.parametrize("trees,warps,soft", [(16, 8, 0), (16, 16, 0), (4, 40, 0), (16, 16, 1), (128, 4, 0)])
 def test_concurrent_traversals_keep_invariants(trees, warps, soft):
     rng = np.random.default_rng(trees * 100 + warps)
