@@ -546,11 +546,12 @@ struct NodeVisits {
 
 // src/puct/puct_gpu_v2.py:291-310: the claims of the first `depth` path entries live on the child each entry leads to.
 template <bool LOCAL>
-__device__ __forceinline__ void rollback_node_path(const NodeSelectArgs &a, const NodeVisits<LOCAL> &visits_of, const int *path, int tree, int depth, int lane,
+__device__ __forceinline__ void rollback_node_path(const NodeSelectArgs &a, const NodeVisits<LOCAL> &visits_of, const Path &path, int tree, int depth, int lane,
                                                    int node_limit) {
-    wait_path_stores();
+    const int stored = depth & ~(kWave - 1);
+    if (stored > 0) wait_path_stores();
     for (int d = lane; d < depth; d += kWave) {
-        const int encoded = load_relaxed(path + d);
+        const int encoded = d < stored ? load_relaxed(path.entries + d) : path.mine;
         if (encoded < 0) continue;
         const int parent = encoded >> 8, slot = encoded & 0xFF;
         if (parent < node_limit && slot < a.edges) {
@@ -572,56 +573,52 @@ __device__ __forceinline__ void rollback_node_path(const NodeSelectArgs &a, cons
 // number S of 64-edge slices that the node's expanded edges fill (1..4, the same for all lanes): what bounds these
 // kernels is the wavefronts' instruction issue, vector and scalar together, and a level written for "up to four slices"
 // spends a third of it on finding out, slice by slice, that a slice is not there.
-template <bool PRECLAIM, bool LOCAL>
-__device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, const NodeVisits<LOCAL> &visits_of, int tree, int wid, int lane) {
+// before_claims is called once, before the counters are looked at, where the launch has a valid shape.
+template <bool PRECLAIM, bool LOCAL, class BeforeClaims>
+__device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, const NodeVisits<LOCAL> &visits_of, int tree, int wid, int lane, BeforeClaims before_claims) {
     static_assert(kPasses == 4, "the levels below are written for one to four slices");
-    const size_t out = (size_t)tree * a.warps + wid;
-    int *path = a.out_path_eids + out * a.path_depth;
-    const int node_limit = a.node_count[tree];
+    const size_t out = (uint64_t)(uint32_t)tree * (uint32_t)a.warps + (uint32_t)wid;
+    int *const entries = a.out_path_eids + out * (uint32_t)a.path_depth;
     const int nodes = a.nodes, edges = a.edges;
-    const size_t trow = (size_t)tree * nodes;
 
     int final_packed = kPackedInvalidV2, final_len = 0;
-    // src/puct/puct_gpu_v2.py:357-366
-    if (a.path_depth >= 1 && nodes > 0 && node_limit > 0 && node_limit <= nodes && node_limit <= PUCT_PACKED_NODE_LIMIT &&
-        edges > 0 && edges <= PUCT_PACKED_EDGE_MASK + 1) {
-        const size_t tree_edges = trow * edges;
-        const int *const tree_c = a.edge_child_id + tree_edges, *const tree_n = a.edge_N + tree_edges;
+    if (valid_select_shape(a.path_depth, nodes, edges)) {   // src/puct/puct_gpu_v2.py:357-366
+        const size_t tree_nodes = (uint64_t)(uint32_t)tree * (uint32_t)nodes, tree_edges = tree_nodes * (uint32_t)edges;
+        const int *const tree_c = a.edge_child_id + tree_edges, *const tree_n = a.edge_N + tree_edges, *const tree_expanded = a.node_expanded + tree_nodes;
         const float *const tree_p = a.edge_prior + tree_edges, *const tree_w = a.edge_W + tree_edges;
+        int *const tree_tickets = a.node_expand_inflight + tree_nodes;
+        // the first 64 edges are requested together with the node's own words, before the node's width is known (lanes beyond the row
+        // read its last edge and take no part), when the level before has chosen the node
+        struct Row { int n, c, info, tickets; float p, w; };
+        const uint32_t lane4 = (uint32_t)(lane < edges ? lane : edges - 1) * 4u;
+        auto request = [=](int node) __attribute__((always_inline)) -> Row {
+            const uint32_t node4 = (uint32_t)node * 4u, at0 = node4 * (uint32_t)edges + lane4;
+            Row r;
+            r.c = *at_bytes(tree_c, at0), r.n = *at_bytes(tree_n, at0), r.p = *at_bytes(tree_p, at0), r.w = *at_bytes(tree_w, at0);
+            r.info = *at_bytes(tree_expanded, node4), r.tickets = load_relaxed(at_bytes(tree_tickets, node4));
+            return r;
+        };
         int node = 0, depth = 0;
-        while (true) {
+        Row row = request(0);
+        const int node_limit = a.node_count[tree];
+        before_claims();
+        Path path{entries};
+        while (valid_node_count(node_limit, nodes)) {
             // (the same in all lanes; said so that the level's addresses and branches are worked out once per wavefront)
             node = __builtin_amdgcn_readfirstlane(node), depth = __builtin_amdgcn_readfirstlane(depth);
-            if (node < 0 || node >= node_limit) {
-                rollback_node_path(a, visits_of, path, tree, depth, lane, node_limit);
-                break;
-            }
-            if (depth >= a.path_depth) {   // the path buffer is full: stop before reading or claiming anything here
-                final_packed = pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, node, 0);
-                final_len = depth + 1;
-                break;
-            }
-            const size_t nrow = trow + node;
-            const uint32_t row4 = (uint32_t)node * (uint32_t)edges * 4u;   // byte offset of the node's edges in the tree's fields
-            // the first 64 edges are requested together with the node's own words, before the node's width is known
-            // (lanes beyond the row read its last edge and take no part)
-            const uint32_t at0 = row4 + (uint32_t)(lane < edges ? lane : edges - 1) * 4u;
-            const int c0 = *at_bytes(tree_c, at0), n0 = *at_bytes(tree_n, at0);
-            const float p0 = *at_bytes(tree_p, at0), w0 = *at_bytes(tree_w, at0);
-            const int node_info = a.node_expanded[nrow];
-            const int expand_inflight = load_relaxed(a.node_expand_inflight + nrow);
+            const uint32_t node4 = (uint32_t)node * 4u, row4 = node4 * (uint32_t)edges;   // byte offsets of the node, and of its edges, in the tree's fields
+            const int n0 = row.n, c0 = row.c, node_info = row.info, tickets = row.tickets;
+            const float p0 = row.p, w0 = row.w;
+            // Where the traversal goes on, or the complement of its selection word where it ends.
+            int next;
             if (node_info == PUCT_NODE_EXPANDED_TERMINAL) {
                 final_packed = pack_selection_v2(PUCT_SELECT_TERMINAL, node, 0);
-                final_len = depth + 1;
                 break;
             }
-            if (node_info < 0 || node_info > edges) {
-                rollback_node_path(a, visits_of, path, tree, depth, lane, node_limit);
-                break;
-            }
+            if (node_info < 0 || node_info > edges) break;
             const int cur_expanded = node_info;
 
-            // The level proper; returns the child the traversal moves on to, or -1 when it ends here.
+            // The level proper.
             auto level = [&](auto slices) __attribute__((always_inline)) -> int {
                 constexpr int S = decltype(slices)::value;   // (S - 1) * 64 < cur_expanded <= S * 64, or no edge at all (S = 1)
                 int n[S], f[S], c[S];
@@ -654,23 +651,17 @@ __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, c
                     // Expansion ticket, :389-403.  Tickets are only given back by the backup, and a ticket beyond the quota is
                     // returned at once, so a counter that already shows the quota used up stays that way for this launch.
                     int expand_slot = -1;
-                    if (cur_expanded + expand_inflight < allowed) {
+                    if (cur_expanded + tickets < allowed) {
                         if (lane == 0) {
-                            const int slot = cur_expanded + atomicAdd(&a.node_expand_inflight[nrow], 1);
+                            const int slot = cur_expanded + atomicAdd(at_bytes(tree_tickets, node4), 1);
                             if (slot < allowed)
                                 expand_slot = slot;
                             else
-                                atomicSub(&a.node_expand_inflight[nrow], 1);
+                                atomicSub(at_bytes(tree_tickets, node4), 1);
                         }
                         expand_slot = __builtin_amdgcn_readfirstlane(expand_slot);
                     }
-                    if (expand_slot >= 0) {
-                        final_packed = pack_selection_v2(PUCT_SELECT_EXPAND, node, expand_slot);
-                        final_len = depth + 1;
-                    } else {
-                        rollback_node_path(a, visits_of, path, tree, depth, lane, node_limit);
-                    }
-                    return -1;
+                    return ~(expand_slot >= 0 ? pack_selection_v2(PUCT_SELECT_EXPAND, node, expand_slot) : kPackedInvalidV2);
                 }
 
                 // puct_score in two parts: the mean value and the numerator of the exploration term do not depend on the
@@ -776,25 +767,32 @@ __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, c
                         }
                     }
                 }
-                if (held == 0) {   // no edge leads anywhere (or the winner's counter cannot be claimed)
-                    rollback_node_path(a, visits_of, path, tree, depth, lane, node_limit);
-                    return -1;
-                }
+                if (held == 0) return ~kPackedInvalidV2;   // no edge leads anywhere (or the winner's counter cannot be claimed)
                 // (only edges that lead to a node of the tree were candidates, so the child is one)
-                if (lane == 0) path[depth] = (node << 8) | best_eid;
+                path.append(depth, (node << 8) | best_eid, lane);
                 return of_edge(c, best_eid);
             };
 
             const int slices = (cur_expanded + kWave - 1) / kWave;
-            int next;
             if (slices <= 1) next = level(std::integral_constant<int, 1>{});
             else if (slices == 2) next = level(std::integral_constant<int, 2>{});
             else if (slices == 3) next = level(std::integral_constant<int, 3>{});
             else next = level(std::integral_constant<int, 4>{});
-            if (next < 0) break;
+            if (next < 0) {
+                final_packed = ~next;
+                break;
+            }
             node = next;
             depth += 1;
+            if (depth >= a.path_depth) {   // the path buffer is full: stop before reading or claiming anything here
+                final_packed = pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, node, 0);
+                break;
+            }
+            row = request(__builtin_amdgcn_readfirstlane(node));
         }
+        if (final_packed >> PUCT_PACKED_KIND_SHIFT == PUCT_SELECT_INVALID) rollback_node_path(a, visits_of, path, tree, depth, lane, node_limit);
+        else final_len = depth + 1;
+        path.finish(depth, lane);
     }
     if (lane == 0) {
         a.out_selected_node[out] = final_packed;

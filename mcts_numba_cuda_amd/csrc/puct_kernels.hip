@@ -13,6 +13,11 @@ __device__ __forceinline__ void fetch_arguments(const SelectArgs &a) {
                  "s"(a.tree_nodes), "s"(a.out_selected_node), "s"(a.out_path_eids), "s"(a.out_path_len), "s"(a.nodes), "s"(a.edges), "s"(a.warps), "s"(a.path_depth),
                  "s"(a.cpuct), "s"(a.c_pw), "s"(a.alpha_pw), "s"(a.soft_winner));
 }
+__device__ __forceinline__ void fetch_arguments(const NodeSelectArgs &a) {
+    asm volatile("" ::"s"(a.edge_child_id), "s"(a.edge_prior), "s"(a.edge_W), "s"(a.edge_N), "s"(a.node_inflight), "s"(a.node_expand_inflight), "s"(a.node_expanded),
+                 "s"(a.node_count), "s"(a.out_selected_node), "s"(a.out_path_eids), "s"(a.out_path_len), "s"(a.nodes), "s"(a.edges), "s"(a.warps), "s"(a.path_depth),
+                 "s"(a.cpuct), "s"(a.c_pw), "s"(a.alpha_pw));
+}
 __device__ __forceinline__ void fetch_arguments(const BackupArgs &a) {
     asm volatile("" ::"s"(a.edge_child_id), "s"(a.edge_W), "s"(a.edge_N), "s"(a.edge_inflight), "s"(a.node_inflight), "s"(a.node_expand_inflight), "s"(a.node_count),
                  "s"(a.out_selected_node), "s"(a.out_path_eids), "s"(a.out_path_len), "s"(a.path_edge_values), "s"(a.virtual_loss), "s"(a.nodes), "s"(a.edges), "s"(a.warps),
@@ -61,18 +66,20 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) __attribute__((amdgpu_wav
 // in the workgroup's dynamic LDS for the launch (a.nodes words).
 template <bool PRECLAIM, bool LOCAL>
 __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) __attribute__((amdgpu_waves_per_eu(8, 8))) void node_select_kernel(const NodeSelectArgs a) {
+    fetch_arguments(a);
     extern __shared__ int tree_visits[];
-    const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * (blockDim.x / kWave) + threadIdx.x / kWave);   // the same in all lanes
-    int *const in_memory = a.node_inflight + (size_t)blockIdx.x * a.nodes;
+    const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * traversals_of_block(a.warps) + threadIdx.x / kWave);   // the same in all lanes
+    int *const in_memory = a.node_inflight + (uint64_t)blockIdx.x * (uint32_t)a.nodes;
     const NodeVisits<LOCAL> visits_of{in_memory, (LdsInts)tree_visits};
-    if (LOCAL) {
-        for (int i = threadIdx.x; i < a.nodes; i += blockDim.x) tree_visits[i] = in_memory[i];
+    auto take_visits = [=]() {   // (while the root's row is on its way)
+        if (!LOCAL) return;
+        copy_words(tree_visits, in_memory, a.nodes);
         __syncthreads();
-    }
-    if (LOCAL || wid < a.warps) node_select_traversal<PRECLAIM, LOCAL>(a, visits_of, blockIdx.x, wid, threadIdx.x & (kWave - 1));
-    if (LOCAL) {
+    };
+    if (LOCAL || wid < a.warps) node_select_traversal<PRECLAIM, LOCAL>(a, visits_of, blockIdx.x, wid, threadIdx.x & (kWave - 1), take_visits);
+    if (LOCAL && valid_select_shape(a.path_depth, a.nodes, a.edges)) {
         __syncthreads();
-        for (int i = threadIdx.x; i < a.nodes; i += blockDim.x) in_memory[i] = tree_visits[i];
+        copy_words(in_memory, tree_visits, a.nodes);
     }
 }
 
@@ -174,8 +181,9 @@ int launch_node_select(float cpuct, float c_pw, float alpha_pw, const int *edge_
                      out_path_eids, out_path_len, trees,             nodes,         edges,        warps,  path_depth};
     dim3 grid, block;
     launch_shape(trees, warps, grid, block);
-    // (the counters of a tree in LDS: up to 16384 nodes)
-    if (grid.y == 1 && nodes > 0 && nodes <= kLocalVisitNodes)
+    // The counters of a tree in LDS: up to 16384 nodes, and a single traversal's only where its path may be long (in memory / in LDS, us a
+    // selection and its backup: 256 trees of 2000 x 128, three levels, 8.9 / 13.2; 4096 of 65 x 64, 512 levels, 1329 / 996).
+    if (grid.y == 1 && nodes > 0 && nodes <= kLocalVisitNodes && (warps > 1 || nodes <= 16 * (long long)path_depth))
         hipLaunchKernelGGL((node_select_kernel<PRECLAIM, true>), grid, block, sizeof(int) * (size_t)nodes, reinterpret_cast<hipStream_t>(stream), a);
     else
         hipLaunchKernelGGL((node_select_kernel<PRECLAIM, false>), grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);
