@@ -278,6 +278,7 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
         int *const tree_tickets = a.node_expand_inflight + tree_nodes;
         const int asked_node_cnt = load_relaxed(a.tree_nodes + tree);
         int node = 0, depth = 0, node_cnt = 0;
+        uint32_t bound = 0;   // a node's expansion word at or beyond which there is more to ask: the root's always, then an end of a game or no width
         Path path{entries};
         while (true) {
             // (the same in all lanes; said so that the level's addresses and branches are worked out once per wavefront)
@@ -294,32 +295,46 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
             const int node_info = *at_bytes(tree_expanded, node4);
             const int tickets = load_relaxed(at_bytes(tree_tickets, node4));
 
-            // Where the traversal goes on, or the complement of its selection word where it ends.
-            int next;
-            if (depth == 0) {   // (how many nodes the tree has is not waited for before the root's row is on its way)
-                int count = asked_node_cnt;
-                asm volatile("" : "+v"(count));
-                node_cnt = __builtin_amdgcn_readfirstlane(count);
-                if (!valid_node_count(node_cnt, nodes)) break;
-            }
-            if (node_info == PUCT_NODE_EXPANDED_TERMINAL) {
-                final_packed = pack_selection(PUCT_SELECT_TERMINAL, node, 0, PUCT_REASON_OK_TERMINAL);
-                break;
-            }
-            if (node_info < 0 || node_info > edges) {
-                final_packed = pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_NODE_INFO);
-                break;
-            }
-            if (depth >= a.path_depth) {
-                final_packed = pack_selection(PUCT_SELECT_DEPTH_LIMIT, node, 0, PUCT_REASON_OK_DEPTH_LIMIT);
-                break;
-            }
-
+            // A node without an edge, or with one: no score to work out.
             const int cur_expanded = node_info;
+            auto try_expand = [&](int allowed) __attribute__((always_inline)) -> int {   // expansion ticket, src/puct/puct_gpu_v3_cpp.cu:219-233; -1: none
+                int expand_slot = -1;
+                if (cur_expanded + tickets < allowed) {
+                    if (lane == 0) {
+                        const int slot = cur_expanded + atomicAdd(at_bytes(tree_tickets, node4), 1);
+                        if (slot < allowed)
+                            expand_slot = slot;
+                        else
+                            atomicSub(at_bytes(tree_tickets, node4), 1);
+                    }
+                    expand_slot = __builtin_amdgcn_readfirstlane(expand_slot);
+                }
+                return expand_slot;
+            };
+            auto narrow = [&]() __attribute__((always_inline)) -> int {
+                int allowed = allowed_children(a.c_pw, 0.5f, 1, edges, 1.0f);   // (no visits: 1 ** alpha_pw is 1, whatever alpha_pw is)
+                if (cur_expanded == 1) {
+                    const int total = __builtin_amdgcn_readfirstlane(n0 + f0), parent_eff = total > 1 ? total : 1;
+                    allowed = a.c_pw != 0.0f ? allowed_children(a.c_pw, a.alpha_pw, parent_eff, edges) : 1;
+                }
+                if (allowed > cur_expanded) {
+                    const int expand_slot = try_expand(allowed);
+                    if (expand_slot >= 0) return ~pack_selection(PUCT_SELECT_EXPAND, node, expand_slot, PUCT_REASON_OK_EXPAND);
+                    if (cur_expanded == 0) return ~pack_selection(PUCT_SELECT_BUSY, node, 0, PUCT_REASON_BUSY_EXPAND_INFLIGHT);
+                }
+                const int child = __builtin_amdgcn_readfirstlane(c0);
+                if ((uint32_t)child >= (uint32_t)node_cnt) return ~pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_CHILD_OOB);
+                if (lane == 0) {
+                    if (WHERE == ClaimsIn::OWN) claims.set(row4, f0 + 1);
+                    else claims.add(row4, 1);
+                }
+                path.append(depth, node << 8, lane);
+                return child;
+            };
 
             // The level proper.
             auto level = [&](auto slices) __attribute__((always_inline)) -> int {
-                constexpr int S = decltype(slices)::value;   // (S - 1) * 64 < cur_expanded <= S * 64, or no edge at all (S = 1)
+                constexpr int S = decltype(slices)::value;   // (S - 1) * 64 < cur_expanded <= S * 64, two at least
                 constexpr int CS = S <= 2 ? S : 1;   // slices whose row of children is requested with the scores' fields (see best_child below)
                 int n[S], f[S], c[CS];
                 // byte offset of the edge that this lane looks at in slice i (lanes beyond the node's edges: its last edge)
@@ -339,35 +354,18 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
 #pragma unroll
                 for (int i = 0; i < S; ++i) in_node[i] = i < S - 1 || lane + i * kWave < cur_expanded;
 
-                int parent_eff = 1, allowed = 1;
-                float sqrt_parent = 1.0f;
-                if (S == 1 && cur_expanded == 0) {   // no visits: 1 ** alpha_pw is 1, whatever alpha_pw is
-                    allowed = allowed_children(a.c_pw, 0.5f, 1, edges, 1.0f);
-                } else if (cur_expanded != 1 || a.c_pw != 0.0f) {
-                    int total = 0;
+                int total = 0;
 #pragma unroll
-                    for (int i = 0; i < S; ++i) total += in_node[i] ? n[i] + f[i] : 0;
-                    total = wave_sum(total);
-                    parent_eff = total > 1 ? total : 1;
-                    sqrt_parent = sqrtf((float)parent_eff);
-                    allowed = allowed_children(a.c_pw, a.alpha_pw, parent_eff, edges, sqrt_parent);
-                }
-
-                if (allowed > cur_expanded) {
-                    // Expansion ticket, src/puct/puct_gpu_v3_cpp.cu:219-233.
-                    int expand_slot = -1;
-                    if (cur_expanded + tickets < allowed) {
-                        if (lane == 0) {
-                            const int slot = cur_expanded + atomicAdd(at_bytes(tree_tickets, node4), 1);
-                            if (slot < allowed)
-                                expand_slot = slot;
-                            else
-                                atomicSub(at_bytes(tree_tickets, node4), 1);
-                        }
-                        expand_slot = __builtin_amdgcn_readfirstlane(expand_slot);
+                for (int i = 0; i < S; ++i) total += in_node[i] ? n[i] + f[i] : 0;
+                total = wave_sum(total);
+                const int parent_eff = total > 1 ? total : 1;
+                const float sqrt_parent = sqrtf((float)parent_eff);
+                if (a.c_pw != 0.0f) {   // (else there is one child allowed, and there are two)
+                    const int allowed = allowed_children(a.c_pw, a.alpha_pw, parent_eff, edges, sqrt_parent);
+                    if (allowed > cur_expanded) {
+                        const int expand_slot = try_expand(allowed);
+                        if (expand_slot >= 0) return ~pack_selection(PUCT_SELECT_EXPAND, node, expand_slot, PUCT_REASON_OK_EXPAND);
                     }
-                    if (expand_slot >= 0) return ~pack_selection(PUCT_SELECT_EXPAND, node, expand_slot, PUCT_REASON_OK_EXPAND);
-                    if (cur_expanded == 0) return ~pack_selection(PUCT_SELECT_BUSY, node, 0, PUCT_REASON_BUSY_EXPAND_INFLIGHT);
                 }
 
                 int tie_offset = WHERE == ClaimsIn::OWN ? 0 : wid;
@@ -386,68 +384,62 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                 // wider node only its first 64, and beyond them just the winner's word is asked for, on its way while the
                 // claim is made (the rest of that row is a sixth of what such a level reads -- and those launches are bound by
                 // what they read -- and three registers per lane; at 128 edges waiting for the word cost more than the row).
-                int best_eid = 0, held = 0, best_child = c0;   // (cur_expanded == 1: lane 0's is read below)
-                if (cur_expanded == 1) {
-                    if (WHERE != ClaimsIn::OWN && lane == 0) claims.add(row4, 1);
-                    held = 1;
-                } else {
-                    // Winner-recalc claim, src/puct/puct_gpu_v3_cpp.cu:235-275: score all edges, try to move the winner's
-                    // in-flight count from the value the score was computed with to that value plus one, rescore once if
-                    // another traversal got there first.  The mean value and the numerator of the exploration term do not
-                    // depend on the in-flight counts, so a second evaluation divides once per edge, and only in the slices
-                    // whose counts have changed (other traversals' claims sit on a few edges).
-                    float q[S], num[S];
+                int best_eid = kNoEdge, held = 0, best_child = 0;
+                // Winner-recalc claim, src/puct/puct_gpu_v3_cpp.cu:235-275: score all edges, try to move the winner's
+                // in-flight count from the value the score was computed with to that value plus one, rescore once if
+                // another traversal got there first.  The mean value and the numerator of the exploration term do not
+                // depend on the in-flight counts, so a second evaluation divides once per edge, and only in the slices
+                // whose counts have changed (other traversals' claims sit on a few edges).
+                float q[S], num[S];
 #pragma unroll
-                    for (int i = 0; i < S; ++i) {
-                        // (of a node of several slices, one none of whose edges has a visit or a value has q = +0 without dividing)
-                        q[i] = 0.0f;
-                        if (S == 1 || __builtin_amdgcn_ballot_w64(n[i] > 0 && __float_as_uint(w[i]) != 0u) != 0) q[i] = n[i] > 0 ? w[i] / (float)n[i] : 0.0f;
-                        num[i] = a.cpuct * p[i] * sqrt_parent;
-                    }
-                    uint32_t keys[S];
-                    auto score_slice = [&](int i, int inflight) {
-                        return in_node[i] ? score_key(q[i] + num[i] / (float)(n[i] + inflight + 1)) : 0u;
-                    };
-                    best_eid = kNoEdge;
-                    for (int attempt = 0; attempt < kRecalcAttempts; ++attempt) {
-                        if (attempt == 0) {
+                for (int i = 0; i < S; ++i) {
+                    // (of a node of several slices, one none of whose edges has a visit or a value has q = +0 without dividing)
+                    q[i] = 0.0f;
+                    if (S == 1 || __builtin_amdgcn_ballot_w64(n[i] > 0 && __float_as_uint(w[i]) != 0u) != 0) q[i] = n[i] > 0 ? w[i] / (float)n[i] : 0.0f;
+                    num[i] = a.cpuct * p[i] * sqrt_parent;
+                }
+                uint32_t keys[S];
+                auto score_slice = [&](int i, int inflight) {
+                    return in_node[i] ? score_key(q[i] + num[i] / (float)(n[i] + inflight + 1)) : 0u;
+                };
+                for (int attempt = 0; attempt < kRecalcAttempts; ++attempt) {
+                    if (attempt == 0) {
 #pragma unroll
-                            for (int i = 0; i < S; ++i) keys[i] = score_slice(i, f[i]);
-                        } else {
+                        for (int i = 0; i < S; ++i) keys[i] = score_slice(i, f[i]);
+                    } else {
 #pragma unroll
-                            for (int i = 0; i < S; ++i) {
-                                const int fi = claims.peek(at(i));
-                                if (__builtin_amdgcn_ballot_w64(fi != f[i]) != 0) {
-                                    f[i] = fi;
-                                    keys[i] = score_slice(i, fi);
-                                }
+                        for (int i = 0; i < S; ++i) {
+                            const int fi = claims.peek(at(i));
+                            if (__builtin_amdgcn_ballot_w64(fi != f[i]) != 0) {
+                                f[i] = fi;
+                                keys[i] = score_slice(i, fi);
                             }
                         }
-                        best_eid = best_edge<S>(keys, lane, -1, tie_offset);
-                        if (best_eid == kNoEdge) break;
-                        if (best_eid < CS * kWave) {
-                            best_child = __builtin_amdgcn_readlane(c[0], best_eid & (kWave - 1));
-                            if (CS > 1 && best_eid >= kWave) best_child = __builtin_amdgcn_readlane(c[CS - 1], best_eid & (kWave - 1));
-                        } else {
-                            best_child = load_relaxed(at_bytes(tree_c, row4 + (uint32_t)best_eid * 4u));   // (every lane the same word)
-                        }
-                        if (WHERE == ClaimsIn::OWN) {
-                            held = 1;
-                            break;
-                        }
-                        const int best_inflight = of_edge(f, best_eid);
-                        int got = 0;
-                        if (lane == 0) {
-                            const int prev = claims.cas(row4 + (uint32_t)best_eid * 4u, best_inflight, best_inflight + 1);
-                            got = prev == best_inflight ? 1 : 0;
-                        }
-                        held = __builtin_amdgcn_readfirstlane(got);
-                        if (held) break;
                     }
-                    if (WHERE != ClaimsIn::OWN && a.soft_winner != 0 && held == 0 && best_eid != kNoEdge) {
-                        if (lane == 0) claims.add(row4 + (uint32_t)best_eid * 4u, 1);
+                    best_eid = best_edge<S>(keys, lane, -1, tie_offset);
+                    if (best_eid == kNoEdge) break;
+                    if (S == CS || best_eid < CS * kWave) {
+                        best_child = __builtin_amdgcn_readlane(c[0], best_eid & (kWave - 1));
+                        if (CS > 1 && best_eid >= kWave) best_child = __builtin_amdgcn_readlane(c[CS - 1], best_eid & (kWave - 1));
+                    } else {
+                        best_child = load_relaxed(at_bytes(tree_c, row4 + (uint32_t)best_eid * 4u));   // (every lane the same word)
+                    }
+                    if (WHERE == ClaimsIn::OWN) {
                         held = 1;
+                        break;
                     }
+                    const int best_inflight = of_edge(f, best_eid);
+                    int got = 0;
+                    if (lane == 0) {
+                        const int prev = claims.cas(row4 + (uint32_t)best_eid * 4u, best_inflight, best_inflight + 1);
+                        got = prev == best_inflight ? 1 : 0;
+                    }
+                    held = __builtin_amdgcn_readfirstlane(got);
+                    if (held) break;
+                }
+                if (WHERE != ClaimsIn::OWN && a.soft_winner != 0 && held == 0 && best_eid != kNoEdge) {
+                    if (lane == 0) claims.add(row4 + (uint32_t)best_eid * 4u, 1);
+                    held = 1;
                 }
 
                 if (held == 0)
@@ -455,7 +447,7 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                                                : ~pack_selection(PUCT_SELECT_BUSY, node, 0, PUCT_REASON_BUSY_WINNER_RECALC);
 
                 best_child = __builtin_amdgcn_readfirstlane(best_child);
-                if (best_child < 0 || best_child >= node_cnt) {
+                if ((uint32_t)best_child >= (uint32_t)node_cnt) {
                     if (WHERE != ClaimsIn::OWN && lane == 0) claims.add(row4 + (uint32_t)best_eid * 4u, -1);
                     return ~pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_CHILD_OOB);
                 }
@@ -468,11 +460,27 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                 return best_child;
             };
 
-            const int slices = (cur_expanded + kWave - 1) / kWave;
-            if (slices <= 1) next = level(std::integral_constant<int, 1>{});
-            else if (slices == 2) next = level(std::integral_constant<int, 2>{});
-            else if (slices == 3) next = level(std::integral_constant<int, 3>{});
-            else next = level(std::integral_constant<int, 4>{});
+            // Where the traversal goes on, or the complement of its selection word where it ends.
+            int next = 0;
+            if (__builtin_expect((uint32_t)node_info >= bound, 0)) {
+                if (bound == 0) {   // (how many nodes the tree has is not waited for before the root's row is on its way)
+                    int count = asked_node_cnt;
+                    asm volatile("" : "+v"(count));
+                    node_cnt = __builtin_amdgcn_readfirstlane(count);
+                    bound = (uint32_t)edges + 1u;
+                    if (!valid_node_count(node_cnt, nodes)) next = ~pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_SHAPE);
+                }
+                if (next == 0 && node_info == PUCT_NODE_EXPANDED_TERMINAL) next = ~pack_selection(PUCT_SELECT_TERMINAL, node, 0, PUCT_REASON_OK_TERMINAL);
+                else if (next == 0 && (uint32_t)node_info >= bound) next = ~pack_selection(PUCT_SELECT_INVALID, PUCT_PACKED_NODE_MASK, 0, PUCT_REASON_INVALID_NODE_INFO);
+            }
+            if (next == 0) {
+                if (depth >= a.path_depth) next = ~pack_selection(PUCT_SELECT_DEPTH_LIMIT, node, 0, PUCT_REASON_OK_DEPTH_LIMIT);
+                else if (cur_expanded <= 1) next = narrow();
+                else if (cur_expanded <= kWave) next = level(std::integral_constant<int, 1>{});
+                else if (cur_expanded <= 2 * kWave) next = level(std::integral_constant<int, 2>{});
+                else if (cur_expanded <= 3 * kWave) next = level(std::integral_constant<int, 3>{});
+                else next = level(std::integral_constant<int, 4>{});
+            }
             if (next < 0) {
                 final_packed = ~next;
                 break;
