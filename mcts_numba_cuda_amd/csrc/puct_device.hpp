@@ -49,10 +49,16 @@ struct SelectArgs {
 
 // ---- cross-lane reductions -------------------------------------------------------------------------------------
 // DPP controls: quad_perm [1,0,3,2], quad_perm [2,3,0,1], row_half_mirror, row_mirror.  After the four steps every
-// lane holds the reduction of its 16-lane row; the four rows are combined through lane reads.
+// lane holds the reduction of its 16-lane row; rows 1 and 3 then take the row before (row_bcast:15), row 3 the lower half
+// (row_bcast:31), so that the last lane has all of it.
 template <int CTRL>
 __device__ __forceinline__ int dpp(int v) {
     return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
+}
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_rows(int v) {   // 0 in the other rows
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
 }
 
 __device__ __forceinline__ int wave_sum(int v) {
@@ -60,8 +66,9 @@ __device__ __forceinline__ int wave_sum(int v) {
     v += dpp<0x4E>(v);
     v += dpp<0x141>(v);
     v += dpp<0x140>(v);
-    return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
-           __builtin_amdgcn_readlane(v, 48);
+    v += dpp_rows<0x142, 0xA>(v);
+    v += dpp_rows<0x143, 0xC>(v);
+    return __builtin_amdgcn_readlane(v, 63);
 }
 
 template <int CTRL>
@@ -111,6 +118,15 @@ __device__ __forceinline__ int pack_selection(int kind, int node, int slot, int 
 __device__ __forceinline__ bool valid_select_shape(int path_depth, int nodes, int edges) { return path_depth >= 1 && nodes > 0 && edges > 0 && edges <= PUCT_PACKED_EDGE_MASK + 1; }
 __device__ __forceinline__ bool valid_node_count(int node_cnt, int nodes) { return node_cnt > 0 && node_cnt <= nodes && node_cnt <= PUCT_PACKED_NODE_LIMIT; }
 
+// sqrtf((float)n), correctly rounded, for n >= 1: the rounding of the hardware's root is put right as the compiler does it, without
+// what it does for arguments that are tiny, infinite or negative.
+__device__ __forceinline__ float sqrt_of_count(int n) {
+    const float x = (float)n, root = __builtin_amdgcn_sqrtf(x);
+    const float below = __uint_as_float(__float_as_uint(root) - 1u), above = __uint_as_float(__float_as_uint(root) + 1u);
+    const float rounded = __builtin_fmaf(-below, root, x) <= 0.0f ? below : root;
+    return __builtin_fmaf(-above, root, x) > 0.0f ? above : rounded;
+}
+
 // Progressive widening, src/puct/puct_gpu_v3_cpp.cu:150-157.
 __device__ __forceinline__ int allowed_children(float c_pw, float alpha_pw, int n_node, int edges, float sqrt_n_node) {
     const float val = __builtin_expect(alpha_pw == 0.5f, 1) ? c_pw * sqrt_n_node : c_pw * powf((float)n_node, alpha_pw);
@@ -119,7 +135,7 @@ __device__ __forceinline__ int allowed_children(float c_pw, float alpha_pw, int 
     return allowed > 1 ? allowed : 1;
 }
 __device__ __forceinline__ int allowed_children(float c_pw, float alpha_pw, int n_node, int edges) {
-    return allowed_children(c_pw, alpha_pw, n_node, edges, sqrtf((float)n_node));
+    return allowed_children(c_pw, alpha_pw, n_node, edges, sqrt_of_count(n_node));
 }
 
 // The score of an edge (src/puct/puct_gpu_v3_cpp.cu:171-180) is q + u with q = n > 0 ? w / n : 0 and
@@ -150,18 +166,14 @@ __device__ __forceinline__ uint32_t score_key(float score) {
 }
 
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-    auto step = [](uint32_t x, auto ctrl) {
-        const uint32_t o = (uint32_t)dpp<decltype(ctrl)::value>((int)x);
-        return o > x ? o : x;
-    };
-    v = step(v, std::integral_constant<int, 0xB1>{});
-    v = step(v, std::integral_constant<int, 0x4E>{});
-    v = step(v, std::integral_constant<int, 0x141>{});
-    v = step(v, std::integral_constant<int, 0x140>{});
-    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
-    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
-    const uint32_t ab = a > b ? a : b, cd = c > d ? c : d;
-    return ab > cd ? ab : cd;
+    auto larger = [](uint32_t x, int o) { return (uint32_t)o > x ? (uint32_t)o : x; };
+    v = larger(v, dpp<0xB1>((int)v));
+    v = larger(v, dpp<0x4E>((int)v));
+    v = larger(v, dpp<0x141>((int)v));
+    v = larger(v, dpp<0x140>((int)v));
+    v = larger(v, dpp_rows<0x142, 0xA>((int)v));
+    v = larger(v, dpp_rows<0x143, 0xC>((int)v));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
 // The edge with the largest key (keys[i] belongs to edge lane + 64 i; `skip` takes no part); among equal keys the one
@@ -359,7 +371,7 @@ __device__ __forceinline__ void select_traversal(const SelectArgs &a, const Edge
                 for (int i = 0; i < S; ++i) total += in_node[i] ? n[i] + f[i] : 0;
                 total = wave_sum(total);
                 const int parent_eff = total > 1 ? total : 1;
-                const float sqrt_parent = sqrtf((float)parent_eff);
+                const float sqrt_parent = sqrt_of_count(parent_eff);
                 if (a.c_pw != 0.0f) {   // (else there is one child allowed, and there are two)
                     const int allowed = allowed_children(a.c_pw, a.alpha_pw, parent_eff, edges, sqrt_parent);
                     if (allowed > cur_expanded) {
@@ -652,7 +664,7 @@ __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, c
                 for (int i = 0; i < S; ++i) total += cand[i] ? n[i] + f[i] : 0;
                 total = wave_sum(total);
                 const int parent_eff = total > 1 ? total : 1;   // :407-416
-                const float sqrt_parent = sqrtf((float)parent_eff);
+                const float sqrt_parent = sqrt_of_count(parent_eff);
                 const int allowed = (PRECLAIM && cur_expanded == 0) ? 1 : allowed_children(a.c_pw, a.alpha_pw, parent_eff, edges, sqrt_parent);
 
                 if (allowed > cur_expanded) {
