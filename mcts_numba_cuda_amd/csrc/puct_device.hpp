@@ -629,18 +629,27 @@ __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, c
             const uint32_t node4 = (uint32_t)node * 4u, row4 = node4 * (uint32_t)edges;   // byte offsets of the node, and of its edges, in the tree's fields
             const int n0 = row.n, c0 = row.c, node_info = row.info, tickets = row.tickets;
             const float p0 = row.p, w0 = row.w;
-            // Where the traversal goes on, or the complement of its selection word where it ends.
-            int next;
-            if (node_info == PUCT_NODE_EXPANDED_TERMINAL) {
-                final_packed = pack_selection_v2(PUCT_SELECT_TERMINAL, node, 0);
-                break;
-            }
-            if (node_info < 0 || node_info > edges) break;
             const int cur_expanded = node_info;
+            // Expansion ticket, :389-403.  Tickets are only given back by the backup, and a ticket beyond the quota is
+            // returned at once, so a counter that already shows the quota used up stays that way for this launch.
+            auto expand = [&](int allowed) __attribute__((always_inline)) -> int {
+                int expand_slot = -1;
+                if (cur_expanded + tickets < allowed) {
+                    if (lane == 0) {
+                        const int slot = cur_expanded + atomicAdd(at_bytes(tree_tickets, node4), 1);
+                        if (slot < allowed)
+                            expand_slot = slot;
+                        else
+                            atomicSub(at_bytes(tree_tickets, node4), 1);
+                    }
+                    expand_slot = __builtin_amdgcn_readfirstlane(expand_slot);
+                }
+                return ~(expand_slot >= 0 ? pack_selection_v2(PUCT_SELECT_EXPAND, node, expand_slot) : kPackedInvalidV2);
+            };
 
             // The level proper.
             auto level = [&](auto slices) __attribute__((always_inline)) -> int {
-                constexpr int S = decltype(slices)::value;   // (S - 1) * 64 < cur_expanded <= S * 64, or no edge at all (S = 1)
+                constexpr int S = decltype(slices)::value;   // (S - 1) * 64 < cur_expanded <= S * 64, one at least
                 int n[S], f[S], c[S];
                 float p[S], w[S];
                 bool cand[S];
@@ -665,23 +674,9 @@ __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, c
                 total = wave_sum(total);
                 const int parent_eff = total > 1 ? total : 1;   // :407-416
                 const float sqrt_parent = sqrt_of_count(parent_eff);
-                const int allowed = (PRECLAIM && cur_expanded == 0) ? 1 : allowed_children(a.c_pw, a.alpha_pw, parent_eff, edges, sqrt_parent);
-
-                if (allowed > cur_expanded) {
-                    // Expansion ticket, :389-403.  Tickets are only given back by the backup, and a ticket beyond the quota is
-                    // returned at once, so a counter that already shows the quota used up stays that way for this launch.
-                    int expand_slot = -1;
-                    if (cur_expanded + tickets < allowed) {
-                        if (lane == 0) {
-                            const int slot = cur_expanded + atomicAdd(at_bytes(tree_tickets, node4), 1);
-                            if (slot < allowed)
-                                expand_slot = slot;
-                            else
-                                atomicSub(at_bytes(tree_tickets, node4), 1);
-                        }
-                        expand_slot = __builtin_amdgcn_readfirstlane(expand_slot);
-                    }
-                    return ~(expand_slot >= 0 ? pack_selection_v2(PUCT_SELECT_EXPAND, node, expand_slot) : kPackedInvalidV2);
+                if (a.c_pw != 0.0f) {   // (else there is one child allowed, and there is one)
+                    const int allowed = allowed_children(a.c_pw, a.alpha_pw, parent_eff, edges, sqrt_parent);
+                    if (allowed > cur_expanded) return expand(allowed);
                 }
 
                 // puct_score in two parts: the mean value and the numerator of the exploration term do not depend on the
@@ -793,21 +788,20 @@ __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, c
                 return of_edge(c, best_eid);
             };
 
-            const int slices = (cur_expanded + kWave - 1) / kWave;
-            if (slices <= 1) next = level(std::integral_constant<int, 1>{});
-            else if (slices == 2) next = level(std::integral_constant<int, 2>{});
-            else if (slices == 3) next = level(std::integral_constant<int, 3>{});
+            // Where the traversal goes on, or the complement of its selection word where it ends.
+            int next;
+            if (__builtin_expect((uint32_t)node_info > (uint32_t)edges, 0)) next = ~(node_info == PUCT_NODE_EXPANDED_TERMINAL ? pack_selection_v2(PUCT_SELECT_TERMINAL, node, 0) : kPackedInvalidV2);
+            else if (cur_expanded == 0) next = expand(PRECLAIM ? 1 : allowed_children(a.c_pw, 0.5f, 1, edges, 1.0f));   // (no visits: 1 ** alpha_pw is 1, whatever alpha_pw is)
+            else if (cur_expanded <= kWave) next = level(std::integral_constant<int, 1>{});
+            else if (cur_expanded <= 2 * kWave) next = level(std::integral_constant<int, 2>{});
+            else if (cur_expanded <= 3 * kWave) next = level(std::integral_constant<int, 3>{});
             else next = level(std::integral_constant<int, 4>{});
+            if (next >= 0 && ++depth >= a.path_depth) next = ~pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, next, 0);   // the path buffer is full: stop before reading or claiming anything there
             if (next < 0) {
                 final_packed = ~next;
                 break;
             }
             node = next;
-            depth += 1;
-            if (depth >= a.path_depth) {   // the path buffer is full: stop before reading or claiming anything here
-                final_packed = pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, node, 0);
-                break;
-            }
             row = request(__builtin_amdgcn_readfirstlane(node));
         }
         if (final_packed >> PUCT_PACKED_KIND_SHIFT == PUCT_SELECT_INVALID) rollback_node_path(a, visits_of, path, tree, depth, lane, node_limit);
