@@ -250,29 +250,6 @@ __device__ __forceinline__ uint32_t score_image(float score) {
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-    auto step = [](uint32_t x, auto ctrl) {
-        const uint32_t o = (uint32_t)dpp<decltype(ctrl)::value>((int)x);
-        return o > x ? o : x;
-    };
-    v = step(v, std::integral_constant<int, 0xB1>{});
-    v = step(v, std::integral_constant<int, 0x4E>{});
-    v = step(v, std::integral_constant<int, 0x141>{});
-    v = step(v, std::integral_constant<int, 0x140>{});
-    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
-    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
-    const uint32_t ab = a > b ? a : b, cd = c > d ? c : d;
-    return ab > cd ? ab : cd;
-}
-
-// Progressive widening, src/puct/puct_gpu_v3_cpp.cu:150-157; sqrt_n = sqrtf((float)n_node), which the score needs too.
-__device__ __forceinline__ int allowed_children(float c_pw, float alpha_pw, int n_node, float sqrt_n, int edges) {
-    const float val = (alpha_pw == 0.5f) ? c_pw * sqrt_n : c_pw * powf((float)n_node, alpha_pw);
-    if (val >= (float)edges) return edges;
-    const int allowed = (int)ceilf(val);
-    return allowed > 1 ? allowed : 1;
-}
-
 // ---- selection ---------------------------------------------------------------------------------------------------
 // The edges of one node as the deciding traversals see them: up to NS per lane.
 template <int NS>
@@ -285,7 +262,7 @@ struct EdgeSet {
 
 template <int NS>
 __device__ __forceinline__ float edge_score(const EdgeSet<NS> &e, int i, float sqrt_parent, int more_claims) {
-    return e.q[i] + e.cp[i] * sqrt_parent / (float)(e.den[i] + more_claims);
+    return prow_score(e.q[i], e.cp[i], sqrt_parent, e.den[i] + more_claims);
 }
 
 // The traversals `members` decide one after another on the edges in `e` (which must include every edge that can come
@@ -299,33 +276,22 @@ __device__ __forceinline__ void decide_in_turn(const LoopArgs &g, StepLds &s, in
     const bool widening = expanded != 1 || g.c_pw != 0.0f;
     const int claims_base = total;
     const int eff_lane = widening ? (total + lane > 1 ? total + lane : 1) : 1;
-    const float sqrt_lane = widening ? sqrtf((float)eff_lane) : 1.0f;
-    const int allowed_lane = widening ? allowed_children(g.c_pw, g.alpha_pw, eff_lane, sqrt_lane, legal) : 1;
+    const float sqrt_lane = widening ? sqrt_of_count(eff_lane) : 1.0f;
+    const int allowed_lane = widening ? allowed_children(g.c_pw, g.alpha_pw, eff_lane, legal, sqrt_lane) : 1;
     for (uint64_t rest = members; rest != 0; rest &= rest - 1) {
         const int j = __builtin_ctzll(rest);   // the traversal deciding now
         const int claimed = total - claims_base;
         const float sqrt_parent = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), claimed));
         const int allowed = __builtin_amdgcn_readlane(allowed_lane, claimed);
-        if (allowed > expanded) {
-            if (expanded + tickets < allowed) {   // expansion ticket
-                if (lane == 0) {
-                    s.sel[j] = pack_sel(PUCT_SELECT_EXPAND, node, expanded + tickets);
-                    s.len[j] = depth + 1;
-                    s.claims[j] = depth;
-                    next[j] = -1;
-                }
-                tickets += 1;
-                continue;
+        if (expanded + tickets < allowed) {   // expansion ticket
+            if (lane == 0) {
+                s.sel[j] = pack_sel(PUCT_SELECT_EXPAND, node, expanded + tickets);
+                s.len[j] = depth + 1;
+                s.claims[j] = depth;
+                next[j] = -1;
             }
-            if (expanded == 0) {   // the node's only allowed child is being created by another traversal
-                if (lane == 0) {
-                    s.sel[j] = pack_sel(PUCT_SELECT_BUSY, node, 0);
-                    s.len[j] = 0;
-                    s.claims[j] = depth;
-                    next[j] = -1;
-                }
-                continue;
-            }
+            tickets += 1;
+            continue;
         }
         // The highest score first: its order-preserving integer image, reduced over the wavefront.  Only if more than
         // one edge attains it does the rotated edge index decide, through the full keys.  (A node's only edge is taken
@@ -408,6 +374,17 @@ __device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {   // over the 16 l
     return step(v, std::integral_constant<int, 0x140>{});
 }
 
+__device__ __forceinline__ float row_max_f32(float v) {   // over the 16 lanes of each row; no NaN
+    float top;
+    asm("s_nop 1\n\t"
+        "v_max_f32_dpp %0, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf bound_ctrl:0\n\ts_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf bound_ctrl:0\n\ts_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:0\n\ts_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf bound_ctrl:0"
+        : "=&v"(top) : "v"(v));
+    return top;
+}
+
 // decide_in_turn for at most 16 edges, one per lane from lane 0 on, all of which lead to a node and have a finite score.  A
 // decision is a chain of dependent instructions on a lone wavefront, 0.5 us by decide_in_turn, most of it not the score:
 // here the maximum stays within a row of 16 lanes, the outcome is one register of the traversal's lane, and what the
@@ -429,11 +406,9 @@ __device__ __forceinline__ void row_decisions(const EdgeSet<1> &e, uint64_t edge
             uint64_t first = 1ull;
             if (!single) {
                 const float sqrt_parent = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), claimed));
-                const uint32_t b = __float_as_uint(prow_score(q, cp, sqrt_parent, den) + 0.0f);   // -0.0f counts as +0.0f
-                const uint32_t image = b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);           // score_image of a finite score
-                const uint32_t top = row_max_u32(image);
-                first = __builtin_amdgcn_uicmp(image, top, 32 /* == */) & edges;
-                if ((first & (first - 1)) != 0) {   // the rotated edge index decides, as in candidate_key
+                const float score = q + prow_quotient(cp * sqrt_parent, (float)den, __builtin_amdgcn_rcpf((float)den));
+                first = __builtin_amdgcn_fcmpf(score, row_max_f32(score), 1 /* == */) & edges;
+                if (__builtin_popcount((uint32_t)first) > 1) {   // the rotated edge index decides, as in candidate_key
                     int tie_offset = __builtin_ctz(bit);
                     if (tie_offset >= expanded) tie_offset %= expanded;
                     const int turned = e.eid[0] - tie_offset + (e.eid[0] < tie_offset ? expanded : 0);
@@ -452,8 +427,8 @@ __device__ __forceinline__ void decide_in_row(const LoopArgs &g, StepLds &s, int
                                               uint32_t members, int depth, int lane, int expanded, int legal, int total, int &tickets, bool single) {
     const bool widening = expanded != 1 || g.c_pw != 0.0f;
     const int eff_lane = widening ? (total + lane > 1 ? total + lane : 1) : 1;
-    const float sqrt_lane = widening ? sqrtf((float)eff_lane) : 1.0f;
-    const int allowed_lane = widening ? allowed_children(g.c_pw, g.alpha_pw, eff_lane, sqrt_lane, legal) : 1;
+    const float sqrt_lane = widening ? sqrt_of_count(eff_lane) : 1.0f;
+    const int allowed_lane = widening ? allowed_children(g.c_pw, g.alpha_pw, eff_lane, legal, sqrt_lane) : 1;
     const int tickets_before = tickets;
     int den = prow_den(e.eid[0] >= 0, e.den[0]), mine = -1;   // mine: lane of the edge that this lane's traversal takes
     uint32_t with_ticket = 0;
@@ -492,11 +467,13 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
     Edge *row = g.edges + nrow * kEdges;
     // all 256 edge slots are requested together with the node's own word, before anything about the node is known: one
     // round trip per level, whatever the node's width
+    const NodeInfo ni = load_info(g.info + nrow);
     Edge loaded[kSlices];
 #pragma unroll
     for (int i = 0; i < kSlices; ++i) loaded[i] = load_edge(row + lane + i * kWave);
-    const NodeInfo ni = load_info(g.info + nrow);
-    const int expanded = ni.expanded;
+    const int expanded = ni.expanded, n_members = __popcll(members);
+    int tickets = ni.tickets;
+    const int legal = ni.legal_turn & 0xFFFF;
     nodes_read += 1;
     if (expanded == PUCT_NODE_EXPANDED_TERMINAL || depth >= g.path_depth) {
         const int kind = expanded == PUCT_NODE_EXPANDED_TERMINAL ? PUCT_SELECT_TERMINAL : PUCT_SELECT_DEPTH_LIMIT;
@@ -508,24 +485,28 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
         }
         return;
     }
+    if (expanded == 0) {
+        // No edge to claim, so the widening limit stays what it is at a count of 1: the first of these traversals get the
+        // tickets that are left, the others find the node's children being created.
+        const int allowed = allowed_children(g.c_pw, 0.5f, 1, legal, 1.0f);   // (1 to any power is 1)
+        if (lane < kTrav && ((members >> lane) & 1ull)) {
+            const int slot = tickets + __popcll(members & lanes_below(lane));
+            const bool with_ticket = slot < allowed;
+            s.sel[lane] = with_ticket ? pack_sel(PUCT_SELECT_EXPAND, node, slot) : pack_sel(PUCT_SELECT_BUSY, node, 0);
+            s.len[lane] = with_ticket ? depth + 1 : 0;
+            s.claims[lane] = depth;
+            next[lane] = -1;
+        }
+        const int left = allowed - tickets > 0 ? allowed - tickets : 0;
+        if (lane == 0 && left > 0) g.info[nrow].tickets = tickets + (n_members < left ? n_members : left);
+        return;
+    }
     edges_scored += (uint32_t)expanded;
 
-    EdgeSet<kSlices> all;
     int total = 0;
 #pragma unroll
-    for (int i = 0; i < kSlices; ++i) {
-        const Edge e = loaded[i];
-        const bool valid = lane + i * kWave < expanded;
-        all.q[i] = valid && e.n > 0 ? e.w / (float)e.n : 0.0f;
-        all.cp[i] = g.cpuct * e.prior;
-        all.link[i] = all.link_loaded[i] = e.link;
-        all.den[i] = e.n + (int)(e.link & 0xFFu) + 1;
-        all.eid[i] = valid ? lane + i * kWave : -1;
-        total += valid ? all.den[i] - 1 : 0;
-    }
+    for (int i = 0; i < kSlices; ++i) total += lane + i * kWave < expanded ? loaded[i].n + (int)(loaded[i].link & 0xFFu) : 0;
     total = wave_sum(total);
-    int tickets = ni.tickets;
-    const int legal = ni.legal_turn & 0xFFFF, n_members = __popcll(members);
 
     // Every one of these traversals takes the same edge: all of them at once, a traversal per lane.
     auto take_all = [&](uint32_t link, int eid) {
@@ -547,45 +528,59 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
     // No expansion ticket is to be had here however many of these traversals have claimed: the widening limit grows with
     // the claims, and its largest value, the one the last of them sees, does not exceed the children there are.
     const auto no_ticket_for_anyone = [&] {
-        if (expanded < 1) return false;
         if (expanded >= legal || (expanded == 1 && g.c_pw == 0.0f)) return true;   // (the limit does not exceed the legal moves)
         const int eff_last = total + n_members - 1 > 1 ? total + n_members - 1 : 1;
-        return allowed_children(g.c_pw, g.alpha_pw, eff_last, sqrtf((float)eff_last), legal) <= expanded;
+        return allowed_children(g.c_pw, g.alpha_pw, eff_last, legal) <= expanded;
     };
 
     // decide_in_row's terms: every edge leads to a node and has a finite score
     const auto fit_for_row = [&](const EdgeSet<1> &e) {
         const int child = (int)(e.link[0] >> 8);
-        return __ballot(e.eid[0] >= 0 && !(child > 0 && child < g.max_nodes && fabsf(e.q[0]) < 1e30f && fabsf(e.cp[0]) < 1e30f && e.den[0] > 0)) == 0;
+        return __ballot(e.eid[0] >= 0 && !(child > 0 && child < g.max_nodes && fabsf(e.q[0]) < 1e30f && prow_cp_fits(e.cp[0]) && e.den[0] > 0)) == 0;
     };
-    // Several traversals on a node with many edges: most edges cannot come first for any of them.  While these
-    // traversals decide, sqrt(parent) only grows (by their own claims) and an edge's claims only grow, and every
-    // operation of the score is monotonic, so an edge's score stays below its score at the largest sqrt(parent) and
-    // its present claims, and the best edge's score stays above the largest score at the present sqrt(parent) with
-    // all of these traversals' claims on it.  Edges whose upper bound is below that lower bound are out; when at
-    // most 64 remain they move to one edge per lane, and a decision costs one division instead of one per 64 edges.
+    const auto slot_of_edge = [&](EdgeSet<1> &e, int n, float w, float cp, uint32_t link, int eid) {
+        e = EdgeSet<1>{{eid >= 0 && n > 0 ? w / (float)n : 0.0f}, {cp}, {n + (int)(link & 0xFFu) + 1}, {link}, {link}, {eid}};
+    };
+    // Most edges of a wide node cannot come first for any of these traversals.  While they decide, sqrt(parent) only
+    // grows (by their own claims) and an edge's claims only grow, and every operation of the score is monotonic, so an
+    // edge's score stays below its score at the largest sqrt(parent) and its present claims, and the best edge's score
+    // stays above the largest score at the present sqrt(parent) with all of these traversals' claims on it.  Edges whose
+    // upper bound is below that lower bound are out, and a decision costs one division instead of one per 64 edges.  The
+    // bounds are worked out with the hardware's reciprocals and roots, each right to an ulp: both are moved apart by 2^-18
+    // of |q| + u, more than four times what the roundings of the bound and of the score come to (the last steps of
+    // subnormal scores: 1e-30).  With the score's own divisions this pass took 2700 clocks a node, more than half of what
+    // sixteen decisions do.
     // Returns how many remain if they are in `few` now, 0 if they are not, -1 if all is decided.
     EdgeSet<1> few{{0.0f}, {0.0f}, {1}, {0u}, {0u}, {-1}};
     const auto keep_the_best = [&](auto slices) -> int {
         constexpr int NS = decltype(slices)::value;
+        constexpr float kApart = 0x1p-18f;
         const int now = total > 1 ? total : 1, then = total + n_members > 1 ? total + n_members : 1;
-        const float sqrt_now = sqrtf((float)now), sqrt_then = sqrtf((float)then);
-        uint32_t low = 0, high[NS];
+        const float sqrt_low = __builtin_amdgcn_sqrtf((float)now) * (1.0f - kApart), sqrt_high = __builtin_amdgcn_sqrtf((float)then) * (1.0f + kApart);
+        float low = -FLT_MAX, high[NS];
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
-            const uint32_t l = all.eid[i] >= 0 ? score_image(edge_score(all, i, sqrt_now, n_members)) : 0u;
-            high[i] = all.eid[i] >= 0 ? score_image(edge_score(all, i, sqrt_then, 0)) : 0u;
-            low = l > low ? l : low;
+            const Edge &e = loaded[i];
+            const bool valid = lane + i * kWave < expanded;
+            const float q = e.n > 0 ? e.w * __builtin_amdgcn_rcpf((float)e.n) : 0.0f, cp = g.cpuct * e.prior;
+            const int den = e.n + (int)(e.link & 0xFFu) + 1;
+            const float l = __builtin_fmaf(cp * sqrt_low, __builtin_amdgcn_rcpf((float)(den + n_members)), __builtin_fmaf(-kApart, fabsf(q), q));
+            const float h = __builtin_fmaf(cp * sqrt_high, __builtin_amdgcn_rcpf((float)den), __builtin_fmaf(kApart, fabsf(q), q));
+            low = valid && l > low ? l : low;   // (a NaN gives no bound)
+            high[i] = h;
         }
-        low = wave_max_u32(low);
-        if (low == 0) return 0;
+        const uint32_t low_bits = __float_as_uint(low);   // the largest of the lanes', by its order-preserving image
+        const uint32_t top = wave_max_u32(low_bits ^ ((uint32_t)((int32_t)low_bits >> 31) | 0x80000000u));
+        low = __uint_as_float((top & 0x80000000u) ? top ^ 0x80000000u : ~top);
+        if (!(low > -FLT_MAX)) return 0;
+        low -= 1e-30f;
         int kept = 0, place[NS];
         uint64_t in_slice[NS];
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
-            const uint64_t mask = __ballot(high[i] >= low);
+            const uint64_t mask = __ballot(lane + i * kWave < expanded && !(high[i] < low));
             in_slice[i] = mask;
-            place[i] = ((mask >> lane) & 1ull) ? kept + __popcll(mask & lanes_below(lane)) : -1;
+            place[i] = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, (uint32_t)kept));
             kept += __popcll(mask);
         }
         // One edge left and no expansion ticket to be had: every one of these traversals takes that edge.
@@ -594,7 +589,7 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
             for (int i = 0; i < NS; ++i)
                 if (in_slice[i] != 0) {
                     const int at = __builtin_ctzll(in_slice[i]);
-                    take_all((uint32_t)__builtin_amdgcn_readlane((int)all.link[i], at), at + i * kWave);
+                    take_all((uint32_t)__builtin_amdgcn_readlane((int)loaded[i].link, at), at + i * kWave);
                 }
             return -1;
         }
@@ -602,80 +597,72 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
         if (kept <= kRow) {   // through LDS into the first row, in one go
 #pragma unroll
             for (int i = 0; i < NS; ++i)
-                if (place[i] >= 0) {
-                    *reinterpret_cast<int4 *>(stage + 4 * place[i]) = make_int4(__float_as_int(all.q[i]), __float_as_int(all.cp[i]), all.den[i], (int)all.link[i]);
-                    stage[4 * kRow + place[i]] = all.eid[i];
+                if (__builtin_amdgcn_inverse_ballot_w64(in_slice[i])) {
+                    *reinterpret_cast<int4 *>(stage + 4 * place[i]) = make_int4(loaded[i].n, __float_as_int(loaded[i].w), __float_as_int(loaded[i].prior), (int)loaded[i].link);
+                    stage[4 * kRow + place[i]] = lane + i * kWave;
                 }
             wave_lds_fence();
-            if (lane < kept) {
-                const int4 v = *reinterpret_cast<const int4 *>(stage + 4 * lane);
-                few = EdgeSet<1>{{__int_as_float(v.x)}, {__int_as_float(v.y)}, {v.z}, {(uint32_t)v.w}, {(uint32_t)v.w}, {stage[4 * kRow + lane]}};
-            }
+            int4 v = make_int4(0, 0, 0, 0);
+            int eid = -1;
+            if (lane < kept) v = *reinterpret_cast<const int4 *>(stage + 4 * lane), eid = stage[4 * kRow + lane];
+            slot_of_edge(few, v.x, __int_as_float(v.y), g.cpuct * __int_as_float(v.z), (uint32_t)v.w, eid);
             wave_lds_fence();
         } else {
             if (NS == 1 || kept > kWave) return 0;
+            int field[5];
 #pragma unroll
             for (int f = 0; f < 5; ++f) {
 #pragma unroll
                 for (int i = 0; i < NS; ++i)
-                    if (place[i] >= 0)
-                        stage[place[i]] = f == 0 ? __float_as_int(all.q[i]) : f == 1 ? __float_as_int(all.cp[i]) : f == 2 ? all.den[i]
-                                        : f == 3 ? (int)all.link[i] : all.eid[i];
+                    if (__builtin_amdgcn_inverse_ballot_w64(in_slice[i]))
+                        stage[place[i]] = f == 0 ? loaded[i].n : f == 1 ? __float_as_int(loaded[i].w) : f == 2 ? __float_as_int(loaded[i].prior)
+                                        : f == 3 ? (int)loaded[i].link : lane + i * kWave;
                 wave_lds_fence();
-                const int v = lane < kept ? stage[lane] : 0;
+                field[f] = lane < kept ? stage[lane] : f == 4 ? -1 : 0;
                 wave_lds_fence();
-                if (f == 0) few.q[0] = __int_as_float(v);
-                if (f == 1) few.cp[0] = __int_as_float(v);
-                if (f == 2) few.den[0] = lane < kept ? v : 1;
-                if (f == 3) few.link[0] = few.link_loaded[0] = (uint32_t)v;
-                if (f == 4) few.eid[0] = lane < kept ? v : -1;
             }
+            slot_of_edge(few, field[0], __int_as_float(field[1]), g.cpuct * __int_as_float(field[2]), (uint32_t)field[3], field[4]);
         }
         return kept;
     };
 
-    const int allowed_now = expanded == 0 ? allowed_children(g.c_pw, g.alpha_pw, total > 1 ? total : 1, sqrtf((float)(total > 1 ? total : 1)), legal) : 0;
-    if (allowed_now > 0) {
-        // No edge to claim, so the widening limit stays as it is: the first of these traversals get the tickets that are
-        // left, the others find the node's children being created.
-        if (lane < kTrav && ((members >> lane) & 1ull)) {
-            const int slot = tickets + __popcll(members & lanes_below(lane));
-            const bool with_ticket = slot < allowed_now;
-            s.sel[lane] = with_ticket ? pack_sel(PUCT_SELECT_EXPAND, node, slot) : pack_sel(PUCT_SELECT_BUSY, node, 0);
-            s.len[lane] = with_ticket ? depth + 1 : 0;
-            s.claims[lane] = depth;
-            next[lane] = -1;
+    int edges = 0;   // how many there are in `few`, one per lane
+    if (expanded > kWave) {
+        edges = keep_the_best(std::integral_constant<int, kSlices>{});
+    } else if (n_members >= 3) {
+        if (expanded > 1) {
+            edges = keep_the_best(std::integral_constant<int, 1>{});
+        } else if (no_ticket_for_anyone()) {   // a node's only edge is taken whatever its score
+            take_all((uint32_t)__builtin_amdgcn_readlane((int)loaded[0].link, 0), 0);
+            edges = -1;
         }
-        const int left = allowed_now - tickets > 0 ? allowed_now - tickets : 0;
-        tickets += n_members < left ? n_members : left;
-    } else {
-        int edges = 0;   // how many there are in `few`, one per lane
-        if (n_members >= 3) {
-            if (expanded > kWave) {
-                edges = keep_the_best(std::integral_constant<int, kSlices>{});
-            } else if (expanded > 1) {
-                edges = keep_the_best(std::integral_constant<int, 1>{});
-            } else if (no_ticket_for_anyone()) {   // a node's only edge is taken whatever its score
-                take_all((uint32_t)__builtin_amdgcn_readlane((int)all.link[0], 0), 0);
-                edges = -1;
-            }
-        }
-        const bool only_one = edges == 1;
-        if (edges == 0 && expanded <= kWave) {
-            few = EdgeSet<1>{{all.q[0]}, {all.cp[0]}, {all.den[0]}, {all.link[0]}, {all.link_loaded[0]}, {all.eid[0]}};
-            edges = expanded;
-        }
-        if (edges >= 1 && edges <= kRow && fit_for_row(few)) {
-            decide_in_row(g, s, paths, next, row, few, node, (uint32_t)members, depth, lane, expanded, legal, total, tickets, edges == 1);
-        } else if (edges > 0 || expanded == 0) {
-            decide_in_turn<1>(g, s, paths, next, few, node, members, depth, lane, expanded, legal, total, tickets, only_one);
-            if (few.eid[0] >= 0 && few.link[0] != few.link_loaded[0]) row[few.eid[0]].link = few.link[0];
-        } else if (edges == 0) {
-            decide_in_turn<kSlices>(g, s, paths, next, all, node, members, depth, lane, expanded, legal, total, tickets);
+    }
+    const bool only_one = edges == 1;
+    if (edges == 0 && expanded <= kWave) {
+        slot_of_edge(few, loaded[0].n, loaded[0].w, g.cpuct * loaded[0].prior, loaded[0].link, lane < expanded ? lane : -1);
+        edges = expanded;
+    }
+    if (edges >= 1 && edges <= kRow && fit_for_row(few)) {
+        decide_in_row(g, s, paths, next, row, few, node, (uint32_t)members, depth, lane, expanded, legal, total, tickets, edges == 1);
+    } else if (edges > 0) {
+        decide_in_turn<1>(g, s, paths, next, few, node, members, depth, lane, expanded, legal, total, tickets, only_one);
+        if (few.eid[0] >= 0 && few.link[0] != few.link_loaded[0]) row[few.eid[0]].link = few.link[0];
+    } else if (edges == 0) {
+        EdgeSet<kSlices> all;
 #pragma unroll
-            for (int i = 0; i < kSlices; ++i)
-                if (all.link[i] != all.link_loaded[i]) row[lane + i * kWave].link = all.link[i];
+        for (int i = 0; i < kSlices; ++i) {
+            const Edge &e = loaded[i];
+            const bool valid = lane + i * kWave < expanded;
+            all.q[i] = valid && e.n > 0 ? e.w / (float)e.n : 0.0f;
+            all.cp[i] = g.cpuct * e.prior;
+            all.link[i] = all.link_loaded[i] = e.link;
+            all.den[i] = e.n + (int)(e.link & 0xFFu) + 1;
+            all.eid[i] = valid ? lane + i * kWave : -1;
         }
+        decide_in_turn<kSlices>(g, s, paths, next, all, node, members, depth, lane, expanded, legal, total, tickets);
+#pragma unroll
+        for (int i = 0; i < kSlices; ++i)
+            if (all.link[i] != all.link_loaded[i]) row[lane + i * kWave].link = all.link[i];
     }
     if (lane == 0 && tickets != ni.tickets) g.info[nrow].tickets = tickets;
 }

@@ -13,6 +13,19 @@ SOURCE = """
 float score(int edge, float q, float cp, int den, float sqrt_parent) {
     return prow_score(prow_q(edge, q), prow_cp(edge, cp), sqrt_parent, prow_den(edge, den));
 }
+/* How many of `count` quotients differ from the division's in any bit, with a reciprocal that is `ulps` off the rounded one. */
+int quotients_that_differ(const float *num, const int *den, int count, int ulps) {
+    int wrong = 0;
+    for (int i = 0; i < count; ++i) {
+        union { float f; int i; } r, a, b;
+        r.f = 1.0f / (float)den[i];
+        r.i += ulps;
+        a.f = prow_quotient(num[i], (float)den[i], r.f);
+        b.f = num[i] / (float)den[i];
+        wrong += a.i != b.i;
+    }
+    return wrong;
+}
 """
 INT_MIN = -2**31
 
@@ -22,7 +35,7 @@ def row(tmp_path_factory):
     at = tmp_path_factory.mktemp("puct_row")
     (at / "row.c").write_text(SOURCE)
     lib = str(at / "row.so")
-    subprocess.check_call(["gcc", "-std=c99", "-O2", "-Wall", "-Werror", "-ffp-contract=off", "-shared", "-fPIC", "-I" + CSRC, "-o", lib, str(at / "row.c")])
+    subprocess.check_call(["gcc", "-std=c99", "-O2", "-Wall", "-Werror", "-ffp-contract=off", "-shared", "-fPIC", "-I" + CSRC, "-o", lib, str(at / "row.c"), "-lm"])
     so, f = ctypes.CDLL(lib), ctypes.c_float
     so.score.argtypes, so.score.restype = [ctypes.c_int, f, f, ctypes.c_int, f], f
     return so
@@ -37,3 +50,17 @@ def test_a_lane_without_an_edge_is_finite_and_last(row, den):
             s = row.score(0, junk, junk, den, sqrt_parent)
             assert np.isfinite(s) and s == np.float32(-np.finfo(np.float32).max), (den, junk, sqrt_parent)
             assert s < lowest_edge
+
+
+@pytest.mark.parametrize("ulps", [-1, 0, 1])
+def test_the_short_division_is_the_division(row, ulps):
+    """Every bit, over the declared range of operands (cp of prow_cp_fits times a root of up to 2^16), small and large counts."""
+    rng = np.random.default_rng(5 + ulps)
+    for low, high in ((1, 64), (1, 70000), (1, 2**24), (2**24, 2**31 - 64)):
+        n = 400000
+        num = np.exp(rng.uniform(np.log(1e-20), np.log(1e15 * 65536), n)).astype(np.float32)
+        num[: n // 2] = rng.uniform(0, 300, n // 2).astype(np.float32)
+        num[: n // 8] = 0.0
+        den = rng.integers(low, high, n).astype(np.int32)
+        p = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+        assert row.quotients_that_differ(p(num), p(den), n, ulps) == 0
