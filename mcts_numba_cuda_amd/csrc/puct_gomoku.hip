@@ -65,15 +65,20 @@ struct LoopArgs {
 
 // What a tree's workgroup hands to its evaluator workgroups, step by step: the non-terminal children the step created.
 struct EvalRequests {
-    int tag;     // step + 1 once the step's entries are complete; -1 when the search is over
+    unsigned long long tag;   // posted() once the step's entries are complete; kSearchOver when there are no more
     int done;    // entries the evaluators have worked off since the search began
     int abort;   // a bounded wait gave up: everybody leaves
-    int n;       // entries of the step
     int child[kMaxWavesPerBlock];       // node to evaluate, -1 = nothing to do for this entry
     uint64_t hash[kMaxWavesPerBlock];   // its position's hash
     int xcc[1 + 8];                     // XCD that the tree's workgroup [0] and its evaluators [1..] run on, -1 = not known yet
 };
 constexpr int kMaxEvaluators = 8;
+// All that an evaluator needs to know before it can ask for a step's entries, in the word that it waits for: the step, how many
+// entries there are (0..16) and the first's node (20 bits; the others follow it).
+constexpr unsigned long long kSearchOver = ~0ull;
+__device__ __forceinline__ unsigned long long posted(int step, int n, int first) {
+    return (uint32_t)(step + 1) | (unsigned long long)n << 32 | (unsigned long long)first << 40;
+}
 static_assert(sizeof(EvalRequests::xcc) == sizeof(int) * (1 + kMaxEvaluators), "one entry per workgroup of a tree");
 
 __device__ __forceinline__ int my_xcc() { return (int)(__builtin_amdgcn_s_getreg(6164) & 0xfu); }   // HW_REG_XCC_ID, bits 3:0
@@ -188,6 +193,20 @@ __device__ __forceinline__ NodeInfo load_info(const NodeInfo *p) {
 }
 __device__ __forceinline__ uint64_t lanes_below(int lane) { return (1ull << lane) - 1ull; }
 
+// psyn_gamma_round: two of its three logarithms only say whether the candidate is accepted.  The hardware's, within 6e-6 of them
+// together (none is above 17), say so unless the two sides are closer than 2^-15, and then the exact ones do.
+__device__ __forceinline__ int gamma_round(float alpha, uint64_t key, int round, float *x) {
+    constexpr float kLn2 = 0.693147181f;
+    float u2;
+    int small;
+    psyn_gamma_candidate(alpha, key, round, x, &u2, &small);
+    const float bound = small ? -*x : (alpha - 1.0f) * (__builtin_amdgcn_logf(*x) * kLn2);
+    const float room = bound - __builtin_amdgcn_logf(u2) * kLn2;
+    int accepted = room > 0.0f;
+    if (!(fabsf(room) > 0x1p-15f)) accepted = psyn_gamma_accepts(alpha, *x, u2, small);
+    return accepted;
+}
+
 // Priors of a new node: one Gamma weight per legal cell, prior = weight / sum, edge slots in descending weight order
 // (ties: smaller cell first), so that progressive widening opens the most promising moves first.  Writes the whole
 // record of every legal slot (no visits, no child, nothing in flight) and the slot's cell.  All 64 lanes must call it
@@ -209,7 +228,7 @@ __device__ void write_priors(const LoopArgs &g, int tree, int node, const uint32
     uint64_t key = i < kPer ? psyn_cell_key(board_hash, lane + i * kWave) : 0;
     while (__ballot(i < kPer) != 0) {
         float x;
-        const int ok = psyn_gamma_round(g.dirichlet_alpha, key, round, &x);
+        const int ok = gamma_round(g.dirichlet_alpha, key, round, &x);
         if (i < kPer) {
             if (ok || round == PSYN_GAMMA_ROUNDS - 1) {
                 const uint32_t weight = psyn_weight_key(x, lane + i * kWave);
@@ -485,20 +504,22 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
         }
         return;
     }
-    if (expanded == 0) {
-        // No edge to claim, so the widening limit stays what it is at a count of 1: the first of these traversals get the
-        // tickets that are left, the others find the node's children being created.
-        const int allowed = allowed_children(g.c_pw, 0.5f, 1, legal, 1.0f);   // (1 to any power is 1)
+    // The first of these traversals get the tickets that are left under a limit, the others find the node's children being
+    // created.
+    const auto give_tickets = [&](int allowed) {
         if (lane < kTrav && ((members >> lane) & 1ull)) {
-            const int slot = tickets + __popcll(members & lanes_below(lane));
+            const int slot = expanded + tickets + __popcll(members & lanes_below(lane));
             const bool with_ticket = slot < allowed;
             s.sel[lane] = with_ticket ? pack_sel(PUCT_SELECT_EXPAND, node, slot) : pack_sel(PUCT_SELECT_BUSY, node, 0);
             s.len[lane] = with_ticket ? depth + 1 : 0;
             s.claims[lane] = depth;
             next[lane] = -1;
         }
-        const int left = allowed - tickets > 0 ? allowed - tickets : 0;
+        const int left = allowed - expanded - tickets > 0 ? allowed - expanded - tickets : 0;
         if (lane == 0 && left > 0) g.info[nrow].tickets = tickets + (n_members < left ? n_members : left);
+    };
+    if (expanded == 0) {   // no edge to claim, so the widening limit stays what it is at a count of 1
+        give_tickets(allowed_children(g.c_pw, 0.5f, 1, legal, 1.0f));   // (1 to any power is 1)
         return;
     }
     edges_scored += (uint32_t)expanded;
@@ -507,6 +528,13 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
 #pragma unroll
     for (int i = 0; i < kSlices; ++i) total += lane + i * kWave < expanded ? loaded[i].n + (int)(loaded[i].link & 0xFFu) : 0;
     total = wave_sum(total);
+    if (expanded != 1 || g.c_pw != 0.0f) {   // as many tickets as traversals: no edge is claimed, and the limit stays too
+        const int allowed = allowed_children(g.c_pw, g.alpha_pw, total > 1 ? total : 1, legal);
+        if (expanded + tickets + n_members <= allowed) {
+            give_tickets(allowed);
+            return;
+        }
+    }
 
     // Every one of these traversals takes the same edge: all of them at once, a traversal per lane.
     auto take_all = [&](uint32_t link, int eid) {
@@ -880,7 +908,6 @@ __global__ __launch_bounds__(kWave) void init_kernel(const LoopArgs g, const uin
         rq.tag = 0;
         rq.done = 0;
         rq.abort = 0;
-        rq.n = 0;
         for (int &x : rq.xcc) x = -1;
     }
     if (n_legal > 0) write_priors(g, tree, 0, board, lane, psyn_board_hash(psyn_tree_seed(g.seed, tree), board), n_legal);
@@ -967,7 +994,7 @@ struct EvalLds {
     uint32_t keys[kEvalNodes][kEvalParts][kWave];
     unsigned long long weight[kEvalNodes][kEvalParts];
     int legal[kEvalNodes][kEvalParts];
-    int tag;
+    unsigned long long tag[2];   // by parity of the step
 };
 __device__ __forceinline__ int eval_nodes_at_once() { return (int)blockDim.x / (kWave * kEvalParts); }   // (2 to 4: 8 to 16 wavefronts)
 
@@ -990,31 +1017,38 @@ __device__ __forceinline__ void sort64_descending(uint32_t &v, int lane) {
     if constexpr (SIZE < kWave) sort64_descending<2 * SIZE>(v, lane);
 }
 
-__device__ __forceinline__ int poll_word(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <class T>
+__device__ __forceinline__ T poll_word(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// Entry `index` of the step (none if it is not below n) by four wavefronts, `part` = 0..3; the whole workgroup must call it.
-__device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index, int n, int group, int part, int lane) {
+// Entry `index` of the step (none if it is not below n), whose node is first_node + index, by four wavefronts, `part` = 0..3; the whole workgroup must call it.
+__device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index, int n, int first_node, int group, int part, int lane) {
     const EvalRequests &rq = g.requests[tree];
-    const int child = index < n ? rq.child[index] : -1;
-    const bool active = child > 0;
     const size_t trow = (size_t)tree * g.max_nodes;
+    int child = -1;
+    uint32_t w = 0u;
+    uint64_t hash = 0;
+    if (index < n) {   // all that there is to know about the entry in one round trip
+        child = rq.child[index];
+        hash = rq.hash[index];
+        if (lane < kBoardWords) w = g.board[(trow + first_node + index) * kBoardWords + lane];
+    }
+    const bool active = child > 0;
     uint32_t key = 0;
     if (active) {
         const int cell = part * kWave + lane;
-        const uint32_t w = lane < kBoardWords ? g.board[(trow + child) * kBoardWords + lane] : 0u;
         // words of the lane's cell: the same for each half of the wavefront
         uint32_t plus = (uint32_t)__builtin_amdgcn_readlane((int)w, 2 * part), minus = (uint32_t)__builtin_amdgcn_readlane((int)w, 8 + 2 * part);
         const uint32_t plus_hi = (uint32_t)__builtin_amdgcn_readlane((int)w, 2 * part + 1);
         const uint32_t minus_hi = (uint32_t)__builtin_amdgcn_readlane((int)w, 8 + 2 * part + 1);
         if (lane >= 32) plus = plus_hi, minus = minus_hi;
         const bool legal = cell < g.cells && !(((plus | minus) >> (lane & 31)) & 1u);
-        const uint64_t stream = psyn_cell_key(rq.hash[index], cell);
+        const uint64_t stream = psyn_cell_key(hash, cell);
         // One round of the sampler for every cell, then, as the rounds of a cell are independent numbers of its stream, several
         // at once for the cells that are left: 1, 2 or 4 lanes a cell, the first round that accepts counts.  (Round after
         // round the wavefront ran five for its unluckiest lane, 500 of its 700 instructions: 12.8 us a step instead of 11.85 at
         // 16 trees x 16 traversals, four evaluators.)
         float x;
-        bool pending = legal && !psyn_gamma_round(g.dirichlet_alpha, stream, 0, &x);
+        bool pending = legal && !gamma_round(g.dirichlet_alpha, stream, 0, &x);
         if (legal && !pending) key = psyn_weight_key(x, cell);
         uint64_t left = __ballot(pending);
         for (int round = 1; left != 0;) {
@@ -1025,7 +1059,7 @@ __device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index
             const int owner = __builtin_amdgcn_ds_bpermute((lane >> shift) << 2, nth) << 2;
             const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(owner, (int)(uint32_t)stream), hi = (uint32_t)__builtin_amdgcn_ds_bpermute(owner, (int)(uint32_t)(stream >> 32));
             const int mine = round + (lane & ((1 << shift) - 1)), first_lane = (rank << shift) & (kWave - 1);   // (of the cell, if it is left)
-            const int ok = psyn_gamma_round(g.dirichlet_alpha, ((uint64_t)hi << 32) | lo, mine, &x);
+            const int ok = gamma_round(g.dirichlet_alpha, ((uint64_t)hi << 32) | lo, mine, &x);
             const uint64_t accepted = __ballot((ok && mine < PSYN_GAMMA_ROUNDS) || mine == PSYN_GAMMA_ROUNDS - 1);
             const uint32_t of_cell = (uint32_t)(accepted >> first_lane) & ((1u << (1 << shift)) - 1u);
             const float gamma = __int_as_float(__builtin_amdgcn_ds_bpermute((first_lane + (of_cell ? __builtin_ctz(of_cell) : 0)) << 2, __float_as_int(x)));
@@ -1068,32 +1102,33 @@ __device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index
 __device__ void evaluator_loop(const LoopArgs &g, EvalLds &L, int tree, int helper, int wave, int lane) {
     EvalRequests &rq = g.requests[tree];
     if (threadIdx.x == 0) __hip_atomic_store(&rq.xcc[1 + helper], my_xcc(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int step = 0;; ++step) {
+    int seen = 0;   // the last step's tag (steps of which this evaluator had nothing to do may pass it by)
+    for (int turn = 0;; turn ^= 1) {
         if (threadIdx.x == 0) {
             const uint64_t start = wall_clock64();
-            int tag;
-            while ((tag = poll_word(&rq.tag)) >= 0 && tag <= step) {
+            unsigned long long tag;
+            while ((int)(uint32_t)(tag = poll_word(&rq.tag)) >= 0 && (int)(uint32_t)tag <= seen) {
                 if (poll_word(&rq.abort) != 0 || wall_clock64() - start > kWaitTicks) {
                     __hip_atomic_store(&rq.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    tag = -1;
+                    tag = kSearchOver;
                     break;
                 }
                 __builtin_amdgcn_s_sleep(2);
             }
-            L.tag = tag;
+            L.tag[turn] = tag;
         }
         if (wave == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");   // for all of the workgroup's wavefronts, which share an L1
         __syncthreads();
-        const int tag = L.tag;
-        __syncthreads();
-        if (tag < 0) return;
-        const int n = rq.n;
+        const unsigned long long tag = L.tag[turn];
+        seen = __builtin_amdgcn_readfirstlane((int)(uint32_t)tag);
+        if (seen < 0) return;
+        const int n = __builtin_amdgcn_readfirstlane((int)(tag >> 32) & 0xFF), first_node = __builtin_amdgcn_readfirstlane((int)(tag >> 40));
         int worked_off = 0;
         // (the step's nodes are dealt to the evaluators one by one, so that a step with few of them keeps all busy)
         const int at_once = eval_nodes_at_once();
         for (int first = helper; first < n; first += at_once * g.evaluators) {
             const int group = wave / kEvalParts;
-            evaluate_node(g, L, tree, first + group * g.evaluators, n, group, wave & (kEvalParts - 1), lane);
+            evaluate_node(g, L, tree, first + group * g.evaluators, n, first_node, group, wave & (kEvalParts - 1), lane);
             for (int i = 0; i < at_once; ++i) worked_off += first + i * g.evaluators < n ? 1 : 0;
         }
         // every wavefront's stores have reached the L2 before one of them reports; the release pushes them on
@@ -1175,7 +1210,6 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
         phase_barrier(farm);   // the claims of the selection and the new nodes are in memory
         if (s.gave_up) break;
         if (farm && threadIdx.x == 0) {   // ... and the evaluators may start on this step's nodes
-            rq.n = s.requests;
             s.requested += s.requests;
             if (!same_l2 && !g.agent_fences) {
                 same_l2 = true;
@@ -1184,9 +1218,8 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
             // The phase barrier above has the step's nodes and requests in the L2.  Evaluators on the same XCD read them
             // there (their acquire drops what their L1 holds); for any other, or one not heard of yet, the L2 is written
             // back first, which is the expensive part of an agent-scope release.
-            if (same_l2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // rq.n
-            else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            __hip_atomic_store(&rq.tag, step + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!same_l2) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            __hip_atomic_store(&rq.tag, posted(step, s.requests, s.node_count - s.requests), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (wave == 0) t2 = wall_clock64();
         backup_phase(g, s, paths, tree, wave, lane, n_waves);
@@ -1203,7 +1236,7 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
         if (threadIdx.x == 0) wait_for_evaluators(rq, s);
         __syncthreads();
     }
-    if (farm && threadIdx.x == 0) __hip_atomic_store(&rq.tag, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (farm && threadIdx.x == 0) __hip_atomic_store(&rq.tag, kSearchOver, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     state_to_memory(g, s, paths, tree, n_waves);
     work.to_memory(g, tree, lane);
 }

@@ -56,22 +56,28 @@ PSYN_FN float psyn_unit(uint32_t h) { return ((float)(h >> 9) + 0.5f) * (1.0f / 
  * accepted.  The acceptance tests are taken in the log domain (log u2 <= -x, resp. log u2 <= (alpha - 1) log x).
  * Single precision throughout (a weight keeps 15 mantissa bits) and without a branch: a wavefront whose lanes take
  * different sides of the sampler runs the same instructions. */
-PSYN_FN int psyn_gamma_round(float alpha, uint64_t key, int round, float *x) {
+PSYN_FN void psyn_gamma_candidate(float alpha, uint64_t key, int round, float *x, float *u2, int *small) {
     const float b = 1.0f + alpha * 0.36787944117f; /* 1 + alpha / e */
     const float inv_alpha = 1.0f / alpha;
     const uint64_t h = psyn_mix64(key + (uint64_t)round);
     const float u1 = psyn_unit((uint32_t)(h >> 32));
-    const float log_u2 = detm_logf(psyn_unit((uint32_t)h));
     const float p = b * u1;
-    const int small = p <= 1.0f;
-    float t = small ? p : (b - p) * inv_alpha;
+    *u2 = psyn_unit((uint32_t)h);
+    *small = p <= 1.0f;
+    float t = *small ? p : (b - p) * inv_alpha;
     t = t < 1.17549435e-38f ? 1.17549435e-38f : t;
     const float log_t = detm_logf(t);
-    const float x_small = detm_expf(log_t * inv_alpha);
-    const float x_large = -log_t; /* > 1 on this side: b - p < alpha / e */
-    const float bound = small ? -x_small : (alpha - 1.0f) * detm_logf(small ? 2.0f : x_large);
-    *x = small ? x_small : x_large;
-    return log_u2 <= bound;
+    *x = *small ? detm_expf(log_t * inv_alpha) : -log_t; /* -log_t > 1 on its side: b - p < alpha / e */
+}
+PSYN_FN int psyn_gamma_accepts(float alpha, float x, float u2, int small) {
+    const float bound = small ? -x : (alpha - 1.0f) * detm_logf(small ? 2.0f : x);
+    return detm_logf(u2) <= bound;
+}
+PSYN_FN int psyn_gamma_round(float alpha, uint64_t key, int round, float *x) {
+    float u2;
+    int small;
+    psyn_gamma_candidate(alpha, key, round, x, &u2, &small);
+    return psyn_gamma_accepts(alpha, *x, u2, small);
 }
 
 #define PSYN_GAMMA_ROUNDS 16 /* the chance of needing more is below 1e-9; the last candidate is taken then */
