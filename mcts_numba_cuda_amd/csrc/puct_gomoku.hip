@@ -138,34 +138,46 @@ __device__ __forceinline__ bool makes_five(const uint32_t *mine, int cell, int m
     return __ballot(1 + __builtin_clz(~(line << 27)) + __builtin_ctz(~(line >> 6)) == 5) != 0;
 }
 
-// Bitonic sort of the wavefront's 256 keys, largest first: element e = 4 * lane + k lives in v[k] of `lane`.  Partners
-// at element distance 1 and 2 are registers of the same lane; lane distances 1, 2 and 8 are DPP moves, 4 and 16 LDS
-// swizzles (no memory), 32 an LDS permute.
+// This lane's key and that of lane ^ LANE_XOR, in any order, by vector instructions alone: DPP moves (4: the two directions, each to
+// its banks of four lanes), and beyond a row of 16 the swaps of rows and halves, after which one register has the lower partner's
+// key on both sides and the other the upper's.
+struct KeyPair {
+    uint32_t a, b;
+};
 template <int LANE_XOR>
-__device__ __forceinline__ uint32_t from_lane_xor(uint32_t x, int lane) {
-    if (LANE_XOR == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);    // quad_perm [1,0,3,2]
-    if (LANE_XOR == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true);    // quad_perm [2,3,0,1]
-    if (LANE_XOR == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, true);   // row_ror:8
-    if (LANE_XOR == 4) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, 0x101F);                      // bit mode: xor 4
-    if (LANE_XOR == 16) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, 0x401F);                     // bit mode: xor 16
-    return (uint32_t)__builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, (int)x);
+__device__ __forceinline__ KeyPair with_partner(uint32_t x) {
+    if constexpr (LANE_XOR == 1) return {x, (uint32_t)dpp<0xB1>((int)x)};    // quad_perm [1,0,3,2]
+    if constexpr (LANE_XOR == 2) return {x, (uint32_t)dpp<0x4E>((int)x)};    // quad_perm [2,3,0,1]
+    if constexpr (LANE_XOR == 4) {
+        const int up = __builtin_amdgcn_update_dpp((int)x, (int)x, 0x104, 0xF, 0x5, false);            // row_shl:4
+        return {x, (uint32_t)__builtin_amdgcn_update_dpp(up, (int)x, 0x114, 0xF, 0xA, false)};         // row_shr:4
+    }
+    if constexpr (LANE_XOR == 8) return {x, (uint32_t)dpp<0x128>((int)x)};   // row_ror:8
+    if constexpr (LANE_XOR == 16) {
+        const auto v = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return {v[0], v[1]};
+    }
+    const auto v = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return {v[0], v[1]};
 }
+__device__ __forceinline__ uint32_t larger_key(KeyPair p) { return p.a > p.b ? p.a : p.b; }
+__device__ __forceinline__ uint32_t smaller_key(KeyPair p) { return p.a > p.b ? p.b : p.a; }
+
+// Bitonic sort of the wavefront's 256 keys, largest first: element e = 4 * lane + k lives in v[k] of `lane`.  Partners
+// at element distance 1 and 2 are registers of the same lane.
 template <int SIZE, int DIST>
 __device__ __forceinline__ void bitonic_step(uint32_t (&v)[4], int lane) {
-    uint32_t p[4];
-    if (DIST < 4) {
+    KeyPair pair[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) p[k] = v[k ^ DIST];
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) p[k] = from_lane_xor<DIST / 4>(v[k], lane);
+    for (int k = 0; k < 4; ++k) {
+        if constexpr (DIST < 4) pair[k] = {v[k], v[k ^ DIST]};
+        else pair[k] = with_partner<DIST / 4>(v[k]);
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const int e = 4 * lane + k;
         const bool descending = (e & SIZE) == 0, first = (e & DIST) == 0;   // SIZE == 256: every block descends
-        const uint32_t hi = v[k] > p[k] ? v[k] : p[k], lo = v[k] > p[k] ? p[k] : v[k];
-        v[k] = (first == descending) ? hi : lo;
+        v[k] = (first == descending) ? larger_key(pair[k]) : smaller_key(pair[k]);
     }
 }
 template <int SIZE, int DIST>
@@ -983,38 +995,38 @@ extern __shared__ int dynamic_lds[];
 // The priors of a new node are a pure function of its position, and nothing reads them before the next step's
 // selection, so they need not be worked out on the compute unit that owns the tree: the tree's workgroup posts the
 // step's new nodes, goes on with its backup, and picks the results up before the next step.  An evaluator workgroup
-// takes up to four nodes at a time, four wavefronts and one cell per lane each.  A wavefront sorts its 64 keys in registers;
-// the slot of a cell is its place there and the number of larger keys in the three other wavefronts' lists, each a binary
-// search in LDS.  Same priors, bit for bit, as write_priors().  Bound by vector instructions: about 450 a wavefront and
-// node, 1200 when every lane compared its key with all 256 and the sampler ran round after round; four evaluators of 8
-// wavefronts then took longer over a step's sixteen nodes than the tree's own step.
+// takes up to four nodes at a time, four wavefronts and one cell per lane each.  A wavefront sorts its 64 keys in registers,
+// the node's four lists are merged through LDS, and every wavefront stores 64 consecutive slots.  Same priors, bit for bit, as
+// write_priors().  Bound by vector instructions, about 400 a wavefront and node, and by the multiplications of the streams among
+// them.  (1200 when every lane compared its key with all 256 and the sampler ran round after round; with a binary search in the
+// three other lists for each key's slot, bank conflicts and scattered stores made a step 10.40 us, now 10.04, at 16 trees x 16
+// traversals and four evaluators.)
 constexpr int kEvalParts = kEdges / kWave;              // wavefronts per node
 constexpr int kEvalNodes = kTrav / kEvalParts;          // nodes at a time, at most
 struct EvalLds {
-    uint32_t keys[kEvalNodes][kEvalParts][kWave];
+    uint32_t keys[2][kEvalNodes][kEvalParts][kWave];   // sorted by 64, by 128
     unsigned long long weight[kEvalNodes][kEvalParts];
     int legal[kEvalNodes][kEvalParts];
     unsigned long long tag[2];   // by parity of the step
 };
 __device__ __forceinline__ int eval_nodes_at_once() { return (int)blockDim.x / (kWave * kEvalParts); }   // (2 to 4: 8 to 16 wavefronts)
 
-// The wavefront's 64 keys, largest first: a bitonic sort with one key per lane.
+// The wavefront's 64 keys, largest first: a bitonic sort with one key per lane.  SIZE == 64, DIST == 32 alone: a bitonic list.
 template <int SIZE, int DIST>
-__device__ __forceinline__ void sort64_step(uint32_t &v, int lane) {
+__device__ __forceinline__ void sort64_step(uint32_t &v) {
     constexpr auto takes_larger = [] {
         uint64_t m = 0;
         for (int i = 0; i < kWave; ++i) m |= (uint64_t)(((i & DIST) == 0) == ((i & SIZE) == 0)) << i;
         return m;
     }();
-    const uint32_t p = from_lane_xor<DIST>(v, lane);
-    const uint32_t hi = v > p ? v : p, lo = v > p ? p : v;
-    v = __builtin_amdgcn_inverse_ballot_w64(takes_larger) ? hi : lo;
-    if constexpr (DIST > 1) sort64_step<SIZE, DIST / 2>(v, lane);
+    const KeyPair p = with_partner<DIST>(v);
+    v = __builtin_amdgcn_inverse_ballot_w64(takes_larger) ? larger_key(p) : smaller_key(p);
+    if constexpr (DIST > 1) sort64_step<SIZE, DIST / 2>(v);
 }
 template <int SIZE = 2>
-__device__ __forceinline__ void sort64_descending(uint32_t &v, int lane) {
-    sort64_step<SIZE, SIZE / 2>(v, lane);
-    if constexpr (SIZE < kWave) sort64_descending<2 * SIZE>(v, lane);
+__device__ __forceinline__ void sort64_descending(uint32_t &v) {
+    sort64_step<SIZE, SIZE / 2>(v);
+    if constexpr (SIZE < kWave) sort64_descending<2 * SIZE>(v);
 }
 
 template <class T>
@@ -1076,27 +1088,35 @@ __device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index
             L.weight[group][part] = part_sum;
             L.legal[group][part] = part_legal;
         }
-        sort64_descending(key, lane);   // (0: not a legal cell, last)
-        L.keys[group][part][lane] = key;
+        sort64_descending(key);   // (0: not a legal cell, last)
+        L.keys[0][group][part][lane] = key;
     }
     __syncthreads();
-    if (key != 0) {
-        const uint64_t sum = L.weight[group][0] + L.weight[group][1] + L.weight[group][2] + L.weight[group][3];
-        const int n_legal = L.legal[group][0] + L.legal[group][1] + L.legal[group][2] + L.legal[group][3];
-        int larger[kEvalParts - 1] = {};   // keys above this one in the other parts' lists
-        const auto list = [&](int i) -> const uint32_t * { return L.keys[group][(part + 1 + i) & (kEvalParts - 1)]; };
-#pragma unroll
-        for (int d = kWave / 2; d > 0; d >>= 1)
-#pragma unroll
-            for (int i = 0; i < kEvalParts - 1; ++i) larger[i] += list(i)[larger[i] + d - 1] > key ? d : 0;
-        int slot = lane;
-#pragma unroll
-        for (int i = 0; i < kEvalParts - 1; ++i) slot += larger[i] + (list(i)[larger[i]] > key ? 1 : 0);
-        const size_t e = (trow + child) * kEdges + slot;
-        store_edge(g.edges + e, 0, 0.0f, psyn_prior(psyn_key_weight(key), sum, n_legal), 0u);
-        g.action[e] = (uint8_t)(255u - (key & 0xFFu));
+    uint64_t sum = 0;
+    int n_legal = 0;
+    if (active) {   // two lists of 64 to one of 128: the first meets the second from its end, the larger keys stay in front
+        sum = L.weight[group][0] + L.weight[group][1] + L.weight[group][2] + L.weight[group][3];
+        n_legal = L.legal[group][0] + L.legal[group][1] + L.legal[group][2] + L.legal[group][3];
+        const KeyPair p{key, L.keys[0][group][part ^ 1][kWave - 1 - lane]};
+        key = (part & 1) == 0 ? larger_key(p) : smaller_key(p);
+        sort64_step<kWave, kWave / 2>(key);
+        L.keys[1][group][part][lane] = key;
     }
-    __syncthreads();   // the keys are free again
+    __syncthreads();
+    if (active) {   // two lists of 128 to one of 256, and that step's first one between two wavefronts at once
+        const auto &list = L.keys[1][group];
+        const KeyPair near{list[0][lane], list[3][kWave - 1 - lane]}, far{list[1][lane], list[2][kWave - 1 - lane]};
+        const KeyPair p = part < 2 ? KeyPair{larger_key(near), larger_key(far)} : KeyPair{smaller_key(near), smaller_key(far)};
+        key = (part & 1) == 0 ? larger_key(p) : smaller_key(p);
+        sort64_step<kWave, kWave / 2>(key);
+        const size_t e = (trow + child) * kEdges + part * kWave + lane;
+        if (key != 0) {
+            store_edge(g.edges + e, 0, 0.0f, psyn_prior(psyn_key_weight(key), sum, n_legal), 0u);
+            g.action[e] = (uint8_t)(255u - (key & 0xFFu));
+        }
+    }
+    // (the next node's first keys and weights replace what all have read before the second barrier, its second keys come behind
+    // its first barrier)
 }
 
 __device__ void evaluator_loop(const LoopArgs &g, EvalLds &L, int tree, int helper, int wave, int lane) {
