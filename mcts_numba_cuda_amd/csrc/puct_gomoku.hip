@@ -742,20 +742,36 @@ __device__ void select_phase(const LoopArgs &g, StepLds &s, int *paths, int tree
 // into the node's next free edge slots in traversal order (the expanded edges of a node stay contiguous whatever the
 // tickets say); when the tree cannot take all expansions of a step none is committed (those traversals evaluate the
 // node they reached instead).
+struct Leaf {   // what the selection has brought the wavefront's traversal to, on its way from memory
+    NodeInfo info;
+    uint32_t board;   // lanes 0..15
+};
+__device__ __forceinline__ bool reached_a_node(int sel) {
+    const int kind = (sel >> PUCT_GOMOKU_SEL_KIND_SHIFT) & 7;
+    return kind == PUCT_SELECT_EXPAND || kind == PUCT_SELECT_TERMINAL || kind == PUCT_SELECT_DEPTH_LIMIT;
+}
+__device__ __forceinline__ Leaf request_leaf(const LoopArgs &g, const StepLds &s, int tree, int wave, int lane) {
+    Leaf leaf{{0, 0, 0, 0.0f}, 0u};
+    const int sel = __builtin_amdgcn_readfirstlane(s.sel[wave]);
+    if (reached_a_node(sel)) {
+        const size_t row = (size_t)tree * g.max_nodes + (sel & PUCT_GOMOKU_SEL_NODE_MASK);
+        leaf.info = load_info(g.info + row);
+        if (lane < kBoardWords) leaf.board = g.board[row * kBoardWords + lane];
+    }
+    return leaf;
+}
 template <bool FARM>
-__device__ void expand_phase(const LoopArgs &g, StepLds &s, int tree, int wave, int lane, int n_waves, uint32_t &created) {
+__device__ void expand_phase(const LoopArgs &g, StepLds &s, const Leaf &leaf, int tree, int wave, int lane, int n_waves, uint32_t &created) {
     const int raw = s.sel[wave];
     const int kind = (raw >> PUCT_GOMOKU_SEL_KIND_SHIFT) & 7;
     const int node = raw & PUCT_GOMOKU_SEL_NODE_MASK, ticket_slot = (raw >> PUCT_GOMOKU_SEL_SLOT_SHIFT) & 0xFF;
     const size_t trow = (size_t)tree * g.max_nodes;
     const uint64_t tree_seed = psyn_tree_seed(g.seed, tree);
-    const bool has_node = kind == PUCT_SELECT_EXPAND || kind == PUCT_SELECT_TERMINAL || kind == PUCT_SELECT_DEPTH_LIMIT;
+    const bool has_node = reached_a_node(raw);
     uint32_t *board = s.board[wave];
-    NodeInfo ni{0, 0, 0, 0.0f};
+    const NodeInfo ni = leaf.info;
     if (has_node) {
-        const uint32_t w = lane < kBoardWords ? g.board[(trow + node) * kBoardWords + lane] : 0u;
-        ni = load_info(g.info + trow + node);
-        if (lane < kBoardWords) board[lane] = w;
+        if (lane < kBoardWords) board[lane] = leaf.board;
         wave_lds_fence();
     }
     const int n_legal = ni.legal_turn & 0xFFFF, turn = (ni.legal_turn & kTurnBit) ? -1 : 1;
@@ -1218,6 +1234,7 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
         work.count_kind(s, wave);
         uint64_t t1 = 0, t2 = 0;
         if (wave == 0) t1 = wall_clock64();
+        const Leaf leaf = request_leaf(g, s, tree, wave, lane);   // (the tree's own work: on its way while the evaluators are waited for)
         if (farm) {
             // A node created in the step before can be expanded now at the earliest (selection hands out tickets without
             // looking at a node's priors), so this is where its priors must be there, not a step's length earlier.
@@ -1226,7 +1243,7 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
             if (threadIdx.x == 0) wait_for_evaluators(rq, s);
             if (wave == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
-        expand_phase<FARM>(g, s, tree, wave, lane, n_waves, work.created);
+        expand_phase<FARM>(g, s, leaf, tree, wave, lane, n_waves, work.created);
         phase_barrier(farm);   // the claims of the selection and the new nodes are in memory
         if (s.gave_up) break;
         if (farm && threadIdx.x == 0) {   // ... and the evaluators may start on this step's nodes
@@ -1280,7 +1297,7 @@ __global__ __launch_bounds__(kTrav *kWave) void expand_step_kernel(const LoopArg
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), n_waves = blockDim.x / kWave;
     Work work;
     state_from_memory(g, s, paths, tree, n_waves);
-    expand_phase<false>(g, s, tree, wave, lane, n_waves, work.created);
+    expand_phase<false>(g, s, request_leaf(g, s, tree, wave, lane), tree, wave, lane, n_waves, work.created);
     __syncthreads();
     state_to_memory(g, s, paths, tree, n_waves);
     work.to_memory(g, tree, lane);
