@@ -416,65 +416,118 @@ __device__ __forceinline__ float row_max_f32(float v) {   // over the 16 lanes o
     return top;
 }
 
-// decide_in_turn for at most 16 edges, one per lane from lane 0 on, all of which lead to a node and have a finite score.  A
-// decision is a chain of dependent instructions on a lone wavefront, 0.5 us by decide_in_turn, most of it not the score:
-// here the maximum stays within a row of 16 lanes, the outcome is one register of the traversal's lane, and what the
-// traversals leave behind is written once, for all of them.  `single`: there is one edge to take.
+// decide_in_turn for at most 16 edges, one per lane from lane 0 on, all of which lead to a node and have a finite score; the n-th
+// decision's edge goes to lane n of `mine`.  A decision is a chain on a lone wavefront, eight clocks for every instruction that
+// waits for the one before it and more on the way through scalar registers and a branch: 330 clocks by decide_in_turn's way with one
+// row (row_decisions).  So where nobody can get a ticket, all decisions are taken by vector instructions alone, without a branch on an
+// outcome, by a score of one fused operation on the hardware's reciprocal (70 clocks with up to four edges, 110 with 16).  While the
+// maximum is looked for, the reciprocal for an edge that is taken is worked out.  The scores are kept from being negative, so that
+// they compare as integers.  An edge is taken if it comes within `apart` of the largest, which is more than both can be off by; if that
+// held for more than one edge at any of the decisions, their number says so in the end, and the scores themselves decide them all.
+template <int EDGES, int J = 0>
+__device__ __forceinline__ void lane_that_took(int takes, int decision, int &lane) {
+    lane = (dpp<0x150 + J>(takes) & decision) != 0 ? J : lane;   // row_newbcast:J
+    if constexpr (J + 1 < EDGES) lane_that_took<EDGES, J + 1>(takes, decision, lane);
+}
+struct QuickRow {
+    float cp, apart, q, cp_by;   // cp_by: cp over the edge's visits and claims and one
+    int den, takes;              // takes: bit n, the n-th decision
+};
+template <int EDGES, int N = 0>
+__device__ __forceinline__ void quick_row_decision(QuickRow &r, int n_members, float sqrt_lane) {
+    const float root = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), N));
+    const float score = __builtin_fmaf(r.cp_by, root, r.q), near = score + r.apart;
+    const float cp_by_if_taken = r.cp * __builtin_amdgcn_rcpf((float)(r.den + 1));
+    int top = __float_as_int(score);
+    const auto larger = [](int a, int b) { return a > b ? a : b; };
+    top = larger(dpp<0xB1>(top), top);
+    top = larger(dpp<0x4E>(top), top);
+    if constexpr (EDGES > 4) {
+        top = larger(dpp<0x141>(top), top);
+        top = larger(dpp<0x140>(top), top);
+    }
+    const bool taken = near >= __int_as_float(top);
+    r.cp_by = taken ? cp_by_if_taken : r.cp_by;
+    r.den += taken ? 1 : 0;
+    r.takes |= taken ? 1 << N : 0;
+    if constexpr (N + 1 < kTrav)
+        if (N + 1 < n_members) quick_row_decision<EDGES, N + 1>(r, n_members, sqrt_lane);
+}
+template <int EDGES>
+__device__ __forceinline__ bool quick_row_decisions(const EdgeSet<1> &e, int n_members, int lane, float sqrt_lane, int &den, int &mine) {
+    const bool edge = e.eid[0] >= 0;
+    const float q = prow_q(edge, e.q[0]);
+    QuickRow r;
+    r.cp = prow_cp(edge, e.cp[0]);
+    r.cp_by = r.cp * __builtin_amdgcn_rcpf((float)den);
+    r.den = den;
+    r.takes = 0;
+    // In units of 2^-24 of the largest |q| + u: an edge's quick score is off by 4 for u, 2 and 2 for the sums (a score is at most
+    // twice that when none is negative), its score by 2 and 1, `near` by 2: 24 for two edges, and 32 are allowed for.
+    const float last_root = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), n_members));
+    r.apart = row_max_f32(edge ? fabsf(q) + r.cp_by * last_root : 0.0f) * 0x1p-19f;
+    const float lift = row_max_f32(edge && q < 0.0f ? -q : 0.0f);
+    r.q = lane >= EDGES ? __builtin_nanf("") : edge ? q + lift : q;   // (lanes behind the edges are never taken)
+    quick_row_decision<EDGES>(r, n_members, sqrt_lane);
+    if (wave_sum(__popc((uint32_t)r.takes)) != n_members) return false;
+    den = r.den;
+    lane_that_took<EDGES>(r.takes, 1 << (lane & (kRow - 1)), mine);
+    return true;
+}
 template <bool TICKETS>
-__device__ __forceinline__ void row_decisions(const EdgeSet<1> &e, uint64_t edges, uint32_t members, int lane, int expanded, float sqrt_lane, int allowed_lane,
-                                              bool single, int &tickets, uint32_t &with_ticket, int &den, int &mine) {
+__device__ __forceinline__ void row_decisions(const EdgeSet<1> &e, uint64_t edges, uint32_t members, int n_members, int lane, int expanded, float sqrt_lane,
+                                              int allowed_lane, int &tickets, uint32_t &with_ticket, int &den, int &mine) {
     const bool edge = e.eid[0] >= 0;
     const float q = prow_q(edge, e.q[0]), cp = prow_cp(edge, e.cp[0]);
     int claimed = 0;
-    uint32_t rest = members;
+    uint32_t bit = 1u;
     do {
-        const uint32_t bit = rest & (0u - rest);
-        rest ^= bit;
         if (TICKETS && expanded + tickets < __builtin_amdgcn_readlane(allowed_lane, claimed)) {
             with_ticket |= bit;
             tickets += 1;
         } else {
-            uint64_t first = 1ull;
-            if (!single) {
-                const float sqrt_parent = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), claimed));
-                const float score = q + prow_quotient(cp * sqrt_parent, (float)den, __builtin_amdgcn_rcpf((float)den));
-                first = __builtin_amdgcn_fcmpf(score, row_max_f32(score), 1 /* == */) & edges;
-                if (__builtin_popcount((uint32_t)first) > 1) {   // the rotated edge index decides, as in candidate_key
-                    int tie_offset = __builtin_ctz(bit);
-                    if (tie_offset >= expanded) tie_offset %= expanded;
-                    const int turned = e.eid[0] - tie_offset + (e.eid[0] < tie_offset ? expanded : 0);
-                    const uint32_t key = __builtin_amdgcn_inverse_ballot_w64(first) ? 0x10000u - (uint32_t)turned : 0u;
-                    const uint32_t top_key = row_max_u32(key);
-                    first &= __builtin_amdgcn_uicmp(key, top_key, 32);
-                }
+            const float root = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), claimed));
+            const float score = q + prow_quotient(cp * root, (float)den, __builtin_amdgcn_rcpf((float)den));
+            uint32_t first = (uint32_t)(__builtin_amdgcn_fcmpf(score, row_max_f32(score), 1 /* == */) & edges);
+            if (__builtin_popcount(first) > 1) {   // the rotated edge index decides, as in candidate_key
+                const uint32_t of_lane = 1u << (lane & (kTrav - 1));   // the deciding traversal: the member with this many before it
+                int tie_offset = __builtin_ctzll(__ballot((members & of_lane) != 0 && 1u << __builtin_popcount(members & (of_lane - 1u)) == bit));
+                if (tie_offset >= expanded) tie_offset %= expanded;
+                const int turned = e.eid[0] - tie_offset + (e.eid[0] < tie_offset ? expanded : 0);
+                const uint32_t key = __builtin_amdgcn_inverse_ballot_w64((uint64_t)first) ? 0x10000u - (uint32_t)turned : 0u;
+                const uint32_t top_key = row_max_u32(key);
+                first &= (uint32_t)__builtin_amdgcn_uicmp(key, top_key, 32);
             }
-            den += __builtin_amdgcn_inverse_ballot_w64(first) ? 1 : 0;
-            mine = __builtin_amdgcn_inverse_ballot_w64(bit) ? __builtin_ctzll(first) : mine;
+            den += __builtin_amdgcn_inverse_ballot_w64((uint64_t)first) ? 1 : 0;
+            mine = __builtin_amdgcn_inverse_ballot_w64((uint64_t)bit) ? __builtin_ctz(first) : mine;
             claimed += 1;
         }
-    } while (rest != 0);
+        bit <<= 1;
+    } while (bit != 1u << n_members);
 }
 __device__ __forceinline__ void decide_in_row(const LoopArgs &g, StepLds &s, int *paths, int *next, Edge *row, const EdgeSet<1> &e, int node,
-                                              uint32_t members, int depth, int lane, int expanded, int legal, int total, int &tickets, bool single) {
+                                              uint32_t members, int depth, int lane, int expanded, int legal, int total, int &tickets) {
     const bool widening = expanded != 1 || g.c_pw != 0.0f;
     const int eff_lane = widening ? (total + lane > 1 ? total + lane : 1) : 1;
     const float sqrt_lane = widening ? sqrt_of_count(eff_lane) : 1.0f;
     const int allowed_lane = widening ? allowed_children(g.c_pw, g.alpha_pw, eff_lane, legal, sqrt_lane) : 1;
-    const int tickets_before = tickets;
-    int den = prow_den(e.eid[0] >= 0, e.den[0]), mine = -1;   // mine: lane of the edge that this lane's traversal takes
-    uint32_t with_ticket = 0;
+    const int tickets_before = tickets, n_members = __builtin_popcount(members);
+    int den = prow_den(e.eid[0] >= 0, e.den[0]), mine = 0;   // mine, in lane n: lane of the edge that the n-th decision takes
+    uint32_t with_ticket = 0;                                // bit n: the n-th decision is a ticket
     const uint64_t edges = __ballot(e.eid[0] >= 0);
     // (the limit grows with the claims: its largest value is the last one's)
-    if (expanded + tickets < __builtin_amdgcn_readlane(allowed_lane, __builtin_popcount(members) - 1))
-        row_decisions<true>(e, edges, members, lane, expanded, sqrt_lane, allowed_lane, single, tickets, with_ticket, den, mine);
-    else
-        row_decisions<false>(e, edges, members, lane, expanded, sqrt_lane, allowed_lane, single, tickets, with_ticket, den, mine);
-    const int from = (mine < 0 ? 0 : mine) << 2;
+    if (expanded + tickets < __builtin_amdgcn_readlane(allowed_lane, n_members - 1))
+        row_decisions<true>(e, edges, members, n_members, lane, expanded, sqrt_lane, allowed_lane, tickets, with_ticket, den, mine);
+    else if (n_members < 4 || !((edges >> 4) == 0 ? quick_row_decisions<4>(e, n_members, lane, sqrt_lane, den, mine)
+                                                  : quick_row_decisions<kRow>(e, n_members, lane, sqrt_lane, den, mine)))
+        row_decisions<false>(e, edges, members, n_members, lane, expanded, sqrt_lane, allowed_lane, tickets, with_ticket, den, mine);
+    const int nth = __builtin_popcount(members & ((1u << (lane & (kTrav - 1))) - 1u));   // which of the decisions is lane's traversal's
+    const int from = __builtin_amdgcn_ds_bpermute(nth << 2, mine) << 2;
     const int child = (int)((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)e.link[0]) >> 8);
     const int eid = __builtin_amdgcn_ds_bpermute(from, e.eid[0]);
     if (lane < kTrav && ((members >> lane) & 1u)) {
-        if ((with_ticket >> lane) & 1u) {
-            s.sel[lane] = pack_sel(PUCT_SELECT_EXPAND, node, expanded + tickets_before + __builtin_popcount(with_ticket & ((1u << lane) - 1u)));
+        if ((with_ticket >> nth) & 1u) {
+            s.sel[lane] = pack_sel(PUCT_SELECT_EXPAND, node, expanded + tickets_before + __builtin_popcount(with_ticket & ((1u << nth) - 1u)));
             s.len[lane] = depth + 1;
             s.claims[lane] = depth;
             next[lane] = -1;
@@ -683,7 +736,7 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
         edges = expanded;
     }
     if (edges >= 1 && edges <= kRow && fit_for_row(few)) {
-        decide_in_row(g, s, paths, next, row, few, node, (uint32_t)members, depth, lane, expanded, legal, total, tickets, edges == 1);
+        decide_in_row(g, s, paths, next, row, few, node, (uint32_t)members, depth, lane, expanded, legal, total, tickets);
     } else if (edges > 0) {
         decide_in_turn<1>(g, s, paths, next, few, node, members, depth, lane, expanded, legal, total, tickets, only_one);
         if (few.eid[0] >= 0 && few.link[0] != few.link_loaded[0]) row[few.eid[0]].link = few.link[0];
