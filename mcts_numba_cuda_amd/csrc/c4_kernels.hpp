@@ -473,25 +473,33 @@ struct Connect4 {
 // ---- kernels ----------------------------------------------------------------------------------------
 
 // MCTSNC._reset (src/mctsnc.py:1259-1290): one thread per tree.
-__global__ void reset_kernel(const TreeRef *refs, int n_refs, const uint64_t *root_bb /* [n_refs][2] */, const int32_t *root_turns) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_refs) return;
-    TreeRef ref = refs[r];
+struct Root { uint64_t bb[2]; int32_t turn; };
+__device__ __forceinline__ void reset_tree(const TreeRef &ref, const Root &root) {
     Node nd;
     for (int i = 0; i < kMaxCols; i++) { nd.child_ns[i] = 0; nd.child_wins[i] = 0; }
-    nd.bb_pos = root_bb[2 * r]; nd.bb_neg = root_bb[2 * r + 1];
-    nd.child_base = -1; nd.parent = -1; nd.depth = 0; nd.turn = (int8_t)root_turns[r]; nd.outcome = 2;
+    nd.bb_pos = root.bb[0]; nd.bb_neg = root.bb[1];
+    nd.child_base = -1; nd.parent = -1; nd.depth = 0; nd.turn = (int8_t)root.turn; nd.outcome = 2;
     nd.child_mask = 0; nd.flags = kLeaf; nd.action = 0; nd.best = 0;
     for (int i = 0; i < 8; i++) nd.reserved[i] = 0;
     ref.nodes[0] = nd;
     TreeHdr *h = ref.hdr;
     h->size = 1; h->root_ns = 0; h->root_wins = 0; h->max_depth = 0; h->depth_sum = 0;
-    h->selected = 0; h->path_len = 0; h->mode = 0; h->error = 0; h->root_turn = root_turns[r];
+    h->selected = 0; h->path_len = 0; h->mode = 0; h->error = 0; h->root_turn = root.turn;
     for (int i = 0; i < kMaxCols; i++) { h->mail[0][i] = 0; h->mail[1][i] = 0; }
     for (int i = 0; i < kMaxWide; i++) { h->wide_mail[0][i] = 0; h->wide_mail[1][i] = 0; }
     h->gen = 0; h->next_job = 0; h->plies = 0; h->u1_events = 0;
     h->stat_levels = 0; h->stat_children = 0; h->stat_expanded = 0; h->stat_played = 0;
     h->t_select = 0; h->t_expand = 0; h->t_playout = 0; h->t_backup = 0; h->t_exchange = 0;
+}
+__global__ void reset_kernel(const TreeRef *refs, int n_refs, const uint64_t *root_bb /* [n_refs][2] */, const int32_t *root_turns) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < n_refs) reset_tree(refs[r], Root{{root_bb[2 * r], root_bb[2 * r + 1]}, root_turns[r]});
+}
+// The trees of one search: its root comes with the launch, so that nothing has to be copied for it.
+__global__ void reset_search_kernel(const TreeRef *refs, int n_refs, Root root, int32_t *abort_flag) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r == 0) *abort_flag = 0;
+    if (r < n_refs) reset_tree(refs[r], root);
 }
 
 // Plies played in every tree since its reset, for the host to order a pass by what its searches cost.

@@ -367,24 +367,33 @@ struct LeafInfo {
 
 // ---- kernels ----------------------------------------------------------------------------------------------------
 
-__global__ void reset_kernel(const TreeRef *refs, int n_refs, const uint32_t *root_bb /* [n_refs][2 W] */, const int32_t *root_turns) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_refs) return;
-    TreeRef ref = refs[r];
+// One thread per tree.
+__device__ __forceinline__ void reset_tree(const TreeRef &ref, const uint32_t *root_bb /* [2 W] */, int turn) {
     Node nd;
-    nd.child_base = -1; nd.parent = -1; nd.n_children = 0; nd.best_child = -1; nd.depth = 0; nd.turn = (int8_t)root_turns[r];
+    nd.child_base = -1; nd.parent = -1; nd.n_children = 0; nd.best_child = -1; nd.depth = 0; nd.turn = (int8_t)turn;
     nd.outcome = 2; nd.flags = kLeaf; nd.pad0 = 0; nd.action = 0; nd.pad1[0] = nd.pad1[1] = 0;
     for (int i = 0; i < 24; i++) nd.bb[i] = 0u;
     ref.nodes[0] = nd;
     uint32_t *const stones = reinterpret_cast<uint32_t *>(ref.nodes) + 8;   // (a record's stone sets follow its 32-byte head)
-    for (int i = 0; i < 2 * ref.words; i++) stones[i] = root_bb[2 * ref.words * r + i];
+    for (int i = 0; i < 2 * ref.words; i++) stones[i] = root_bb[i];
     Stat st; st.ns = 0; st.wins = 0; st.action = 0; st.pad = 0;
     ref.stats[0] = st;
     TreeHdr *h = ref.hdr;
-    h->size = 1; h->max_depth = 0; h->depth_sum = 0; h->selected = 0; h->path_len = 0; h->mode = 0; h->root_turn = root_turns[r]; h->error = 0;
+    h->size = 1; h->max_depth = 0; h->depth_sum = 0; h->selected = 0; h->path_len = 0; h->mode = 0; h->root_turn = turn; h->error = 0;
     h->plies = 0; h->u1_events = 0; h->stat_levels = 0; h->stat_children = 0; h->stat_expanded = 0; h->stat_played = 0;
     h->t_select = 0; h->t_expand = 0; h->t_playout = 0; h->t_backup = 0; h->t_exchange = 0;
     h->arrive = 0; h->gen = 0;
+}
+__global__ void reset_kernel(const TreeRef *refs, int n_refs, const uint32_t *root_bb /* [n_refs][2 W] */, const int32_t *root_turns) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < n_refs) reset_tree(refs[r], root_bb + 2 * refs[r].words * r, root_turns[r]);
+}
+// The trees of one search: its root comes with the launch, so that nothing has to be copied for it.
+struct Root { uint32_t bb[2 * kMaxWords]; int32_t turn; };
+__global__ void reset_search_kernel(const TreeRef *refs, int n_refs, Root root, int32_t *abort_flag) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r == 0) *abort_flag = 0;
+    if (r < n_refs) reset_tree(refs[r], root.bb, root.turn);
 }
 
 // Draws the whole list of one playout, `count` cells: list[i * 64] is the lane's entry i; afterwards entry count - 1 - k

@@ -91,8 +91,7 @@ struct mctsnc_engine {
     uint64_t *d_rng_playout = nullptr, *d_rng_expand = nullptr;
     c4::TreeRef *d_refs = nullptr;
     unsigned char *d_reduced = nullptr;   // what the final reductions leave for the host (one search)
-    uint64_t *d_root_bb = nullptr;
-    int32_t *d_root_turns = nullptr, *d_abort = nullptr;
+    int32_t *d_abort = nullptr;
     int64_t n_rng_playout = 0, n_rng_expand = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -109,7 +108,6 @@ struct mctsnc_engine {
     gomoku::TreeRef *g_refs = nullptr;
     int16_t *g_ae = nullptr, *g_root_ae = nullptr;
     int32_t *g_poc = nullptr, *g_path = nullptr;
-    uint32_t *g_root_bb = nullptr;
     bool is_gomoku() const { return cfg.game == MCTSNC_GAME_GOMOKU; }
 };
 
@@ -155,18 +153,16 @@ void free_device(mctsnc_engine *e) {
     if (e->d_rng_expand) (void)hipFree(e->d_rng_expand);
     if (e->d_refs) (void)hipFree(e->d_refs);
     if (e->d_reduced) (void)hipFree(e->d_reduced);
-    if (e->d_root_bb) (void)hipFree(e->d_root_bb);
-    if (e->d_root_turns) (void)hipFree(e->d_root_turns);
     if (e->d_abort) (void)hipFree(e->d_abort);
-    void *gp[] = {e->g_nodes, e->g_stats, e->g_hdrs, e->g_refs, e->g_ae, e->g_root_ae, e->g_poc, e->g_path, e->g_root_bb};
+    void *gp[] = {e->g_nodes, e->g_stats, e->g_hdrs, e->g_refs, e->g_ae, e->g_root_ae, e->g_poc, e->g_path};
     for (void *q : gp) if (q) (void)hipFree(q);
     e->g_nodes = nullptr; e->g_stats = nullptr; e->g_hdrs = nullptr; e->g_refs = nullptr; e->g_ae = nullptr;
-    e->g_root_ae = nullptr; e->g_poc = nullptr; e->g_path = nullptr; e->g_root_bb = nullptr;
+    e->g_root_ae = nullptr; e->g_poc = nullptr; e->g_path = nullptr;
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     e->d_nodes = nullptr; e->d_hdrs = nullptr; e->d_rng_playout = nullptr; e->d_rng_expand = nullptr; e->d_refs = nullptr;
-    e->d_reduced = nullptr; e->d_root_bb = nullptr; e->d_root_turns = nullptr; e->d_abort = nullptr;
+    e->d_reduced = nullptr; e->d_abort = nullptr;
     e->ev0 = e->ev1 = nullptr; e->stream = nullptr;
     e->inited = false;
 }
@@ -282,12 +278,44 @@ int check_batch(mctsnc_engine **engines, int n, const int32_t *turns) {
     return MCTSNC_OK;
 }
 
+// Final reductions over trees and actions (src/mctsnc.py:2222-2375) on the device, one workgroup per search, and the
+// copy of their small result blocks for the host.  The trees of search j of the launch order are at refs[j * T .. (j + 1) * T).
+// They follow the search's last launch in the stream, so that the host waits once for both and reads the abort flag in the blocks:
+// with two waits and a copy of the flag, and a copy of the root, a memset and a wait before the search (see reset_search_kernel), a search of
+// 32 playouts and 100 steps took 622 us instead of 584.  (Blocks in pinned memory took 10 us less a search, but 80 more an engine.)
+template <class Game>
+struct Reduction {
+    mctsnc_engine *e0;
+    int n;
+    const typename Game::Ref *d_refs;
+    unsigned char *d_blocks;
+    std::vector<unsigned char> blocks;
+    bool enqueued = false;
+    ReducedHeader header(int j) const {
+        ReducedHeader h;
+        memcpy(&h, blocks.data() + reduced_stride(e0->cfg.max_actions) * (size_t)j, sizeof h);
+        return h;
+    }
+    int enqueue() {
+        const mctsnc_config &c = e0->cfg;
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(reduce_kernel<Game>), dim3(n), dim3(kReduceThreads), 0, e0->stream, d_refs, c.n_trees, c.max_actions,
+                           e0->thrifty ? 1 : 0, e0->d_abort, d_blocks);
+        HIP_TRY(hipGetLastError());
+        blocks.resize(reduced_stride(c.max_actions) * (size_t)n);
+        HIP_TRY(hipMemcpyAsync(blocks.data(), d_blocks, blocks.size(), hipMemcpyDeviceToHost, e0->stream));
+        enqueued = true;
+        return MCTSNC_OK;
+    }
+};
+constexpr double kTick = 1e-8;   // wall_clock64 counts at 100 MHz
+
 // The search loop: chunks of steps on the device, the budget checked between chunks.  launch(nsteps) enqueues one
 // launch of the persistent kernel on the engine's stream.
 // first_chunk > 0 caps the first launch at that many steps and calls after_first() once it has completed (with the
-// stream drained), if steps remain: where a pass orders its trees by what they turned out to cost.
-template <typename Launch, typename After>
-int budget_loop(mctsnc_engine *e0, const Budget &bud, Launch launch, int64_t &steps, double &dev_time, double &time_loop, int32_t first_chunk, After after_first) {
+// stream drained), if steps remain: where a pass orders its trees by what they turned out to cost.  A launch that uses the step
+// budget up is followed by the reductions; a search that ends by its time budget leaves them to the caller.
+template <class Game, typename Launch, typename After>
+int budget_loop(mctsnc_engine *e0, const Budget &bud, Reduction<Game> &reduction, Launch launch, int64_t &steps, double &dev_time, double &time_loop, int32_t first_chunk, After after_first) {
     hipStream_t stream = e0->stream;
     const bool forced = bud.forced < INFINITY;
     double step_budget = forced ? bud.forced : bud.steps_limit;
@@ -324,48 +352,46 @@ int budget_loop(mctsnc_engine *e0, const Budget &bud, Launch launch, int64_t &st
         int rc = launch(nsteps);
         if (rc) return rc;
         HIP_TRY(hipEventRecord(e0->ev1, stream));
+        const bool last = (double)(steps + nsteps) >= step_budget;
+        if (last && (rc = reduction.enqueue())) return rc;
         HIP_TRY(hipStreamSynchronize(stream));
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, e0->ev0, e0->ev1));
         dev_time += ms * 1e-3;
         steps += nsteps;
         int32_t aborted = 0;
-        HIP_TRY(hipMemcpy(&aborted, e0->d_abort, sizeof aborted, hipMemcpyDeviceToHost));
+        if (last) aborted = reduction.header(0).aborted;
+        else HIP_TRY(hipMemcpy(&aborted, e0->d_abort, sizeof aborted, hipMemcpyDeviceToHost));
         if (aborted) return MCTSNC_E_DEVICE_SYNC;   // the caller puts the engines back into a defined state and reports
         if (first_chunk > 0 && steps == nsteps && (double)steps < step_budget) {
             rc = after_first();
             if (rc) return rc;
         }
     }
-    time_loop = now_s() - t_loop;
+    time_loop = now_s() - t_loop - (reduction.enqueued ? reduction.header(0).t_reduce * kTick : 0.0);
     return MCTSNC_OK;
 }
-template <typename Launch>
-int budget_loop(mctsnc_engine *e0, const Budget &bud, Launch launch, int64_t &steps, double &dev_time, double &time_loop) {
-    return budget_loop(e0, bud, launch, steps, dev_time, time_loop, 0, [] { return MCTSNC_OK; });
+template <class Game, typename Launch>
+int budget_loop(mctsnc_engine *e0, const Budget &bud, Reduction<Game> &reduction, Launch launch, int64_t &steps, double &dev_time, double &time_loop) {
+    return budget_loop(e0, bud, reduction, launch, steps, dev_time, time_loop, 0, [] { return MCTSNC_OK; });
 }
 
-// Final reductions over trees and actions (src/mctsnc.py:2222-2375) on the device, one workgroup per search, and the
-// copy of their small result blocks into the callers' structs.  The trees of search j of the launch order are at
-// refs[j * T .. (j + 1) * T); search_of[j] is its index in the caller's arrays.
+// The result blocks in the callers' structs; search_of[j] is the index there of search j of the launch order.
 template <class Game>
-int reduce_and_finish(mctsnc_engine **engines, int n, const typename Game::Ref *d_refs, unsigned char *d_reduced, const std::vector<int> &search_of,
-                      int64_t steps, double t_start, double time_loop, double dev_time, mctsnc_result *out) {
+int finish(mctsnc_engine **engines, Reduction<Game> &reduction, const std::vector<int> &search_of, int64_t steps, double t_start, double time_loop, double dev_time,
+           mctsnc_result *out) {
     mctsnc_engine *e0 = engines[0];
-    const mctsnc_config &c = e0->cfg;
-    const int A = c.max_actions, T = c.n_trees;
+    const int A = e0->cfg.max_actions, n = reduction.n;
     const size_t stride = reduced_stride(A);
+    double time_reduce = reduction.enqueued ? reduction.header(0).t_reduce * kTick : 0.0;
     const double t_red = now_s();
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(reduce_kernel<Game>), dim3(n), dim3(kReduceThreads), 0, e0->stream, d_refs, T, A, e0->thrifty ? 1 : 0, d_reduced);
-    HIP_TRY(hipGetLastError());
-    std::vector<unsigned char> host(stride * (size_t)n);
-    HIP_TRY(hipMemcpyAsync(host.data(), d_reduced, host.size(), hipMemcpyDeviceToHost, e0->stream));
-    HIP_TRY(hipStreamSynchronize(e0->stream));
-    const double tick = 1e-8;  // wall_clock64 counts at 100 MHz
+    if (!reduction.enqueued) {
+        if (int rc = reduction.enqueue()) return rc;
+        HIP_TRY(hipStreamSynchronize(e0->stream));
+    }
     for (int j = 0; j < n; j++) {
-        const unsigned char *blk = host.data() + stride * (size_t)j;
-        ReducedHeader h;
-        memcpy(&h, blk, sizeof h);
+        const unsigned char *blk = reduction.blocks.data() + stride * (size_t)j;
+        const ReducedHeader h = reduction.header(j);
         mctsnc_result *o = out + search_of[j];
         memset(o, 0, sizeof *o);
         o->steps = steps;
@@ -379,13 +405,14 @@ int reduce_and_finish(mctsnc_engine **engines, int n, const typename Game::Ref *
         o->depth_sum = h.depth_sum; o->size_sum = h.size_sum; o->max_depth = h.max_depth; o->max_size = h.max_size;
         o->playout_plies = h.plies; o->u1_events = h.u1_events;
         o->stat_levels = h.stat_levels; o->stat_children = h.stat_children; o->stat_expanded = h.stat_expanded; o->stat_played = h.stat_played;
-        o->time_select = h.t_select * tick; o->time_expand = h.t_expand * tick; o->time_playout = h.t_playout * tick;
-        o->time_backup = h.t_backup * tick; o->time_exchange = h.t_exchange * tick;
+        o->time_select = h.t_select * kTick; o->time_expand = h.t_expand * kTick; o->time_playout = h.t_playout * kTick;
+        o->time_backup = h.t_backup * kTick; o->time_exchange = h.t_exchange * kTick;
         engines[search_of[j]]->has_run = true;
     }
     const double t_end = now_s();
+    time_reduce += t_end - t_red;
     for (int i = 0; i < n; i++) {
-        out[i].time_loop = time_loop; out[i].time_reduce = t_end - t_red; out[i].time_total = t_end - t_start; out[i].time_device_loop = dev_time;
+        out[i].time_loop = time_loop; out[i].time_reduce = time_reduce; out[i].time_total = t_end - t_start; out[i].time_device_loop = dev_time;
     }
     return MCTSNC_OK;
 }
@@ -494,7 +521,7 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
         bb.swap(bb2); tr.swap(tr2);
     }
     // one search with allocation allowed: the engine's own buffers; otherwise pieces of one block
-    C4BatchBuffers buf{e0->d_refs, e0->d_root_bb, e0->d_root_turns, e0->d_reduced};
+    C4BatchBuffers buf{e0->d_refs, nullptr, nullptr, e0->d_reduced};
     BlockHolder block_holder;
     if (n > 1 || fixed) {
         Workspace count, ws;
@@ -510,12 +537,18 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
     uint64_t *const d_bb = buf.root_bb;
     int32_t *const d_turns = buf.turns;
     hipStream_t stream = e0->stream;
-    HIP_TRY(hipMemcpyAsync(d_bb, bb.data(), sizeof(uint64_t) * 2 * n_refs, hipMemcpyHostToDevice, stream));
-    HIP_TRY(hipMemcpyAsync(d_turns, tr.data(), sizeof(int32_t) * n_refs, hipMemcpyHostToDevice, stream));
-    HIP_TRY(hipMemsetAsync(e0->d_abort, 0, sizeof(int32_t), stream));
-    hipLaunchKernelGGL(c4::reset_kernel, dim3((n_refs + 63) / 64), dim3(64), 0, stream, d_refs, n_refs, d_bb, d_turns);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(stream));
+    if (n > 1) {
+        HIP_TRY(hipMemcpyAsync(d_bb, bb.data(), sizeof(uint64_t) * 2 * n_refs, hipMemcpyHostToDevice, stream));
+        HIP_TRY(hipMemcpyAsync(d_turns, tr.data(), sizeof(int32_t) * n_refs, hipMemcpyHostToDevice, stream));
+        HIP_TRY(hipMemsetAsync(e0->d_abort, 0, sizeof(int32_t), stream));
+        hipLaunchKernelGGL(c4::reset_kernel, dim3((n_refs + 63) / 64), dim3(64), 0, stream, d_refs, n_refs, d_bb, d_turns);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(stream));   // (the copies are from pageable memory)
+    } else {
+        const c4::Root root{{bb[0], bb[1]}, tr[0]};
+        hipLaunchKernelGGL(c4::reset_search_kernel, dim3((n_refs + 63) / 64), dim3(64), 0, stream, d_refs, n_refs, root, e0->d_abort);
+        HIP_TRY(hipGetLastError());
+    }
 
     c4::SearchArgs args;
     args.refs = d_refs; args.n_refs = n_refs; args.m = c.board_m; args.n = c.board_n; args.P = c.n_playouts; args.G = e0->G; args.parts = 1;
@@ -619,7 +652,8 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
     const bool plain_launch = opt[MCTSNC_OPT_PLAIN_LAUNCH] != 0;
     static std::atomic<uint32_t> launch_counter{0};
     int64_t steps; double dev_time, time_loop;
-    int rc = budget_loop(e0, bud, [&](int32_t nsteps) -> int {
+    Reduction<c4::RootView> reduction{e0, n, d_refs, buf.reduced, {}};
+    int rc = budget_loop(e0, bud, reduction, [&](int32_t nsteps) -> int {
         args.nsteps = nsteps;
         if (e0->acp) {
             if (args.queue) {
@@ -674,7 +708,7 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
     // the trees of a search stay together and in order under the sorts above: search j of the launch order
     std::vector<int> search_of((size_t)n);
     for (int j = 0; j < n; j++) search_of[j] = order[(size_t)j * T] / T;
-    return reduce_and_finish<c4::RootView>(engines, n, d_refs, buf.reduced, search_of, steps, t_start, time_loop, dev_time, out);
+    return finish(engines, reduction, search_of, steps, t_start, time_loop, dev_time, out);
 }
 
 int run_many_gomoku(mctsnc_engine **engines, int n, const int8_t *boards, const int32_t *turns, const Budget &bud, mctsnc_result *out, Workspace *fixed) {
@@ -707,7 +741,7 @@ int run_many_gomoku(mctsnc_engine **engines, int n, const int8_t *boards, const 
         for (int k = 0; k < n_refs; k++) { memcpy(&bb2[RW * (size_t)k], &bb[RW * (size_t)order[k]], RW * sizeof(uint32_t)); tr2[k] = tr[order[k]]; }
         bb.swap(bb2); tr.swap(tr2);
     }
-    GomokuBatchBuffers buf{e0->g_refs, e0->g_root_bb, e0->d_root_turns, e0->d_reduced};
+    GomokuBatchBuffers buf{e0->g_refs, nullptr, nullptr, e0->d_reduced};
     BlockHolder block_holder;
     if (n > 1 || fixed) {
         Workspace count, ws;
@@ -723,12 +757,19 @@ int run_many_gomoku(mctsnc_engine **engines, int n, const int8_t *boards, const 
     uint32_t *const d_bb = buf.root_bb;
     int32_t *const d_turns = buf.turns;
     hipStream_t stream = e0->stream;
-    HIP_TRY(hipMemcpyAsync(d_bb, bb.data(), sizeof(uint32_t) * RW * n_refs, hipMemcpyHostToDevice, stream));
-    HIP_TRY(hipMemcpyAsync(d_turns, tr.data(), sizeof(int32_t) * n_refs, hipMemcpyHostToDevice, stream));
-    HIP_TRY(hipMemsetAsync(e0->d_abort, 0, sizeof(int32_t), stream));
-    hipLaunchKernelGGL(gomoku::reset_kernel, dim3((n_refs + 63) / 64), dim3(64), 0, stream, d_refs, n_refs, d_bb, d_turns);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(stream));
+    if (n > 1) {
+        HIP_TRY(hipMemcpyAsync(d_bb, bb.data(), sizeof(uint32_t) * RW * n_refs, hipMemcpyHostToDevice, stream));
+        HIP_TRY(hipMemcpyAsync(d_turns, tr.data(), sizeof(int32_t) * n_refs, hipMemcpyHostToDevice, stream));
+        HIP_TRY(hipMemsetAsync(e0->d_abort, 0, sizeof(int32_t), stream));
+        hipLaunchKernelGGL(gomoku::reset_kernel, dim3((n_refs + 63) / 64), dim3(64), 0, stream, d_refs, n_refs, d_bb, d_turns);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(stream));   // (the copies are from pageable memory)
+    } else {
+        gomoku::Root root{{}, tr[0]};
+        memcpy(root.bb, bb.data(), sizeof(uint32_t) * RW);
+        hipLaunchKernelGGL(gomoku::reset_search_kernel, dim3((n_refs + 63) / 64), dim3(64), 0, stream, d_refs, n_refs, root, e0->d_abort);
+        HIP_TRY(hipGetLastError());
+    }
 
     gomoku::SearchArgs args;
     int cus_now = 0;
@@ -764,7 +805,8 @@ int run_many_gomoku(mctsnc_engine **engines, int n, const int8_t *boards, const 
     }
     const bool plain_launch = opt[MCTSNC_OPT_PLAIN_LAUNCH] != 0;
     int64_t steps; double dev_time, time_loop;
-    int rc = budget_loop(e0, bud, [&](int32_t nsteps) -> int {
+    Reduction<gomoku::RootView> reduction{e0, n, d_refs, buf.reduced, {}};
+    int rc = budget_loop(e0, bud, reduction, [&](int32_t nsteps) -> int {
         args.nsteps = nsteps;
         for (int start = 0; start < n_refs; start += group) {
             args.refs = d_refs + start;
@@ -785,7 +827,7 @@ int run_many_gomoku(mctsnc_engine **engines, int n, const int8_t *boards, const 
 
     std::vector<int> search_of((size_t)n);
     for (int j = 0; j < n; j++) search_of[j] = order[(size_t)j * T] / T;
-    return reduce_and_finish<gomoku::RootView>(engines, n, d_refs, buf.reduced, search_of, steps, t_start, time_loop, dev_time, out);
+    return finish(engines, reduction, search_of, steps, t_start, time_loop, dev_time, out);
 }
 
 // use_static: take the per-call device buffers from the static scratch instead of allocating them.
@@ -937,7 +979,6 @@ static int init_device_impl(mctsnc_engine *e) {
     e->n_rng_expand = e->acp ? 0 : T;
     HIP_TRY(hipMalloc(&e->d_rng_playout, sizeof(uint64_t) * 2 * e->n_rng_playout));
     if (!e->acp) HIP_TRY(hipMalloc(&e->d_rng_expand, sizeof(uint64_t) * 2 * T));
-    HIP_TRY(hipMalloc(&e->d_root_turns, sizeof(int32_t) * T));
     HIP_TRY(hipMalloc(&e->d_reduced, reduced_stride(c.max_actions)));
     HIP_TRY(hipMalloc(&e->d_abort, 2 * sizeof(int32_t)));   // [0] abort flag, [1] head of the tree queue of a batch launch
     const size_t rng_per_tree = (size_t)(e->acp ? c.max_actions * c.n_playouts : c.n_playouts);
@@ -946,7 +987,6 @@ static int init_device_impl(mctsnc_engine *e) {
         HIP_TRY(hipMalloc(&e->d_hdrs, sizeof(c4::TreeHdr) * T));
         HIP_TRY(hipMemset(e->d_hdrs, 0, sizeof(c4::TreeHdr) * T));
         HIP_TRY(hipMalloc(&e->d_refs, sizeof(c4::TreeRef) * T));
-        HIP_TRY(hipMalloc(&e->d_root_bb, sizeof(uint64_t) * 2 * T));
         std::vector<c4::TreeRef> refs((size_t)T);
         for (int t = 0; t < T; t++) {
             refs[t].nodes = e->d_nodes + (size_t)t * S;
@@ -971,7 +1011,6 @@ static int init_device_impl(mctsnc_engine *e) {
         HIP_TRY(hipMalloc(&e->g_poc, sizeof(int32_t) * 2 * A * T));
         HIP_TRY(hipMemset(e->g_poc, 0, sizeof(int32_t) * 2 * A * T));
         HIP_TRY(hipMalloc(&e->g_path, sizeof(int32_t) * gomoku::kMaxPath * T));
-        HIP_TRY(hipMalloc(&e->g_root_bb, sizeof(uint32_t) * 2 * gomoku::kMaxWords * T));
         std::vector<gomoku::TreeRef> refs((size_t)T);
         for (int t = 0; t < T; t++) {
             refs[t].nodes = reinterpret_cast<gomoku::Node *>(e->g_nodes + (size_t)t * S * rec);

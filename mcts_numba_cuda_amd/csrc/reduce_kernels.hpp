@@ -22,10 +22,11 @@ constexpr int kReduceThreads = 512;   // MAX_STATE_MAX_ACTIONS of the reference 
 // root_actions_expanded[A + 2] (int16), actions_win_flags[A] (uint8); blocks of consecutive searches are
 // reduced_stride(A) bytes apart.
 struct __attribute__((aligned(256))) ReducedHeader {
-    int32_t best_action, best_win_flag, n_root_entries, max_depth, max_size, pad0[3];
+    int32_t best_action, best_win_flag, n_root_entries, max_depth, max_size, aborted, pad0[2];   // aborted: the search was, and nothing else is set
     int64_t best_n, best_n_wins, depth_sum, size_sum;
     unsigned long long plies, u1_events, stat_levels, stat_children, stat_expanded, stat_played;
     unsigned long long t_select, t_expand, t_playout, t_backup, t_exchange;   // of tree 0
+    unsigned long long t_reduce;   // of this kernel
 };
 static_assert(sizeof(ReducedHeader) == 256, "header of a reduced block");
 
@@ -39,11 +40,17 @@ __host__ __device__ inline size_t reduced_stride(int A) { return (reduced_off_fl
 #ifdef __HIPCC__
 // refs: the trees of the launch, those of search j at [j * T, (j + 1) * T) with its tree 0 first.
 template <class Game>
-__global__ void __launch_bounds__(kReduceThreads) reduce_kernel(const typename Game::Ref *refs, int T, int A, int thrifty, unsigned char *out) {
+__global__ void __launch_bounds__(kReduceThreads) reduce_kernel(const typename Game::Ref *refs, int T, int A, int thrifty, const int32_t *abort_flag, unsigned char *out) {
     using Ref = typename Game::Ref;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const unsigned long long t_start = wall_clock64();
     refs += (size_t)blockIdx.x * T;
     unsigned char *const o = out + (size_t)blockIdx.x * reduced_stride(A);
+    // (the launch before it may not have been waited for: what an abandoned search leaves is not looked at)
+    if (*abort_flag != 0) {
+        if (tid == 0) reinterpret_cast<ReducedHeader *>(o)->aborted = 1;
+        return;
+    }
     int A_pad = 1;
     while (A_pad < A) A_pad <<= 1;   // slots of the tournament: the next power of two (any larger padding gives the same winner)
 
@@ -154,12 +161,13 @@ __global__ void __launch_bounds__(kReduceThreads) reduce_kernel(const typename G
             hd.best_win_flag = f; hd.best_n = n; hd.best_n_wins = w;
             hd.n_root_entries = nb;
             hd.max_depth = s_max[0]; hd.max_size = s_max[1];
-            hd.pad0[0] = hd.pad0[1] = hd.pad0[2] = 0;
+            hd.aborted = 0; hd.pad0[0] = hd.pad0[1] = 0;
             hd.depth_sum = (int64_t)s_tot[1]; hd.size_sum = (int64_t)s_tot[2];
             hd.plies = s_tot[3]; hd.u1_events = s_tot[4];
             hd.stat_levels = s_tot[5]; hd.stat_children = s_tot[6]; hd.stat_expanded = s_tot[7]; hd.stat_played = s_tot[8];
             const auto *h0 = ref0.hdr;
             hd.t_select = h0->t_select; hd.t_expand = h0->t_expand; hd.t_playout = h0->t_playout; hd.t_backup = h0->t_backup; hd.t_exchange = h0->t_exchange;
+            hd.t_reduce = wall_clock64() - t_start;
             *reinterpret_cast<ReducedHeader *>(o) = hd;
         }
     }
