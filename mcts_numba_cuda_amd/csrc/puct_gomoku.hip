@@ -1074,11 +1074,27 @@ constexpr int kEvalParts = kEdges / kWave;              // wavefronts per node
 constexpr int kEvalNodes = kTrav / kEvalParts;          // nodes at a time, at most
 struct EvalLds {
     uint32_t keys[2][kEvalNodes][kEvalParts][kWave];   // sorted by 64, by 128
-    unsigned long long weight[kEvalNodes][kEvalParts];
+    double weight[kEvalNodes][kEvalParts];
     int legal[kEvalNodes][kEvalParts];
     unsigned long long tag[2];   // by parity of the step
 };
 __device__ __forceinline__ int eval_nodes_at_once() { return (int)blockDim.x / (kWave * kEvalParts); }   // (2 to 4: 8 to 16 wavefronts)
+
+// psyn_key_weight as a double, which it is exactly, and so are the sums (below 2^48): psyn_prior's quotient without the conversions.
+__device__ __forceinline__ double key_weight(uint32_t key) { return trunc((double)__uint_as_float(key & 0x7FFFFF00u) * 4294967296.0); }
+__device__ __forceinline__ double wave_sum_f64(double v) {
+    const auto step = [](double x, auto ctrl) {
+        const uint64_t b = (uint64_t)__double_as_longlong(x);
+        const uint32_t lo = (uint32_t)dpp<decltype(ctrl)::value>((int)(uint32_t)b), hi = (uint32_t)dpp<decltype(ctrl)::value>((int)(uint32_t)(b >> 32));
+        return x + __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+    };
+    v = step(v, std::integral_constant<int, 0xB1>{});
+    v = step(v, std::integral_constant<int, 0x4E>{});
+    v = step(v, std::integral_constant<int, 0x141>{});
+    v = step(v, std::integral_constant<int, 0x140>{});
+    const auto row = [&](int lane) { return __longlong_as_double((long long)read_lane64((uint64_t)__double_as_longlong(v), lane)); };
+    return (row(0) + row(16)) + (row(32) + row(48));
+}
 
 // The wavefront's 64 keys, largest first: a bitonic sort with one key per lane.  SIZE == 64, DIST == 32 alone: a bitonic list.
 template <int SIZE, int DIST>
@@ -1151,7 +1167,7 @@ __device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index
             left = __ballot(pending);
             round += 1 << shift;
         }
-        const uint64_t part_sum = wave_sum64(key ? psyn_key_weight(key) : 0);
+        const double part_sum = wave_sum_f64(key ? key_weight(key) : 0.0);
         const int part_legal = __popcll(__ballot(legal));
         if (lane == 0) {
             L.weight[group][part] = part_sum;
@@ -1161,7 +1177,7 @@ __device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index
         L.keys[0][group][part][lane] = key;
     }
     __syncthreads();
-    uint64_t sum = 0;
+    double sum = 0.0;
     int n_legal = 0;
     if (active) {   // two lists of 64 to one of 128: the first meets the second from its end, the larger keys stay in front
         sum = L.weight[group][0] + L.weight[group][1] + L.weight[group][2] + L.weight[group][3];
@@ -1180,7 +1196,7 @@ __device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index
         sort64_step<kWave, kWave / 2>(key);
         const size_t e = (trow + child) * kEdges + part * kWave + lane;
         if (key != 0) {
-            store_edge(g.edges + e, 0, 0.0f, psyn_prior(psyn_key_weight(key), sum, n_legal), 0u);
+            store_edge(g.edges + e, 0, 0.0f, sum == 0.0 ? (float)(1.0 / (double)n_legal) : (float)(key_weight(key) / sum), 0u);
             g.action[e] = (uint8_t)(255u - (key & 0xFFu));
         }
     }
