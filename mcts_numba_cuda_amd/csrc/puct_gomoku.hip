@@ -1207,6 +1207,7 @@ __device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index
 __device__ void evaluator_loop(const LoopArgs &g, EvalLds &L, int tree, int helper, int wave, int lane) {
     EvalRequests &rq = g.requests[tree];
     if (threadIdx.x == 0) __hip_atomic_store(&rq.xcc[1 + helper], my_xcc(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bool asked = false, same_l2 = false;
     int seen = 0;   // the last step's tag (steps of which this evaluator had nothing to do may pass it by)
     for (int turn = 0;; turn ^= 1) {
         if (threadIdx.x == 0) {
@@ -1242,8 +1243,13 @@ __device__ void evaluator_loop(const LoopArgs &g, EvalLds &L, int tree, int help
         __syncthreads();
         if (threadIdx.x == 0 && worked_off > 0) {
             // The tree's workgroup wrote its XCD down before it handed out its first step.  On the same XCD the priors
-            // are where it reads them, in the L2 that both share; anywhere else the L2 must be written back first.
-            if (g.agent_fences || poll_word(&rq.xcc[0]) != my_xcc()) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            // are where it reads them, in the L2 that both share; anywhere else the L2 must be written back first.  (Asked
+            // once: the answer took a round trip to the L2 of every step that the tree waited for.)
+            if (!asked) {
+                asked = true;
+                same_l2 = !g.agent_fences && poll_word(&rq.xcc[0]) == my_xcc();
+            }
+            if (!same_l2) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
             __hip_atomic_fetch_add(&rq.done, worked_off, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
