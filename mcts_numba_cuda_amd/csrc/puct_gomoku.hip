@@ -132,7 +132,8 @@ __device__ __forceinline__ bool stone_at(const uint32_t *colour, int cell) { ret
 // row does not win)?  Lane 16 d + 5 + k looks at the cell k steps along direction d; the result is uniform.
 __device__ __forceinline__ bool makes_five(const uint32_t *mine, int cell, int m, int n, int lane) {
     const int d = lane >> 4, k = (lane & 15) - 5;
-    const int r = cell / n + (d == 0 ? 0 : k), c = cell % n + (d == 0 || d == 2 ? k : (d == 1 ? 0 : -k));
+    const int row = (int)(((float)cell + 0.5f) * __builtin_amdgcn_rcpf((float)n));   // (cell < 256: half a cell is far more than the reciprocal's error)
+    const int r = row + (d == 0 ? 0 : k), c = cell - row * n + (d == 0 || d == 2 ? k : (d == 1 ? 0 : -k));
     const uint64_t like = __ballot(k <= 5 && r >= 0 && r < m && c >= 0 && c < n && stone_at(mine, r * n + c));
     const uint32_t line = (uint32_t)(like >> (16 * (lane & 3))) & 0x7FFu;   // bit 5: the stone itself
     return __ballot(1 + __builtin_clz(~(line << 27)) + __builtin_ctz(~(line >> 6)) == 5) != 0;
@@ -280,6 +281,9 @@ __device__ __forceinline__ uint32_t score_image(float score) {
     const uint32_t b = __float_as_uint(score + 0.0f);
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
+
+template <class T>
+__device__ __forceinline__ T poll_word(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // ---- selection ---------------------------------------------------------------------------------------------------
 // The edges of one node as the deciding traversals see them: up to NS per lane.
@@ -762,8 +766,11 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
 
 // Selection of one step for the traversals of one tree; all wavefronts of the workgroup call it.  Ends behind a
 // workgroup barrier with every traversal's result in `s` and its path in `paths`.
+// FARM: thread 0 asks for *done, the entries that the evaluators have worked off, with every level and keeps the last answer, so that
+// it seldom has to ask, and wait a round trip for it, afterwards.
+template <bool FARM>
 __device__ void select_phase(const LoopArgs &g, StepLds &s, int *paths, int tree, int wave, int lane, int n_waves,
-                             uint32_t &nodes_read, uint32_t &edges_scored) {
+                             uint32_t &nodes_read, uint32_t &edges_scored, const int *done, int &worked_off) {
     if (threadIdx.x < kTrav) {
         const int t = threadIdx.x;
         s.cur[0][t] = t < n_waves ? 0 : -1;
@@ -779,6 +786,7 @@ __device__ void select_phase(const LoopArgs &g, StepLds &s, int *paths, int tree
         int *next = s.cur[(depth & 1) ^ 1];
         const int at = lane < kTrav ? cur[lane] : -1;
         if (__ballot(at >= 0) == 0) break;   // every wavefront reads the same words: all leave together
+        if (FARM && threadIdx.x == 0) worked_off = poll_word(done);
         const int mine = __builtin_amdgcn_readlane(at, wave);
         const uint64_t members = __ballot(at >= 0 && at == mine);
         if (mine < 0) {
@@ -814,12 +822,11 @@ __device__ __forceinline__ Leaf request_leaf(const LoopArgs &g, const StepLds &s
     return leaf;
 }
 template <bool FARM>
-__device__ void expand_phase(const LoopArgs &g, StepLds &s, const Leaf &leaf, int tree, int wave, int lane, int n_waves, uint32_t &created) {
+__device__ void expand_phase(const LoopArgs &g, StepLds &s, const Leaf &leaf, uint64_t hash_seed, int tree, int wave, int lane, int n_waves, uint32_t &created) {
     const int raw = s.sel[wave];
     const int kind = (raw >> PUCT_GOMOKU_SEL_KIND_SHIFT) & 7;
     const int node = raw & PUCT_GOMOKU_SEL_NODE_MASK, ticket_slot = (raw >> PUCT_GOMOKU_SEL_SLOT_SHIFT) & 0xFF;
     const size_t trow = (size_t)tree * g.max_nodes;
-    const uint64_t tree_seed = psyn_tree_seed(g.seed, tree);
     const bool has_node = reached_a_node(raw);
     uint32_t *board = s.board[wave];
     const NodeInfo ni = leaf.info;
@@ -874,7 +881,7 @@ __device__ void expand_phase(const LoopArgs &g, StepLds &s, const Leaf &leaf, in
             float u = 0.0f;   // value of the reached node for the player who moved into it
             if (r.x == kReachedValued) u = s.value[lane];
             if (r.x >= kReachedPosition) {
-                const uint64_t bh = psyn_board_hash(tree_seed, s.board[lane]);
+                const uint64_t bh = psyn_board_hash_from(hash_seed, s.board[lane]);
                 s.hash[lane] = bh;
                 const bool terminal = r.x == kReachedWin || r.x == kReachedDraw;
                 const float v = r.x == kReachedWin ? -1.0f : (terminal ? 0.0f : psyn_value(bh));
@@ -1114,9 +1121,6 @@ __device__ __forceinline__ void sort64_descending(uint32_t &v) {
     if constexpr (SIZE < kWave) sort64_descending<2 * SIZE>(v);
 }
 
-template <class T>
-__device__ __forceinline__ T poll_word(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-
 // Entry `index` of the step (none if it is not below n), whose node is first_node + index, by four wavefronts, `part` = 0..3; the whole workgroup must call it.
 __device__ void evaluate_node(const LoopArgs &g, EvalLds &L, int tree, int index, int n, int first_node, int group, int part, int lane) {
     const EvalRequests &rq = g.requests[tree];
@@ -1302,10 +1306,12 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
         if (farm) __hip_atomic_store(&rq.xcc[0], my_xcc(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
+    const uint64_t hash_seed = psyn_mix64(psyn_tree_seed(g.seed, tree));
     bool same_l2 = false;   // known: every evaluator of the tree runs on this workgroup's XCD
     uint64_t t0 = wave == 0 ? wall_clock64() : 0;
     for (int step = 0; step < g.steps; ++step) {
-        select_phase(g, s, paths, tree, wave, lane, n_waves, work.nodes_read, work.edges_scored);
+        int worked_off = 0;
+        select_phase<FARM>(g, s, paths, tree, wave, lane, n_waves, work.nodes_read, work.edges_scored, &rq.done, worked_off);
         work.count_kind(s, wave);
         uint64_t t1 = 0, t2 = 0;
         if (wave == 0) t1 = wall_clock64();
@@ -1315,10 +1321,10 @@ __global__ __launch_bounds__(kTrav *kWave) void search_kernel(const LoopArgs g, 
             // looking at a node's priors), so this is where its priors must be there, not a step's length earlier.
             // Selection has read rows of such nodes while they were being written: the L1 drops what it holds.  The first
             // wavefront's acquire does that for all of them, which read no evaluator's work before expand_phase's barrier.
-            if (threadIdx.x == 0) wait_for_evaluators(rq, s);
+            if (threadIdx.x == 0 && worked_off < s.requested) wait_for_evaluators(rq, s);
             if (wave == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
-        expand_phase<FARM>(g, s, leaf, tree, wave, lane, n_waves, work.created);
+        expand_phase<FARM>(g, s, leaf, hash_seed, tree, wave, lane, n_waves, work.created);
         phase_barrier(farm);   // the claims of the selection and the new nodes are in memory
         if (s.gave_up) break;
         if (farm && threadIdx.x == 0) {   // ... and the evaluators may start on this step's nodes
@@ -1360,7 +1366,8 @@ __global__ __launch_bounds__(kTrav *kWave) void select_step_kernel(const LoopArg
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), n_waves = blockDim.x / kWave;
     Work work;
     if (threadIdx.x == 0) s.node_count = g.node_count[tree];
-    select_phase(g, s, paths, tree, wave, lane, n_waves, work.nodes_read, work.edges_scored);
+    int no_evaluators = 0;
+    select_phase<false>(g, s, paths, tree, wave, lane, n_waves, work.nodes_read, work.edges_scored, nullptr, no_evaluators);
     work.count_kind(s, wave);
     state_to_memory(g, s, paths, tree, n_waves);
     work.to_memory(g, tree, lane);
@@ -1372,7 +1379,7 @@ __global__ __launch_bounds__(kTrav *kWave) void expand_step_kernel(const LoopArg
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), n_waves = blockDim.x / kWave;
     Work work;
     state_from_memory(g, s, paths, tree, n_waves);
-    expand_phase<false>(g, s, request_leaf(g, s, tree, wave, lane), tree, wave, lane, n_waves, work.created);
+    expand_phase<false>(g, s, request_leaf(g, s, tree, wave, lane), psyn_mix64(psyn_tree_seed(g.seed, tree)), tree, wave, lane, n_waves, work.created);
     __syncthreads();
     state_to_memory(g, s, paths, tree, n_waves);
     work.to_memory(g, tree, lane);

@@ -36,11 +36,11 @@ PSYN_FN uint64_t psyn_tree_seed(uint64_t seed, int tree) { return psyn_mix64(see
 
 /* Hash of a position given as 16 words: words 0..7 the stones of the player with token +1 (bit = cell index), words
  * 8..15 those of the player with token -1.  The side to move follows from the stone counts. */
-PSYN_FN uint64_t psyn_board_hash(uint64_t tree_seed, const uint32_t *w) {
-    uint64_t h = psyn_mix64(tree_seed);
+PSYN_FN uint64_t psyn_board_hash_from(uint64_t h /* psyn_mix64(tree_seed) */, const uint32_t *w) {
     for (int i = 0; i < 8; ++i) h = psyn_mix64(h ^ (((uint64_t)w[2 * i + 1] << 32) | w[2 * i]));
     return h;
 }
+PSYN_FN uint64_t psyn_board_hash(uint64_t tree_seed, const uint32_t *w) { return psyn_board_hash_from(psyn_mix64(tree_seed), w); }
 
 /* Value of the position for the player to move, in [-1, 1): 24 hash bits, exactly representable. */
 PSYN_FN float psyn_value(uint64_t board_hash) {
