@@ -282,7 +282,7 @@ int check_batch(mctsnc_engine **engines, int n, const int32_t *turns) {
 // copy of their small result blocks for the host.  The trees of search j of the launch order are at refs[j * T .. (j + 1) * T).
 // They follow the search's last launch in the stream, so that the host waits once for both and reads the abort flag in the blocks:
 // with two waits and a copy of the flag, and a copy of the root, a memset and a wait before the search (see reset_search_kernel), a search of
-// 32 playouts and 100 steps took 622 us instead of 584.  (Blocks in pinned memory took 10 us less a search, but 80 more an engine.)
+// 32 playouts and 100 steps took 622 us instead of 584.  (Blocks in pinned memory took 10 us less a search, but 30 to 130 more an engine.)
 template <class Game>
 struct Reduction {
     mctsnc_engine *e0;
