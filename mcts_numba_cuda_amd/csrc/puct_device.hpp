@@ -835,18 +835,33 @@ struct BackupArgs {
 // selection word has no reason field).  NODE_LEVEL = false: the same conversion of virtual visits into real ones for
 // the edge-level virtual loss of select_kernel; BUSY selections hold nothing and are skipped, as in
 // src/puct/test_puct_gpu_v3.py:297-302.
-template <bool NODE_LEVEL, bool COUNTED = false>
-__device__ __forceinline__ void backup_traversal(const BackupArgs &a, LdsInts counted, int tree, int wid, int lane) {
-    // All that a path of up to 64 levels needs is requested at once: a launch of few traversals is as long as its chain of loads,
-    // which was four long, each asked for when the one before was known to matter (16 trees x 8 traversals 3.5 -> 2.7 us, 1024 x 8
-    // 4.1 -> 3.8).
+// All that a path of up to 64 levels needs is requested at once: a launch of few traversals is as long as its chain of loads,
+// which was four long, each asked for when the one before was known to matter (16 trees x 8 traversals 3.5 -> 2.7 us, 1024 x 8
+// 4.1 -> 3.8).
+struct BackupRequest {
+    const int *path;
+    const float *values;
+    int node_limit, raw, plen, encoded;
+    float value;
+};
+__device__ __forceinline__ BackupRequest request_backup(const BackupArgs &a, int tree, int wid, int lane) {
     const size_t out = (uint64_t)(uint32_t)tree * (uint32_t)a.warps + (uint32_t)wid, first = out * (uint32_t)a.path_depth;
-    const int *const path = a.out_path_eids + first;
-    const float *const values = a.path_edge_values == nullptr ? nullptr : a.path_edge_values + first;
-    const int node_limit = a.node_count[tree], raw = a.out_selected_node[out], plen = a.out_path_len[out];
-    int encoded = lane < a.path_depth ? path[lane] : -1;
-    float value = values != nullptr && lane < a.path_depth ? values[lane] : 0.0f;
+    BackupRequest r;
+    r.path = a.out_path_eids + first;
+    r.values = a.path_edge_values == nullptr ? nullptr : a.path_edge_values + first;
+    r.node_limit = a.node_count[tree], r.raw = a.out_selected_node[out], r.plen = a.out_path_len[out];
+    r.encoded = lane < a.path_depth ? r.path[lane] : -1;
+    r.value = r.values != nullptr && lane < a.path_depth ? r.values[lane] : 0.0f;
     asm volatile("" ::: "memory");
+    return r;
+}
+template <bool NODE_LEVEL, bool COUNTED = false>
+__device__ __forceinline__ void backup_traversal(const BackupArgs &a, LdsInts counted, int tree, int lane, const BackupRequest &request) {
+    const int *const path = request.path;
+    const float *const values = request.values;
+    const int node_limit = request.node_limit, raw = request.raw, plen = request.plen;
+    int encoded = request.encoded;
+    float value = request.value;
     if (node_limit <= 0 || node_limit > a.nodes || node_limit > PUCT_PACKED_NODE_LIMIT) return;
     if (raw < 0) return;
     const int kind = NODE_LEVEL ? raw >> PUCT_PACKED_KIND_SHIFT : (raw >> PUCT_PACKED_KIND_SHIFT) & PUCT_PACKED_KIND_MASK;

@@ -4,6 +4,14 @@
 namespace {
 using namespace puct;
 
+// Trees of a workgroup of counted_backup_kernel (up to kMaxWavesPerBlock traversals each), a traversal for each of its wavefronts where there are
+// many trees.  Where paths are short they share what it costs to start a workgroup with its LDS; where they are long they are counted
+// one after the other, which costs more the fewer workgroups there are.
+constexpr int kMostCountedTrees = 8;
+inline int trees_of_counting_block(int trees, int warps, int threads) {
+    const int waves = threads / kWave / warps, spread = trees / 2048, most = waves < kMostCountedTrees ? waves : kMostCountedTrees;
+    return spread < 1 || most < 1 ? 1 : spread < most ? spread : most;
+}
 inline __host__ __device__ int traversals_of_block(int warps) { return warps < kMaxWavesPerBlock ? warps : kMaxWavesPerBlock; }
 
 // Has a launch's arguments read at once: the compiler asks for them where they are used, three waits one after the other (16 trees of
@@ -88,43 +96,77 @@ __global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void backup_kernel(const 
     fetch_arguments(a);
     const int wid = __builtin_amdgcn_readfirstlane(blockIdx.y * traversals_of_block(a.warps) + threadIdx.x / kWave);   // the same in all lanes
     if (wid >= a.warps) return;
-    backup_traversal<NODE_LEVEL>(a, nullptr, blockIdx.x, wid, threadIdx.x & (kWave - 1));
+    const int lane = threadIdx.x & (kWave - 1);
+    backup_traversal<NODE_LEVEL>(a, nullptr, blockIdx.x, lane, request_backup(a, blockIdx.x, wid, lane));
 }
 
-// The backup of small trees with long paths, whose traversals are wavefronts of this workgroup (grid.y == 1): how often each edge is passed
+// Whether a tree's backup is counted (see below): by the levels that its paths have together, which only the device knows.  Both forms take as long at
+// some 40 + slots / 85 levels where paths wander evenly over all edges (us a release of 16384 trees, atomics / counted: 65 x 64 with
+// paths of 64 levels 37 / 42, of 128 72 / 68; 10 x 9 with 32 9.2 / 11, with 64 15 / 11), and at some 15 + slots / 300 where they keep
+// coming back to the same ones, which is what selections do (65 x 64 with 55 levels on average 47 / 23; 10 x 9 with 33 21 / 11).
+inline __host__ __device__ bool counting_pays(long long levels, long long slots) { return levels >= 24 + slots / 128; }
+
+// The backup of small trees whose paths may be long, a few trees a workgroup, so that each of its wavefronts has a traversal (grid.y == 1).
+// Where a tree's paths are short, its traversals are backed up as by backup_kernel.  Otherwise how often each edge is passed
 // is counted in LDS (a.nodes * a.edges words, and at node level a.nodes more), and the edges that were passed, and the nodes that they
-// lead to, are then updated in one sweep, an atomic each and lanes side by side, instead of one a level wherever the path leads.  (Values
-// are added one by one, in the order in which they come, as before.)  Bound by the lines that the sweep updates: 16384 trees of 65 x 64
-// edges with one path of 512 levels, some 0.55 GB in 86 us, where 8.4 M scattered atomics took 324.  Loads and stores in the sweep
-// instead of atomics: 100 us, with values 463 instead of 580, but then two launches on the same trees would no longer add up.
+// lead to, are then updated in one sweep by the whole workgroup, an atomic each and lanes side by side, instead of one a level wherever the
+// path leads.  (Values are added one by one, in the order in which they come, as before.)  Loads and stores in the sweep
+// instead of atomics would be faster with values and slower without, but then two launches on the same trees would no longer add up.
 template <bool NODE_LEVEL>
-__global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void counted_backup_kernel(const BackupArgs a) {
+__global__ __launch_bounds__(kMaxWavesPerBlock *kWave) void counted_backup_kernel(const BackupArgs a, int at_once) {
     fetch_arguments(a);
     extern __shared__ int times_passed[];
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), words = a.nodes * a.edges, threads = blockDim.x;
-    int *const times_reached = times_passed + words;
-    const int node_limit = a.node_count[blockIdx.x];
-    for (int i = threadIdx.x; i < words + (NODE_LEVEL ? a.nodes : 0); i += threads) times_passed[i] = 0;
-    __syncthreads();
-    if (wid < a.warps) backup_traversal<NODE_LEVEL, true>(a, (LdsInts)times_passed, blockIdx.x, wid, threadIdx.x & (kWave - 1));
-    __syncthreads();
-    const uint64_t first_node = (uint64_t)blockIdx.x * (uint32_t)a.nodes, first = first_node * (uint32_t)a.edges;
-    for (int i = threadIdx.x; i < words; i += threads) {
-        const int passed = times_passed[i];
-        if (passed == 0) continue;
-        if (!NODE_LEVEL) {
-            atomicAdd(&a.edge_inflight[first + i], (int)(0u - (uint32_t)passed * (uint32_t)a.virtual_loss));
-        } else {
-            const int child = a.edge_child_id[first + i];
-            if (child >= 0 && child < node_limit) __hip_atomic_fetch_add((LdsInts)times_reached + child, passed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-        if (a.path_edge_values != nullptr) atomicAdd(&a.edge_N[first + i], passed);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+    const int words = a.nodes * a.edges, threads = blockDim.x;
+    const auto tree_at = [&](int k) { return (int)(blockIdx.x + (uint32_t)k * gridDim.x); };   // the workgroup's k-th (neighbours go to neighbours)
+    const auto nth_tree = [&](int traversal) {   // (by divisions, and with sums over lanes where a tree has one traversal, a launch on short paths took 8.3 us, not 7.0)
+        int n = 0;
+#pragma unroll
+        for (int k = 1; k <= kMostCountedTrees; ++k) n += traversal >= k * a.warps ? 1 : 0;
+        return n;
+    };
+    const int tree_of_lane = nth_tree(lane), tree_of_wave = nth_tree(wave);
+    const bool has_traversal = tree_of_wave < at_once && tree_at(tree_of_wave) < a.trees;
+    BackupRequest mine{};
+    if (has_traversal) mine = request_backup(a, tree_at(tree_of_wave), wave - tree_of_wave * a.warps, lane);
+    int levels = 0;   // of traversal `lane` of the workgroup's
+    if (tree_of_lane < at_once && tree_at(tree_of_lane) < a.trees) {
+        const int len = a.out_path_len[(uint64_t)(uint32_t)tree_at(tree_of_lane) * (uint32_t)a.warps + (uint32_t)(lane - tree_of_lane * a.warps)];
+        const int most = a.path_depth < 1 << 20 ? a.path_depth : 1 << 20;
+        levels = len <= 1 ? 0 : len - 1 < most ? len - 1 : most;
     }
-    if (NODE_LEVEL) {
+    uint32_t counted = 0;   // bit k: the workgroup's k-th tree
+    if (a.warps == 1) counted = (uint32_t)__ballot(counting_pays(levels, words));
+    else
+        for (int k = 0; k < at_once; ++k) counted |= counting_pays(wave_sum(tree_of_lane == k ? levels : 0), words) ? 1u << k : 0u;
+    if (has_traversal && !((counted >> tree_of_wave) & 1u)) backup_traversal<NODE_LEVEL>(a, nullptr, tree_at(tree_of_wave), lane, mine);
+
+    int *const times_reached = times_passed + words;
+    for (uint32_t rest = counted; rest != 0; rest &= rest - 1) {   // (the same in all wavefronts)
+        const int kth = __builtin_ctz(rest), tree = tree_at(kth), node_limit = a.node_count[tree];
+        __syncthreads();   // (nobody reads the tree before any more)
+        for (int i = threadIdx.x; i < words + (NODE_LEVEL ? a.nodes : 0); i += threads) times_passed[i] = 0;
         __syncthreads();
-        for (int c = threadIdx.x; c < a.nodes; c += threads) {
-            const int reached = times_reached[c];
-            if (reached != 0) atomicAdd(&a.node_inflight[first_node + c], (int)(0u - (uint32_t)reached * (uint32_t)a.virtual_loss));
+        if (tree_of_wave == kth) backup_traversal<NODE_LEVEL, true>(a, (LdsInts)times_passed, tree, lane, mine);
+        __syncthreads();
+        const uint64_t first_node = (uint64_t)(uint32_t)tree * (uint32_t)a.nodes, first = first_node * (uint32_t)a.edges;
+        for (int i = threadIdx.x; i < words; i += threads) {
+            const int passed = times_passed[i];
+            if (passed == 0) continue;
+            if (!NODE_LEVEL) {
+                atomicAdd(&a.edge_inflight[first + i], (int)(0u - (uint32_t)passed * (uint32_t)a.virtual_loss));
+            } else {
+                const int child = a.edge_child_id[first + i];
+                if (child >= 0 && child < node_limit) __hip_atomic_fetch_add((LdsInts)times_reached + child, passed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            if (a.path_edge_values != nullptr) atomicAdd(&a.edge_N[first + i], passed);
+        }
+        if (NODE_LEVEL) {
+            __syncthreads();
+            for (int c = threadIdx.x; c < a.nodes; c += threads) {
+                const int reached = times_reached[c];
+                if (reached != 0) atomicAdd(&a.node_inflight[first_node + c], (int)(0u - (uint32_t)reached * (uint32_t)a.virtual_loss));
+            }
         }
     }
 }
@@ -219,18 +261,21 @@ template <bool NODE_LEVEL>
 int launch_backup(const BackupArgs &a, hipStream_t stream) {
     dim3 grid, block;
     launch_shape(a.trees, a.warps, grid, block);
-    // Counted in LDS where paths can only be that long by coming back to nodes, so that they pass a good part of a small tree's edges, and
-    // where there are many of them.  Atomics on scattered words go at 25 G a second, whatever the occupancy, one for a release and
-    // three with values.  us, atomics / counted, release and with values: 16384 trees of 65 x 64, paths of 512 324 / 86 and 1043 / 580, of
-    // 128 81 / 50 and 255 / 187; of 91 x 90 (512 threads) 316 / 131 and 1038 / 649; of 21 x 20, paths of 64, 39 / 18 and 122 / 71; 2048
-    // trees of 65 x 64 with 8 traversals of up to 512 98 / 15 and 309 / 144.  Few trees, which take a few us: 64 of 65 x 64 with one path
-    // of 128 4.3 / 6.4, with 8 traversals 4.6 / 5.1.  (Threads, us a release of 16384 x 512 by loads and stores with 64 / 128 / 256 / 512:
-    // 65 x 64 179 / 124 / 98 / 116, 91 x 90 627 / 415 / 291 / 213.)
+    // Counted in LDS where paths may be so long that they can only come back to nodes, so that they pass a good part of a small tree's edges, and
+    // where there are many of them; whether they are that long the kernel sees for each tree.  Atomics on scattered words go at 25 G a second,
+    // whatever the occupancy, one for a release and three with values.  us, atomics / counted, release and with values, paths as
+    // selections of recurrent trees leave them: 16384 trees of 65 x 64, paths of 512 368 / 65 and 1140 / 581, of 128 88 / 31 and
+    // 281 / 166; of 91 x 90 (512 threads), 512, 364 / 106 and 1183 / 671; of 21 x 20, 64, 47 / 13 and 146 / 76; 2048
+    // trees of 65 x 64 with 8 traversals of up to 512 111 / 13 and 347 / 152.  Paths of two levels in the same room: 5.2 / 7.0 with one traversal a
+    // tree, whatever the tree, 4.0 / 6.6 with 8 or 16 (when they were counted too, 26 with 65 x 64, 48 with 91 x 90).  Few trees, which
+    // take a few us, have nothing to gain: 1030 of 65 x 64 with one path of 64 4.1 / 5.5, of 512 20 / 14.  (Threads, us a release of
+    // 16384 x 512 by loads and stores with 64 / 128 / 256 / 512: 65 x 64 179 / 124 / 98 / 116, 91 x 90 627 / 415 / 291 / 213.)
     const long long slots = (long long)a.nodes * a.edges, walked = (long long)a.warps * a.path_depth;
-    if (grid.y == 1 && slots > 0 && slots <= kLocalClaimSlots && a.path_depth >= a.nodes && walked * 40 >= slots && a.trees * walked >= 1 << 19) {
-        const unsigned threads = slots <= 4608 ? 256 : 512;
-        hipLaunchKernelGGL(counted_backup_kernel<NODE_LEVEL>, grid, dim3(block.x < threads ? threads : block.x),
-                           sizeof(int) * (size_t)(slots + (NODE_LEVEL ? a.nodes : 0)), stream, a);
+    if (grid.y == 1 && slots > 0 && slots <= kLocalClaimSlots && a.path_depth >= a.nodes && walked * 40 >= slots && counting_pays(walked, slots) && a.trees * walked >= 1 << 19) {
+        const unsigned least = slots <= 4608 ? 256 : 512, threads = block.x < least ? least : block.x;
+        const int at_once = trees_of_counting_block(a.trees, a.warps, (int)threads);
+        hipLaunchKernelGGL(counted_backup_kernel<NODE_LEVEL>, dim3((unsigned)((a.trees - 1) / at_once + 1)), dim3(threads),
+                           sizeof(int) * (size_t)(slots + (NODE_LEVEL ? a.nodes : 0)), stream, a, at_once);
     } else {
         hipLaunchKernelGGL(backup_kernel<NODE_LEVEL>, grid, block, 0, stream, a);
     }

@@ -169,6 +169,85 @@ def test_backup_of_long_paths_matches_oracle(trees, actions, nodes, depth, warps
             assert np.array_equal(got[k], at_nodes[k], equal_nan=True), (rnd, k)
 
 
+@pytest.mark.parametrize("trees,actions,nodes,depth,warps", [(16390, 9, 10, 40, 1), (8197, 20, 21, 70, 1), (2050, 90, 91, 300, 1), (4101, 20, 21, 70, 2), (1367, 64, 65, 130, 3),
+                                                             (1025, 30, 31, 100, 8), (530, 90, 91, 91, 16), (600, 8, 1024, 1024, 1)])
+def test_backup_of_short_and_long_paths_matches_oracle(trees, actions, nodes, depth, warps):
+    """Where paths may be long, a tree is counted by the levels that its paths have together: trees on either side of that line (24 + nodes *
+    actions / 128 levels), with paths of no, one and two levels and of all that there is room for, next to each other, and numbers of
+    trees that are no multiple of a workgroup's.  Values and sums are multiples of 1/64, exact in every order of adding them."""
+    from mcts_numba_cuda_amd import puct
+    from mcts_numba_cuda_amd.hipmem import DeviceArray
+    rng = np.random.default_rng(trees + actions)
+    line, shape = 24 + nodes * actions // 128, (trees, nodes, actions)
+    d = {"edge_child": rng.integers(-1, nodes + 1, shape).astype(np.int32), "edge_w": np.zeros(shape, np.float32), "edge_n": rng.integers(0, 50, shape).astype(np.int32),
+         "edge_inflight": rng.integers(0, 50, shape).astype(np.int32), "node_expand_inflight": rng.integers(0, 9, shape[:2]).astype(np.int32),
+         "node_count": rng.integers(nodes // 2, nodes + 1, trees).astype(np.int32)}
+    # how the levels of a tree are shared out among its traversals: evenly, or all to the last
+    levels = rng.choice([0, 1, 2, line - 1, line, line + 1, depth, warps * depth], trees)
+    each = np.minimum(np.diff(np.floor(levels[:, None] * np.arange(warps + 1) / warps).astype(np.int64), axis=1), depth)
+    alone = rng.random(trees) < 0.3
+    each[alone] = 0
+    each[alone, -1] = np.minimum(levels[alone], depth)
+    kind = np.where(each > 0, rng.choice([pc.EXPAND, pc.TERMINAL_KIND, pc.DEPTH_LIMIT], each.shape), rng.choice([pc.INVALID, pc.BUSY, pc.EXPAND, pc.TERMINAL_KIND], each.shape))
+    d["out_selected"] = ((kind << 22) | rng.integers(0, nodes, each.shape)).astype(np.int32)
+    d["out_len"] = np.where((kind == pc.INVALID) | (kind == pc.BUSY), 0, each + 1).astype(np.int32)
+    d["out_path"] = (rng.integers(0, nodes, (trees, warps, depth)) << 8 | rng.integers(0, actions, (trees, warps, depth))).astype(np.int32)
+    d["out_path"][rng.random(d["out_path"].shape) < 0.01] = -1
+    assert depth >= nodes and nodes * actions <= 8192 and 40 * warps * depth >= nodes * actions and trees * warps * depth >= 1 << 19 and line <= warps * depth
+    sums = each.sum(1)
+    assert all(np.any(sums == n) for n in ((line - 1, line) if line <= depth else ()))
+    for node_level in (False, True):
+        h = copy.deepcopy(d)
+        if node_level:
+            del h["edge_inflight"]
+            h["node_inflight"] = rng.integers(0, 999, (trees, nodes)).astype(np.int32)
+            h["out_selected"] = np.where(kind == pc.BUSY, 0x3FFF, h["out_selected"]).astype(np.int32)
+        for with_values in ((True,) if node_level else (True, False)):
+            got = to_device(h)
+            values = (np.floor(rng.uniform(-64, 64, h["out_path"].shape)) / 64).astype(np.float32) if with_values else None
+            (puct.launch_node_backup if node_level else puct.launch_edge_backup)(got, None if values is None else DeviceArray(values))
+            synchronize()
+            po.backup(h, values, node_level=node_level)
+            got = to_host(got)
+            for k in h:
+                assert np.array_equal(got[k], h[k]), (node_level, with_values, k)
+
+
+def launch_times(launch, launches=60, rounds=7):
+    """Fastest of `rounds` mean times of a launch, in us."""
+    from mcts_numba_cuda_amd.hipmem import Event
+    best = np.inf
+    for _ in range(rounds):
+        start, end = Event(), Event()
+        start.record()
+        for _ in range(launches):
+            launch()
+        end.record()
+        synchronize()
+        best = min(best, 1e3 * start.elapsed_ms(end) / launches)
+    return best
+
+
+def test_backup_of_short_paths_does_not_pay_for_the_room_that_they_have():
+    """Paths of one and two levels where 512 would fit, which is more than the trees have nodes, and where 64 would, which is less: 7.0 and 5.2 us;
+    when all trees of the first kind were counted it took 26."""
+    from mcts_numba_cuda_amd import puct
+    from mcts_numba_cuda_amd.hipmem import DeviceArray
+    trees, nodes, actions = 16384, 65, 64
+    rng = np.random.default_rng(3)
+    d = {k: DeviceArray(np.zeros((trees, nodes, actions), t)) for k, t in (("edge_w", np.float32), ("edge_n", np.int32), ("edge_inflight", np.int32))}
+    d.update({"node_expand_inflight": DeviceArray(np.zeros((trees, nodes), np.int32)), "node_count": DeviceArray(np.full(trees, nodes, np.int32)),
+              "out_selected": DeviceArray(np.full((trees, 1), pc.TERMINAL_KIND << 22, np.int32)), "out_len": DeviceArray(rng.integers(2, 4, (trees, 1)).astype(np.int32))})
+    path = (rng.integers(0, nodes, (trees, 1, 512)) << 8 | rng.integers(0, actions, (trees, 1, 512))).astype(np.int32)
+    roomy, tight = (dict(d, out_path=DeviceArray(path[:, :, :n])) for n in (512, 64))
+    launch, fields = puct._lib().puct_edge_backup_launch, ("edge_w", "edge_n", "edge_inflight", "node_expand_inflight", "node_count", "out_selected", "out_path", "out_len")
+    times = []
+    for x in (roomy, tight):   # (the C function itself: the arguments' checks take longer than the launch)
+        arguments = (1, *(x[k].data_ptr() for k in fields), None, trees, nodes, actions, 1, x["out_path"].shape[2], None)
+        times.append(launch_times(lambda: launch(*arguments)))
+    assert times[0] < 2.5 * times[1], times
+
+
 @pytest.mark.parametrize("trees,warps,soft", [(16, 8, 0), (16, 16, 0), (4, 40, 0), (16, 16, 1), (128, 4, 0)])
 def test_concurrent_traversals_keep_invariants(trees, warps, soft):
     rng = np.random.default_rng(trees * 100 + warps)
