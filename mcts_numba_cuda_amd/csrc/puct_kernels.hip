@@ -223,9 +223,15 @@ int launch_node_select(float cpuct, float c_pw, float alpha_pw, const int *edge_
                      out_path_eids, out_path_len, trees,             nodes,         edges,        warps,  path_depth};
     dim3 grid, block;
     launch_shape(trees, warps, grid, block);
-    // The counters of a tree in LDS: up to 16384 nodes, and a single traversal's only where its path may be long (in memory / in LDS, us a
-    // selection and its backup: 256 trees of 2000 x 128, three levels, 8.9 / 13.2; 4096 of 65 x 64, 512 levels, 1329 / 996).
-    if (grid.y == 1 && nodes > 0 && nodes <= kLocalVisitNodes && (warps > 1 || nodes <= 16 * (long long)path_depth))
+    // The counters of a tree in LDS: up to 16384 nodes, and a single traversal's where copying them costs little beside reading them in memory at every
+    // level that its path may have.  The copy costs by the nodes, a level in memory by its edges, and how long the paths really are the
+    // launch does not know: beyond the line, paths of a few levels are two to five times as fast with the counters in memory, and those that
+    // fill path_depth up to 1.5 times as slow (before the copy was made eight words at a time they were no slower either).
+    // In memory / in LDS, us a preclaim selection and its backup, 64 trees: 700 nodes of 16 edges, 3 levels 8.2 / 9.0, 50 levels 71 / 38;
+    // 2000 of 64, 8 levels 14.6 / 13.1, 20 levels 31 / 21; 5000 of 64, 20 levels 31 / 23; 12000 of 64, 50 levels 73 / 49; 5000
+    // of 256, 8 levels 31 / 24.  1024 trees: 2000 of 64, 8 levels 16.5 / 15.7, 20 levels 35 / 26; 5000 of 64, 20 levels 35 / 31.
+    const long long slices = (edges + kWave - 1) / kWave;
+    if (grid.y == 1 && nodes > 0 && nodes <= kLocalVisitNodes && (warps > 1 || nodes <= 200 * slices * path_depth))
         hipLaunchKernelGGL((node_select_kernel<PRECLAIM, true>), grid, block, sizeof(int) * (size_t)nodes, reinterpret_cast<hipStream_t>(stream), a);
     else
         hipLaunchKernelGGL((node_select_kernel<PRECLAIM, false>), grid, block, 0, reinterpret_cast<hipStream_t>(stream), a);

@@ -164,6 +164,30 @@ def test_deep_wide_shape_of_the_reference_benchmark(variant):
     assert nc.inflight_sum(h2) == 0 and int(h2["edge_n"].sum()) == int(c["edge_n"].sum()) + trees * warps * depth
 
 
+@pytest.mark.parametrize("variant", nc.VARIANTS)
+def test_a_single_traversals_counters_cost_no_jump(variant):
+    """64 trees of 700 nodes with 16 edges, one traversal of 43 and of 44 levels: 29 and 30 us (winner-recalc 39 and 40).
+    When a tree of more than 16 * path_depth nodes had its counters in memory, 43 levels took 58 and 62."""
+    from mcts_numba_cuda_amd import puct
+    from mcts_numba_cuda_amd.hipmem import DeviceArray
+    from test_gpu_puct import launch_times
+    trees, actions, nodes = 64, 16, 700
+    launch = {"preclaim": puct._lib().puct_node_select_preclaim_launch, "winner_recalc": puct._lib().puct_node_select_winner_recalc_launch}[variant]
+    times = []
+    for depth in (43, 44):
+        c = nc.make_case(trees=trees, nodes=nodes, actions=actions, warps=1, path_depth=depth)
+        c["node_expanded"][:] = actions
+        c["edge_child"][:] = np.arange(1, actions + 1, dtype=np.int32)
+        c["edge_n"][:] = 1
+        d = to_device(c)
+        arguments = (1.0, 0.0, 0.5, *(d[k].data_ptr() for k in ("edge_child", "edge_prior", "edge_w", "edge_n", "node_inflight", "node_expand_inflight", "node_expanded", "node_count",
+                                                             "out_selected", "out_path", "out_len")), trees, nodes, actions, 1, depth, None)
+        times.append(launch_times(lambda: launch(*arguments)))
+        h = to_host(d)
+        assert np.all(h["out_len"] == depth + 1)
+    assert times[0] < 1.3 * times[1], times
+
+
 def test_launch_errors_are_reported():
     from mcts_numba_cuda_amd import puct
     from mcts_numba_cuda_amd.hipmem import DeviceArray
