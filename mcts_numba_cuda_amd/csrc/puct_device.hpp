@@ -597,6 +597,12 @@ __device__ __forceinline__ void rollback_node_path(const NodeSelectArgs &a, cons
 template <bool PRECLAIM, bool LOCAL, class BeforeClaims>
 __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, const NodeVisits<LOCAL> &visits_of, int tree, int wid, int lane, BeforeClaims before_claims) {
     static_assert(kPasses == 4, "the levels below are written for one to four slices");
+    // Preclaims in memory: the traversals of a tree (more than 16, where it matters) are bound by their atomics on the same few lines, and the sooner
+    // each comes to them the more they are in each other's way.  A widening limit that nobody needs is worked out between the
+    // reads and the claims, and the depth asked for apart from the other ends.  us a selection and its backup with neither /
+    // the first / both: 64 trees of 129 x 128, 24 traversals, 128 levels 1750 / 1575 / 1370, one tree with 32 920 / 802 / 728, 256 of 257 x 256 with 32,
+    // 256 levels 10700 / 9850 / 9310, 64 of 65 x 64 with 24 915 / 902 / 856.
+    constexpr bool CONTENDED = PRECLAIM && !LOCAL;
     const size_t out = (uint64_t)(uint32_t)tree * (uint32_t)a.warps + (uint32_t)wid;
     int *const entries = a.out_path_eids + out * (uint32_t)a.path_depth;
     const int nodes = a.nodes, edges = a.edges;
@@ -674,7 +680,7 @@ __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, c
                 total = wave_sum(total);
                 const int parent_eff = total > 1 ? total : 1;   // :407-416
                 const float sqrt_parent = sqrt_of_count(parent_eff);
-                if (a.c_pw != 0.0f) {   // (else there is one child allowed, and there is one)
+                if (CONTENDED || a.c_pw != 0.0f) {   // (else there is one child allowed, and there is one)
                     const int allowed = allowed_children(a.c_pw, a.alpha_pw, parent_eff, edges, sqrt_parent);
                     if (allowed > cur_expanded) return expand(allowed);
                 }
@@ -796,12 +802,17 @@ __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, c
             else if (cur_expanded <= 2 * kWave) next = level(std::integral_constant<int, 2>{});
             else if (cur_expanded <= 3 * kWave) next = level(std::integral_constant<int, 3>{});
             else next = level(std::integral_constant<int, 4>{});
-            if (next >= 0 && ++depth >= a.path_depth) next = ~pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, next, 0);   // the path buffer is full: stop before reading or claiming anything there
+            // the path buffer is full: stop before reading or claiming anything there
+            if (!CONTENDED && next >= 0 && ++depth >= a.path_depth) next = ~pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, next, 0);
             if (next < 0) {
                 final_packed = ~next;
                 break;
             }
             node = next;
+            if (CONTENDED && ++depth >= a.path_depth) {
+                final_packed = pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, node, 0);
+                break;
+            }
             row = request(__builtin_amdgcn_readfirstlane(node));
         }
         if (final_packed >> PUCT_PACKED_KIND_SHIFT == PUCT_SELECT_INVALID) rollback_node_path(a, visits_of, path, tree, depth, lane, node_limit);
