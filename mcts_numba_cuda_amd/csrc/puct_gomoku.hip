@@ -519,8 +519,8 @@ __device__ __forceinline__ void decide_in_row(const LoopArgs &g, StepLds &s, int
     int den = prow_den(e.eid[0] >= 0, e.den[0]), mine = 0;   // mine, in lane n: lane of the edge that the n-th decision takes
     uint32_t with_ticket = 0;                                // bit n: the n-th decision is a ticket
     const uint64_t edges = __ballot(e.eid[0] >= 0);
-    // (the limit grows with the claims: its largest value is the last one's)
-    if (expanded + tickets < __builtin_amdgcn_readlane(allowed_lane, n_members - 1))
+    // (nobody can get a ticket if none of the limits that the decisions may see leaves one: with a negative alpha_pw the first is the largest)
+    if (__ballot(lane < n_members && expanded + tickets < allowed_lane) != 0)
         row_decisions<true>(e, edges, members, n_members, lane, expanded, sqrt_lane, allowed_lane, tickets, with_ticket, den, mine);
     else if (n_members < 4 || !((edges >> 4) == 0 ? quick_row_decisions<4>(e, n_members, lane, sqrt_lane, den, mine)
                                                   : quick_row_decisions<kRow>(e, n_members, lane, sqrt_lane, den, mine)))
@@ -622,12 +622,12 @@ __device__ void select_group(const LoopArgs &g, StepLds &s, int *paths, int *nex
         }
         if (leads_somewhere && lane == 0) row[eid].link = link + (uint32_t)n_members;
     };
-    // No expansion ticket is to be had here however many of these traversals have claimed: the widening limit grows with
-    // the claims, and its largest value, the one the last of them sees, does not exceed the children there are.
+    // No expansion ticket is to be had here however many of these traversals have claimed: none of the widening limits that they may
+    // see, one a lane, exceeds the children there are.
     const auto no_ticket_for_anyone = [&] {
         if (expanded >= legal || (expanded == 1 && g.c_pw == 0.0f)) return true;   // (the limit does not exceed the legal moves)
-        const int eff_last = total + n_members - 1 > 1 ? total + n_members - 1 : 1;
-        return allowed_children(g.c_pw, g.alpha_pw, eff_last, legal) <= expanded;
+        const int eff_lane = total + lane > 1 ? total + lane : 1;
+        return __ballot(lane < n_members && allowed_children(g.c_pw, g.alpha_pw, eff_lane, legal) > expanded) == 0;
     };
 
     // decide_in_row's terms: every edge leads to a node and has a finite score
