@@ -66,7 +66,10 @@ typedef struct mctsnc_result {
     int64_t actions_ns[MCTSNC_MAX_ACTIONS];
     int64_t actions_ns_wins[MCTSNC_MAX_ACTIONS];
     uint8_t actions_win_flags[MCTSNC_MAX_ACTIONS];
-    double time_total, time_loop, time_reduce;      /* host wall clock, seconds */
+    /* seconds; time_total is the host's wall clock around the call, time_loop the search's part of it (up to the end of its last
+     * launch; of one search the resetting of its trees too, a few microseconds) and time_reduce that of the final reductions of
+     * all searches of the call, the copy of their results and the filling of these structs, however the search ended */
+    double time_total, time_loop, time_reduce;
     double time_device_loop;                        /* HIP-event time of the search kernels, seconds */
     int64_t depth_sum;                              /* sum of node depths over all trees */
     int64_t size_sum;                               /* sum of tree sizes */

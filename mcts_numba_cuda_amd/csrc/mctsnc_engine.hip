@@ -94,7 +94,7 @@ struct mctsnc_engine {
     int32_t *d_abort = nullptr;
     int64_t n_rng_playout = 0, n_rng_expand = 0;
     hipStream_t stream = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;   // around a launch of the search; ev2: behind its reductions
     bool has_run = false;
     bool stage_timing = true;
     int options[MCTSNC_OPT_COUNT] = {0, -1, 0, -1, 0, -1, 0, -1, 0, -1};   // mctsnc_set_option(): defaults, see include/mctsnc_hip.h
@@ -160,10 +160,11 @@ void free_device(mctsnc_engine *e) {
     e->g_root_ae = nullptr; e->g_poc = nullptr; e->g_path = nullptr;
     if (e->ev0) (void)hipEventDestroy(e->ev0);
     if (e->ev1) (void)hipEventDestroy(e->ev1);
+    if (e->ev2) (void)hipEventDestroy(e->ev2);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     e->d_nodes = nullptr; e->d_hdrs = nullptr; e->d_rng_playout = nullptr; e->d_rng_expand = nullptr; e->d_refs = nullptr;
     e->d_reduced = nullptr; e->d_abort = nullptr;
-    e->ev0 = e->ev1 = nullptr; e->stream = nullptr;
+    e->ev0 = e->ev1 = e->ev2 = nullptr; e->stream = nullptr;
     e->inited = false;
 }
 
@@ -291,6 +292,7 @@ struct Reduction {
     unsigned char *d_blocks;
     std::vector<unsigned char> blocks;
     bool enqueued = false;
+    double time = 0.0;
     ReducedHeader header(int j) const {
         ReducedHeader h;
         memcpy(&h, blocks.data() + reduced_stride(e0->cfg.max_actions) * (size_t)j, sizeof h);
@@ -303,7 +305,15 @@ struct Reduction {
         HIP_TRY(hipGetLastError());
         blocks.resize(reduced_stride(c.max_actions) * (size_t)n);
         HIP_TRY(hipMemcpyAsync(blocks.data(), d_blocks, blocks.size(), hipMemcpyDeviceToHost, e0->stream));
+        HIP_TRY(hipEventRecord(e0->ev2, e0->stream));
         enqueued = true;
+        return MCTSNC_OK;
+    }
+    // From the end of the launch before it to the copy's, once the stream has been waited for: the time of the search loop ends where this begins.
+    int take_time() {
+        float ms = 0.f;
+        HIP_TRY(hipEventElapsedTime(&ms, e0->ev1, e0->ev2));
+        time = ms * 1e-3;
         return MCTSNC_OK;
     }
 };
@@ -363,12 +373,13 @@ int budget_loop(mctsnc_engine *e0, const Budget &bud, Reduction<Game> &reduction
         if (last) aborted = reduction.header(0).aborted;
         else HIP_TRY(hipMemcpy(&aborted, e0->d_abort, sizeof aborted, hipMemcpyDeviceToHost));
         if (aborted) return MCTSNC_E_DEVICE_SYNC;   // the caller puts the engines back into a defined state and reports
+        if (last && (rc = reduction.take_time())) return rc;
         if (first_chunk > 0 && steps == nsteps && (double)steps < step_budget) {
             rc = after_first();
             if (rc) return rc;
         }
     }
-    time_loop = now_s() - t_loop - (reduction.enqueued ? reduction.header(0).t_reduce * kTick : 0.0);
+    time_loop = now_s() - t_loop - reduction.time;
     return MCTSNC_OK;
 }
 template <class Game, typename Launch>
@@ -383,7 +394,6 @@ int finish(mctsnc_engine **engines, Reduction<Game> &reduction, const std::vecto
     mctsnc_engine *e0 = engines[0];
     const int A = e0->cfg.max_actions, n = reduction.n;
     const size_t stride = reduced_stride(A);
-    double time_reduce = reduction.enqueued ? reduction.header(0).t_reduce * kTick : 0.0;
     const double t_red = now_s();
     if (!reduction.enqueued) {
         if (int rc = reduction.enqueue()) return rc;
@@ -410,7 +420,7 @@ int finish(mctsnc_engine **engines, Reduction<Game> &reduction, const std::vecto
         engines[search_of[j]]->has_run = true;
     }
     const double t_end = now_s();
-    time_reduce += t_end - t_red;
+    const double time_reduce = reduction.time + (t_end - t_red);
     for (int i = 0; i < n; i++) {
         out[i].time_loop = time_loop; out[i].time_reduce = time_reduce; out[i].time_total = t_end - t_start; out[i].time_device_loop = dev_time;
     }
@@ -975,6 +985,7 @@ static int init_device_impl(mctsnc_engine *e) {
     HIP_TRY(hipStreamCreate(&e->stream));
     HIP_TRY(hipEventCreate(&e->ev0));
     HIP_TRY(hipEventCreate(&e->ev1));
+    HIP_TRY(hipEventCreate(&e->ev2));
     e->n_rng_playout = e->acp ? (int64_t)T * c.max_actions * c.n_playouts : (int64_t)T * c.n_playouts;
     e->n_rng_expand = e->acp ? 0 : T;
     HIP_TRY(hipMalloc(&e->d_rng_playout, sizeof(uint64_t) * 2 * e->n_rng_playout));

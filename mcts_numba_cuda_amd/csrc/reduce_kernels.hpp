@@ -26,7 +26,6 @@ struct __attribute__((aligned(256))) ReducedHeader {
     int64_t best_n, best_n_wins, depth_sum, size_sum;
     unsigned long long plies, u1_events, stat_levels, stat_children, stat_expanded, stat_played;
     unsigned long long t_select, t_expand, t_playout, t_backup, t_exchange;   // of tree 0
-    unsigned long long t_reduce;   // of this kernel
 };
 static_assert(sizeof(ReducedHeader) == 256, "header of a reduced block");
 
@@ -43,7 +42,6 @@ template <class Game>
 __global__ void __launch_bounds__(kReduceThreads) reduce_kernel(const typename Game::Ref *refs, int T, int A, int thrifty, const int32_t *abort_flag, unsigned char *out) {
     using Ref = typename Game::Ref;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const unsigned long long t_start = wall_clock64();
     refs += (size_t)blockIdx.x * T;
     unsigned char *const o = out + (size_t)blockIdx.x * reduced_stride(A);
     // (the launch before it may not have been waited for: what an abandoned search leaves is not looked at)
@@ -167,7 +165,6 @@ __global__ void __launch_bounds__(kReduceThreads) reduce_kernel(const typename G
             hd.stat_levels = s_tot[5]; hd.stat_children = s_tot[6]; hd.stat_expanded = s_tot[7]; hd.stat_played = s_tot[8];
             const auto *h0 = ref0.hdr;
             hd.t_select = h0->t_select; hd.t_expand = h0->t_expand; hd.t_playout = h0->t_playout; hd.t_backup = h0->t_backup; hd.t_exchange = h0->t_exchange;
-            hd.t_reduce = wall_clock64() - t_start;
             *reinterpret_cast<ReducedHeader *>(o) = hd;
         }
     }

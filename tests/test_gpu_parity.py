@@ -503,3 +503,25 @@ def test_time_limited_batch_over_several_launches_through_the_queue():
         for ti in range(4):
             for name in ("trees", "ns", "ns_wins"):
                 np.testing.assert_array_equal(batch[k].read_array(name, ti), single.read_array(name, ti))
+
+
+def test_times_of_loop_and_reductions_mean_the_same_however_a_pass_ends():
+    """Sixty-four Gomoku searches in a pass: their reductions and the copy of their 0.4 MB of results, some 0.2 ms (less where the
+    host's memory is warm), are time_reduce and no part of time_loop, both where the steps end the searches (the reductions
+    follow the last launch unasked) and where the time does."""
+    from mcts_numba_cuda_amd import MCTSNC, run_batch
+    loops, reduced = {}, {}
+    board = np.zeros((15, 15), np.int8)
+    for how, steps, seconds in (("steps", 20, np.inf), ("time", np.inf, 0.002)):
+        engines = [MCTSNC((15, 15), 0, 225, game="gomoku", search_time_limit=seconds, search_steps_limit=steps, n_trees=4, n_playouts=32, variant="ocp_thrifty",
+                          device_memory=0.02, ucb_c=2.0, seed=i, verbose_info=False) for i in range(64)]
+        for e in engines:
+            e.init_device_side_arrays()
+        seen = []
+        for _ in range(10):
+            run_batch(engines, [board] * 64, None, [1] * 64)
+            e = engines[0]
+            assert e.time_device_loop <= e.time_loop and e.time_loop + e.time_reduce_over_trees <= e.time_total
+            seen.append((e.time_loop - e.time_device_loop, e.time_reduce_over_trees))
+        loops[how], reduced[how] = np.min(seen, axis=0)
+    assert loops["steps"] < 0.5 * reduced["steps"] and loops["steps"] < 2 * loops["time"], (loops, reduced)
