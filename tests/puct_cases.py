@@ -475,3 +475,41 @@ def recurrent_forest(rng, trees, nodes, actions, path_depth, claims=0.1, dead_en
     held = rng.random(shape) < claims
     c["edge_inflight"][held] = rng.integers(1, 4, int(held.sum()))
     return c
+
+
+def settled_forest(rng, trees, nodes, actions, warps, path_depth, ends=0.02, all_lead_nowhere=False):
+    """Trees on which what a traversal does does not depend on the claims of others, so that a launch of several has one outcome: at every node either
+    one edge is ahead of the others by more than claims can change (with cpuct = 1e-3), or several are equally good and nothing else counts
+    (priors of 0), so that the traversal's number decides.  No node is without edges (nobody asks for a ticket with c_pw = 0).  Edges lead
+    anywhere, so paths come back to nodes that they have been to; a share `ends` of the nodes is terminal or, in equal parts, malformed,
+    without a score that can win, or has its best edges (or all) lead nowhere.  In every other tree the best edges lead from node to node, and the
+    last node is such an end."""
+    c = make_case(trees=trees, nodes=nodes, actions=actions, warps=warps, path_depth=path_depth)
+    shape = (trees, nodes, actions)
+    widths = [w for w in (1, 2, 33, 64, 65, 100, 128, 129, 180, 192, 193, 230, 256) if w <= actions] + 3 * [actions]
+    expanded = rng.choice(widths, (trees, nodes)).astype(np.int32)
+    expanded[:, 0] = actions
+    there = np.arange(actions) < expanded[..., None]
+    tied = (rng.random((trees, nodes)) < 0.5)[..., None]
+    order = np.where(there, rng.random(shape), -1.0)
+    best = order >= np.where(tied, np.sort(order, axis=2)[..., -4:-3], order.max(axis=2, keepdims=True)) if actions >= 4 else order == order.max(axis=2, keepdims=True)
+    best &= there
+    c["node_expanded"][:] = expanded
+    c["edge_child"][:] = rng.integers(0, nodes, shape)
+    c["edge_n"][:] = np.where(rng.random(shape) < 0.8, 1 << rng.integers(0, 5, shape), 0)
+    c["edge_n"][best] = 1 << rng.integers(0, 5, int(best.sum()))
+    c["edge_w"][:] = np.where(best, 1.0, rng.integers(-4, 6, shape) / 8) * c["edge_n"]   # (value sums whose quotients are exact)
+    c["edge_prior"][:] = np.where(tied, 0.0, rng.uniform(0.01, 1.0, shape))
+    c["edge_inflight"][:] = np.where(rng.random(shape) < 0.2, rng.integers(1, 4, shape), 0)
+    fate = np.where(rng.random((trees, nodes)) < ends, rng.integers(1, 8, (trees, nodes)), 0)
+    fate[:, 0] = 0
+    chained = np.arange(trees) % 2 == 1
+    c["edge_child"][chained] = np.where(best[chained], np.minimum(np.arange(1, nodes + 1), nodes - 1)[None, :, None], c["edge_child"][chained])
+    fate[chained], fate[chained, -1] = 0, np.arange(int(chained.sum())) % 4 + 4
+    c["node_expanded"][(fate >= 1) & (fate <= 4)] = TERMINAL
+    c["node_expanded"][fate == 5] = rng.choice([-3, actions + 1], int((fate == 5).sum()))
+    no_score = (fate == 6)[..., None] & there
+    c["edge_w"][no_score], c["edge_n"][no_score] = np.nan, 1
+    nowhere = (fate == 7)[..., None] & (there if all_lead_nowhere else best)
+    c["edge_child"][nowhere] = rng.choice([-1, nodes], int(nowhere.sum()))
+    return c

@@ -390,3 +390,11 @@ def wide_forest(rng, trees, nodes, actions, warps, path_depth, hubs=2, visits=0.
     broken = expanded & (rng.random(c["edge_child"].shape) < broken_edges)
     c["edge_child"][broken] = -1
     return c
+
+
+def settled_forest(rng, trees, nodes, actions, warps, path_depth):
+    """puct_cases.settled_forest with node-level counters, a third of which already hold some visits."""
+    c = pc.settled_forest(rng, trees, nodes, actions, warps, path_depth, all_lead_nowhere=True)
+    del c["edge_inflight"]
+    c["node_inflight"] = np.where(rng.random((trees, nodes)) < 0.3, rng.integers(1, 9, (trees, nodes)), 0).astype(np.int32)
+    return c

@@ -55,9 +55,9 @@ def test_known_answers(case):
                                                             (8, 1024, 24, 1.2, 1.0), (8, 1025, 24, 1.2, 1.0)])
 def test_single_traversal_matches_oracle_exactly(actions, nodes, depth, cpuct, c_pw):
     """One traversal per tree is deterministic: every array must equal the oracle's, over several select/backup
-    rounds on the same trees (the statistics drift apart as soon as one score comparison differs).  (Up to 8192 edge
-    slots per tree a single traversal's claims are plain stores, beyond that atomics: the last two cases sit on either
-    side.)"""
+    rounds on the same trees (the statistics drift apart as soon as one score comparison differs).  (A single traversal's claims
+    are plain stores, whatever the size of the tree; up to 8192 edge slots, on either side of which the last two cases
+    are, several would keep theirs in LDS.)"""
     rng = np.random.default_rng(actions * 1000 + nodes)
     case = pc.random_forest(rng, trees=64, nodes=nodes, actions=actions, warps=1, path_depth=depth)
     h = copy.deepcopy(case)
@@ -80,7 +80,7 @@ def test_single_traversal_matches_oracle_exactly(actions, nodes, depth, cpuct, c
                                                                       (225, 40, 1, 0.0, 0.0, 100.0, 0)])
 def test_wide_nodes_with_claims_in_flight_match_oracle_exactly(actions, nodes, hubs, claims, cpuct, c_pw, soft):
     """As above on trees whose top levels fill two to four 64-edge slices, with random statistics, repeated priors and
-    claims already held on some edges (so the scores see virtual loss and a strict claim can find its edge taken)."""
+    claims already held on some edges (so the scores see virtual loss)."""
     rng = np.random.default_rng(actions * 1000 + nodes)
     case = pc.wide_forest(rng, trees=32, nodes=nodes, actions=actions, warps=1, path_depth=12, hubs=hubs, claims=claims)
     h = copy.deepcopy(case)
@@ -104,7 +104,8 @@ def test_wide_nodes_with_claims_in_flight_match_oracle_exactly(actions, nodes, h
 def test_single_traversals_of_recurrent_trees_match_oracle_exactly(actions, nodes, depth, claims, cpuct, c_pw, soft):
     """One traversal a tree on few nodes of one to four 64-edge slices, with claims already held, some of them on the edges
     that win; paths come back to edges that they hold a claim on, and some end at an edge that leads nowhere and give all of
-    it back.  nodes * edges lies on both sides of 8192, where the claims change from plain stores to atomics."""
+    it back.  nodes * edges lies on both sides of 8192, which makes no difference to a single traversal (its claims are
+    plain stores)."""
     rng = np.random.default_rng(actions * 1000 + nodes)
     case = pc.recurrent_forest(rng, trees=48, nodes=nodes, actions=actions, path_depth=depth, claims=claims, dead_ends=1.0 / min(depth, actions))
     h = copy.deepcopy(case)
@@ -132,7 +133,8 @@ def test_single_traversals_of_recurrent_trees_match_oracle_exactly(actions, node
     (16, 64, 65, 300, 4, False), (4095, 9, 10, 128, 1, False), (8, 90, 92, 200, 16, False)])
 def test_backup_of_long_paths_matches_oracle(trees, actions, nodes, depth, warps, counted):
     """Paths that come back to the nodes of a small tree, longer than a wavefront, by one to sixteen traversals; those that give way or end
-    nowhere hold nothing.  On either side of where the backup counts in LDS what was passed (`counted`).  Values are multiples of 1/64
+    nowhere hold nothing.  On either side of where the backup may count in LDS what was passed (`counted`; it does for trees whose paths
+    are long).  Values are multiples of 1/64
     small enough for their sums to be exact, so that every order of adding them gives the same."""
     from mcts_numba_cuda_amd import puct
     from mcts_numba_cuda_amd.hipmem import DeviceArray
@@ -246,6 +248,40 @@ def test_backup_of_short_paths_does_not_pay_for_the_room_that_they_have():
         arguments = (1, *(x[k].data_ptr() for k in fields), None, trees, nodes, actions, 1, x["out_path"].shape[2], None)
         times.append(launch_times(lambda: launch(*arguments)))
     assert times[0] < 2.5 * times[1], times
+
+
+@pytest.mark.parametrize("actions,nodes,depth,warps", [
+    (256, 32, 200, 8), (256, 33, 200, 8), (193, 42, 150, 16), (193, 43, 150, 16), (129, 63, 200, 3), (129, 64, 200, 3), (65, 126, 140, 16), (65, 127, 140, 16), (64, 128, 200, 2),
+    (64, 129, 200, 2), (192, 20, 128, 16), (128, 70, 90, 5), (256, 20, 150, 17), (193, 60, 130, 24), (65, 40, 200, 33), (5, 9, 90, 16), (100, 80, 120, 8),
+    (256, 90, 100, 8), (193, 140, 200, 20)])
+def test_settled_traversals_match_oracle_exactly(actions, nodes, depth, warps):
+    """Several traversals a tree, where their order does not matter: every array must equal the oracle's.  Nodes of one to four 64-edge slices; up to
+    16 traversals with claims in LDS (nodes * edges <= 8192) or in memory, and more than 16, in several workgroups.  Claims are lost to others and
+    taken again, paths are longer than a wavefront, and those that end nowhere are given back."""
+    trees = 24
+    rng = np.random.default_rng(actions * 1000 + nodes + warps)
+    case = pc.settled_forest(rng, trees=trees, nodes=nodes, actions=actions, warps=warps, path_depth=depth)
+    h, other = copy.deepcopy(case), copy.deepcopy(case)
+    other["edge_inflight"][:] = rng.integers(0, 2 * warps, other["edge_inflight"].shape)
+    po.select(other, cpuct=1e-3, c_pw=0.0, soft_winner=1)
+    r = HipRunner()
+    for rnd in range(2):
+        got = r.select(case if rnd == 0 else to_host(r.d), cpuct=1e-3, c_pw=0.0, soft_winner=1)
+        po.select(h, cpuct=1e-3, c_pw=0.0, soft_winner=1)
+        if rnd == 0:   # (whatever is claimed already)
+            assert all(np.array_equal(h[k], other[k]) for k in ("out_selected", "out_path", "out_len"))
+        for k in h:
+            assert np.array_equal(got[k], h[k], equal_nan=True), (rnd, k)
+    kinds, reasons = (h["out_selected"] >> 22) & 7, (h["out_selected"] >> 25) & 0x3F
+    assert {pc.INVALID, pc.TERMINAL_KIND} <= set(kinds.ravel().tolist()) <= {pc.INVALID, pc.TERMINAL_KIND, pc.DEPTH_LIMIT}
+    given_back = (kinds == pc.INVALID) & np.isin(reasons, (11, 14, 15))
+    assert set(reasons[given_back].tolist()) == {11, 14, 15} and np.any((case["edge_inflight"] > 0) & (h["edge_inflight"] > case["edge_inflight"] + 1))
+    levels = (h["out_path"] >= 0).sum(axis=2)
+    assert levels.max() > 64 and (min(nodes, depth) <= 66 or levels[given_back].max() > 64)
+    got = r.backup(None)
+    po.backup(h, None)
+    for k in h:
+        assert np.array_equal(got[k], h[k], equal_nan=True), k
 
 
 @pytest.mark.parametrize("trees,warps,soft", [(16, 8, 0), (16, 16, 0), (4, 40, 0), (16, 16, 1), (128, 4, 0)])

@@ -57,8 +57,8 @@ def test_single_traversal_matches_oracle_exactly(actions, nodes, depth, cpuct, c
     """One traversal per tree is deterministic: every array must equal the oracle's, over several select/backup rounds on
     the same trees (the statistics drift apart as soon as one score comparison differs).  In every other round the
     claims of the selection are left in place for the next one, so that the kernels also score against virtual visits.
-    (Up to 16384 nodes per tree the kernels keep a tree's virtual-visit counters in LDS during a launch, beyond that in
-    device memory: the last two cases sit on either side.)"""
+    (A tree's counters are in LDS during a launch up to 200 * path_depth nodes for every 64 edges, here 300 and 4000 nodes,
+    and in device memory beyond; the test below is about that line.)"""
     rng = np.random.default_rng(actions * 1000 + nodes)
     case = nc.random_forest(rng, trees=64, nodes=nodes, actions=actions, warps=1, path_depth=depth)
     h = copy.deepcopy(case)
@@ -75,6 +75,77 @@ def test_single_traversal_matches_oracle_exactly(actions, nodes, depth, cpuct, c
         po.backup(h, values, node_level=True)
         for k in h:
             assert np.array_equal(got[k], h[k], equal_nan=True), (rnd, k)
+
+
+@pytest.mark.parametrize("variant", nc.VARIANTS)
+@pytest.mark.parametrize("actions,nodes,depth", [(5, 800, 4), (5, 801, 4), (64, 1000, 5), (64, 1001, 5), (65, 800, 2), (65, 801, 2), (129, 1200, 2), (129, 1201, 2), (256, 1600, 2), (256, 1601, 2),
+                                                 (5, 16384, 82), (5, 16384, 81), (5, 16385, 82), (3, 16384, 1024), (3, 16385, 1024)])
+def test_single_traversals_on_either_side_of_counters_in_lds(actions, nodes, depth, variant):
+    """Counters in LDS up to 200 * path_depth nodes for every 64 edges and up to 16384 nodes, in memory beyond: as above, with visits already on some of
+    the nodes, those beyond the last among them, which nobody may change."""
+    rng = np.random.default_rng(actions * 1000 + nodes + depth)
+    trees = 3 if nodes > 2000 else 8
+    case = nc.random_forest(rng, trees=trees, nodes=nodes, actions=actions, warps=1, path_depth=depth)
+    case["node_inflight"][:] = np.where(rng.random(case["node_inflight"].shape) < 0.5, rng.integers(1, 5, case["node_inflight"].shape), 0)
+    case["node_count"][0] = nodes if nodes <= 16384 else 16384
+    h = copy.deepcopy(case)
+    r = HipRunner()
+    for rnd in range(4):
+        got = r.select(case if rnd == 0 else to_host(r.d), variant, cpuct=1.2, c_pw=1.0)
+        po.node_select(h, cpuct=1.2, c_pw=1.0, variant=variant)
+        for k in h:
+            assert np.array_equal(got[k], h[k], equal_nan=True), (rnd, k)
+        values = rng.uniform(-1, 1, h["out_path"].shape).astype(np.float32)
+        got = r.backup(values)
+        po.backup(h, values, node_level=True)
+        for k in h:
+            assert np.array_equal(got[k], h[k], equal_nan=True), (rnd, k)
+
+
+@pytest.mark.parametrize("actions,nodes,depth,warps", [(64, 130, 200, 2), (256, 90, 120, 16), (193, 100, 120, 7), (129, 70, 90, 3), (65, 5003, 90, 2), (9, 12007, 70, 16), (9, 16384, 70, 11),
+                                                       (9, 16385, 70, 4), (256, 90, 100, 17), (193, 40, 100, 24), (129, 140, 200, 33), (64, 80, 100, 20)])
+def test_settled_preclaims_match_oracle_exactly(actions, nodes, depth, warps):
+    """Several traversals a tree, where their order does not matter: every array must equal the oracle's, with up to 16 traversals (counters in LDS up to
+    16384 nodes, copied eight words at a time and then one by one: neither 5003 nor 12007 nor 16384 is a multiple of what that takes) and
+    more of them (counters in memory).  Visits are on some of the nodes beforehand, most of which nobody comes to."""
+    rng = np.random.default_rng(actions * 1000 + nodes + warps)
+    case = nc.settled_forest(rng, trees=4 if nodes > 2000 else 24, nodes=nodes, actions=actions, warps=warps, path_depth=depth)
+    if nodes > 16384:
+        case["node_count"][:] = 16384
+    h, other = copy.deepcopy(case), copy.deepcopy(case)
+    other["node_inflight"][:] = rng.integers(0, 2 * warps, other["node_inflight"].shape)
+    po.node_select(other, cpuct=1e-3, c_pw=0.0, variant="preclaim")
+    r = HipRunner()
+    for rnd in range(2):
+        got = r.select(case if rnd == 0 else to_host(r.d), "preclaim", cpuct=1e-3, c_pw=0.0)
+        po.node_select(h, cpuct=1e-3, c_pw=0.0, variant="preclaim")
+        if rnd == 0:   # (whatever is claimed already)
+            assert all(np.array_equal(h[k], other[k]) for k in ("out_selected", "out_path", "out_len"))
+        for k in h:
+            assert np.array_equal(got[k], h[k], equal_nan=True), (rnd, k)
+    assert (h["out_path"] >= 0).sum(axis=2).max() > 64 or nodes > 2000
+    got = r.backup(nc.zeros_like_path(h))
+    po.backup(h, nc.zeros_like_path(h), node_level=True)
+    for k in h:
+        assert np.array_equal(got[k], h[k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("variant", nc.VARIANTS)
+@pytest.mark.parametrize("nodes,warps", [(5003, 2), (5003, 3), (12007, 16), (16384, 16), (4099, 17)])
+def test_counters_of_nodes_that_nobody_comes_to_stay(nodes, warps, variant):
+    """Several traversals, whose claims depend on each other, on trees of several thousand nodes with visits on them: what has been added to the counters
+    is one for every path edge, on the node it leads to, and nothing on any other node, whoever keeps them."""
+    rng = np.random.default_rng(nodes + warps)
+    case = nc.random_forest(rng, trees=4, nodes=nodes, actions=12, warps=warps, path_depth=24)
+    case["node_inflight"][:] = rng.integers(0, 4, case["node_inflight"].shape)
+    h = HipRunner().select(case, variant, cpuct=1.5, c_pw=0.6)
+    kinds = h["out_selected"] >> 22
+    assert np.any(kinds != nc.INVALID) and np.all(h["out_len"][kinds == nc.INVALID] == 0)
+    want = case["node_inflight"].copy()
+    for t, w in zip(*np.nonzero(kinds != nc.INVALID)):
+        for enc in h["out_path"][t, w, :h["out_len"][t, w] - 1]:
+            want[t, case["edge_child"][t, enc >> 8, enc & 0xFF]] += 1
+    assert np.array_equal(h["node_inflight"], want)
 
 
 @pytest.mark.parametrize("variant", nc.VARIANTS)
