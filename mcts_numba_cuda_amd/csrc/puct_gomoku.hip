@@ -296,8 +296,8 @@ struct EdgeSet {
 };
 
 template <int NS>
-__device__ __forceinline__ float edge_score(const EdgeSet<NS> &e, int i, float sqrt_parent, int more_claims) {
-    return prow_score(e.q[i], e.cp[i], sqrt_parent, e.den[i] + more_claims);
+__device__ __forceinline__ float edge_score(const EdgeSet<NS> &e, int i, float sqrt_parent) {
+    return prow_score(e.q[i], e.cp[i], sqrt_parent, e.den[i]);
 }
 
 // The traversals `members` decide one after another on the edges in `e` (which must include every edge that can come
@@ -337,7 +337,7 @@ __device__ __forceinline__ void decide_in_turn(const LoopArgs &g, StepLds &s, in
             uint32_t image[NS], lane_top = 0;
 #pragma unroll
             for (int i = 0; i < NS; ++i) {
-                score[i] = edge_score(e, i, sqrt_parent, 0);
+                score[i] = edge_score(e, i, sqrt_parent);
                 image[i] = e.eid[i] >= 0 ? score_image(score[i]) : 0u;
                 lane_top = image[i] > lane_top ? image[i] : lane_top;
             }
@@ -440,7 +440,7 @@ struct QuickRow {
 template <int EDGES, int N = 0>
 __device__ __forceinline__ void quick_row_decision(QuickRow &r, int n_members, float sqrt_lane) {
     const float root = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), N));
-    const float score = __builtin_fmaf(r.cp_by, root, r.q), near = score + r.apart;
+    const float score = prow_quick_score(r.q, r.cp_by, root), near = score + r.apart;
     const float cp_by_if_taken = r.cp * __builtin_amdgcn_rcpf((float)(r.den + 1));
     int top = __float_as_int(score);
     const auto larger = [](int a, int b) { return a > b ? a : b; };
@@ -466,10 +466,8 @@ __device__ __forceinline__ bool quick_row_decisions(const EdgeSet<1> &e, int n_m
     r.cp_by = r.cp * __builtin_amdgcn_rcpf((float)den);
     r.den = den;
     r.takes = 0;
-    // In units of 2^-24 of the largest |q| + u: an edge's quick score is off by 4 for u, 2 and 2 for the sums (a score is at most
-    // twice that when none is negative), its score by 2 and 1, `near` by 2: 24 for two edges, and 32 are allowed for.
     const float last_root = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), n_members));
-    r.apart = row_max_f32(edge ? fabsf(q) + r.cp_by * last_root : 0.0f) * 0x1p-19f;
+    r.apart = prow_quick_apart(row_max_f32(edge ? prow_quick_size(q, r.cp_by, last_root) : 0.0f));
     const float lift = row_max_f32(edge && q < 0.0f ? -q : 0.0f);
     r.q = lane >= EDGES ? __builtin_nanf("") : edge ? q + lift : q;   // (lanes behind the edges are never taken)
     quick_row_decision<EDGES>(r, n_members, sqrt_lane);
@@ -491,7 +489,7 @@ __device__ __forceinline__ void row_decisions(const EdgeSet<1> &e, uint64_t edge
             tickets += 1;
         } else {
             const float root = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sqrt_lane), claimed));
-            const float score = q + prow_quotient(cp * root, (float)den, __builtin_amdgcn_rcpf((float)den));
+            const float score = prow_row_score(q, cp, root, den, __builtin_amdgcn_rcpf((float)den));
             uint32_t first = (uint32_t)(__builtin_amdgcn_fcmpf(score, row_max_f32(score), 1 /* == */) & edges);
             if (__builtin_popcount(first) > 1) {   // the rotated edge index decides, as in candidate_key
                 const uint32_t of_lane = 1u << (lane & (kTrav - 1));   // the deciding traversal: the member with this many before it
