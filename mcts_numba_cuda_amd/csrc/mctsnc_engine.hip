@@ -530,7 +530,8 @@ int run_many_c4(mctsnc_engine **engines, int n, const int8_t *boards, const int8
         for (int k = 0; k < n_refs; k++) { bb2[2 * (size_t)k] = bb[2 * (size_t)order[k]]; bb2[2 * (size_t)k + 1] = bb[2 * (size_t)order[k] + 1]; tr2[k] = tr[order[k]]; }
         bb.swap(bb2); tr.swap(tr2);
     }
-    // one search with allocation allowed: the engine's own buffers; otherwise pieces of one block
+    // one search with allocation allowed: the engine's own buffers; otherwise pieces of one block (of one search the roots' part stays unused,
+    // so that a static scratch has the size that it is documented to need)
     C4BatchBuffers buf{e0->d_refs, nullptr, nullptr, e0->d_reduced};
     BlockHolder block_holder;
     if (n > 1 || fixed) {

@@ -518,6 +518,8 @@ __device__ __forceinline__ void decide_in_row(const LoopArgs &g, StepLds &s, int
     uint32_t with_ticket = 0;                                // bit n: the n-th decision is a ticket
     const uint64_t edges = __ballot(e.eid[0] >= 0);
     // (nobody can get a ticket if none of the limits that the decisions may see leaves one: with a negative alpha_pw the first is the largest)
+    // From how many decisions on the quick way is tried matters little: from two, three, four or six on a step of 1 to 16 trees takes as long to
+    // within 1 %; without it 1.5 to 2.5 % longer with 16 traversals (8.96 -> 9.17 us, 12.5 -> 12.8).
     if (__ballot(lane < n_members && expanded + tickets < allowed_lane) != 0)
         row_decisions<true>(e, edges, members, n_members, lane, expanded, sqrt_lane, allowed_lane, tickets, with_ticket, den, mine);
     else if (n_members < 4 || !((edges >> 4) == 0 ? quick_row_decisions<4>(e, n_members, lane, sqrt_lane, den, mine)

@@ -172,7 +172,7 @@ def test_backup_of_long_paths_matches_oracle(trees, actions, nodes, depth, warps
 
 
 @pytest.mark.parametrize("trees,actions,nodes,depth,warps", [(16390, 9, 10, 40, 1), (8197, 20, 21, 70, 1), (2050, 90, 91, 300, 1), (4101, 20, 21, 70, 2), (1367, 64, 65, 130, 3),
-                                                             (1025, 30, 31, 100, 8), (530, 90, 91, 91, 16), (600, 8, 1024, 1024, 1)])
+                                                             (1025, 30, 31, 100, 8), (530, 90, 91, 91, 16), (600, 8, 1024, 1024, 1), (64, 1, 8192, 8192, 1)])
 def test_backup_of_short_and_long_paths_matches_oracle(trees, actions, nodes, depth, warps):
     """Where paths may be long, a tree is counted by the levels that its paths have together: trees on either side of that line (24 + nodes *
     actions / 128 levels), with paths of no, one and two levels and of all that there is room for, next to each other, and numbers of
