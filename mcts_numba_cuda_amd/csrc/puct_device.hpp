@@ -598,10 +598,11 @@ template <bool PRECLAIM, bool LOCAL, class BeforeClaims>
 __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, const NodeVisits<LOCAL> &visits_of, int tree, int wid, int lane, BeforeClaims before_claims) {
     static_assert(kPasses == 4, "the levels below are written for one to four slices");
     // Preclaims in memory: the traversals of a tree (more than 16, where it matters) are bound by their atomics on the same few lines, and the sooner
-    // each comes to them the more they are in each other's way.  A widening limit that nobody needs is worked out between the
-    // reads and the claims, and the depth asked for apart from the other ends.  us a selection and its backup with neither /
-    // the first / both: 64 trees of 129 x 128, 24 traversals, 128 levels 1750 / 1575 / 1370, one tree with 32 920 / 802 / 728, 256 of 257 x 256 with 32,
-    // 256 levels 10700 / 9850 / 9310, 64 of 65 x 64 with 24 915 / 902 / 856.
+    // each comes to them the more they are in each other's way.  A widening limit that nobody needs is worked out between the reads and the
+    // claims, and beyond 64 edges the depth is asked for apart from the other ends.  us a selection and its backup of 64 trees, before levels asked
+    // for ends once / with neither / the first / both: 129 x 128, 32 traversals, 256 levels 3223 / 3649 / 3390 / 3129, 24 traversals, 128 levels
+    // 1483 / 1732 / 1570 / 1444; 65 x 64, 32 traversals, 256 levels 1968 / 2009 / 1981 / 2000, 64 traversals, 128 levels 1571 / 1515 / 1521 / 1549 (2518
+    // with the depth apart at 64 edges too); 256 of 257 x 256, 32 traversals, 256 levels 10600 / 10700 / 9890 / 9850.
     constexpr bool CONTENDED = PRECLAIM && !LOCAL;
     const size_t out = (uint64_t)(uint32_t)tree * (uint32_t)a.warps + (uint32_t)wid;
     int *const entries = a.out_path_eids + out * (uint32_t)a.path_depth;
@@ -803,13 +804,14 @@ __device__ __forceinline__ void node_select_traversal(const NodeSelectArgs &a, c
             else if (cur_expanded <= 3 * kWave) next = level(std::integral_constant<int, 3>{});
             else next = level(std::integral_constant<int, 4>{});
             // the path buffer is full: stop before reading or claiming anything there
-            if (!CONTENDED && next >= 0 && ++depth >= a.path_depth) next = ~pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, next, 0);
+            const bool apart = CONTENDED && cur_expanded > kWave;
+            if (!apart && next >= 0 && ++depth >= a.path_depth) next = ~pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, next, 0);
             if (next < 0) {
                 final_packed = ~next;
                 break;
             }
             node = next;
-            if (CONTENDED && ++depth >= a.path_depth) {
+            if (apart && ++depth >= a.path_depth) {
                 final_packed = pack_selection_v2(PUCT_SELECT_DEPTH_LIMIT, node, 0);
                 break;
             }
